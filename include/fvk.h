@@ -253,17 +253,27 @@ int fvk_sys_get_x(fvk_ctx *ctx, double *x);
    restart, default).  DIC / DILU factor and sweeps (solv_precond,
    solv_direct): "sweep_one_launch" (1, default when no row has more than 8
    slots: one launch each, rows waiting for their values; 0: one launch per
-   level), "sweep_parts" (1, default: each block owns ranges of
-   "sweep_part_rows" rows consecutive in the reference numbering, default
-   4096, 256..6400, and walks them level by level, values inside a range
-   passing through LDS; 0: rows taken in level order in chunks by
-   "sweep_blocks_per_cu" resident blocks per CU, default 1).  All give the
-   same bits.  "sweep_fail" 1 (a test of the failure path): records that a
-   sweep's wait ran past its bound, as a wait that never ends would; rows
-   of the ranges form that wait give up within 256 passes, blocks stop
-   taking ranges, and this and every later factorisation or sweep of the
+   level), "sweep_parts" (1, default: each block walks parts of at most
+   "sweep_part_rows" rows, default 4096, 256..6400, values inside a part
+   passing through LDS (fvk_sweep_plan); 0: rows taken in level order in
+   chunks by "sweep_blocks_per_cu" resident blocks per CU, default 1).  All
+   give the same bits.  "sweep_fail" 1 (a test of the failure path): records
+   that a sweep's wait ran past its bound, as a wait that never ends would;
+   parts that wait give up within 256 polls, blocks stop taking parts, and
+   this and every later factorisation or sweep of the
    context returns FVK_ERR_HIP. */
 int fvk_ctx_set_param(fvk_ctx *ctx, const char *name, double value);
+/* How the one-launch sweeps split a pattern (1-based CSR with its diagonal,
+   as solv_m receives it): parts of at most max_rows rows that depend on
+   each other in one direction only, grid cells over the paths' entry
+   distances ("bricks") where a few distances carry nearly all entries, else
+   ranges of consecutive rows; inside a part chunks of up to 64 independent
+   rows.  Builds the plan and walks it as the kernels do: FVK_ERR_STATE when
+   a value would be read before it is there.  info: parts, chunks,
+   dependency levels, 1 for bricks, LDS bytes of a block with one and with
+   three right-hand sides, values passed between parts forward and backward.
+   Host only; no counterpart in the reference. */
+int fvk_sweep_plan(int n, const int *ia, const int *ja, int max_rows, int *info);
 
 /* The factorised preconditioner z = G G^T r, G = D^-1/2 (I + L) Delta, with
    D the diagonal of the current matrix, L strictly lower triangular on the
@@ -504,10 +514,10 @@ void fvk_fl_ctx_destroy(fvk_fl_ctx *ctx);
 /* "sweep_one_launch" 1 (default when every row has at most 8 lower and 8
    upper entries): the factor and direct_solve's sweeps in one launch each,
    rows waiting for their values; 0: one launch per level.  "sweep_parts" 1
-   (default with one launch): each block of the launch owns ranges of
-   "sweep_part_rows" consecutive rows (default 4096, 256..6400) and walks them
-   level by level, values inside a range passing through LDS; 0: rows taken
-   in level order in chunks.  "sweep_blocks" (0: one per CU): blocks of the
+   (default with one launch): each block of the launch walks parts of at most
+   "sweep_part_rows" rows (default 4096, 256..6400), values inside a part
+   passing through LDS (fvk_sweep_plan); 0: rows taken in level order in
+   chunks.  "sweep_blocks" (0: one per CU): blocks of the
    one-launch kernels.  All give the same bits.  "sweep_fail" 1 (a test of
    the failure path): as fvk_ctx_set_param's; the context's solves then
    return FVK_ERR_HIP.  No counterpart in the reference. */

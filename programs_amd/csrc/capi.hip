@@ -362,6 +362,7 @@ static void ctx_free(Ctx &c) {
   if (c.stream) hipStreamSynchronize(c.stream);
   for (void *p : c.owned) hipFree(p);
   c.owned.clear();
+  sweep_exec_free(c.sw);
   if (c.ev0) hipEventDestroy(c.ev0);
   if (c.ev1) hipEventDestroy(c.ev1);
   for (int k = 0; k < 2; ++k)
@@ -671,7 +672,7 @@ int fvk_set_matrix(fvk_ctx *cc, const double *pl, const double *ng_p, const doub
   FVK_HIP(hipMemcpy(c.ngn, ng_n, sizeof(double) * c.nf, hipMemcpyHostToDevice));
   k_spv_from_faces<<<grid_for(c.n), BS, 0, c.stream>>>(c.M, c.ngp, c.ngn, c.spv);
   FVK_HIP(hipGetLastError());
-  c.pc_valid = false;
+  matrix_changed(c);
   return FVK_OK;
 }
 
@@ -693,6 +694,7 @@ int fvk_solv_direct(fvk_ctx *cc, int imat, const double *cv, const double *c_r, 
     GUARD(to_dev(c, c_r, 1, 1, c.n, &c.perm, c.pc_cr));
     c.pc_imat = imat;
     c.pc_valid = true;
+    c.sw_fac = false;
   } else if (!c.pc_valid || c.pc_imat != imat) {
     GUARD(precond_build(c, imat));
   }

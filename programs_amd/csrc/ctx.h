@@ -9,6 +9,7 @@
 
 #include "../../include/fvk.h"
 #include "dev.h"
+#include "sweepexec.h"
 
 namespace fvk {
 
@@ -99,17 +100,12 @@ struct Ctx {
   double *sweep_t = nullptr;      // forward sweep output (3 x n)
   int *sweep_int = nullptr;       // tickets: forward, backward, factor; [3] = wait-bound error
   unsigned char *sweep_lmask = nullptr, *sweep_umask = nullptr;  // lower / upper slots of each row
-  // partitioned one-launch sweeps (sweep_parts in sweep.h): ranges of
-  // sweep_part_rows rows consecutive in the reference numbering, each walked
-  // level by level by one block
-  struct SweepParts {
-    int P = 0, R = 0, W = 0, wmax = 0;  // wmax: the most rows of one level of a range
-    int *hd = nullptr, *jc = nullptr, *lc = nullptr;  // descriptors (sweep_pack), 16-byte words
-    int *step = nullptr, *sp = nullptr;
-  };
-  SweepParts spf, spb;
+  // the default form: parts of rows, each walked by one block (sweep.hip)
+  SweepExec sw;
   bool sweep_parts = true;
-  int sweep_part_rows = 4096;
+  int sweep_part_rows = 4096;     // rows of a part at most
+  // the packed copies in sw are of the current matrix / of pc_c, pc_cr
+  bool sw_mat = false, sw_fac = false;
   // Krylov workspace (3 components)
   double *wk = nullptr;           // 8 vectors x 3 components x n
   KS *ks = nullptr;               // 3 components: state after the last kernel / solve
@@ -236,9 +232,11 @@ int precond_apply(Ctx &c, int imat, int nvc, const double *b, double *x, const K
 // FVK_ERR_HIP if a one-launch factorisation or sweep exceeded its wait bound
 int sweep_status(Ctx &c);
 int sweep_masks_build(Ctx &c);
-// the tables of the partitioned sweeps (after sweep_masks_build); frees the
-// previous ones
+// the plan and tables of the partitioned sweeps (after sweep_masks_build);
+// frees the previous ones
 int sweep_parts_build(Ctx &c);
+// diag, spv, ngp, ngn hold another matrix: its factor and packed copies are stale
+inline void matrix_changed(Ctx &c) { c.pc_valid = c.sw_mat = c.sw_fac = false; }
 int spmv(Ctx &c, int nvc, const double *x, double *y);
 // a[0..n) = v and b = a as kernels (capturable in a HIP graph)
 int fill(Ctx &c, double *a, size_t n, double v);

@@ -709,7 +709,7 @@ int mom_setup(Flow &F, int it, bool &skipped) {
   k_mom_cell<<<grid_for(n), BS, 0, c.stream>>>(c.M, P, nvc, F.u, F.ub, c.ngp, c.ngn, F.cor, F.cfl, F.dpdx, c.diag,
                                                c.spv, F.rhs, F.cs, F.frc_vol);
   FVK_HIP(hipGetLastError());
-  c.pc_valid = false;
+  matrix_changed(c);
   rc = krylov(c, 1, F.cfg.imat_u, F.cfg.reduc_u, F.cfg.n_bicg, nvc, F.u, F.rhs, false);
   if (rc) return rc;
   k_mom_norm<<<1, 1, 0, c.stream>>>(it, nvc, c.ks, F.sc);
@@ -731,7 +731,7 @@ static int pp_assemble(Flow &F) {
   k_pp_cell<<<grid_for(n), BS, 0, c.stream>>>(c.M, c.ngp, c.ngn, F.cpp, F.cs, c.diag, c.spv, F.rhs);
   if (fill(c, F.pc, n, 0.0)) return FVK_ERR_HIP;
   FVK_HIP(hipGetLastError());
-  c.pc_valid = false;
+  matrix_changed(c);
   return 0;
 }
 
@@ -1046,15 +1046,15 @@ int flow_run_graph(Flow &F, int it0, int n, fvk_outer_hist *h, int &replayed) {
     // preconditioner vector stale, so the host does that after each launch.
     for (; it < it0 + n; ++it) {
       FVK_HIP(hipGraphLaunch(F.graphs[0], c.stream));
-      c.pc_valid = false;
+      matrix_changed(c);
       if (host) {
         if ((rc = pp_solve(F, F.pc, F.rhs))) return rc;
         FVK_HIP(hipGraphLaunch(F.graphs[1], c.stream));
-        c.pc_valid = false;
+        matrix_changed(c);
         if (F.cfg.simpler) {
           if ((rc = p_solve_simpler(F))) return rc;
           FVK_HIP(hipGraphLaunch(F.graphs[2], c.stream));
-          c.pc_valid = false;
+          matrix_changed(c);
         }
       }
       ++replayed;

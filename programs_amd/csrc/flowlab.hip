@@ -58,19 +58,11 @@ struct FlCtx {
   bool one_launch = true;
   int n_cu = 256;
   int sweep_blocks = 0;  // blocks of the one-launch kernels (0: one per CU)
-  // partitioned one-launch sweeps (sweep_parts): forward / backward level
-  // order of each row range, for ranges of R1 rows (one component, the
-  // factor) and R3 rows (two or three components)
-  struct Parts {
-    int P = 0, R = 0, W = 0, wmax = 0;  // wmax: the most rows of one level of a range
-    int *hd = nullptr, *jc = nullptr, *lc = nullptr;  // descriptors (sweep_pack), 16-byte words
-    int *step = nullptr, *sp = nullptr;
-    SweepTabs tabs() const { return SweepTabs{(const int4 *)hd, (const int4 *)jc, (const int4 *)lc}; }
-  };
-  Parts pf, pb;
+  // the default form: parts of rows, each walked by one block (sweep.hip)
+  SweepExec sw;
   bool parts = false;
-  int part_rows = 4096;  // R: LDS of one block = components x R doubles
-  std::vector<int> h_levf, h_levb, h_kii, h_klo, h_kup;
+  int part_rows = 4096;  // rows of a part at most
+  std::vector<int> h_kii, h_klo, h_kup, h_tpos;
   int *sweep_int = nullptr;  // tickets: forward, backward, factor; [3] wait-bound error
   // Krylov work: 6 vectors x 3 components, partials, scalars
   double *wk = nullptr, *pc = nullptr, *part = nullptr;
@@ -728,165 +720,59 @@ __global__ __launch_bounds__(BS) void k_fl_sweep_sf(int n, const int *__restrict
   sweep_chunks(n, ticket, err, row);
 }
 
-// the same rows for sweep_parts: a position's descriptor holds the row, its
-// first entry (forward: ia; backward: the last entry, walked down), the
-// entry count and (factor) the diagonal entry
-template <bool FWD, int NC>
-struct FlPtSweep {
-  const double *a, *pc, *src;
-  int n;
-  double cc, s[NC];
-  double av[kSweepSlots];
-  __device__ void fetch(const SweepDesc &d, int MW) {
-    constexpr int st = FWD ? 1 : -1;
-#pragma unroll
-    for (int t = 0; t < kSweepSlots; ++t)
-      if (t < MW) av[t] = a[t < d.nl ? d.first + st * t : d.first];
-    cc = pc[d.r];
-#pragma unroll
-    for (int q = 0; q < NC; ++q) s[q] = src[(size_t)q * n + d.r];
-  }
-  __device__ void begin() {
-    if (!FWD) {
-      const double cof = 1.0 / (cc + SMALL);
-#pragma unroll
-      for (int q = 0; q < NC; ++q) s[q] = cof * s[q];
-    }
-  }
-  __device__ void take(int t, const double *w) {
-#pragma unroll
-    for (int q = 0; q < NC; ++q) s[q] = s[q] - av[t] * w[q];
-  }
-  __device__ double result(int q) const { return s[q] * cc; }
-  __device__ void done(const SweepDesc &) {}
-};
-
-struct FlPtPc {
-  const double *a;
-  const int *tpos;
-  double s;
-  double a1[kSweepSlots], a2[kSweepSlots];
-  __device__ void fetch(const SweepDesc &d, int MW) {
-    s = a[d.aux];
-#pragma unroll
-    for (int t = 0; t < kSweepSlots; ++t)
-      if (t < MW) {
-        const int k = t < d.nl ? d.first + t : d.aux;
-        a1[t] = a[k];
-        a2[t] = a[t < d.nl ? tpos[k] : k];
-      }
-  }
-  __device__ void begin() {}
-  __device__ void take(int t, const double *w) { s = s - a1[t] * w[0] * a2[t]; }
-  __device__ double result(int) const { return 1.0 / (s + SMALL); }
-  __device__ void done(const SweepDesc &) {}
-};
-
-template <int MW, int TB>
-__global__ __launch_bounds__(TB) void k_fl_pc_pt(int n, int R, int P, SweepTabs T, const int *__restrict__ step,
-                                                 const int *__restrict__ sp, const int *__restrict__ tpos,
-                                                 const double *__restrict__ a, double *pc, int *ticket, int *err) {
-  FlPtPc row;
-  row.a = a; row.tpos = tpos;
-  sweep_parts<1, MW, FlPtPc, TB>(n, R, P, T, step, sp, pc, ticket, err, row);
-}
-
-template <bool FWD, int NC, int MW, int TB>
-__global__ __launch_bounds__(TB) void k_fl_sweep_pt(int n, int R, int P, SweepTabs T, const int *__restrict__ step,
-                                                    const int *__restrict__ sp, const double *__restrict__ a,
-                                                    const double *__restrict__ pc, const double *__restrict__ src,
-                                                    double *out, int *ticket, int *err, const FlKS *ks) {
-  if (fl_all_done(ks, NC)) return;
-  FlPtSweep<FWD, NC> row;
-  row.a = a; row.pc = pc; row.src = src; row.n = n;
-  sweep_parts<NC, MW, FlPtSweep<FWD, NC>, TB>(n, R, P, T, step, sp, out, ticket, err, row);
-}
-
 // ---------------------------------------------------------------- host
-// Ranges of R rows in the sweep's order and, in each, its rows by level
-// (ties by row), with each position's descriptor: the tables of sweep_parts.
-static int fl_parts_build(FlCtx &c, const std::vector<int> &lev, bool fwd, int R, FlCtx::Parts &pt) {
-  const int n = c.n;
-  const std::vector<int> &ia = c.h_ia, &ja = c.h_ja;
-  pt.R = R;
-  pt.P = (n + R - 1) / R;
-  std::vector<int> rows, first(n), cnt(n), aux(n), lrow(n), step, sp;
-  rows.reserve(n);
-  std::vector<std::pair<int, int>> buf;
-  for (int q = 0; q < pt.P; ++q) {
-    const int lo = fwd ? q * R : std::max(0, n - (q + 1) * R);
-    const int hi = fwd ? std::min(n, (q + 1) * R) : n - q * R;
-    buf.clear();
-    for (int r = lo; r < hi; ++r) buf.emplace_back(lev[r], r);
-    std::sort(buf.begin(), buf.end());
-    sp.push_back((int)step.size());
-    for (size_t t = 0; t < buf.size(); ++t) {
-      if (t == 0 || buf[t].first != buf[t - 1].first) step.push_back((int)rows.size());
-      rows.push_back(buf[t].second);
+// The sweeps' pattern: lower entries in column order, upper entries from the
+// row's last column down, as direct_solve takes them.
+static SweepGraph fl_sweep_graph(int n, const std::vector<int> &ia, const std::vector<int> &ja,
+                                 const std::vector<int> &klo, const std::vector<int> &kup,
+                                 const std::vector<int> &tpos) {
+  SweepGraph g;
+  g.n = n;
+  g.row.resize(n);
+  for (int r = 0; r < n; ++r) g.row[r] = r;
+  g.lptr.assign(n + 1, 0);
+  g.uptr.assign(n + 1, 0);
+  bool sorted = true;
+  for (int r = 0; r < n; ++r) {
+    g.lptr[r + 1] = g.lptr[r] + klo[r] - ia[r];
+    g.uptr[r + 1] = g.uptr[r] + ia[r + 1] - kup[r];
+    for (int k = ia[r] + 1; k < ia[r + 1]; ++k) sorted = sorted && ja[k - 1] < ja[k];
+  }
+  // every lower entry has its transpose (checked with tpos); in sorted rows
+  // with as many upper entries these are all of them
+  g.symmetric = sorted && g.lptr[n] == g.uptr[n];
+  g.lcol.reserve(g.lptr[n]);
+  g.lval.reserve(g.lptr[n]);
+  g.tval.reserve(g.lptr[n]);
+  g.ucol.reserve(g.uptr[n]);
+  g.uval.reserve(g.uptr[n]);
+  for (int r = 0; r < n; ++r) {
+    for (int k = ia[r]; k < klo[r]; ++k) {
+      g.lcol.push_back(ja[k]);
+      g.lval.push_back(k);
+      g.tval.push_back(tpos[k]);
     }
-    step.push_back((int)rows.size());
-  }
-  sp.push_back((int)step.size());
-  pt.wmax = 0;
-  for (int q = 0; q < pt.P; ++q)
-    for (int k = sp[q]; k + 1 < sp[q + 1]; ++k) pt.wmax = std::max(pt.wmax, step[k + 1] - step[k]);
-  int W = 1;
-  for (int p = 0; p < n; ++p) {
-    const int r = rows[p];
-    first[p] = fwd ? ia[r] : ia[r + 1] - 1;
-    cnt[p] = fwd ? c.h_klo[r] - ia[r] : ia[r + 1] - c.h_kup[r];
-    aux[p] = c.h_kii[r];
-    W = std::max(W, cnt[p]);
-  }
-  if (W > kSweepSlots) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
-  pt.W = W;
-  // a range's rows: forward [qR, (q+1)R), backward counted from the end
-  auto range_lo = [&](int r) { return fwd ? r / R * R : std::max(0, n - (n - 1 - r) / R * R - R); };
-  std::vector<int> cols((size_t)W * n, 0), lcol((size_t)W * n, -1);
-  for (int p = 0; p < n; ++p) {
-    const int r = rows[p], lo = range_lo(r);
-    lrow[p] = r - lo;
-    for (int t = 0; t < cnt[p]; ++t) {
-      const int j = ja[fwd ? first[p] + t : first[p] - t];
-      cols[(size_t)t * n + p] = j;
-      if (range_lo(j) == lo) lcol[(size_t)t * n + p] = j - lo;
+    for (int k = ia[r + 1] - 1; k >= kup[r]; --k) {
+      g.ucol.push_back(ja[k]);
+      g.uval.push_back(k);
     }
   }
-  std::vector<int> hd, jc, lc;
-  sweep_pack(n, W, rows, first, cnt, aux, lrow, cols, lcol, hd, jc, lc);
-  int rc = fl_up(c, &pt.hd, hd);
-  if (!rc) rc = fl_up(c, &pt.jc, jc);
-  if (!rc) rc = fl_up(c, &pt.lc, lc);
-  if (!rc) rc = fl_up(c, &pt.step, step);
-  if (!rc) rc = fl_up(c, &pt.sp, sp);
-  return rc;
+  return g;
 }
 
 static int fl_parts_setup(FlCtx &c) {
-  for (FlCtx::Parts *pt : {&c.pf, &c.pb}) {
-    for (int *q : {pt->hd, pt->jc, pt->lc, pt->step, pt->sp}) fl_free(c, q);
-    *pt = FlCtx::Parts();
-  }
-  int rc = fl_parts_build(c, c.h_levf, true, c.part_rows, c.pf);
-  if (!rc) rc = fl_parts_build(c, c.h_levb, false, c.part_rows, c.pb);
-  if (rc) return rc;
-  const int bytes = 3 * c.part_rows * 8;
-  if (bytes > 65536) {
-    const void *k[] = {
-#define K_(D, C, MW) (const void *)k_fl_sweep_pt<D, C, MW, 64>, (const void *)k_fl_sweep_pt<D, C, MW, BS>
-#define K2_(C, MW) K_(true, C, MW), K_(false, C, MW)
-        K2_(1, 4), K2_(2, 4), K2_(3, 4), K2_(1, 8), K2_(2, 8), K2_(3, 8)
-#undef K2_
-#undef K_
-    };
-    for (const void *f : k) FVK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-  }
-  return 0;
+  sweep_exec_free(c.sw);
+  const SweepGraph g = fl_sweep_graph(c.n, c.h_ia, c.h_ja, c.h_klo, c.h_kup, c.h_tpos);
+  SweepPlan p;
+  const std::string e = sweep_plan(g, c.part_rows, p);
+  if (!e.empty()) { set_error(e); return FVK_ERR_ARG; }
+  c.sw.n_cu = c.n_cu;
+  return sweep_exec_build(c.sw, p, c.stream);
 }
 
 static int fl_levels(const std::vector<int> &ia, const std::vector<int> &ja, int n, bool fwd,
-                     std::vector<int> &ptr, std::vector<int> &rows, std::vector<int> &lev) {
-  lev.assign(n, 0);
+                     std::vector<int> &ptr, std::vector<int> &rows) {
+  std::vector<int> lev(n, 0);
   int nl = 0;
   for (int s = 0; s < n; ++s) {
     const int i = fwd ? s : n - 1 - s;
@@ -912,55 +798,10 @@ static int fl_sweep_grid(const FlCtx &c) {
 }
 static int fl_mark_grid(size_t cnt) { return (int)std::max<size_t>(1, std::min<size_t>((cnt + BS - 1) / BS, 4096)); }
 
-// blocks of the partitioned kernels (sweep_blocks 0: as many per CU as the
-// LDS of a block lets reside, at most four of 64 threads or two of 256)
-static int fl_pt_grid(const FlCtx &c, const FlCtx::Parts &pt, size_t lds, int tb) {
-  const int per_cu = std::max(1, std::min<int>(tb == 64 ? 4 : 2, (int)(163840 / (lds + 1024))));
-  return std::max(1, std::min(pt.P, c.sweep_blocks > 0 ? c.sweep_blocks : c.n_cu * per_cu));
-}
-
-// one partitioned sweep: one wave a block when no level of a range has more
-// than 64 rows
-template <bool FWD, int C, int MW>
-static void fl_sweep_launch(FlCtx &c, const FlCtx::Parts &X, size_t lds, const double *a, const double *src,
-                            double *out, int *ticket, const FlKS *ks) {
-  if (X.wmax <= 64)
-    k_fl_sweep_pt<FWD, C, MW, 64><<<fl_pt_grid(c, X, lds, 64), 64, lds, c.stream>>>(
-        c.n, X.R, X.P, X.tabs(), X.step, X.sp, a, c.pc, src, out, ticket, c.sweep_int + 3, ks);
-  else
-    k_fl_sweep_pt<FWD, C, MW, BS><<<fl_pt_grid(c, X, lds, BS), BS, lds, c.stream>>>(
-        c.n, X.R, X.P, X.tabs(), X.step, X.sp, a, c.pc, src, out, ticket, c.sweep_int + 3, ks);
-}
-
-template <bool FWD>
-static void fl_sweep_any(FlCtx &c, int ncmp, const FlCtx::Parts &X, size_t lds, const double *a, const double *src,
-                         double *out, int *ticket, const FlKS *ks) {
-  if (X.W <= 4) {
-    if (ncmp == 1) fl_sweep_launch<FWD, 1, 4>(c, X, lds, a, src, out, ticket, ks);
-    else if (ncmp == 2) fl_sweep_launch<FWD, 2, 4>(c, X, lds, a, src, out, ticket, ks);
-    else fl_sweep_launch<FWD, 3, 4>(c, X, lds, a, src, out, ticket, ks);
-  } else {
-    if (ncmp == 1) fl_sweep_launch<FWD, 1, 8>(c, X, lds, a, src, out, ticket, ks);
-    else if (ncmp == 2) fl_sweep_launch<FWD, 2, 8>(c, X, lds, a, src, out, ticket, ks);
-    else fl_sweep_launch<FWD, 3, 8>(c, X, lds, a, src, out, ticket, ks);
-  }
-}
-
 static int fl_precond(FlCtx &c, const double *a) {
   if (c.one_launch && c.parts) {
-    const FlCtx::Parts &P = c.pf;
-    const size_t lds = (size_t)P.R * 8;
-    k_fl_mark<<<fl_mark_grid(c.n), BS, 0, c.stream>>>(c.n, c.pc, c.sweep_int + 2, nullptr, 1);
-#define PC_(MW, TB) k_fl_pc_pt<MW, TB><<<fl_pt_grid(c, P, lds, TB), TB, lds, c.stream>>>(c.n, P.R, P.P, P.tabs(), \
-    P.step, P.sp, c.tpos, a, c.pc, c.sweep_int + 2, c.sweep_int + 3)
-    if (P.W <= 4) {
-      if (P.wmax <= 64) PC_(4, 64); else PC_(4, BS);
-    } else {
-      if (P.wmax <= 64) PC_(8, 64); else PC_(8, BS);
-    }
-#undef PC_
-    FVK_HIP(hipGetLastError());
-    return 0;
+    const int rc = sweep_pack(c.sw, c.stream, a, a);
+    return rc ? rc : sweep_factor(c.sw, c.stream, SWEEP_FL, a, c.kii, c.pc, nullptr, c.sweep_int + 3);
   }
   if (c.one_launch) {
     k_fl_mark<<<fl_mark_grid(c.n), BS, 0, c.stream>>>(c.n, c.pc, c.sweep_int + 2, nullptr, 1);
@@ -981,14 +822,9 @@ static int fl_precond(FlCtx &c, const double *a) {
 // x = M^-1 b (direct_solve), t: scratch
 static int fl_direct(FlCtx &c, int ncmp, const double *a, const double *b, double *t, double *x, const FlKS *ks) {
   if (c.one_launch && c.parts) {
-    const size_t cnt = (size_t)ncmp * c.n;
-    const size_t lds = (size_t)ncmp * c.part_rows * 8;
-    k_fl_mark<<<fl_mark_grid(cnt), BS, 0, c.stream>>>(cnt, t, c.sweep_int, ks, ncmp);
-    fl_sweep_any<true>(c, ncmp, c.pf, lds, a, b, t, c.sweep_int, ks);
-    k_fl_mark<<<fl_mark_grid(cnt), BS, 0, c.stream>>>(cnt, x, c.sweep_int + 1, ks, ncmp);
-    fl_sweep_any<false>(c, ncmp, c.pb, lds, a, t, x, c.sweep_int + 1, ks);
-    FVK_HIP(hipGetLastError());
-    return 0;
+    SweepGate G;
+    if (ks) G = SweepGate{&ks->done, (int)(sizeof(FlKS) / sizeof(int)), ncmp};
+    return sweep_apply(c.sw, c.stream, ncmp, b, x, G, c.sweep_int + 3);
   }
   if (c.one_launch) {
     const size_t cnt = (size_t)ncmp * c.n;
@@ -1425,16 +1261,21 @@ int fl_grad(FlCtx &c, int ncmp, const double *phi, double *phib, double *g, int 
 
 // ---------------------------------------------------------------- host set-up
 // The cell matrix pattern (1-based CSR) and the Krylov workspace.
-static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
-  c.n = n;
-  c.nnz = ngp[n] - 1;
-  if (ngp[0] != 1 || c.nnz < n) { set_error("bad matrix pattern"); return FVK_ERR_ARG; }
-  std::vector<int> ia(n + 1), ja(c.nnz);
+struct FlPattern {
+  std::vector<int> ia, ja, kii, klo, kup, tpos;
+  int widest = 0;  // the most lower or upper entries of a row
+};
+static int fl_pattern(int n, const int *ngp, const int *ngc, FlPattern &p) {
+  const int nnz = ngp[n] - 1;
+  if (ngp[0] != 1 || nnz < n) { set_error("bad matrix pattern"); return FVK_ERR_ARG; }
+  p.ia.resize(n + 1);
+  p.ja.resize(nnz);
+  std::vector<int> &ia = p.ia, &ja = p.ja;
   for (int i = 0; i <= n; ++i) {
     ia[i] = ngp[i] - 1;
     if (i && ia[i] < ia[i - 1]) { set_error("bad matrix pattern"); return FVK_ERR_ARG; }
   }
-  for (int k = 0; k < c.nnz; ++k) {
+  for (int k = 0; k < nnz; ++k) {
     ja[k] = ngc[k] - 1;
     if (ja[k] < 0 || ja[k] >= n) { set_error("matrix column out of range"); return FVK_ERR_ARG; }
   }
@@ -1443,26 +1284,42 @@ static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
       if (ja[k] == j) return k;
     return -1;
   };
-  std::vector<int> kii(n), klo(n), kup(n), tpos(c.nnz, -1);
-  int mx = 0;
+  p.kii.resize(n);
+  p.klo.resize(n);
+  p.kup.resize(n);
+  p.tpos.assign(nnz, -1);
   for (int i = 0; i < n; ++i) {
-    if ((kii[i] = csr_index(i, i)) < 0) { set_error("matrix pattern lacks a diagonal entry"); return FVK_ERR_ARG; }
+    if ((p.kii[i] = csr_index(i, i)) < 0) { set_error("matrix pattern lacks a diagonal entry"); return FVK_ERR_ARG; }
     int k = ia[i];
     while (k < ia[i + 1] && ja[k] < i) ++k;
-    klo[i] = k;
+    p.klo[i] = k;
     k = ia[i + 1];
     while (k > ia[i] && ja[k - 1] > i) --k;
-    kup[i] = k;
-    mx = std::max({mx, klo[i] - ia[i], ia[i + 1] - kup[i]});
-    for (int q = ia[i]; q < klo[i]; ++q)
-      if ((tpos[q] = csr_index(ja[q], i)) < 0) { set_error("matrix pattern is not symmetric"); return FVK_ERR_ARG; }
+    p.kup[i] = k;
+    p.widest = std::max({p.widest, p.klo[i] - ia[i], ia[i + 1] - p.kup[i]});
+    for (int q = ia[i]; q < p.klo[i]; ++q)
+      if ((p.tpos[q] = csr_index(ja[q], i)) < 0) { set_error("matrix pattern is not symmetric"); return FVK_ERR_ARG; }
   }
+  return 0;
+}
+
+static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
+  c.n = n;
+  FlPattern p;
+  {
+    const int rc = fl_pattern(n, ngp, ngc, p);
+    if (rc) return rc;
+  }
+  c.nnz = (int)p.ja.size();
+  const std::vector<int> &ia = p.ia, &ja = p.ja, &kii = p.kii, &klo = p.klo, &kup = p.kup, &tpos = p.tpos;
+  const int mx = p.widest;
   c.one_launch = mx <= kSweepSlots;
   c.h_ia = ia;
   c.h_ja = ja;
   c.h_kii = kii;
   c.h_klo = klo;
   c.h_kup = kup;
+  c.h_tpos = tpos;
   int rc = 0;
 #define A(ptr, cnt_) if (!rc) rc = fl_alloc(c, &ptr, cnt_)
 #define U(ptr, vec) if (!rc) rc = fl_up(c, &ptr, vec)
@@ -1474,9 +1331,9 @@ static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
   if (rc) return rc;
   FVK_HIP(hipDeviceGetAttribute(&c.n_cu, hipDeviceAttributeMultiprocessorCount, c.device));
   std::vector<int> lrows;
-  fl_levels(ia, ja, n, true, c.lf_ptr, lrows, c.h_levf);
+  fl_levels(ia, ja, n, true, c.lf_ptr, lrows);
   if ((rc = fl_up(c, &c.lf_rows, lrows))) return rc;
-  fl_levels(ia, ja, n, false, c.lb_ptr, lrows, c.h_levb);
+  fl_levels(ia, ja, n, false, c.lb_ptr, lrows);
   if ((rc = fl_up(c, &c.lb_rows, lrows))) return rc;
   if (c.one_launch) {
     if ((rc = fl_parts_setup(c))) return rc;
@@ -1581,6 +1438,7 @@ static void fl_ctx_free(FlCtx &c) {
   if (c.stream) hipStreamSynchronize(c.stream);
   for (void *p : c.owned) hipFree(p);
   c.owned.clear();
+  sweep_exec_free(c.sw);
   if (c.stream) hipStreamDestroy(c.stream);
   c.stream = nullptr;
 }
@@ -1858,6 +1716,22 @@ int fvk_fl_csr_create(int n, const int *ia, const int *ja, int device, fvk_fl_ct
   return FVK_OK;
 }
 
+int fvk_sweep_plan(int n, const int *ia, const int *ja, int max_rows, int *info) {
+  if (!ia || !ja || !info || n < 1 || max_rows < 64) { set_error("bad argument"); return FVK_ERR_ARG; }
+  FlPattern q;
+  const int rc = fl_pattern(n, ia, ja, q);
+  if (rc) return rc;
+  const SweepGraph g = fl_sweep_graph(n, q.ia, q.ja, q.klo, q.kup, q.tpos);
+  SweepPlan p;
+  std::string e = sweep_plan(g, max_rows, p);
+  if (!e.empty()) { set_error(e); return FVK_ERR_ARG; }
+  e = sweep_plan_check(g, p);
+  if (!e.empty()) { set_error("sweep plan: " + e); return FVK_ERR_STATE; }
+  const int v[8] = {p.P, p.np / kChunk, p.levels, p.bricks ? 1 : 0, (int)p.lds(1), (int)p.lds(3), p.d[0].NE, p.d[1].NE};
+  std::copy(v, v + 8, info);
+  return FVK_OK;
+}
+
 int fvk_fl_csr_matches(const fvk_fl_ctx *cc, int n, const int *ia, const int *ja) {
   if (!cc || !ia || !ja) return 0;
   const FlCtx &c = cc->c;
@@ -1973,18 +1847,18 @@ int fvk_fl_ctx_set_param(fvk_fl_ctx *cc, const char *name, double value) {
     return FVK_OK;
   }
   if (!std::strcmp(name, "sweep_parts") && (value == 0 || value == 1)) {
-    if (value == 1 && !c.pf.hd) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
+    if (value == 1 && !c.sw.built()) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
     c.parts = value != 0;
     return FVK_OK;
   }
   if (!std::strcmp(name, "sweep_part_rows") && value >= 256 && value <= 6400 && value == (int)value) {
-    if (!c.pf.hd) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
+    if (!c.sw.built()) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
     FVK_HIP(hipStreamSynchronize(c.stream));
     c.part_rows = (int)value;
     return fl_parts_setup(c);
   }
   if (!std::strcmp(name, "sweep_blocks") && value >= 0 && value <= 65536 && value == (int)value) {
-    c.sweep_blocks = (int)value;
+    c.sweep_blocks = c.sw.blocks = (int)value;
     return FVK_OK;
   }
   if (!std::strcmp(name, "sweep_fail") && value == 1 && c.sweep_int) {

@@ -323,102 +323,6 @@ __global__ __launch_bounds__(BS) void k_sweep_bwd_sf(DMesh M, const int *__restr
   sweep_run<false, NVC>(M, order, umask, spv, c, cr, t, x, ticket, err);
 }
 
-// The same factor and sweeps for sweep_parts: a position's descriptor holds
-// the row, its slot mask (first), the number of lower (upper) slots and the
-// columns of those slots in slot order.
-__device__ __forceinline__ void slots_of(unsigned m, int (&sl)[kSweepSlots]) {
-#pragma unroll
-  for (int t = 0; t < kSweepSlots; ++t) {
-    sl[t] = m ? __builtin_ctz(m) : 0;
-    m &= m - 1u;
-  }
-}
-
-struct PtPrecond {
-  const int *spf;
-  size_t ld;
-  int imat;
-  const double *diag, *ngp, *ngn;
-  double *cr;
-  double d;
-  double a1[kSweepSlots], a2[kSweepSlots];
-  __device__ void fetch(const SweepDesc &q, int MW) {
-    int sl[kSweepSlots];
-    slots_of((unsigned)q.first, sl);
-    d = diag[q.r];
-#pragma unroll
-    for (int t = 0; t < kSweepSlots; ++t)
-      if (t < MW) {
-        const int f0 = spf[(size_t)sl[t] * ld + q.r];
-        const int f = t < q.nl ? f0 : 0;
-        a1[t] = imat == 1 ? ngn[f] : ngp[f];
-        a2[t] = ngn[f];
-      }
-  }
-  __device__ void begin() {}
-  __device__ void take(int t, const double *w) {
-    if (imat == 1) d = d - a1[t] * a2[t] * w[0];
-    else d = d - a1[t] * w[0] * a2[t];
-  }
-  __device__ double result(int) const { return 1.0 / (d + SMALL); }
-  __device__ void done(const SweepDesc &q) { cr[q.r] = d; }
-};
-
-template <bool FWD, int NVC>
-struct PtSweep {
-  const double *spv, *c, *cr, *src;
-  size_t ld;
-  int n;
-  double cc, crr, acc[NVC];
-  double a[kSweepSlots];
-  __device__ void fetch(const SweepDesc &q, int MW) {
-    int sl[kSweepSlots];
-    slots_of((unsigned)q.first, sl);
-#pragma unroll
-    for (int t = 0; t < kSweepSlots; ++t)
-      if (t < MW) a[t] = spv[(size_t)sl[t] * ld + q.r];
-    cc = c[q.r];
-    if (!FWD) crr = cr[q.r];
-#pragma unroll
-    for (int v = 0; v < NVC; ++v) acc[v] = src[v * n + q.r];
-  }
-  __device__ void begin() {
-    if (!FWD) {
-#pragma unroll
-      for (int v = 0; v < NVC; ++v) acc[v] = acc[v] * crr;
-    }
-  }
-  __device__ void take(int t, const double *w) {
-#pragma unroll
-    for (int v = 0; v < NVC; ++v) acc[v] = acc[v] - a[t] * w[v];
-  }
-  __device__ double result(int v) const { return acc[v] * cc; }
-  __device__ void done(const SweepDesc &) {}
-};
-
-template <int MW, int TB>
-__global__ __launch_bounds__(TB) void k_precond_pt(int n, int R, int P, SweepTabs T, const int *__restrict__ step,
-                                                   const int *__restrict__ sp, DMesh M, int imat,
-                                                   const double *__restrict__ diag, const double *__restrict__ ngp,
-                                                   const double *__restrict__ ngn, double *c, double *__restrict__ cr,
-                                                   int *ticket, int *err) {
-  PtPrecond row;
-  row.spf = M.spf; row.ld = M.ld; row.imat = imat; row.diag = diag; row.ngp = ngp; row.ngn = ngn; row.cr = cr;
-  sweep_parts<1, MW, PtPrecond, TB>(n, R, P, T, step, sp, c, ticket, err, row);
-}
-
-template <bool FWD, int NVC, int MW, int TB>
-__global__ __launch_bounds__(TB) void k_sweep_pt(int n, int R, int P, SweepTabs T, const int *__restrict__ step,
-                                                 const int *__restrict__ sp, size_t ld, const double *__restrict__ spv,
-                                                 const double *__restrict__ c, const double *__restrict__ cr,
-                                                 const double *__restrict__ src, double *out, int *ticket, int *err,
-                                                 const KS *ks) {
-  if (all_done(ks, NVC)) return;
-  PtSweep<FWD, NVC> row;
-  row.spv = spv; row.c = c; row.cr = cr; row.src = src; row.ld = ld; row.n = n;
-  sweep_parts<NVC, MW, PtSweep<FWD, NVC>, TB>(n, R, P, T, step, sp, out, ticket, err, row);
-}
-
 template <int WS>
 __global__ __launch_bounds__(BS) void k_spmv(DMesh M, int nvc, const double *__restrict__ diag,
                                              const double *__restrict__ spv, const double *__restrict__ x,
@@ -883,165 +787,67 @@ int sweep_masks_build(Ctx &c) {
   return 0;
 }
 
-static void free_owned(Ctx &c, void *p) {
-  if (!p) return;
-  for (size_t k = 0; k < c.owned.size(); ++k)
-    if (c.owned[k] == p) {
-      hipFree(p);
-      c.owned.erase(c.owned.begin() + (long)k);
-      return;
-    }
-}
-
-template <class T>
-static int upload_v(Ctx &c, T **dst, const std::vector<T> &src) {
-  int rc = dalloc(c, dst, src.size());
-  if (rc) return rc;
-  if (!src.empty()) FVK_HIP(hipMemcpy(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice));
-  return 0;
-}
-
-// Ranges of R rows consecutive in the reference numbering (the order of
-// the sweeps: forward ascending, backward descending) and, in each, its
-// rows by level (ties by rank), with the descriptors of sweep_parts.
-static int parts_build(Ctx &c, bool fwd, const std::vector<int> &rank, const std::vector<int> &spc,
-                       const std::vector<unsigned char> &mask, Ctx::SweepParts &pt) {
-  const int n = c.n, R = c.sweep_part_rows, Ws = c.M.Ws;
-  const size_t ld = (size_t)c.M.ld;
-  std::vector<int> row_of(n);
-  for (int r = 0; r < n; ++r) row_of[rank[r]] = r;
-  // sweep position of each row (0 = first reached) and its level
-  auto pos_of = [&](int r) { return fwd ? rank[r] : n - 1 - rank[r]; };
-  std::vector<int> lev(n, 0);
-  for (int k = 0; k < n; ++k) {
-    const int r = row_of[fwd ? k : n - 1 - k];
-    int l = 0;
-    for (int s = 0; s < Ws; ++s)
-      if ((mask[r] >> s) & 1u) l = std::max(l, lev[spc[(size_t)s * ld + r]] + 1);
-    lev[r] = l;
-  }
-  pt.R = R;
-  pt.P = (n + R - 1) / R;
-  std::vector<int> rows, first(n), cnt(n), aux(n, 0), lrow(n), step, sp;
-  rows.reserve(n);
-  std::vector<std::pair<int, int>> buf;
-  for (int q = 0; q < pt.P; ++q) {
-    buf.clear();
-    for (int k = q * R; k < std::min(n, (q + 1) * R); ++k) {
-      const int r = row_of[fwd ? k : n - 1 - k];
-      buf.emplace_back(lev[r], k);
-    }
-    std::sort(buf.begin(), buf.end());
-    sp.push_back((int)step.size());
-    for (size_t t = 0; t < buf.size(); ++t) {
-      if (t == 0 || buf[t].first != buf[t - 1].first) step.push_back((int)rows.size());
-      rows.push_back(row_of[fwd ? buf[t].second : n - 1 - buf[t].second]);
-    }
-    step.push_back((int)rows.size());
-  }
-  sp.push_back((int)step.size());
-  pt.wmax = 0;
-  for (int q = 0; q < pt.P; ++q)
-    for (int k = sp[q]; k + 1 < sp[q + 1]; ++k) pt.wmax = std::max(pt.wmax, step[k + 1] - step[k]);
-  int W = 1;
-  for (int p = 0; p < n; ++p) {
-    first[p] = mask[rows[p]];
-    cnt[p] = __builtin_popcount(mask[rows[p]]);
-    W = std::max(W, cnt[p]);
-  }
-  pt.W = W;
-  std::vector<int> cols((size_t)W * n, 0), lcol((size_t)W * n, -1);
-  for (int p = 0; p < n; ++p) {
-    const int r = rows[p], q = pos_of(r) / R;
-    lrow[p] = pos_of(r) - q * R;
-    int t = 0;
-    for (int s = 0; s < Ws; ++s)
-      if ((mask[r] >> s) & 1u) {
-        const int j = spc[(size_t)s * ld + r];
-        cols[(size_t)t * n + p] = j;
-        if (pos_of(j) / R == q) lcol[(size_t)t * n + p] = pos_of(j) - q * R;
-        ++t;
-      }
-  }
-  std::vector<int> hd, jc, lc;
-  sweep_pack(n, W, rows, first, cnt, aux, lrow, cols, lcol, hd, jc, lc);
-  int rc = upload_v(c, &pt.hd, hd);
-  if (!rc) rc = upload_v(c, &pt.jc, jc);
-  if (!rc) rc = upload_v(c, &pt.lc, lc);
-  if (!rc) rc = upload_v(c, &pt.step, step);
-  if (!rc) rc = upload_v(c, &pt.sp, sp);
-  return rc;
-}
-
+// The sweeps' pattern in the reference numbering: entry values are places in
+// the slot table spv, transposed ones faces (ngp of the entry's face).
 int sweep_parts_build(Ctx &c) {
-  for (Ctx::SweepParts *pt : {&c.spf, &c.spb}) {
-    for (int *q : {pt->hd, pt->jc, pt->lc, pt->step, pt->sp}) free_owned(c, q);
-    *pt = Ctx::SweepParts();
-  }
+  sweep_exec_free(c.sw);
+  c.sw_mat = c.sw_fac = false;
   if (!c.sweep_one_launch) return 0;
-  const int n = c.n;
+  const int n = c.n, Ws = c.M.Ws;
   const size_t ld = (size_t)c.M.ld;
-  std::vector<int> rank(n), spc((size_t)c.M.Ws * ld);
+  std::vector<int> rank(n), spc((size_t)Ws * ld), spf((size_t)Ws * ld);
   std::vector<unsigned char> lm(n), um(n);
   FVK_HIP(hipStreamSynchronize(c.stream));
   FVK_HIP(hipMemcpy(rank.data(), c.M.rank, (size_t)n * sizeof(int), hipMemcpyDeviceToHost));
   FVK_HIP(hipMemcpy(spc.data(), c.M.spc, spc.size() * sizeof(int), hipMemcpyDeviceToHost));
+  FVK_HIP(hipMemcpy(spf.data(), c.M.spf, spf.size() * sizeof(int), hipMemcpyDeviceToHost));
   FVK_HIP(hipMemcpy(lm.data(), c.sweep_lmask, n, hipMemcpyDeviceToHost));
   FVK_HIP(hipMemcpy(um.data(), c.sweep_umask, n, hipMemcpyDeviceToHost));
-  int rc = parts_build(c, true, rank, spc, lm, c.spf);
-  if (!rc) rc = parts_build(c, false, rank, spc, um, c.spb);
-  if (rc) return rc;
-  const int bytes = 3 * c.sweep_part_rows * 8;
-  if (bytes > 65536) {
-    const void *k[] = {
-#define K_(D, V, MW) (const void *)k_sweep_pt<D, V, MW, 64>, (const void *)k_sweep_pt<D, V, MW, BS>
-#define K2_(V, MW) K_(true, V, MW), K_(false, V, MW)
-        K2_(1, 4), K2_(2, 4), K2_(3, 4), K2_(1, 8), K2_(2, 8), K2_(3, 8)
-#undef K2_
-#undef K_
-    };
-    for (const void *f : k) FVK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  SweepGraph g;
+  g.n = n;
+  g.symmetric = true;
+  g.row.resize(n);
+  for (int r = 0; r < n; ++r) g.row[rank[r]] = r;
+  g.lptr.assign(n + 1, 0);
+  g.uptr.assign(n + 1, 0);
+  for (int k = 0; k < n; ++k) {
+    g.lptr[k + 1] = g.lptr[k] + __builtin_popcount(lm[g.row[k]]);
+    g.uptr[k + 1] = g.uptr[k] + __builtin_popcount(um[g.row[k]]);
   }
-  return 0;
-}
-
-static SweepTabs tabs_of(const Ctx::SweepParts &p) {
-  return SweepTabs{(const int4 *)p.hd, (const int4 *)p.jc, (const int4 *)p.lc};
-}
-// blocks of the partitioned kernels: as many per CU as the LDS of a block
-// lets reside, at most four of 64 threads or two of 256 (the ranges a grid
-// cannot hold at once wait for a block to finish)
-static int pt_grid(const Ctx &c, const Ctx::SweepParts &p, size_t lds, int tb) {
-  const int per_cu = std::max(1, std::min<int>(tb == 64 ? 4 : 2, (int)(163840 / (lds + 1024))));
-  return std::max(1, std::min(p.P, c.n_cu * per_cu));
-}
-
-// one partitioned sweep: one wave a block when no level of a range has more
-// than 64 rows
-template <bool FWD, int V, int MW>
-static void sweep_pt_launch(Ctx &c, const Ctx::SweepParts &X, size_t lds, const double *cr, const double *src,
-                            double *out, int *ticket, const KS *gate) {
-  const size_t ld = (size_t)c.M.ld;
-  if (X.wmax <= 64)
-    k_sweep_pt<FWD, V, MW, 64><<<pt_grid(c, X, lds, 64), 64, lds, c.stream>>>(
-        c.n, X.R, X.P, tabs_of(X), X.step, X.sp, ld, c.spv, c.pc_c, cr, src, out, ticket, c.sweep_int + 3, gate);
-  else
-    k_sweep_pt<FWD, V, MW, BS><<<pt_grid(c, X, lds, BS), BS, lds, c.stream>>>(
-        c.n, X.R, X.P, tabs_of(X), X.step, X.sp, ld, c.spv, c.pc_c, cr, src, out, ticket, c.sweep_int + 3, gate);
-}
-
-template <bool FWD>
-static void sweep_pt_any(Ctx &c, int nvc, const Ctx::SweepParts &X, size_t lds, const double *cr, const double *src,
-                         double *out, int *ticket, const KS *gate) {
-  if (X.W <= 4) {
-    if (nvc == 1) sweep_pt_launch<FWD, 1, 4>(c, X, lds, cr, src, out, ticket, gate);
-    else if (nvc == 2) sweep_pt_launch<FWD, 2, 4>(c, X, lds, cr, src, out, ticket, gate);
-    else sweep_pt_launch<FWD, 3, 4>(c, X, lds, cr, src, out, ticket, gate);
-  } else {
-    if (nvc == 1) sweep_pt_launch<FWD, 1, 8>(c, X, lds, cr, src, out, ticket, gate);
-    else if (nvc == 2) sweep_pt_launch<FWD, 2, 8>(c, X, lds, cr, src, out, ticket, gate);
-    else sweep_pt_launch<FWD, 3, 8>(c, X, lds, cr, src, out, ticket, gate);
+  g.lcol.resize(g.lptr[n]);
+  g.lval.resize(g.lptr[n]);
+  g.tval.resize(g.lptr[n]);
+  g.ucol.resize(g.uptr[n]);
+  g.uval.resize(g.uptr[n]);
+  for (int k = 0; k < n; ++k) {
+    const int r = g.row[k];
+    int l = g.lptr[k], u = g.uptr[k];
+    for (int s = 0; s < Ws; ++s) {
+      const size_t o = (size_t)s * ld + r;
+      if ((lm[r] >> s) & 1u) {
+        g.lcol[l] = rank[spc[o]];
+        g.lval[l] = (int)o;
+        g.tval[l++] = spf[o];
+      } else if ((um[r] >> s) & 1u) {
+        g.ucol[u] = rank[spc[o]];
+        g.uval[u++] = (int)o;
+      }
+    }
   }
+  SweepPlan p;
+  const std::string e = sweep_plan(g, c.sweep_part_rows, p);
+  if (!e.empty()) {
+    set_error(e);
+    return FVK_ERR_ARG;
+  }
+  c.sw.n_cu = c.n_cu;
+  return sweep_exec_build(c.sw, p, c.stream);
+}
+
+static int sweep_pack_matrix(Ctx &c) {
+  const int rc = sweep_pack(c.sw, c.stream, c.spv, c.ngp);
+  c.sw_mat = rc == 0;
+  return rc;
 }
 
 int precond_build(Ctx &c, int imat) {
@@ -1049,17 +855,11 @@ int precond_build(Ctx &c, int imat) {
   if (imat == 0) {
     k_precond_jacobi<<<grid_for(n), BS, 0, c.stream>>>(n, c.diag, c.pc_c, c.pc_cr);
   } else if (c.sweep_one_launch && c.sweep_parts) {
-    const Ctx::SweepParts &P = c.spf;
-    const size_t lds = (size_t)P.R * 8;
-    k_sweep_mark<<<mark_grid(n), BS, 0, c.stream>>>(n, c.pc_c, c.sweep_int + 2, nullptr, 1);
-#define PC_(MW, TB) k_precond_pt<MW, TB><<<pt_grid(c, P, lds, TB), TB, lds, c.stream>>>(n, P.R, P.P, tabs_of(P), \
-    P.step, P.sp, c.M, imat, c.diag, c.ngp, c.ngn, c.pc_c, c.pc_cr, c.sweep_int + 2, c.sweep_int + 3)
-    if (P.W <= 4) {
-      if (P.wmax <= 64) PC_(4, 64); else PC_(4, BS);
-    } else {
-      if (P.wmax <= 64) PC_(8, 64); else PC_(8, BS);
-    }
-#undef PC_
+    int rc = sweep_pack_matrix(c);
+    if (!rc)
+      rc = sweep_factor(c.sw, c.stream, imat == 1 ? SWEEP_DIC : SWEEP_DILU, c.diag, nullptr, c.pc_c, c.pc_cr,
+                        c.sweep_int + 3);
+    if (rc) return rc;
   } else if (c.sweep_one_launch) {
     k_sweep_mark<<<mark_grid(n), BS, 0, c.stream>>>(n, c.pc_c, c.sweep_int + 2, nullptr, 1);
     k_precond_sf<<<sweep_grid(c), BS, 0, c.stream>>>(c.M, c.lf.rows, c.sweep_lmask, imat, c.diag, c.ngp, c.ngn,
@@ -1074,6 +874,7 @@ int precond_build(Ctx &c, int imat) {
   FVK_HIP(hipGetLastError());
   c.pc_imat = imat;
   c.pc_valid = true;
+  c.sw_fac = imat != 0 && c.sweep_one_launch && c.sweep_parts;
   return 0;
 }
 
@@ -1082,12 +883,16 @@ int precond_apply(Ctx &c, int imat, int nvc, const double *b, double *x, const K
   if (imat == 0) {
     k_jacobi_apply<<<grid_for(n), BS, 0, c.stream>>>(n, nvc, c.pc_c, b, x, gate);
   } else if (c.sweep_one_launch && c.sweep_parts) {
-    const size_t cnt = (size_t)nvc * n;
-    const size_t lds = (size_t)nvc * c.sweep_part_rows * 8;
-    k_sweep_mark<<<mark_grid(cnt), BS, 0, c.stream>>>(cnt, c.sweep_t, c.sweep_int, gate, nvc);
-    sweep_pt_any<true>(c, nvc, c.spf, lds, nullptr, b, c.sweep_t, c.sweep_int, gate);
-    k_sweep_mark<<<mark_grid(cnt), BS, 0, c.stream>>>(cnt, x, c.sweep_int + 1, gate, nvc);
-    sweep_pt_any<false>(c, nvc, c.spb, lds, c.pc_cr, c.sweep_t, x, c.sweep_int + 1, gate);
+    // a factor that another form built, or that the caller gave
+    int rc = c.sw_mat ? 0 : sweep_pack_matrix(c);
+    if (!rc && !c.sw_fac) {
+      rc = sweep_factor_from(c.sw, c.stream, c.pc_c, c.pc_cr);
+      c.sw_fac = rc == 0;
+    }
+    SweepGate G;
+    if (gate) G = SweepGate{&gate->done, (int)(sizeof(KS) / sizeof(int)), nvc};
+    if (!rc) rc = sweep_apply(c.sw, c.stream, nvc, b, x, G, c.sweep_int + 3);
+    if (rc) return rc;
   } else if (c.sweep_one_launch) {
     const size_t cnt = (size_t)nvc * n;
     k_sweep_mark<<<mark_grid(cnt), BS, 0, c.stream>>>(cnt, c.sweep_t, c.sweep_int, gate, nvc);

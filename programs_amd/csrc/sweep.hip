@@ -1,0 +1,557 @@
+// The one-launch triangular sweeps and factorisations (SweepPlan): DIC /
+// DILU of spray-simulation (solv_precond.f90:10-29, solv_direct.f90:11-42)
+// and flowlab's factor (solv_m.f90:224-286).  Each row performs the
+// reference's operations in its order; only the order between independent
+// rows differs, so results equal the sequential loops bit for bit.
+//
+// A block takes parts of the plan from a ticket counter, in an order in
+// which a part only needs values of parts taken before it (no deadlock
+// whatever the residency), and runs a part with three waves:
+//   wave 0 computes: it walks the part's chunks (64 rows that do not depend
+//     on each other) in order.  All values it reads sit in LDS, its own
+//     rows' and the halo's; a wave's LDS operations are in order, so chunk
+//     after chunk needs no barrier.  Matrix entries, factor and records are
+//     stored by position, so that a chunk's loads are consecutive, and are
+//     issued up to eight chunks ahead.  Values that other parts need go to
+//     the export buffer at once (agent scope).
+//   waves 1 and 2 fetch the halo: each polls the export buffer for the
+//     values of other parts, in the order in which the chunks need them,
+//     puts them into LDS and publishes how many are there.  Two waves poll
+//     twice as often as one (the wait for the next poll is part of every
+//     crossing).
+// Results go from LDS to memory by all waves when the part is done.
+//
+// Export slots hold kSweepMark (a signalling NaN: no arithmetic result has
+// this pattern) until their value arrives.  A launch marks the buffer of the
+// other direction, so no launch is spent on marking.  The halo waves'
+// waits are bounded (kSweepSpin polls; 256 once an error is recorded); past
+// the bound they record the error, the compute wave runs through what is
+// left on what is there and the block stops taking parts.
+//
+// What bounds it: the chain of chunks a path runs through (0.11 us a chunk:
+// LDS read, five dependent FP64 operations, LDS write) and the crossings
+// between parts (1 us: store, poll, reload), not bandwidth.  One application
+// of DIC to one right-hand side (both sweeps), against the form it replaced
+// (ranges of 4096 consecutive rows, a level at a time): 24^3 42 us (177),
+// 96^3 189 us (620), 128^3 294 us (1232); DILU to three at 128^3 445 us
+// (1823); 40,000 triangles of a Delaunay channel 64 us (155).
+#include <algorithm>
+#include <climits>
+#include <cmath>
+
+#include "ctx.h"
+#include "sweep.h"
+#include "sweepexec.h"
+
+namespace fvk {
+
+constexpr int SW_TB = 192;   // one compute wave, two halo waves
+constexpr int kHaloWin = 2;  // groups of 64 halo values polled together
+// chunks whose loads are in flight: at most 8, and at most 56 loads and
+// exports (a wave counts 63)
+constexpr int sweep_ahead(int MW, int KIND) {
+  const int ops = (MW == 8 ? 2 : 1) + MW * (KIND == 2 ? 2 : 1) + (KIND == 0 ? 1 : 0) + 1;
+  return ops * 8 <= 56 ? 8 : 56 / ops;
+}
+
+struct SweepArgs {
+  int P, np, slots, NE, NEo, n;
+  const int *part, *prow, *ppos, *hsrc;
+  const unsigned short *pslot, *rec;
+  const double *a, *a2, *c;   // by position
+  const double *src, *cr;     // initial values of the rows; backward: their scale
+  const int *dix;
+  double *dst;
+  double *E, *Eo;
+  int *ticket, *ticket_o, *err;
+  double *crow, *drow, *cpos, *crr;  // factor
+  SweepGate gate;
+};
+
+// LDS scalars shared by a block's waves
+struct SweepShared {
+  int q, have, abort;
+};
+
+__device__ __forceinline__ int lds_get(const int *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// this wave's LDS operations so far are done
+__device__ __forceinline__ void lds_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+typedef const __attribute__((address_space(1))) char *global_p;
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+template <class T>
+__device__ __forceinline__ T ld_at(global_p base, unsigned byte) {
+  return *(const __attribute__((address_space(1))) T *)(base + byte);
+}
+
+// what a lane needs to run its row of a chunk
+template <int MW>
+struct SweepStage {
+  unsigned w[MW <= 4 ? 4 : 6];  // the record's 16-bit words in pairs
+  double a[MW], a2[MW], c;
+  __device__ __forceinline__ unsigned word(int t) const { return t & 1 ? w[t / 2] >> 16 : w[t / 2] & 0xffffu; }
+  __device__ __forceinline__ int need() const { return (int)word(MW <= 4 ? 5 : 9); }
+  __device__ __forceinline__ int exp() const { return (int)w[MW <= 4 ? 3 : 5]; }
+};
+
+// uniform base pointers of the loads by position (opaque, so that each load
+// is one instruction with a scalar base and a 32-bit offset)
+template <int MW>
+struct SweepBase {
+  global_p rec, a[MW], a2[MW], c;
+};
+__device__ __forceinline__ global_p opaque(const void *p) {
+  global_p q = (global_p)p;
+  asm volatile("" : "+s"(q));
+  return q;
+}
+
+// KIND 0: sweep; 1: DIC factor, entries (a a) v; 2: factor, entries (a v) a2
+template <int MW, int KIND>
+__device__ __forceinline__ void sweep_load(const SweepBase<MW> &B, unsigned bo, SweepStage<MW> &S) {
+  const u32x4 x = ld_at<u32x4>(B.rec, bo * (MW <= 4 ? 2u : 4u));
+#pragma unroll
+  for (int k = 0; k < 4; ++k) S.w[k] = x[k];
+  if (MW > 4) {
+    const u32x2 y = ld_at<u32x2>(B.rec, bo * 4u + 16u);
+    S.w[MW > 4 ? 4 : 0] = y[0];
+    S.w[MW > 4 ? 5 : 0] = y[1];
+  }
+#pragma unroll
+  for (int t = 0; t < MW; ++t) {
+    S.a[t] = ld_at<double>(B.a[t], bo);
+    if (KIND == 2) S.a2[t] = ld_at<double>(B.a2[t], bo);
+  }
+  if (KIND == 0) S.c = ld_at<double>(B.c, bo);
+}
+
+// The chunks of a part.  The groups of kAhead + 1 chunks are straight code
+// but for the (rare) wait for the halo, so that the compiler can count the
+// loads in flight and waits for the oldest only; a chunk's loads go to the
+// stage that the chunk before has freed, while this chunk's LDS reads are
+// on their way.
+template <bool FWD, int NC, int MW, int KIND>
+__device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nch, char *lv, unsigned ld,
+                                              SweepShared &sh) {
+  constexpr int kAhead = sweep_ahead(MW, KIND), kRing = kAhead + 1;
+  SweepBase<MW> B;
+  B.rec = opaque(A.rec);
+#pragma unroll
+  for (int t = 0; t < MW; ++t) {
+    B.a[t] = opaque(A.a + (size_t)t * A.np);
+    if (KIND == 2) B.a2[t] = opaque(A.a2 + (size_t)t * A.np);
+  }
+  if (KIND == 0) B.c = opaque(A.c);
+  const unsigned lane8 = threadIdx.x * 8u;
+  // byte offset of the j-th chunk in the sweep's direction (clamped to the part's last)
+  auto at = [&](int j) {
+    const int jj = min(j, nch - 1);
+    return (unsigned)(FWD ? c0 + jj : c0 + nch - 1 - jj) * (kChunk * 8u) + lane8;
+  };
+  SweepStage<MW> S[kRing];
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) sweep_load<MW, KIND>(B, at(u), S[u]);
+  int have = 0;
+  // the chunk about to run: its LDS addresses and halo need, taken while
+  // the reads of the chunk before are on their way
+  unsigned off[MW + 1];
+  int nd = 0;
+  auto prep = [&](const SweepStage<MW> &Y) {
+#pragma unroll
+    for (int t = 0; t <= MW; ++t) off[t] = Y.word(t);
+    nd = __builtin_amdgcn_readfirstlane(Y.need());
+  };
+  auto run = [&](const SweepStage<MW> &X, const SweepStage<MW> &Y, auto ahead) {
+    while (nd > have) {
+      have = __builtin_amdgcn_readfirstlane(lds_get(&sh.have));
+      // the halo waves gave up: the rest of the part runs on what is there
+      if (nd > have && __builtin_amdgcn_readfirstlane(lds_get(&sh.abort))) have = INT_MAX;
+    }
+    asm volatile("" ::: "memory");
+    double acc[NC], v[MW][NC], r[NC];
+#pragma unroll
+    for (int q = 0; q < NC; ++q) acc[q] = *(const double *)(lv + (off[0] + q * ld));
+#pragma unroll
+    for (int t = 0; t < MW; ++t)
+#pragma unroll
+      for (int q = 0; q < NC; ++q) v[t][q] = *(const double *)(lv + (off[1 + t] + q * ld));
+    __builtin_amdgcn_sched_barrier(0);
+    ahead();
+    const unsigned own = off[0];
+    prep(Y);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < MW; ++t)
+#pragma unroll
+      for (int q = 0; q < NC; ++q) {
+        if (KIND == 0) acc[q] = acc[q] - X.a[t] * v[t][q];
+        else if (KIND == 1) acc[q] = acc[q] - X.a[t] * X.a[t] * v[t][q];
+        else acc[q] = acc[q] - X.a[t] * v[t][q] * X.a2[t];
+      }
+    if (KIND == 0) {
+#pragma unroll
+      for (int q = 0; q < NC; ++q) *(double *)(lv + (own + q * ld)) = r[q] = acc[q] * X.c;
+    } else {
+      *(double *)(lv + own) = r[0] = 1.0 / (acc[0] + SMALL);
+      *(double *)(lv + (own + ld)) = acc[0];
+    }
+    const int e = X.exp();
+    if (e >= 0)
+#pragma unroll
+      for (int q = 0; q < NC; ++q) st_agent(A.E + (size_t)q * A.NE + e, r[q]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  prep(S[0]);
+  int j0 = 0;
+  for (; j0 + kRing <= nch; j0 += kRing) {
+#pragma unroll
+    for (int u = 0; u < kRing; ++u)
+      run(S[u], S[(u + 1) % kRing],
+          [&] { sweep_load<MW, KIND>(B, at(j0 + u + kAhead), S[(u + kAhead) % kRing]); });
+  }
+  // fewer than kRing chunks are left, all of them loaded
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u)
+    if (j0 + u < nch) run(S[u], S[(u + 1) % kRing], [] {});
+}
+
+template <int NC>
+__device__ __forceinline__ void sweep_halo(const SweepArgs &A, int nh, int nr, char *lv, unsigned ld, const int *s_hsrc,
+                                           SweepShared &sh) {
+  const int lane = threadIdx.x & 63, ng = (nh + 63) / 64;
+  int src[kHaloWin];
+  bool pend[kHaloWin];
+  auto start = [&](int g, int &s, bool &p) {
+    const int e = g * 64 + lane;
+    p = e < nh;
+    s = p ? s_hsrc[e] : 0;
+  };
+#pragma unroll
+  for (int w = 0; w < kHaloWin; ++w) start(w, src[w], pend[w]);
+  unsigned spin = 0;
+  int g = 0, pub = 0;
+  while (g < ng) {
+    unsigned long long v[kHaloWin][NC];
+#pragma unroll
+    for (int w = 0; w < kHaloWin; ++w)
+      if (pend[w])
+#pragma unroll
+        for (int q = 0; q < NC; ++q) v[w][q] = ld_agent(A.E + (size_t)q * A.NE + src[w]);
+#pragma unroll
+    for (int w = 0; w < kHaloWin; ++w)
+      if (pend[w]) {
+        bool ready = true;
+#pragma unroll
+        for (int q = 0; q < NC; ++q) ready = ready && v[w][q] != kSweepMark;
+        if (ready) {
+          const unsigned o = (unsigned)(nr + (g + w) * 64 + lane) * 8u;
+#pragma unroll
+          for (int q = 0; q < NC; ++q) *(double *)(lv + (o + q * ld)) = __longlong_as_double((long long)v[w][q]);
+          pend[w] = false;
+        }
+      }
+    unsigned long long m = __ballot(pend[0]);
+    while (m == 0 && g < ng) {
+      ++g;
+#pragma unroll
+      for (int w = 0; w + 1 < kHaloWin; ++w) {
+        pend[w] = pend[w + 1];
+        src[w] = src[w + 1];
+      }
+      start(g + kHaloWin - 1, src[kHaloWin - 1], pend[kHaloWin - 1]);
+      m = __ballot(pend[0]);
+    }
+    const int have = min(nh, g * 64 + (m ? __builtin_ctzll(m) : 0));
+    if (have > pub) {
+      pub = have;
+      spin = 0;
+      lds_done();
+      __hip_atomic_fetch_max(&sh.have, have, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else if (++spin > kSweepSpin ||
+               ((spin & 255u) == 0 && __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+      __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&sh.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      return;
+    }
+  }
+}
+
+template <bool FWD, int NC, int MW, int KIND>
+__global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
+  if (A.gate.done) {
+    bool all = true;
+    for (int q = 0; q < A.gate.n; ++q) all = all && A.gate.done[q * A.gate.stride];
+    if (all) return;
+  }
+  extern __shared__ double lds[];
+  __shared__ SweepShared sh;
+  constexpr int NV = KIND == 0 ? NC : 2;  // values per slot (factor: c and d)
+  const unsigned ld = (unsigned)A.slots * 8u;
+  char *lv = (char *)lds;
+  int *s_hsrc = (int *)(lv + (size_t)NV * ld);
+  const int tid = threadIdx.x, wave = tid >> 6;
+  if (KIND == 0) {
+    // the other direction's export buffer, for the launch after this one
+    const size_t m = (size_t)NC * A.NEo;
+    for (size_t i = blockIdx.x * (size_t)SW_TB + tid; i < m; i += (size_t)gridDim.x * SW_TB)
+      ((unsigned long long *)A.Eo)[i] = kSweepMark;
+    if (blockIdx.x == 0 && tid == 0) *A.ticket_o = 0;
+  }
+  if (tid == 0) sh.abort = 0;
+  for (;;) {
+    if (tid == 0) {
+      sh.q = atomicAdd(A.ticket, 1);
+      sh.have = 0;
+    }
+    __syncthreads();
+    const int o = __builtin_amdgcn_readfirstlane(sh.q);
+    if (o >= A.P) return;
+    const int q = FWD ? o : A.P - 1 - o;
+    const int *Q = A.part + 8 * q;
+    const int c0 = Q[0], nch = Q[1], r0 = Q[2], nr = Q[3], h0 = FWD ? Q[4] : Q[6], nh = FWD ? Q[5] : Q[7];
+    // rows' initial values and the part's tables into LDS
+    for (int k0 = tid; k0 < nr; k0 += 4 * SW_TB) {
+      int kk[4], row[4];
+      unsigned off[4];
+      double v[4][NC], s[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        kk[i] = r0 + min(k0 + i * SW_TB, nr - 1);
+        off[i] = A.pslot[kk[i]];
+        if (FWD) row[i] = A.prow[kk[i]];
+        else s[i] = A.cr[kk[i]];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int z = !FWD ? kk[i] : KIND != 0 && A.dix ? A.dix[row[i]] : row[i];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[i][c] = A.src[(size_t)c * A.n + z];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (k0 + i * SW_TB < nr)
+#pragma unroll
+          for (int c = 0; c < NC; ++c) *(double *)(lv + (off[i] + c * ld)) = FWD ? v[i][c] : v[i][c] * s[i];
+    }
+    for (int h = tid; h < nh; h += SW_TB) s_hsrc[h] = A.hsrc[h0 + h];
+    if (tid < 2 * NV) *(double *)(lv + ((unsigned)(nr + nh + (tid & 1)) * 8u + (tid >> 1) * ld)) = 0.0;
+    __syncthreads();
+    // the halo waves of other blocks poll on the same SIMD
+    if (wave == 0) __builtin_amdgcn_s_setprio(3);
+    if (wave == 0) sweep_compute<FWD, NC, MW, KIND>(A, c0, nch, lv, ld, sh);
+    else sweep_halo<NC>(A, nh, nr, lv, ld, s_hsrc, sh);
+    __syncthreads();
+    if (sh.abort) return;
+    for (int k = tid; k < nr; k += SW_TB) {
+      const unsigned off = A.pslot[r0 + k];
+      if (KIND == 0) {
+        const int z = FWD ? r0 + k : A.prow[r0 + k];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) A.dst[(size_t)c * A.n + z] = *(const double *)(lv + (off + c * ld));
+      } else {
+        const int row = A.prow[r0 + k];
+        const double c = *(const double *)(lv + off), d = *(const double *)(lv + (off + ld));
+        A.crow[row] = c;
+        if (A.drow) A.drow[row] = d;
+        A.cpos[A.ppos[r0 + k]] = c;
+        A.crr[r0 + k] = A.drow ? d : 1.0 / (c + SMALL);
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(BS) void k_export_mark(size_t cnt, double *__restrict__ out) {
+  for (size_t i = blockIdx.x * (size_t)BS + threadIdx.x; i < cnt; i += (size_t)gridDim.x * BS)
+    ((unsigned long long *)out)[i] = kSweepMark;
+}
+
+// entry values by position; the factorisation's export buffer and ticket
+__global__ __launch_bounds__(BS) void k_sweep_pack(int np, int MW, const int *__restrict__ lval,
+                                                   const int *__restrict__ uval, const int *__restrict__ tval,
+                                                   const double *__restrict__ vals, const double *__restrict__ tvals,
+                                                   double *__restrict__ aL, double *__restrict__ aU,
+                                                   double *__restrict__ aT, int NE, double *__restrict__ Ec,
+                                                   int *ticket) {
+  const size_t i = blockIdx.x * (size_t)BS + threadIdx.x;
+  if (i < (size_t)NE) ((unsigned long long *)Ec)[i] = kSweepMark;
+  if (i == 0) *ticket = 0;
+  if (i >= (size_t)np) return;
+  for (int t = 0; t < MW; ++t) {
+    const size_t o = (size_t)t * np + i;
+    const int l = lval[o], u = uval[o];
+    aL[o] = l >= 0 ? vals[l] : 0.0;
+    aU[o] = u >= 0 ? vals[u] : 0.0;
+    if (tvals) {
+      const int x = tval[o];
+      aT[o] = x >= 0 ? tvals[x] : 0.0;
+    }
+  }
+}
+
+__global__ __launch_bounds__(BS) void k_sweep_factor_from(int n, const int *__restrict__ prow,
+                                                          const int *__restrict__ ppos,
+                                                          const double *__restrict__ crow,
+                                                          const double *__restrict__ drow, double *__restrict__ cpos,
+                                                          double *__restrict__ crr) {
+  const int k = blockIdx.x * BS + threadIdx.x;
+  if (k >= n) return;
+  cpos[ppos[k]] = crow[prow[k]];
+  crr[k] = drow[prow[k]];
+}
+
+// ---------------------------------------------------------------- host
+template <class T>
+static int up(SweepExec &X, T **d, const std::vector<T> &v, size_t extra = 0) {
+  void *q = nullptr;
+  FVK_HIP(hipMalloc(&q, std::max<size_t>(1, v.size() + extra) * sizeof(T)));
+  X.mem.push_back(q);
+  if (!v.empty()) FVK_HIP(hipMemcpy(q, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+  *d = (T *)q;
+  return 0;
+}
+// zeroed; the clear has finished when the build returns (it ends with a wait)
+static int room(SweepExec &X, double **d, size_t n, hipStream_t s) {
+  void *q = nullptr;
+  FVK_HIP(hipMalloc(&q, std::max<size_t>(1, n) * sizeof(double)));
+  X.mem.push_back(q);
+  FVK_HIP(hipMemsetAsync(q, 0, std::max<size_t>(1, n) * sizeof(double), s));
+  *d = (double *)q;
+  return 0;
+}
+static int mark(double *p, size_t cnt, hipStream_t s) {
+  k_export_mark<<<(int)std::max<size_t>(1, std::min<size_t>((cnt + BS - 1) / BS, 4096)), BS, 0, s>>>(cnt, p);
+  FVK_HIP(hipGetLastError());
+  return 0;
+}
+
+template <int MW>
+static int allow_lds() {
+  const void *k[] = {(const void *)k_sweep<true, 1, MW, 0>,  (const void *)k_sweep<true, 2, MW, 0>,
+                     (const void *)k_sweep<true, 3, MW, 0>,  (const void *)k_sweep<false, 1, MW, 0>,
+                     (const void *)k_sweep<false, 2, MW, 0>, (const void *)k_sweep<false, 3, MW, 0>,
+                     (const void *)k_sweep<true, 1, MW, 1>,  (const void *)k_sweep<true, 1, MW, 2>};
+  for (const void *f : k) FVK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kSweepLds));
+  return 0;
+}
+
+int sweep_exec_build(SweepExec &X, const SweepPlan &p, hipStream_t s) {
+  X.n = p.n; X.P = p.P; X.MW = p.MW; X.np = p.np; X.slots = p.slots; X.bricks = p.bricks;
+  for (int k = 1; k <= 3; ++k) X.lds_[k] = p.lds(k);
+  int rc = 0;
+#define U(dst, src) if (!rc) rc = up(X, &dst, src)
+#define R(dst, cnt) if (!rc) rc = room(X, &dst, cnt, s)
+  U(X.part, p.part); U(X.prow, p.prow); U(X.ppos, p.ppos); U(X.pslot, p.pslot); U(X.tval, p.tval);
+  const size_t mnp = (size_t)p.MW * p.np;
+  for (int k = 0; k < 2; ++k) {
+    SweepExec::Dir &D = X.d[k];
+    const SweepPlan::Dir &S = p.d[k];
+    D.NE = S.NE;
+    U(D.rec, S.rec); U(D.val, S.val); U(D.hsrc, S.hsrc);
+    R(D.E, (size_t)3 * D.NE); R(D.a, mnp);
+    if (!rc) rc = mark(D.E, (size_t)3 * D.NE, s);
+  }
+  R(X.aT, mnp); R(X.c, p.np); R(X.cr, p.n); R(X.Ec, X.d[0].NE); R(X.t, (size_t)3 * p.n);
+  double *tk = nullptr;
+  R(tk, 2);
+  X.ticket = (int *)tk;
+#undef U
+#undef R
+  if (rc) return rc;
+  if ((rc = X.MW == 3 ? allow_lds<3>() : X.MW == 4 ? allow_lds<4>() : allow_lds<8>())) return rc;
+  FVK_HIP(hipStreamSynchronize(s));
+  return 0;
+}
+
+void sweep_exec_free(SweepExec &X) {
+  for (void *q : X.mem) hipFree(q);
+  const int n_cu = X.n_cu, blocks = X.blocks;
+  X = SweepExec();
+  X.n_cu = n_cu;
+  X.blocks = blocks;
+}
+
+static SweepArgs args(const SweepExec &X, int dir) {
+  SweepArgs A;
+  const SweepExec::Dir &D = X.d[dir], &O = X.d[1 - dir];
+  A.P = X.P; A.np = X.np; A.slots = X.slots; A.NE = D.NE; A.NEo = O.NE; A.n = X.n;
+  A.part = X.part; A.prow = X.prow; A.ppos = X.ppos; A.pslot = X.pslot;
+  A.rec = D.rec; A.hsrc = D.hsrc;
+  A.a = D.a; A.a2 = nullptr; A.c = X.c; A.src = nullptr; A.cr = X.cr; A.dix = nullptr; A.dst = nullptr;
+  A.E = D.E; A.Eo = O.E;
+  A.ticket = X.ticket + dir; A.ticket_o = X.ticket + 1 - dir; A.err = nullptr;
+  A.crow = A.drow = A.cpos = A.crr = nullptr;
+  return A;
+}
+
+// Blocks of a launch.  A block that waits for its part's first values polls,
+// which slows the ones at work, so of a brick plan no more are resident than
+// run at a time: the front through the brick grid is about 2.25 P^(2/3)
+// parts wide.  At least one per CU, at most what their LDS lets reside.
+// Measured (DIC, both sweeps, 128^3, 1331 bricks: 272 blocks by the rule):
+// 256 blocks 294 us, 512 309 us, 1024 334 us; 96^3 (512 bricks): 189 us
+// with 256, 199 us with 512.
+static int grid(const SweepExec &X, size_t lds) {
+  const int fit = X.n_cu * std::max(1, std::min(8, (int)(163840 / (lds + 512))));
+  const int front = X.bricks ? std::max(X.n_cu, (int)(2.25 * std::cbrt((double)X.P * X.P))) : fit;
+  return std::max(1, std::min({X.P, fit, X.blocks > 0 ? X.blocks : front}));
+}
+
+template <bool FWD, int NC, int KIND>
+static void launch(const SweepExec &X, const SweepArgs &A, hipStream_t s) {
+  const size_t lds = X.lds_[KIND == 0 ? NC : 2];
+  const int G = grid(X, lds);
+  if (X.MW == 3) k_sweep<FWD, NC, 3, KIND><<<G, SW_TB, lds, s>>>(A);
+  else if (X.MW == 4) k_sweep<FWD, NC, 4, KIND><<<G, SW_TB, lds, s>>>(A);
+  else k_sweep<FWD, NC, 8, KIND><<<G, SW_TB, lds, s>>>(A);
+}
+
+int sweep_pack(SweepExec &X, hipStream_t s, const double *vals, const double *tvals) {
+  const int cnt = std::max(X.np, X.d[0].NE);
+  k_sweep_pack<<<(cnt + BS - 1) / BS, BS, 0, s>>>(X.np, X.MW, X.d[0].val, X.d[1].val, X.tval, vals, tvals, X.d[0].a,
+                                                  X.d[1].a, X.aT, X.d[0].NE, X.Ec, X.ticket + 2);
+  FVK_HIP(hipGetLastError());
+  return 0;
+}
+
+int sweep_factor(SweepExec &X, hipStream_t s, int kind, const double *diag, const int *dix, double *crow, double *drow,
+                 int *err) {
+  SweepArgs A = args(X, 0);
+  A.src = diag; A.dix = dix; A.err = err; A.E = X.Ec; A.ticket = X.ticket + 2;
+  A.crow = crow; A.drow = drow; A.cpos = X.c; A.crr = X.cr;
+  // DIC: d - ngn ngn c; DILU: d - ngp c ngn; flowlab: s - a pc a^T
+  A.a = kind == SWEEP_DILU ? X.aT : X.d[0].a;
+  A.a2 = kind == SWEEP_DILU ? X.d[0].a : X.aT;
+  if (kind == SWEEP_DIC) launch<true, 1, 1>(X, A, s);
+  else launch<true, 1, 2>(X, A, s);
+  FVK_HIP(hipGetLastError());
+  return 0;
+}
+
+int sweep_factor_from(SweepExec &X, hipStream_t s, const double *crow, const double *drow) {
+  k_sweep_factor_from<<<(X.n + BS - 1) / BS, BS, 0, s>>>(X.n, X.prow, X.ppos, crow, drow, X.c, X.cr);
+  FVK_HIP(hipGetLastError());
+  return 0;
+}
+
+int sweep_apply(SweepExec &X, hipStream_t s, int nc, const double *b, double *x, SweepGate gate, int *err) {
+  SweepArgs A = args(X, 0), B = args(X, 1);
+  A.src = b; A.dst = X.t; A.err = err; A.gate = gate;
+  B.src = X.t; B.dst = x; B.err = err; B.gate = gate;
+  if (nc == 1) {
+    launch<true, 1, 0>(X, A, s);
+    launch<false, 1, 0>(X, B, s);
+  } else if (nc == 2) {
+    launch<true, 2, 0>(X, A, s);
+    launch<false, 2, 0>(X, B, s);
+  } else {
+    launch<true, 3, 0>(X, A, s);
+    launch<false, 3, 0>(X, B, s);
+  }
+  FVK_HIP(hipGetLastError());
+  return 0;
+}
+
+}  // namespace fvk

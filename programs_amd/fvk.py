@@ -149,6 +149,7 @@ def lib():
         "fvk_sys_solve": [_vp, C.c_int, C.c_int, C.c_double, C.c_int, C.c_int, C.POINTER(SolveInfo)],
         "fvk_sys_get_x": [_vp, _dp],
         "fvk_ctx_set_param": [_vp, C.c_char_p, C.c_double],
+        "fvk_sweep_plan": [C.c_int, _ip, _ip, C.c_int, _ip],
         "fvk_factor_set": [_vp, _fp, _fp],
         "fvk_factor_apply": [_vp, _dp, _dp],
         "fvk_factor_get": [_vp, _fp, _fp],
@@ -517,6 +518,15 @@ def sys_solve(ctx: Ctx, method=SOLVE_PCG64, imat=0, tol=1e-8, max_iter=100000, t
 
 def set_param(ctx: Ctx, name, value):
     _check(lib().fvk_ctx_set_param(ctx.h, name.encode(), float(value)))
+
+
+def sweep_plan(ia, ja, max_rows=4096):
+    """How the one-launch sweeps split a pattern (1-based CSR with its
+    diagonal), checked by walking it; host only."""
+    a, b = np.ascontiguousarray(ia, np.int32), np.ascontiguousarray(ja, np.int32)
+    o = np.zeros(8, np.int32)
+    _check(lib().fvk_sweep_plan(len(a) - 1, _i(a), _i(b), max_rows, _i(o)))
+    return dict(zip(("parts", "chunks", "levels", "bricks", "lds1", "lds3", "passed_fwd", "passed_bwd"), map(int, o)))
 
 
 def factor_set(ctx: Ctx, l, sig):

@@ -1,0 +1,71 @@
+"""The plan of the one-launch triangular sweeps (host only): which rows a
+block walks together and which values pass between blocks.  fvk_sweep_plan
+walks every plan as the kernels do and fails when a value would be read
+before it is there, when a part needs a part taken after it, or when a row
+is not run once; the cases are where that can go wrong: one row, one part,
+ragged boxes, chains, unstructured and unsorted patterns, rows with one to
+eight entries on a side."""
+import numpy as np
+import pytest
+
+from programs_amd import fvk
+
+LDS = 163840  # bytes of LDS of a compute unit
+
+
+def csr(n, pairs, unsorted=None):
+    """1-based CSR of the pattern pairs + transposed + diagonal; unsorted: a
+    generator that shuffles the columns of some rows."""
+    cols = [{i} for i in range(n)]
+    for i, j in pairs:
+        cols[i].add(j)
+        cols[j].add(i)
+    ia, ja = [1], []
+    for c in cols:
+        c = sorted(c)
+        if unsorted is not None and unsorted.random() < 0.3:
+            unsorted.shuffle(c)
+        ja += [j + 1 for j in c]
+        ia.append(len(ja) + 1)
+    return ia, ja
+
+
+def box(nx, ny, nz):
+    k = np.arange(nx * ny * nz).reshape(nz, ny, nx)
+    e = [(k[:, :, 1:], k[:, :, :-1]), (k[:, 1:], k[:, :-1]), (k[1:], k[:-1])]
+    return nx * ny * nz, np.concatenate([np.stack([a.ravel(), b.ravel()], 1) for a, b in e])
+
+
+@pytest.mark.parametrize("rows", [64, 100, 1728, 6400])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 1, 1), (65, 1, 1), (7, 5, 3), (13, 12, 11), (40, 33, 1), (25, 24, 23)])
+def test_boxes(dims, rows):
+    n, pairs = box(*dims)
+    p = fvk.sweep_plan(*csr(n, pairs.tolist()), rows)
+    assert p["levels"] == sum(dims) - 2
+    assert p["lds3"] <= LDS and p["chunks"] * 64 >= n
+    if min(dims) > 1:
+        assert p["bricks"] == 1
+        # a brick passes on the values of its faces only
+        assert p["passed_fwd"] < n or rows < 100
+
+
+@pytest.mark.parametrize("rows", [64, 300, 4096])
+@pytest.mark.parametrize("n,span,width", [(50, 1, 1), (700, 3, 2), (3000, 40, 3), (3000, 3000, 4), (2000, 900, 8)])
+def test_unstructured(n, span, width, rows):
+    rng = np.random.default_rng(n + span)
+    pairs, deg = [], np.zeros((n, 2), int)
+    for i in range(1, n):
+        for j in set((i - 1 - rng.integers(0, min(i, span), width)).tolist()):
+            if deg[i, 0] < 8 and deg[j, 1] < 8:
+                deg[i, 0] += 1
+                deg[j, 1] += 1
+                pairs.append((i, j))
+    p = fvk.sweep_plan(*csr(n, pairs), rows)
+    assert p["lds3"] <= LDS
+    # the reference's loops leave entries out where columns are not sorted
+    fvk.sweep_plan(*csr(n, pairs, np.random.default_rng(1)), rows)
+
+
+def test_too_many_entries_is_refused():
+    with pytest.raises(fvk.FvkError):
+        fvk.sweep_plan(*csr(10, [(9, j) for j in range(9)]), 64)
