@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libfvk.so")
 BUILD = os.path.join(HERE, "_build")
 
-HIP_SOURCES = ["sweep.hip", "krylov.hip", "mixed.hip", "learn.hip", "flow.hip", "meshdev.hip", "flowlab.hip", "capi.hip"]
+HIP_SOURCES = ["hostio.hip", "sweep.hip", "krylov.hip", "mixed.hip", "learn.hip", "flow.hip", "meshdev.hip", "flowlab.hip", "capi.hip"]
 CPP_SOURCES = ["mesh.cpp", "output.cpp", "flmesh.cpp", "sweepplan.cpp"]
 ARCH = os.environ.get("FVK_OFFLOAD_ARCH", "gfx950")
 

@@ -242,6 +242,7 @@ static int ctx_build(Ctx &c, const Topo &t, int device, int flags) {
     if (rc) return rc;
   }
   FVK_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
+  c.io.stream = c.stream;
   FVK_HIP(hipEventCreate(&c.ev0));
   FVK_HIP(hipEventCreate(&c.ev1));
   FVK_HIP(hipHostMalloc((void **)&c.poll_h, 2 * sizeof(KS), hipHostMallocDefault));
@@ -305,6 +306,9 @@ static int ctx_build(Ctx &c, const Topo &t, int device, int flags) {
 #define UP(field, vec) do { if ((rc = upload(c, &p, vec))) return rc; M.field = p; } while (0)
 #define UPI(field, vec) do { if ((rc = upload(c, &ip, vec))) return rc; M.field = ip; } while (0)
   UP(cx, cx); UP(cy, cy); UP(cz, cz); UP(v, v); UP(vr, vr);
+  if (flags & FVK_CTX_RCM) {
+    if ((rc = upload(c, &c.where, c.iperm))) return rc;
+  }
   UPI(rank, c.perm); UPI(fip, fip); UPI(fin, fin); UPI(fib, t.fib); UPI(fbty, t.fbty);
   UP(fs, t.fs); UP(flpn, t.flpn); UP(fwfp, t.fwfp);
   UP(fx, comp(t.fx, 0)); UP(fy, comp(t.fx, 1)); UP(fz, comp(t.fx, 2));
@@ -363,6 +367,7 @@ static void ctx_free(Ctx &c) {
   for (void *p : c.owned) hipFree(p);
   c.owned.clear();
   sweep_exec_free(c.sw);
+  c.io.free();
   if (c.ev0) hipEventDestroy(c.ev0);
   if (c.ev1) hipEventDestroy(c.ev1);
   for (int k = 0; k < 2; ++k)
@@ -373,27 +378,22 @@ static void ctx_free(Ctx &c) {
   c.stream = nullptr;
 }
 
-// reference entity-major host array (stride ld, ncomp components) <-> device
-// rows (component-major)
-static int to_dev(Ctx &c, const double *h, int ncomp, int ld, int count, const std::vector<int> *perm, double *d) {
-  std::vector<double> tmp((size_t)ncomp * count);
-  for (int r = 0; r < count; ++r) {
-    const int o = perm ? (*perm)[r] : r;
-    for (int q = 0; q < ncomp; ++q) tmp[(size_t)q * count + r] = h[(size_t)o * ld + q];
-  }
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  FVK_HIP(hipMemcpy(d, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice));
-  return 0;
+// reference-order entity-major host array <-> device rows (component-major)
+static int cells_in(Ctx &c, const double *h, int ncomp, double *d) { return c.io.put(h, ncomp, c.n, c.where, d, c.n); }
+static int cells_out(Ctx &c, const double *d, int ncomp, double *h) { return c.io.get(d, c.n, ncomp, c.n, c.where, h); }
+// res0(n_vol, n_vc), column-major
+static int cols_in(Ctx &c, const double *h, int nvc, double *d) {
+  return c.io.put(h, nvc, c.n, c.where, d, c.n, IO_COLUMN);
 }
-static int to_host(Ctx &c, const double *d, int ncomp, int ld, int count, const std::vector<int> *perm, double *h) {
-  std::vector<double> tmp((size_t)ncomp * count);
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  FVK_HIP(hipMemcpy(tmp.data(), d, tmp.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int r = 0; r < count; ++r) {
-    const int o = perm ? (*perm)[r] : r;
-    for (int q = 0; q < ncomp; ++q) h[(size_t)o * ld + q] = tmp[(size_t)q * count + r];
-  }
-  return 0;
+static int cols_out(Ctx &c, const double *d, int nvc, double *h) {
+  return c.io.get(d, c.n, nvc, c.n, c.where, h, IO_COLUMN);
+}
+// faces and boundary slots keep the reference's order
+static int plain_in(Ctx &c, const double *h, int ncomp, int count, double *d) {
+  return c.io.put(h, ncomp, count, nullptr, d, count);
+}
+static int plain_out(Ctx &c, const double *d, int ncomp, int count, double *h) {
+  return c.io.get(d, count, ncomp, count, nullptr, h);
 }
 
 __global__ __launch_bounds__(BS) void k_spv_from_faces(DMesh M, const double *ngp, const double *ngn, double *spv) {
@@ -666,10 +666,9 @@ int fvk_ctx_levels(const fvk_ctx *c, int *n_fwd, int *n_bwd) {
 int fvk_set_matrix(fvk_ctx *cc, const double *pl, const double *ng_p, const double *ng_n) {
   if (!cc || !pl || !ng_p || !ng_n) { set_error("null argument"); return FVK_ERR_ARG; }
   Ctx &c = cc->c;
-  GUARD(to_dev(c, pl, 1, 1, c.n, &c.perm, c.diag));
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  FVK_HIP(hipMemcpy(c.ngp, ng_p, sizeof(double) * c.nf, hipMemcpyHostToDevice));
-  FVK_HIP(hipMemcpy(c.ngn, ng_n, sizeof(double) * c.nf, hipMemcpyHostToDevice));
+  GUARD(cells_in(c, pl, 1, c.diag));
+  GUARD(plain_in(c, ng_p, 1, c.nf, c.ngp));
+  GUARD(plain_in(c, ng_n, 1, c.nf, c.ngn));
   k_spv_from_faces<<<grid_for(c.n), BS, 0, c.stream>>>(c.M, c.ngp, c.ngn, c.spv);
   FVK_HIP(hipGetLastError());
   matrix_changed(c);
@@ -679,19 +678,20 @@ int fvk_set_matrix(fvk_ctx *cc, const double *pl, const double *ng_p, const doub
 int fvk_solv_precond(fvk_ctx *cc, int imat, double *cv, double *c_r) {
   if (!cc || imat < 0 || imat > 2) { set_error("bad argument"); return FVK_ERR_ARG; }
   Ctx &c = cc->c;
+  IoCall call(c.io);
   GUARD(precond_build(c, imat));
   GUARD(sweep_status(c));
-  if (cv) GUARD(to_host(c, c.pc_c, 1, 1, c.n, &c.perm, cv));
-  if (c_r) GUARD(to_host(c, c.pc_cr, 1, 1, c.n, &c.perm, c_r));
-  return FVK_OK;
+  if (cv) GUARD(cells_out(c, c.pc_c, 1, cv));
+  if (c_r) GUARD(cells_out(c, c.pc_cr, 1, c_r));
+  return c.io.finish();
 }
 
 int fvk_solv_direct(fvk_ctx *cc, int imat, const double *cv, const double *c_r, const double *b, double *x) {
   if (!cc || !b || !x || imat < 0 || imat > 2 || (!cv) != (!c_r)) { set_error("bad argument"); return FVK_ERR_ARG; }
   Ctx &c = cc->c;
   if (cv) {
-    GUARD(to_dev(c, cv, 1, 1, c.n, &c.perm, c.pc_c));
-    GUARD(to_dev(c, c_r, 1, 1, c.n, &c.perm, c.pc_cr));
+    GUARD(cells_in(c, cv, 1, c.pc_c));
+    GUARD(cells_in(c, c_r, 1, c.pc_cr));
     c.pc_imat = imat;
     c.pc_valid = true;
     c.sw_fac = false;
@@ -699,41 +699,26 @@ int fvk_solv_direct(fvk_ctx *cc, int imat, const double *cv, const double *c_r, 
     GUARD(precond_build(c, imat));
   }
   double *db = wk_slot(c, 5), *dx = wk_slot(c, 6);
-  GUARD(to_dev(c, b, 1, 1, c.n, &c.perm, db));
+  IoCall call(c.io);
+  GUARD(cells_in(c, b, 1, db));
   GUARD(precond_apply(c, imat, 1, db, dx, nullptr));
   GUARD(sweep_status(c));
-  GUARD(to_host(c, dx, 1, 1, c.n, &c.perm, x));
-  return FVK_OK;
-}
-
-static int col_to_dev(Ctx &c, const double *res0, int nvc, double *d) {
-  // res0(n_vol, n_vc) column-major -> component-major rows
-  std::vector<double> tmp((size_t)nvc * c.n);
-  for (int q = 0; q < nvc; ++q)
-    for (int r = 0; r < c.n; ++r) tmp[(size_t)q * c.n + r] = res0[(size_t)q * c.n + c.perm[r]];
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  FVK_HIP(hipMemcpy(d, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice));
-  return 0;
-}
-static int col_to_host(Ctx &c, const double *d, int nvc, double *res0) {
-  std::vector<double> tmp((size_t)nvc * c.n);
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  FVK_HIP(hipMemcpy(tmp.data(), d, tmp.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int q = 0; q < nvc; ++q)
-    for (int r = 0; r < c.n; ++r) res0[(size_t)q * c.n + c.perm[r]] = tmp[(size_t)q * c.n + r];
-  return 0;
+  GUARD(cells_out(c, dx, 1, x));
+  return c.io.finish();
 }
 
 int fvk_solv_res(fvk_ctx *cc, int n_vc, const double *phi, double *res0, double *res0_n, int not_r0) {
   if (!cc || !res0 || !res0_n || n_vc < 1 || n_vc > 3 || (!not_r0 && !phi)) { set_error("bad argument"); return FVK_ERR_ARG; }
   Ctx &c = cc->c;
   double *dx = wk_slot(c, 5), *dr = wk_slot(c, 6);
-  if (!not_r0) GUARD(to_dev(c, phi, n_vc, n_vc, c.n, &c.perm, dx));
-  GUARD(col_to_dev(c, res0, n_vc, dr));
+  IoCall call(c.io);
+  if (!not_r0) GUARD(cells_in(c, phi, n_vc, dx));
+  GUARD(cols_in(c, res0, n_vc, dr));
   GUARD(residual(c, n_vc, dx, dr, not_r0 != 0));
-  GUARD(col_to_host(c, dr, n_vc, res0));
+  GUARD(cols_out(c, dr, n_vc, res0));
   KS h[3];
-  FVK_HIP(hipMemcpy(h, c.ks, sizeof h, hipMemcpyDeviceToHost));
+  GUARD(c.io.get_raw(c.ks, sizeof h, h));
+  GUARD(c.io.finish());
   for (int q = 0; q < n_vc; ++q) res0_n[q] = h[q].res0_n;
   return FVK_OK;
 }
@@ -757,15 +742,17 @@ static int solve_common(fvk_ctx *cc, int kind, int imat, double reduc, int n_ite
   }
   Ctx &c = cc->c;
   double *dx = wk_slot(c, 5), *dr = wk_slot(c, 6);
-  GUARD(to_dev(c, phi, n_vc, n_vc, c.n, &c.perm, dx));
-  GUARD(col_to_dev(c, res0, n_vc, dr));
+  IoCall call(c.io);
+  GUARD(cells_in(c, phi, n_vc, dx));
+  GUARD(cols_in(c, res0, n_vc, dr));
   FVK_HIP(hipEventRecord(c.ev0, c.stream));
   GUARD(krylov(c, kind, imat, reduc, n_iter, n_vc, dx, dr, not_r0 != 0));
   FVK_HIP(hipEventRecord(c.ev1, c.stream));
-  GUARD(to_host(c, dx, n_vc, n_vc, c.n, &c.perm, phi));
-  GUARD(col_to_host(c, dr, n_vc, res0));
+  GUARD(cells_out(c, dx, n_vc, phi));
+  GUARD(cols_out(c, dr, n_vc, res0));
   KS h[3];
-  FVK_HIP(hipMemcpy(h, c.ks, sizeof h, hipMemcpyDeviceToHost));
+  GUARD(c.io.get_raw(c.ks, sizeof h, h));
+  GUARD(c.io.finish());
   for (int q = 0; q < n_vc; ++q) res0_n[q] = h[q].res0_n;
   if (st) {
     std::memset(st, 0, sizeof *st);
@@ -795,18 +782,15 @@ int fvk_solv_grad(fvk_ctx *cc, int n_vc, const double *phi, double *gout, int n_
   if (!c.bnd_buf) GUARD(dalloc(c, &c.bnd_buf, (size_t)3 * std::max(nb, 1)));
   // g and g0 hold 3 n_vc x n doubles: three slots each
   double *dphi = wk_slot(c, 0), *dphib = c.bnd_buf, *g = wk_slot(c, 2), *g0 = wk_slot(c, 5);
-  GUARD(to_dev(c, phi, n_vc, n_vc, n, &c.perm, dphi));
-  if (nb) GUARD(to_dev(c, phi + (size_t)n * n_vc, n_vc, n_vc, nb, nullptr, dphib));
+  IoCall call(c.io);
+  GUARD(cells_in(c, phi, n_vc, dphi));
+  if (nb) GUARD(plain_in(c, phi + (size_t)n * n_vc, n_vc, nb, dphib));
   GUARD(grad(c, n_vc, dphi, dphib, g, n_iter, neu, nullptr, g0));
-  std::vector<double> tmp((size_t)9 * n);
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  FVK_HIP(hipMemcpy(tmp.data(), g, sizeof(double) * 3 * n_vc * n, hipMemcpyDeviceToHost));
-  for (int r = 0; r < n; ++r) {
-    const int o = c.perm[r];
-    for (int q = 0; q < n_vc; ++q)
-      for (int d = 0; d < nd; ++d) gout[((size_t)o * n_vc + q) * nd + d] = tmp[(size_t)(q * 3 + d) * n + r];
-  }
-  return FVK_OK;
+  int comp[9];
+  for (int q = 0; q < n_vc; ++q)
+    for (int d = 0; d < nd; ++d) comp[q * nd + d] = q * 3 + d;
+  GUARD(c.io.get(g, n, n_vc * nd, n, c.where, gout, IO_ENTITY, comp));
+  return c.io.finish();
 }
 
 // ---------------------------------------------------------------- systems
@@ -838,7 +822,7 @@ int fvk_sys_set(fvk_ctx *cc, const double *pl, const double *a, const double *b)
   std::vector<double> ng(c.nf);
   for (int f = 0; f < c.nf; ++f) ng[f] = -a[f];
   GUARD(fvk_set_matrix(cc, pl, ng.data(), ng.data()));
-  GUARD(to_dev(c, b, 1, 1, c.n, &c.perm, c.sys_b));
+  GUARD(cells_in(c, b, 1, c.sys_b));
   return FVK_OK;
 }
 
@@ -868,19 +852,21 @@ int fvk_sys_random(fvk_ctx *cc, uint64_t seed, double sigma, double *b_out) {
 
 int fvk_sys_get_x(fvk_ctx *cc, double *x) {
   if (!cc || !x || !cc->c.sys_x) { set_error("no system"); return FVK_ERR_STATE; }
-  return to_host(cc->c, cc->c.sys_x, 1, 1, cc->c.n, &cc->c.perm, x);
+  IoCall call(cc->c.io);
+  GUARD(cells_out(cc->c, cc->c.sys_x, 1, x));
+  return cc->c.io.finish();
 }
 
 int fvk_sys_get(fvk_ctx *cc, double *pl, double *a, double *b) {
   if (!cc || !cc->c.sys_b) { set_error("no system"); return FVK_ERR_STATE; }
   Ctx &c = cc->c;
-  if (pl) GUARD(to_host(c, c.diag, 1, 1, c.n, &c.perm, pl));
-  if (a) {
-    FVK_HIP(hipStreamSynchronize(c.stream));
-    FVK_HIP(hipMemcpy(a, c.ngp, sizeof(double) * c.nf, hipMemcpyDeviceToHost));
+  IoCall call(c.io);
+  if (pl) GUARD(cells_out(c, c.diag, 1, pl));
+  if (a) GUARD(plain_out(c, c.ngp, 1, c.nf, a));
+  if (b) GUARD(cells_out(c, c.sys_b, 1, b));
+  GUARD(c.io.finish());
+  if (a)
     for (int f = 0; f < c.nf; ++f) a[f] = -a[f];
-  }
-  if (b) GUARD(to_host(c, c.sys_b, 1, 1, c.n, &c.perm, b));
   return FVK_OK;
 }
 
@@ -1036,9 +1022,11 @@ int fvk_factor_apply(fvk_ctx *cc, const double *r, double *z) {
   Ctx &c = cc->c;
   GUARD(mix_build(c));
   double *dr = c.stage, *dz = c.stage + c.n;
-  GUARD(to_dev(c, r, 1, 1, c.n, &c.perm, dr));
+  IoCall call(c.io);
+  GUARD(cells_in(c, r, 1, dr));
   GUARD(factor_apply(c, dr, dz));
-  return to_host(c, dz, 1, 1, c.n, &c.perm, z);
+  GUARD(cells_out(c, dz, 1, z));
+  return c.io.finish();
 }
 
 int fvk_bench_spmv(fvk_ctx *cc, int reps, double *sec) {
@@ -1338,12 +1326,11 @@ int fvk_flow_set_state(fvk_flow *ff, const double *u_cell, const double *u_bnd, 
   if (!ff) return FVK_ERR_ARG;
   Flow &F = ff->f;
   Ctx &c = *F.c;
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  if (u_cell) GUARD(to_dev(c, u_cell, F.nvc, F.nvc, c.n, &c.perm, F.u));
-  if (u_bnd && c.nbf) GUARD(to_dev(c, u_bnd, F.nvc, F.nvc, c.nbf, nullptr, F.ub));
-  if (p) GUARD(to_dev(c, p, 1, 1, c.n, &c.perm, F.p));
-  if (dpdx) GUARD(to_dev(c, dpdx, c.ndx, c.ndx, c.n, &c.perm, F.dpdx));
-  if (spd) FVK_HIP(hipMemcpy(F.spd, spd, sizeof(double) * c.nf, hipMemcpyHostToDevice));
+  if (u_cell) GUARD(cells_in(c, u_cell, F.nvc, F.u));
+  if (u_bnd && c.nbf) GUARD(plain_in(c, u_bnd, F.nvc, c.nbf, F.ub));
+  if (p) GUARD(cells_in(c, p, 1, F.p));
+  if (dpdx) GUARD(cells_in(c, dpdx, c.ndx, F.dpdx));
+  if (spd) GUARD(plain_in(c, spd, 1, c.nf, F.spd));
   return FVK_OK;
 }
 
@@ -1352,38 +1339,43 @@ int fvk_flow_get_state(fvk_flow *ff, double *u_cell, double *u_bnd, double *p, d
   if (!ff) return FVK_ERR_ARG;
   Flow &F = ff->f;
   Ctx &c = *F.c;
-  if (u_cell) GUARD(to_host(c, F.u, F.nvc, F.nvc, c.n, &c.perm, u_cell));
-  if (u_bnd && c.nbf) GUARD(to_host(c, F.ub, F.nvc, F.nvc, c.nbf, nullptr, u_bnd));
-  if (p) GUARD(to_host(c, F.p, 1, 1, c.n, &c.perm, p));
-  if (dpdx) GUARD(to_host(c, F.dpdx, c.ndx, c.ndx, c.n, &c.perm, dpdx));
-  if (cs) GUARD(to_host(c, F.cs, 1, 1, c.n, &c.perm, cs));
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  if (spd) FVK_HIP(hipMemcpy(spd, F.spd, sizeof(double) * c.nf, hipMemcpyDeviceToHost));
-  if (frc_dns) FVK_HIP(hipMemcpy(frc_dns, F.frc_dns, sizeof(double) * c.nf, hipMemcpyDeviceToHost));
-  return FVK_OK;
+  IoCall call(c.io);
+  if (u_cell) GUARD(cells_out(c, F.u, F.nvc, u_cell));
+  if (u_bnd && c.nbf) GUARD(plain_out(c, F.ub, F.nvc, c.nbf, u_bnd));
+  if (p) GUARD(cells_out(c, F.p, 1, p));
+  if (dpdx) GUARD(cells_out(c, F.dpdx, c.ndx, dpdx));
+  if (cs) GUARD(cells_out(c, F.cs, 1, cs));
+  if (spd) GUARD(plain_out(c, F.spd, 1, c.nf, spd));
+  if (frc_dns) GUARD(plain_out(c, F.frc_dns, 1, c.nf, frc_dns));
+  return c.io.finish();
 }
 
 int fvk_flow_get_matrix(fvk_flow *ff, double *pl, double *ng_p, double *ng_n) {
   if (!ff) return FVK_ERR_ARG;
   Flow &F = ff->f;
   Ctx &c = *F.c;
-  if (pl) GUARD(to_host(c, c.diag, 1, 1, c.n, &c.perm, pl));
-  FVK_HIP(hipStreamSynchronize(c.stream));
-  if (ng_p) FVK_HIP(hipMemcpy(ng_p, c.ngp, sizeof(double) * c.nf, hipMemcpyDeviceToHost));
-  if (ng_n) FVK_HIP(hipMemcpy(ng_n, c.ngn, sizeof(double) * c.nf, hipMemcpyDeviceToHost));
-  return FVK_OK;
+  IoCall call(c.io);
+  if (pl) GUARD(cells_out(c, c.diag, 1, pl));
+  if (ng_p) GUARD(plain_out(c, c.ngp, 1, c.nf, ng_p));
+  if (ng_n) GUARD(plain_out(c, c.ngn, 1, c.nf, ng_n));
+  return c.io.finish();
 }
 
 int fvk_flow_get_rhs(fvk_flow *ff, double *rhs) {
   if (!ff || !rhs) { set_error("null argument"); return FVK_ERR_ARG; }
   Flow &F = ff->f;
-  return to_host(*F.c, F.rhs, 1, 1, F.c->n, &F.c->perm, rhs);
+  IoCall call(F.c->io);
+  GUARD(cells_out(*F.c, F.rhs, 1, rhs));
+  return F.c->io.finish();
 }
 
 static int read_hist(Flow &F, fvk_outer_hist *h) {
   FlowSc s;
-  FVK_HIP(hipStreamSynchronize(F.c->stream));
-  FVK_HIP(hipMemcpy(&s, F.sc, sizeof s, hipMemcpyDeviceToHost));
+  int failed = 0;
+  IoCall call(F.c->io);
+  GUARD(F.c->io.get_raw(F.sc, sizeof s, &s));
+  GUARD(F.c->io.get_raw(F.c->sweep_int + 3, sizeof failed, &failed));
+  GUARD(F.c->io.finish());
   if (h) {
     h->reduc = s.h_reduc; h->redpp = s.h_redpp; h->redpp_sum = s.h_redpp_sum;
     h->red_p = s.h_red_p; h->red_p_sum = s.h_red_p_sum; h->mx_res_n = s.mx_res_n;
@@ -1394,7 +1386,7 @@ static int read_hist(Flow &F, fvk_outer_hist *h) {
     h->res0_n_p = s.res0_n_p;
   }
   if (s.diverged) { set_error("momentum residual exceeded large"); return FVK_ERR_DIVERGED; }
-  return sweep_status(*F.c);
+  return failed ? sweep_status(*F.c) : FVK_OK;
 }
 
 int fvk_flow_setup_eqn(fvk_flow *ff, int it, fvk_outer_hist *h) {

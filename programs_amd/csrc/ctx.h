@@ -9,6 +9,7 @@
 
 #include "../../include/fvk.h"
 #include "dev.h"
+#include "hostio.h"
 #include "sweepexec.h"
 
 namespace fvk {
@@ -83,6 +84,8 @@ struct Ctx {
   int n = 0, nf = 0, nbf = 0, W = 0, Ws = 0, ndx = 0;
   std::vector<int> perm, iperm;  // perm[row] = reference cell (0-based)
   std::vector<int> h_fip, h_fin, h_fib, h_fbty;  // rows
+  HostIo io;
+  int *where = nullptr;           // device: row of each reference cell (null: the same)
   DMesh M{};
   std::vector<void *> owned;      // device allocations freed at destroy
   // matrix on the device

@@ -684,8 +684,10 @@ int mom_setup(Flow &F, int it, bool &skipped) {
   // non-zero boundary values it is never taken again
   if (!F.capture) {
     double mx[2];
-    FVK_HIP(hipMemcpyAsync(mx, &F.sc->phi_mx_cell, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    FVK_HIP(hipStreamSynchronize(c.stream));
+    IoCall call(c.io);
+    int rc = c.io.get_raw(&F.sc->phi_mx_cell, sizeof mx, mx);
+    if (!rc) rc = c.io.finish();
+    if (rc) return rc;
     if (mx[1] < SMALL) {
       if (fill(c, c.diag, n, 0.0) || fill(c, F.cs, n, 0.0)) return FVK_ERR_HIP;
       skipped = true;

@@ -37,6 +37,7 @@ struct FlCtx {
   hipStream_t stream = nullptr;
   int nd = 0, n = 0, nb = 0, nf = 0, nnz = 0, n_vrt = 0;
   std::vector<void *> owned;
+  HostIo io;
   std::vector<int> h_ia, h_ja, h_j1, h_jn, h_btag;
   // geometry
   double *xvc = nullptr, *vol = nullptr, *volr = nullptr, *ls = nullptr;
@@ -68,6 +69,11 @@ struct FlCtx {
   double *wk = nullptr, *pc = nullptr, *part = nullptr;
   FlKS *ks = nullptr;
   double *scal = nullptr;  // c_rat and scratch scalars
+  // workspaces of the calls on host arrays, kept once made: matrix values,
+  // solution and right-hand side; boundary values and boundary faces
+  double *lin = nullptr, *bval = nullptr;
+  int *bfl = nullptr;
+  int n_bf = 0;
 };
 
 // zeroed allocation; the clear has finished when this returns (an upload
@@ -1439,27 +1445,14 @@ static void fl_ctx_free(FlCtx &c) {
   for (void *p : c.owned) hipFree(p);
   c.owned.clear();
   sweep_exec_free(c.sw);
+  c.io.free();
   if (c.stream) hipStreamDestroy(c.stream);
   c.stream = nullptr;
 }
 
 // device (component-major, SoA) <-> Fortran column-major a(ncmp, m)
-static int fl_to_dev(hipStream_t s, const double *h, int ncmp, int m, double *d) {
-  std::vector<double> t((size_t)ncmp * m);
-  for (int i = 0; i < m; ++i)
-    for (int q = 0; q < ncmp; ++q) t[(size_t)q * m + i] = h[(size_t)i * ncmp + q];
-  FVK_HIP(hipStreamSynchronize(s));
-  FVK_HIP(hipMemcpy(d, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-  return 0;
-}
-static int fl_to_host(hipStream_t s, const double *d, int ncmp, int m, double *h) {
-  std::vector<double> t((size_t)ncmp * m);
-  FVK_HIP(hipStreamSynchronize(s));
-  FVK_HIP(hipMemcpy(t.data(), d, t.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int i = 0; i < m; ++i)
-    for (int q = 0; q < ncmp; ++q) h[(size_t)i * ncmp + q] = t[(size_t)q * m + i];
-  return 0;
-}
+static int fl_in(FlCtx &c, const double *h, int ncmp, int m, double *d) { return c.io.put(h, ncmp, m, nullptr, d, m); }
+static int fl_out(FlCtx &c, const double *d, int ncmp, int m, double *h) { return c.io.get(d, m, ncmp, m, nullptr, h); }
 
 static int ff_build(FlFlow &F) {
   FlCtx &c = *F.c;
@@ -1540,8 +1533,10 @@ static int ff_construct_pde(FlFlow &F) {
 // bound (its results are then invalid)
 static int fl_sweep_status(FlCtx &c) {
   int e = 0;
-  FVK_HIP(hipMemcpyAsync(&e, c.sweep_int + 3, sizeof e, hipMemcpyDeviceToHost, c.stream));
-  FVK_HIP(hipStreamSynchronize(c.stream));
+  IoCall call(c.io);
+  int rc = c.io.get_raw(c.sweep_int + 3, sizeof e, &e);
+  if (!rc) rc = c.io.finish();
+  if (rc) return rc;
   if (e) {
     set_error("triangular sweep: a wait exceeded its bound; the preconditioner's results are invalid");
     return FVK_ERR_HIP;
@@ -1554,10 +1549,13 @@ static int ff_solve(FlFlow &F, int isol, int ncmp, double *phi, double *rhs, int
   int rc = fl_solve(c, isol, ncmp, F.val, phi, rhs, n_iter, reduc);
   if (rc) return rc;
   FlKS k[3];
-  FVK_HIP(hipMemcpyAsync(k, c.ks, sizeof(FlKS) * ncmp, hipMemcpyDeviceToHost, c.stream));
-  FVK_HIP(hipStreamSynchronize(c.stream));
+  int failed = 0;
+  IoCall call(c.io);
+  if ((rc = c.io.get_raw(c.ks, sizeof(FlKS) * ncmp, k)) ||
+      (rc = c.io.get_raw(c.sweep_int + 3, sizeof failed, &failed)) || (rc = c.io.finish()))
+    return rc;
   for (int q = 0; q < ncmp; ++q) res0[q] = k[q].norm;
-  return fl_sweep_status(c);
+  return failed ? fl_sweep_status(c) : 0;
 }
 
 static int ff_construct_pp(FlFlow &F) {
@@ -1695,6 +1693,7 @@ int fvk_fl_ctx_create(int n_dim, int n_vrt, const double *x3, int n_bnd, const i
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking);
   if (e != hipSuccess) { delete cc; set_error(hipGetErrorString(e)); return FVK_ERR_HIP; }
+  c.io.stream = c.stream;
   const int rc = fl_ctx_build(c, n_dim, n_vrt, x3, n_bnd, bnd_tag, n_dmn, elm_vptr, elm_vrt, n_fce, fce_elm, fce_vptr,
                               fce_vrt, ng_ptr, ng_col);
   if (rc) { fl_ctx_free(c); delete cc; return rc; }
@@ -1710,6 +1709,7 @@ int fvk_fl_csr_create(int n, const int *ia, const int *ja, int device, fvk_fl_ct
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking);
   if (e != hipSuccess) { delete cc; set_error(hipGetErrorString(e)); return FVK_ERR_HIP; }
+  c.io.stream = c.stream;
   const int rc = fl_csr_setup(c, n, ia, ja);
   if (rc) { fl_ctx_free(c); delete cc; return rc; }
   *out = cc;
@@ -1755,17 +1755,18 @@ int fvk_fl_geometry(fvk_fl_ctx *cc, double *x_vc, double *vol, double *x_fc, dou
   FlCtx &c = cc->c;
   const int nd = c.nd;
   int rc = 0;
-  if (x_vc && (rc = fl_to_host(c.stream, c.xvc, nd, c.n, x_vc))) return rc;
-  if (vol && (rc = fl_to_host(c.stream, c.vol, 1, c.n, vol))) return rc;
-  if (x_fc && (rc = fl_to_host(c.stream, c.xfc, nd, c.nf, x_fc))) return rc;
-  if (norm && (rc = fl_to_host(c.stream, c.nrm, nd, c.nf, norm))) return rc;
-  if (area && (rc = fl_to_host(c.stream, c.area, 1, c.nf, area))) return rc;
-  if (x_pc && (rc = fl_to_host(c.stream, c.xpc, nd, c.nf, x_pc))) return rc;
-  if (x_nc && (rc = fl_to_host(c.stream, c.xnc, nd, c.nf, x_nc))) return rc;
-  if (l_pn && (rc = fl_to_host(c.stream, c.lpn, 1, c.nf, l_pn))) return rc;
-  if (w_fp && (rc = fl_to_host(c.stream, c.wfp, 1, c.nf, w_fp))) return rc;
-  if (ls && (rc = fl_to_host(c.stream, c.ls, nd * nd, c.n, ls))) return rc;
-  return FVK_OK;
+  IoCall call(c.io);
+  if (x_vc && (rc = fl_out(c, c.xvc, nd, c.n, x_vc))) return rc;
+  if (vol && (rc = fl_out(c, c.vol, 1, c.n, vol))) return rc;
+  if (x_fc && (rc = fl_out(c, c.xfc, nd, c.nf, x_fc))) return rc;
+  if (norm && (rc = fl_out(c, c.nrm, nd, c.nf, norm))) return rc;
+  if (area && (rc = fl_out(c, c.area, 1, c.nf, area))) return rc;
+  if (x_pc && (rc = fl_out(c, c.xpc, nd, c.nf, x_pc))) return rc;
+  if (x_nc && (rc = fl_out(c, c.xnc, nd, c.nf, x_nc))) return rc;
+  if (l_pn && (rc = fl_out(c, c.lpn, 1, c.nf, l_pn))) return rc;
+  if (w_fp && (rc = fl_out(c, c.wfp, 1, c.nf, w_fp))) return rc;
+  if (ls && (rc = fl_out(c, c.ls, nd * nd, c.n, ls))) return rc;
+  return c.io.finish();
 }
 
 int fvk_fl_ls_gradient(fvk_fl_ctx *cc, int n_cmp, const double *phi, double *phi_bnd, double *grad, int neu_bnd) {
@@ -1774,30 +1775,23 @@ int fvk_fl_ls_gradient(fvk_fl_ctx *cc, int n_cmp, const double *phi, double *phi
     return FVK_ERR_ARG;
   }
   FlCtx &c = cc->c;
-  double *d = wkv(c, 0), *db = nullptr, *dg = wkv(c, 2);
-  void *q = nullptr;
-  FVK_HIP(hipMalloc(&q, sizeof(double) * 3 * (size_t)std::max(c.nb, 1)));
-  db = (double *)q;
-  std::vector<int> bfl;
-  for (int f = 0; f < c.nf; ++f)
-    if (c.h_jn[f] < 0) bfl.push_back(f);
-  int *dbfl = nullptr;
+  double *d = wkv(c, 0), *dg = wkv(c, 2);
   int rc = 0;
-  if (hipMalloc(&q, sizeof(int) * std::max<size_t>(bfl.size(), 1)) != hipSuccess) {
-    hipFree(db);
-    set_error("hipMalloc failed");
-    return FVK_ERR_HIP;
+  if (!c.bval) {
+    std::vector<int> bfl;
+    for (int f = 0; f < c.nf; ++f)
+      if (c.h_jn[f] < 0) bfl.push_back(f);
+    c.n_bf = (int)bfl.size();
+    if ((rc = fl_up(c, &c.bfl, bfl))) return rc;
+    if ((rc = fl_alloc(c, &c.bval, (size_t)3 * std::max(c.nb, 1)))) return rc;
   }
-  dbfl = (int *)q;
-  if (!bfl.empty()) hipMemcpy(dbfl, bfl.data(), bfl.size() * sizeof(int), hipMemcpyHostToDevice);
-  if (!rc) rc = fl_to_dev(c.stream, phi, n_cmp, c.n, d);
-  if (!rc && c.nb) rc = fl_to_dev(c.stream, phi_bnd, n_cmp, c.nb, db);
-  if (!rc) rc = fl_grad(c, n_cmp, d, db, dg, neu_bnd, dbfl, (int)bfl.size());
-  if (!rc) rc = fl_to_host(c.stream, dg, c.nd * n_cmp, c.n, grad);
-  if (!rc && neu_bnd && c.nb) rc = fl_to_host(c.stream, db, n_cmp, c.nb, phi_bnd);
-  hipFree(dbfl);
-  hipFree(db);
-  return rc;
+  IoCall call(c.io);
+  if ((rc = fl_in(c, phi, n_cmp, c.n, d))) return rc;
+  if (c.nb && (rc = fl_in(c, phi_bnd, n_cmp, c.nb, c.bval))) return rc;
+  if ((rc = fl_grad(c, n_cmp, d, c.bval, dg, neu_bnd, c.bfl, c.n_bf))) return rc;
+  if ((rc = fl_out(c, dg, c.nd * n_cmp, c.n, grad))) return rc;
+  if (neu_bnd && c.nb && (rc = fl_out(c, c.bval, n_cmp, c.nb, phi_bnd))) return rc;
+  return c.io.finish();
 }
 
 int fvk_fl_lin_eqns_solver(fvk_fl_ctx *cc, const double *a_ij, double *phi, double *rhs, double *norm, int n_iter,
@@ -1807,26 +1801,20 @@ int fvk_fl_lin_eqns_solver(fvk_fl_ctx *cc, const double *a_ij, double *phi, doub
     return FVK_ERR_ARG;
   }
   FlCtx &c = cc->c;
-  void *q = nullptr;
-  FVK_HIP(hipMalloc(&q, sizeof(double) * ((size_t)c.nnz + 2 * (size_t)c.n)));
-  double *da = (double *)q, *dphi = da + c.nnz, *drhs = dphi + c.n;
-  hipError_t e = hipStreamSynchronize(c.stream);
-  if (e == hipSuccess) e = hipMemcpy(da, a_ij, sizeof(double) * c.nnz, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(dphi, phi, sizeof(double) * c.n, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(drhs, rhs, sizeof(double) * c.n, hipMemcpyHostToDevice);
-  int rc = e == hipSuccess ? fl_solve(c, isol, 1, da, dphi, drhs, n_iter, reduc) : FVK_ERR_HIP;
-  if (e != hipSuccess) set_error(hipGetErrorString(e));
+  int rc = 0;
+  if (!c.lin && (rc = fl_alloc(c, &c.lin, (size_t)c.nnz + 2 * (size_t)c.n))) return rc;
+  double *da = c.lin, *dphi = da + c.nnz, *drhs = dphi + c.n;
+  IoCall call(c.io);
+  if ((rc = fl_in(c, a_ij, 1, c.nnz, da)) || (rc = fl_in(c, phi, 1, c.n, dphi)) || (rc = fl_in(c, rhs, 1, c.n, drhs)))
+    return rc;
+  if ((rc = fl_solve(c, isol, 1, da, dphi, drhs, n_iter, reduc))) return rc;
   FlKS k;
-  if (!rc) {
-    e = hipMemcpyAsync(&k, c.ks, sizeof k, hipMemcpyDeviceToHost, c.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
-    if (e == hipSuccess) e = hipMemcpy(phi, dphi, sizeof(double) * c.n, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(rhs, drhs, sizeof(double) * c.n, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) { set_error(hipGetErrorString(e)); rc = FVK_ERR_HIP; }
-    else *norm = k.norm;
-  }
-  hipFree(q);
-  return rc ? rc : fl_sweep_status(c);
+  int failed = 0;
+  if ((rc = fl_out(c, dphi, 1, c.n, phi)) || (rc = fl_out(c, drhs, 1, c.n, rhs))) return rc;
+  if ((rc = c.io.get_raw(c.ks, sizeof k, &k)) || (rc = c.io.get_raw(c.sweep_int + 3, sizeof failed, &failed))) return rc;
+  if ((rc = c.io.finish())) return rc;
+  *norm = k.norm;
+  return failed ? fl_sweep_status(c) : FVK_OK;
 }
 
 int fvk_fl_ctx_set_param(fvk_fl_ctx *cc, const char *name, double value) {
@@ -1898,10 +1886,10 @@ int fvk_fl_flow_set(fvk_fl_flow *ff, const double *vel, const double *vel_bnd, c
   FlFlow &F = ff->f;
   FlCtx &c = *F.c;
   int rc = 0;
-  if (vel && (rc = fl_to_dev(c.stream, vel, c.nd, c.n, F.u))) return rc;
-  if (vel_bnd && c.nb && (rc = fl_to_dev(c.stream, vel_bnd, c.nd, c.nb, F.ub))) return rc;
-  if (pres && (rc = fl_to_dev(c.stream, pres, 1, c.n, F.p))) return rc;
-  if (pres_bnd && c.nb && (rc = fl_to_dev(c.stream, pres_bnd, 1, c.nb, F.pb))) return rc;
+  if (vel && (rc = fl_in(c, vel, c.nd, c.n, F.u))) return rc;
+  if (vel_bnd && c.nb && (rc = fl_in(c, vel_bnd, c.nd, c.nb, F.ub))) return rc;
+  if (pres && (rc = fl_in(c, pres, 1, c.n, F.p))) return rc;
+  if (pres_bnd && c.nb && (rc = fl_in(c, pres_bnd, 1, c.nb, F.pb))) return rc;
   return FVK_OK;
 }
 
@@ -1911,13 +1899,14 @@ int fvk_fl_flow_get(fvk_fl_flow *ff, double *vel, double *vel_bnd, double *pres,
   FlFlow &F = ff->f;
   FlCtx &c = *F.c;
   int rc = 0;
-  if (vel && (rc = fl_to_host(c.stream, F.u, c.nd, c.n, vel))) return rc;
-  if (vel_bnd && c.nb && (rc = fl_to_host(c.stream, F.ub, c.nd, c.nb, vel_bnd))) return rc;
-  if (pres && (rc = fl_to_host(c.stream, F.p, 1, c.n, pres))) return rc;
-  if (pres_bnd && c.nb && (rc = fl_to_host(c.stream, F.pb, 1, c.nb, pres_bnd))) return rc;
-  if (pp && (rc = fl_to_host(c.stream, F.q, 1, c.n, pp))) return rc;
-  if (spd && (rc = fl_to_host(c.stream, F.spd, 1, c.nf, spd))) return rc;
-  return FVK_OK;
+  IoCall call(c.io);
+  if (vel && (rc = fl_out(c, F.u, c.nd, c.n, vel))) return rc;
+  if (vel_bnd && c.nb && (rc = fl_out(c, F.ub, c.nd, c.nb, vel_bnd))) return rc;
+  if (pres && (rc = fl_out(c, F.p, 1, c.n, pres))) return rc;
+  if (pres_bnd && c.nb && (rc = fl_out(c, F.pb, 1, c.nb, pres_bnd))) return rc;
+  if (pp && (rc = fl_out(c, F.q, 1, c.n, pp))) return rc;
+  if (spd && (rc = fl_out(c, F.spd, 1, c.nf, spd))) return rc;
+  return c.io.finish();
 }
 
 // intermediate arrays of the current iteration: the matrix values (nnz),
@@ -1929,17 +1918,15 @@ int fvk_fl_flow_get_system(fvk_fl_flow *ff, double *val, double *rhs, double *di
   FlFlow &F = ff->f;
   FlCtx &c = *F.c;
   int rc = 0;
-  if (val) {
-    FVK_HIP(hipStreamSynchronize(c.stream));
-    FVK_HIP(hipMemcpy(val, F.val, sizeof(double) * c.nnz, hipMemcpyDeviceToHost));
-  }
-  if (rhs && (rc = fl_to_host(c.stream, F.rhs, c.nd, c.n, rhs))) return rc;
-  if (diag && (rc = fl_to_host(c.stream, F.diag, 1, c.n, diag))) return rc;
-  if (vel_grad && (rc = fl_to_host(c.stream, F.ug, c.nd * c.nd, c.n, vel_grad))) return rc;
-  if (pres_grad && (rc = fl_to_host(c.stream, F.pg, c.nd, c.n, pres_grad))) return rc;
-  if (pp_grad && (rc = fl_to_host(c.stream, F.qg, c.nd, c.n, pp_grad))) return rc;
-  if (pp_bnd && c.nb && (rc = fl_to_host(c.stream, F.qb, 1, c.nb, pp_bnd))) return rc;
-  return FVK_OK;
+  IoCall call(c.io);
+  if (val && (rc = fl_out(c, F.val, 1, c.nnz, val))) return rc;
+  if (rhs && (rc = fl_out(c, F.rhs, c.nd, c.n, rhs))) return rc;
+  if (diag && (rc = fl_out(c, F.diag, 1, c.n, diag))) return rc;
+  if (vel_grad && (rc = fl_out(c, F.ug, c.nd * c.nd, c.n, vel_grad))) return rc;
+  if (pres_grad && (rc = fl_out(c, F.pg, c.nd, c.n, pres_grad))) return rc;
+  if (pp_grad && (rc = fl_out(c, F.qg, c.nd, c.n, pp_grad))) return rc;
+  if (pp_bnd && c.nb && (rc = fl_out(c, F.qb, 1, c.nb, pp_bnd))) return rc;
+  return c.io.finish();
 }
 
 // One step of navierstokes' outer loop, by name of the reference routine

@@ -989,8 +989,10 @@ int residual_to(Ctx &c, int nvc, const double *x, double *r, bool not_r0, double
 int sweep_status(Ctx &c) {
   if (!c.sweep_int) return 0;
   int e = 0;
-  FVK_HIP(hipMemcpyAsync(&e, c.sweep_int + 3, sizeof e, hipMemcpyDeviceToHost, c.stream));
-  FVK_HIP(hipStreamSynchronize(c.stream));
+  IoCall call(c.io);
+  int rc = c.io.get_raw(c.sweep_int + 3, sizeof e, &e);
+  if (!rc) rc = c.io.finish();
+  if (rc) return rc;
   if (e) {
     set_error("triangular sweep: a wait exceeded its bound; the preconditioner's results are invalid");
     return FVK_ERR_HIP;
