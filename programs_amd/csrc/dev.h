@@ -229,15 +229,22 @@ __device__ __forceinline__ int xcd_block() {
   return b < per * kXcd ? (b % kXcd) * per + b / kXcd : b;
 }
 
-// The FP64 Krylov kernels (krylov.hip) run 1024-thread blocks, at most 512
-// of them: measured 2.6 % faster than 512 x 512 on the plain FP64 solve, and
-// 4.5 % slower on the FP32 inner solve, which keeps RB.
+// The FP64 Krylov kernels (krylov.hip): blocks of TB64 threads up to
+// kSmall64 rows, where blocks of RB64 would leave compute units without one
+// and a launch lasts as long as one block (48^3, per CG iteration with the
+// gaps: 22.8 us with RB64, 10.7 us with TB64); above, RB64 threads and at
+// most RG64 blocks (2.6 % faster than 512 x 512 on the plain FP64 solve at
+// 128^3).
 constexpr int RB64 = 1024;
 constexpr int RG64 = 512;
+constexpr int TB64 = 256;
+constexpr int kSmall64 = 512 * 1024;
+inline bool small64(int n) { return n <= kSmall64; }
 inline int red_grid64(int n) {
-  int g = (n + RB64 - 1) / RB64;
+  const int tb = small64(n) ? TB64 : RB64, most = small64(n) ? RG : RG64;
+  int g = (n + tb - 1) / tb;
   if (g < 1) g = 1;
-  if (g > RG64) g = RG64;
+  if (g > most) g = most;
   if (g >= 16) g = g / 8 * 8;
   return g;
 }

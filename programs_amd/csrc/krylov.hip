@@ -335,8 +335,8 @@ __global__ __launch_bounds__(BS) void k_spmv(DMesh M, int nvc, const double *__r
 // r = b - A x (or r = b) with partials {|r|_1[q], s2[q]} where s2 = r.(c r)
 // and z = c r (mode 1, Jacobi PCG), s2 = r.r (mode 2, BiCGStab) or 0.
 // (solv_res.f90; solv_cg.f90:19-33; solv_bicg.f90:19-38)
-template <int WS>
-__global__ __launch_bounds__(RB64) void k_residual(DMesh M, int nvc, const double *__restrict__ diag,
+template <int WS, int TB>
+__global__ __launch_bounds__(TB) void k_residual(DMesh M, int nvc, const double *__restrict__ diag,
                                                  const double *__restrict__ spv, const double *__restrict__ x,
                                                  double *__restrict__ r, int not_r0, int mode,
                                                  const double *__restrict__ c, double *__restrict__ z,
@@ -344,8 +344,8 @@ __global__ __launch_bounds__(RB64) void k_residual(DMesh M, int nvc, const doubl
   const int n = M.n;
   double a[6] = {0, 0, 0, 0, 0, 0};
   int r0, r1;
-  block_rows<RB64>(n, r0, r1);
-  for (int i = r0 + threadIdx.x; i < r1; i += RB64)
+  block_rows<TB>(n, r0, r1);
+  for (int i = r0 + threadIdx.x; i < r1; i += TB)
     for (int q = 0; q < nvc; ++q) {
       double v = r[q * n + i];
       if (!not_r0) {
@@ -368,19 +368,18 @@ __global__ __launch_bounds__(RB64) void k_residual(DMesh M, int nvc, const doubl
         a[3 + q] += v * v;
       }
     }
-  store_partials<6, RB64>(a, part);
+  store_partials<6, TB>(a, part);
 }
 
 // Decide iteration it, then p = z + beta p ; q = A p ; partial p.q.  p of the
 // neighbours is formed on the fly from (z, p_old): p_new is written once.
 // Each thread takes two rows per pass so that both rows' loads are in flight
 // together.
-template <int NVC, int WS>
+template <int WS>
 __device__ __forceinline__ void cg_pq_row(const DMesh &M, int i, const double *__restrict__ diag,
                                           const double *__restrict__ spv, const double *__restrict__ zq,
                                           const double *__restrict__ po, double beta, double *__restrict__ pn,
                                           double *__restrict__ qq, double &pq) {
-  const int n = M.n;
   const double pi = zq[i] + beta * po[i];
   double y = diag[i] * pi;
 #pragma unroll
@@ -394,23 +393,71 @@ __device__ __forceinline__ void cg_pq_row(const DMesh &M, int i, const double *_
   pq += pi * y;
 }
 
-template <int NVC, int WS>
-__global__ __launch_bounds__(RB64) void k_cg_pq(DMesh M, int it, const double *__restrict__ diag,
+// The same row in two halves: its loads do not depend on beta, so a thread's
+// first row is loaded before the partials are reduced.  A block of a small
+// system runs one row a thread and lasts as long as its dependent loads: with
+// the smaller blocks, 13.3 -> 6.1 us at 48^3 (k_cg_upd likewise, 9 -> 5 us).
+template <int WS>
+struct CgRow {
+  double z, po, d, a[WS > 0 ? WS : 1], zj[WS > 0 ? WS : 1], pj[WS > 0 ? WS : 1];
+  unsigned has;
+  __device__ __forceinline__ void load(const DMesh &M, int i, const double *__restrict__ diag,
+                                       const double *__restrict__ spv, const double *__restrict__ zq,
+                                       const double *__restrict__ pold) {
+    z = zq[i];
+    po = pold[i];
+    d = diag[i];
+    has = 0;
+#pragma unroll
+    for (int k = 0; k < WS; ++k) {
+      const int j = M.spc[(size_t)k * M.ld + i];
+      a[k] = spv[(size_t)k * M.ld + i];
+      const int jj = j >= 0 ? j : i;
+      zj[k] = zq[jj];
+      pj[k] = pold[jj];
+      has |= j >= 0 ? 1u << k : 0u;
+    }
+  }
+  __device__ __forceinline__ void finish(int i, double beta, double *__restrict__ pn, double *__restrict__ qq,
+                                         double &pq) const {
+    const double pi = z + beta * po;
+    double y = d * pi;
+#pragma unroll
+    for (int k = 0; k < WS; ++k) {
+      const double t = y + a[k] * (zj[k] + beta * pj[k]);
+      y = (has >> k) & 1u ? t : y;
+    }
+    pn[i] = pi;
+    qq[i] = y;
+    pq += pi * y;
+  }
+};
+
+// partR: r.z of DIC / DILU (null: Jacobi's, with |r|_1 in partU)
+template <int NVC, int WS, int TB>
+__global__ __launch_bounds__(TB) void k_cg_pq(DMesh M, int it, const double *__restrict__ diag,
                                               const double *__restrict__ spv, const double *__restrict__ z,
                                               const double *__restrict__ pold, double *__restrict__ pnew,
-                                              double *__restrict__ qv, const double *__restrict__ partU, int PU,
-                                              const double *__restrict__ partR, int PR, double *__restrict__ partQ,
-                                              KS *ring, KS *out) {
+                                              double *__restrict__ qv, const double *__restrict__ partU, int P,
+                                              const double *__restrict__ partR, double *__restrict__ partQ, KS *ring,
+                                              KS *out) {
+  const int n = M.n;
+  int r0, r1;
+  block_rows<TB>(n, r0, r1);
+  int i = r0 + threadIdx.x;
+  constexpr bool ahead = NVC == 1 && WS > 0 && TB == TB64;
+  CgRow<WS> first;
+  if (ahead && i < r1) first.load(M, i, diag, spv, z, pold);
   // |r|_1 (components 0..NVC) and, for Jacobi, r.z (components 3..3+NVC)
   double L1[NVC], rz[NVC];
   if (partR) {
-    load_totals<NVC, RB64>(partU, PU, L1);
-    load_totals<NVC, RB64>(partR, PR, rz);
+    load_totals<NVC, TB>(partU, P, L1);
+    load_totals<NVC, TB>(partR, P, rz);
   } else {
     int cs[2 * NVC];
     double t[2 * NVC];
     for (int q = 0; q < NVC; ++q) { cs[q] = q; cs[NVC + q] = 3 + q; }
-    load_sel<2 * NVC, RB64>(partU, PU, cs, t);
+    load_sel<2 * NVC, TB>(partU, P, cs, t);
     for (int q = 0; q < NVC; ++q) { L1[q] = t[q]; rz[q] = t[NVC + q]; }
   }
   __shared__ KS sk[3];
@@ -429,44 +476,57 @@ __global__ __launch_bounds__(RB64) void k_cg_pq(DMesh M, int it, const double *_
     any = any || !dn[q];
   }
   if (!any) return;
-  const int n = M.n;
   double pq[NVC];
   for (int q = 0; q < NVC; ++q) pq[q] = 0.0;
-  int r0, r1;
-  block_rows<RB64>(n, r0, r1);
-  int i = r0 + threadIdx.x;
-  for (; i + RB64 < r1; i += 2 * RB64)
+  if (ahead) {
+    if (i < r1) first.finish(i, beta[0], pnew, qv, pq[0]);
+    i += TB;
+  }
+  for (; i + TB < r1; i += 2 * TB)
 #pragma unroll
     for (int q = 0; q < NVC; ++q) {
       if (dn[q]) continue;
       const double *zq = z + q * n, *po = pold + q * n;
       double *pn = pnew + q * n, *qq = qv + q * n;
-      cg_pq_row<NVC, WS>(M, i, diag, spv, zq, po, beta[q], pn, qq, pq[q]);
-      cg_pq_row<NVC, WS>(M, i + RB64, diag, spv, zq, po, beta[q], pn, qq, pq[q]);
+      cg_pq_row<WS>(M, i, diag, spv, zq, po, beta[q], pn, qq, pq[q]);
+      cg_pq_row<WS>(M, i + TB, diag, spv, zq, po, beta[q], pn, qq, pq[q]);
     }
   if (i < r1)
 #pragma unroll
     for (int q = 0; q < NVC; ++q) {
       if (dn[q]) continue;
-      cg_pq_row<NVC, WS>(M, i, diag, spv, z + q * n, pold + q * n, beta[q], pnew + q * n, qv + q * n, pq[q]);
+      cg_pq_row<WS>(M, i, diag, spv, z + q * n, pold + q * n, beta[q], pnew + q * n, qv + q * n, pq[q]);
     }
-  store_partials<NVC, RB64>(pq, partQ);
+  store_partials<NVC, TB>(pq, partQ);
 }
 
 // alpha = s/(p.q + small) ; x += alpha p ; r -= alpha q ; partials |r|_1 and
 // (Jacobi) r.z with z = c r.
-template <int NVC>
-__global__ __launch_bounds__(RB64) void k_cg_upd(int n, int it, double *__restrict__ x, double *__restrict__ r,
+template <int NVC, int TB>
+__global__ __launch_bounds__(TB) void k_cg_upd(int n, int it, double *__restrict__ x, double *__restrict__ r,
                                                const double *__restrict__ p, const double *__restrict__ qv,
                                                const double *__restrict__ c, int jacobi, double *__restrict__ z,
                                                const double *__restrict__ partQ, int PQ, double *__restrict__ partU,
                                                KS *ring) {
+  int r0, r1;
+  block_rows<TB>(n, r0, r1);
+  int i = r0 + threadIdx.x;
+  // the first row's loads before the partials are reduced
+  constexpr bool ahead = NVC == 1 && TB == TB64;
+  double x0 = 0.0, p0 = 0.0, ri0 = 0.0, q0 = 0.0, c0 = 0.0;
+  if (ahead && i < r1) {
+    x0 = x[i];
+    p0 = p[i];
+    ri0 = r[i];
+    q0 = qv[i];
+    if (jacobi) c0 = c[i];
+  }
   const KS *cur = ring + (it & 1) * 3;
   bool any = false;
   for (int q = 0; q < NVC; ++q) any = any || !cur[q].done;
   if (!any) return;
   double t[NVC];
-  load_totals<NVC, RB64>(partQ, PQ, t);
+  load_totals<NVC, TB>(partQ, PQ, t);
   double alpha[NVC];
   int dn[NVC];
   for (int q = 0; q < NVC; ++q) {
@@ -474,52 +534,54 @@ __global__ __launch_bounds__(RB64) void k_cg_upd(int n, int it, double *__restri
     alpha[q] = cur[q].s / (t[q] + SMALL);
   }
   double a[6] = {0, 0, 0, 0, 0, 0};
-  int r0, r1;
-  block_rows<RB64>(n, r0, r1);
-  for (int i = r0 + threadIdx.x; i < r1; i += RB64)
+  auto row = [&](int q, int o, double xo, double po, double ro, double qo, double co) {
+    x[o] = xo + alpha[q] * po;
+    const double ri = ro - alpha[q] * qo;
+    r[o] = ri;
+    a[q] += fabs(ri);
+    if (jacobi) {
+      const double zi = ri * co;
+      z[o] = zi;
+      a[3 + q] += ri * zi;
+    }
+  };
+  if (ahead) {
+    if (i < r1) row(0, i, x0, p0, ri0, q0, c0);
+    i += TB;
+  }
+  for (; i < r1; i += TB)
 #pragma unroll
     for (int q = 0; q < NVC; ++q) {
       if (dn[q]) continue;
       const int o = q * n + i;
-      x[o] = x[o] + alpha[q] * p[o];
-      const double ri = r[o] - alpha[q] * qv[o];
-      r[o] = ri;
-      a[q] += fabs(ri);
-      if (jacobi) {
-        const double zi = ri * c[i];
-        z[o] = zi;
-        a[3 + q] += ri * zi;
-      }
+      row(q, o, x[o], p[o], r[o], qv[o], jacobi ? c[i] : 0.0);
     }
-  store_partials<6, RB64>(a, partU);
+  store_partials<6, TB>(a, partU);
   if (blockIdx.x == 0 && threadIdx.x == 0)
     for (int q = 0; q < NVC; ++q) ring[(it & 1) * 3 + q].alpha = alpha[q];
 }
 
 // r.z after the sweeps (DIC / DILU)
-__global__ __launch_bounds__(RB64) void k_dot(int n, int nvc, const double *__restrict__ a,
+template <int TB>
+__global__ __launch_bounds__(TB) void k_dot(int n, int nvc, const double *__restrict__ a,
                                             const double *__restrict__ b, double *__restrict__ part, const KS *gate) {
   double s[3] = {0, 0, 0};
   if (!all_done(gate, nvc)) {
     int r0, r1;
-    block_rows<RB64>(n, r0, r1);
-    for (int i = r0 + threadIdx.x; i < r1; i += RB64)
+    block_rows<TB>(n, r0, r1);
+    for (int i = r0 + threadIdx.x; i < r1; i += TB)
       for (int q = 0; q < nvc; ++q) s[q] += a[q * n + i] * b[q * n + i];
   }
-  store_partials<3, RB64>(s, part);
+  store_partials<3, TB>(s, part);
 }
 
 // Final decision after the last queued iteration (1 block).
-__global__ __launch_bounds__(RB64) void k_cg_final(int it, int nvc, const double *partU, int PU, const double *partR,
-                                                 int PR, KS *ring, KS *out) {
+__global__ __launch_bounds__(RB64) void k_cg_final(int it, int nvc, const double *partU, int P, const double *partR,
+                                                   KS *ring, KS *out) {
   double t[6];
-  load_totals<6, RB64>(partU, PU, t);
+  load_totals<6, RB64>(partU, P, t);
   double rz[3] = {t[3], t[4], t[5]};
-  if (partR) {
-    double tr[3];
-    load_totals<3, RB64>(partR, PR, tr);
-    rz[0] = tr[0]; rz[1] = tr[1]; rz[2] = tr[2];
-  }
+  if (partR) load_totals<3, RB64>(partR, P, rz);
   if (threadIdx.x == 0) {
     KS cur[3];
     cg_decide(it, nvc, t, rz, ring + ((it + 1) & 1) * 3, cur);
@@ -558,12 +620,13 @@ __device__ __forceinline__ void bi_decide(int it, int nvc, const double *L1, con
 }
 
 // Decide iteration it ; p = r + w6 (p - w2 u) ; Jacobi: z = c p
-__global__ __launch_bounds__(RB64) void k_bi_p(int n, int it, int nvc, const double *__restrict__ r,
+template <int TB>
+__global__ __launch_bounds__(TB) void k_bi_p(int n, int it, int nvc, const double *__restrict__ r,
                                              double *__restrict__ p, const double *__restrict__ u,
                                              const double *__restrict__ c, int jacobi, double *__restrict__ z,
                                              const double *__restrict__ partU, int PU, KS *ring, KS *out) {
   double t[6];
-  load_totals<6, RB64>(partU, PU, t);
+  load_totals<6, TB>(partU, PU, t);
   __shared__ KS sk[3];
   if (threadIdx.x == 0) {
     bi_decide(it, nvc, t, t + 3, ring + ((it + 1) & 1) * 3, sk);
@@ -579,8 +642,8 @@ __global__ __launch_bounds__(RB64) void k_bi_p(int n, int it, int nvc, const dou
     dn[q] = sk[q].done;
   }
   int r0, r1;
-  block_rows<RB64>(n, r0, r1);
-  for (int i = r0 + threadIdx.x; i < r1; i += RB64)
+  block_rows<TB>(n, r0, r1);
+  for (int i = r0 + threadIdx.x; i < r1; i += TB)
     for (int q = 0; q < nvc; ++q) {
       if (dn[q]) continue;
       const int o = q * n + i;
@@ -591,8 +654,8 @@ __global__ __launch_bounds__(RB64) void k_bi_p(int n, int it, int nvc, const dou
 }
 
 // y = A z with partials y.other (and y.y when mode = 1)
-template <int WS>
-__global__ __launch_bounds__(RB64) void k_bi_spmv(DMesh M, int it, int nvc, int mode, const double *__restrict__ diag,
+template <int WS, int TB>
+__global__ __launch_bounds__(TB) void k_bi_spmv(DMesh M, int it, int nvc, int mode, const double *__restrict__ diag,
                                                 const double *__restrict__ spv, const double *__restrict__ z,
                                                 double *__restrict__ y, const double *__restrict__ other,
                                                 double *__restrict__ part, const KS *ring) {
@@ -601,8 +664,8 @@ __global__ __launch_bounds__(RB64) void k_bi_spmv(DMesh M, int it, int nvc, int 
   if (!all_done(cur, nvc)) {
     const int n = M.n;
     int r0, r1;
-    block_rows<RB64>(n, r0, r1);
-    for (int i = r0 + threadIdx.x; i < r1; i += RB64)
+    block_rows<TB>(n, r0, r1);
+    for (int i = r0 + threadIdx.x; i < r1; i += TB)
       for (int q = 0; q < nvc; ++q) {
         if (cur[q].done) continue;
         const double yi = row_spmv<WS>(M, diag, spv, z + q * n, i);
@@ -611,18 +674,19 @@ __global__ __launch_bounds__(RB64) void k_bi_spmv(DMesh M, int it, int nvc, int 
         if (mode) a[3 + q] += yi * yi;
       }
   }
-  store_partials<6, RB64>(a, part);
+  store_partials<6, TB>(a, part);
 }
 
 // gam = beta/(u.r0 + small) ; x += gam z ; r -= gam u ; Jacobi: z = c r
-__global__ __launch_bounds__(RB64) void k_bi_upd1(int n, int it, int nvc, double *__restrict__ x,
+template <int TB>
+__global__ __launch_bounds__(TB) void k_bi_upd1(int n, int it, int nvc, double *__restrict__ x,
                                                 double *__restrict__ r, double *__restrict__ z,
                                                 const double *__restrict__ u, const double *__restrict__ c, int jacobi,
                                                 const double *__restrict__ partB, int PB, KS *ring) {
   KS *cur = ring + (it & 1) * 3;
   if (all_done(cur, nvc)) return;
   double t[6];
-  load_totals<6, RB64>(partB, PB, t);
+  load_totals<6, TB>(partB, PB, t);
   double w5[3];
   int dn[3];
   for (int q = 0; q < nvc; ++q) {
@@ -636,8 +700,8 @@ __global__ __launch_bounds__(RB64) void k_bi_upd1(int n, int it, int nvc, double
     for (int q = 0; q < nvc; ++q)
       if (!dn[q]) cur[q].w5 = w5[q];
   int r0, r1;
-  block_rows<RB64>(n, r0, r1);
-  for (int i = r0 + threadIdx.x; i < r1; i += RB64)
+  block_rows<TB>(n, r0, r1);
+  for (int i = r0 + threadIdx.x; i < r1; i += TB)
     for (int q = 0; q < nvc; ++q) {
       if (dn[q]) continue;
       const int o = q * n + i;
@@ -649,7 +713,8 @@ __global__ __launch_bounds__(RB64) void k_bi_upd1(int n, int it, int nvc, double
 }
 
 // omega = (v.r)/(v.v + small) ; x += omega z ; r -= omega v ; partials |r|_1, r.r0
-__global__ __launch_bounds__(RB64) void k_bi_upd2(int n, int it, int nvc, double *__restrict__ x,
+template <int TB>
+__global__ __launch_bounds__(TB) void k_bi_upd2(int n, int it, int nvc, double *__restrict__ x,
                                                 double *__restrict__ r, const double *__restrict__ z,
                                                 const double *__restrict__ v, const double *__restrict__ r0v,
                                                 const double *__restrict__ partD, int PD, double *__restrict__ partU,
@@ -658,7 +723,7 @@ __global__ __launch_bounds__(RB64) void k_bi_upd2(int n, int it, int nvc, double
   double a[6] = {0, 0, 0, 0, 0, 0};
   if (!all_done(cur, nvc)) {
     double t[6];
-    load_totals<6, RB64>(partD, PD, t);
+    load_totals<6, TB>(partD, PD, t);
     double w1[3], w2[3];
     int dn[3];
     for (int q = 0; q < nvc; ++q) {
@@ -671,8 +736,8 @@ __global__ __launch_bounds__(RB64) void k_bi_upd2(int n, int it, int nvc, double
       for (int q = 0; q < nvc; ++q)
         if (!dn[q]) { cur[q].w1 = w1[q]; cur[q].w2 = w2[q]; }
     int r0, r1;
-    block_rows<RB64>(n, r0, r1);
-    for (int i = r0 + threadIdx.x; i < r1; i += RB64)
+    block_rows<TB>(n, r0, r1);
+    for (int i = r0 + threadIdx.x; i < r1; i += TB)
       for (int q = 0; q < nvc; ++q) {
         if (dn[q]) continue;
         const int o = q * n + i;
@@ -683,7 +748,7 @@ __global__ __launch_bounds__(RB64) void k_bi_upd2(int n, int it, int nvc, double
         a[3 + q] += ri * r0v[o];
       }
   }
-  store_partials<6, RB64>(a, partU);
+  store_partials<6, TB>(a, partU);
 }
 
 __global__ __launch_bounds__(RB64) void k_bi_final(int it, int nvc, const double *partU, int PU, KS *ring, KS *out) {
@@ -705,21 +770,21 @@ __global__ __launch_bounds__(RB64) void k_res_final(int nvc, const double *partU
 }
 
 // FP64 true residual {|b-Ax|_1, |b-Ax|_2^2, |b|_1, |b|_2^2} as partials
-template <int WS>
-__global__ __launch_bounds__(RB64) void k_true_res(DMesh M, const double *__restrict__ diag,
+template <int WS, int TB>
+__global__ __launch_bounds__(TB) void k_true_res(DMesh M, const double *__restrict__ diag,
                                                  const double *__restrict__ spv, const double *__restrict__ x,
                                                  const double *__restrict__ b, double *__restrict__ part) {
   double a[4] = {0, 0, 0, 0};
   int r0, r1;
-  block_rows<RB64>(M.n, r0, r1);
-  for (int i = r0 + threadIdx.x; i < r1; i += RB64) {
+  block_rows<TB>(M.n, r0, r1);
+  for (int i = r0 + threadIdx.x; i < r1; i += TB) {
     const double bi = b[i], ri = bi - row_spmv<WS>(M, diag, spv, x, i);
     a[0] += fabs(ri);
     a[1] += ri * ri;
     a[2] += fabs(bi);
     a[3] += bi * bi;
   }
-  store_partials<4, RB64>(a, part);
+  store_partials<4, TB>(a, part);
 }
 
 __global__ __launch_bounds__(RB64) void k_totals4(const double *part, int P, double *out) {
@@ -932,6 +997,13 @@ int precond_apply(Ctx &c, int imat, int nvc, const double *b, double *x, const K
     default: F(0); break; \
   }
 
+// f(block size) of the reduction kernels at the context's size
+template <class F>
+static void with_tb(const Ctx &c, F f) {
+  if (small64(c.n)) f(std::integral_constant<int, TB64>{});
+  else f(std::integral_constant<int, RB64>{});
+}
+
 int spmv(Ctx &c, int nvc, const double *x, double *y) {
 #define L(W) k_spmv<W><<<grid_for(c.n), BS, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, y)
   FVK_WS(c.M.Ws, L);
@@ -951,10 +1023,13 @@ static int ks_init(Ctx &c, int nvc, double reduc, int n_iter, bool bicg) {
 
 int residual(Ctx &c, int nvc, const double *x, double *r, bool not_r0) {
   const int G = red_grid64(c.n);
+  with_tb(c, [&](auto tb) {
+  constexpr int TB = decltype(tb)::value;
 #define L(W) \
-  k_residual<W><<<G, RB64, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r, not_r0 ? 1 : 0, 0, nullptr, nullptr, pbuf(c, 0))
+  k_residual<W, TB><<<G, TB, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r, not_r0 ? 1 : 0, 0, nullptr, nullptr, pbuf(c, 0))
   FVK_WS(c.M.Ws, L);
 #undef L
+  });
   k_res_final<<<1, RB64, 0, c.stream>>>(nvc, pbuf(c, 0), G, c.ks);
   FVK_HIP(hipGetLastError());
   return 0;
@@ -977,10 +1052,13 @@ int residual_to(Ctx &c, int nvc, const double *x, double *r, bool not_r0, double
     set_error("partials exceed the scratch");
     return FVK_ERR_ARG;
   }
+  with_tb(c, [&](auto tb) {
+  constexpr int TB = decltype(tb)::value;
 #define L(W) \
-  k_residual<W><<<G, RB64, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r, not_r0 ? 1 : 0, 0, nullptr, nullptr, part)
+  k_residual<W, TB><<<G, TB, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r, not_r0 ? 1 : 0, 0, nullptr, nullptr, part)
   FVK_WS(c.M.Ws, L);
 #undef L
+  });
   k_res_final_to<<<1, RB64, 0, c.stream>>>(nvc, part, G, out_dev);
   FVK_HIP(hipGetLastError());
   return 0;
@@ -1012,25 +1090,44 @@ static int all_done_host(Ctx &c, int nvc, bool &done) {
 template <int NVC>
 static void launch_cg_pq(Ctx &c, int G, int it, double *z, double *pold, double *pnew, double *q, const double *pU,
                          const double *pR, KTimer *T) {
-  hipEvent_t a, b;
-  if (T && T->take(a, b)) {
-    const double *zc = z, *pc = pold;
-#define L(W)                                                                                                   \
-  hipExtLaunchKernelGGL(k_cg_pq<NVC, W>, dim3(G), dim3(RB64), 0, c.stream, a, b, 0, c.M, it, (const double *)c.diag, \
-                        (const double *)c.spv, zc, pc, pnew, q, pU, G, pR, G, pbuf(c, 1), c.ksr, c.ks)
-    FVK_WS(c.M.Ws, L);
+  hipEvent_t ea, eb;
+  const bool stamp = T && T->take(ea, eb);
+  const double *zc = z, *pc = pold, *dg = c.diag, *sv = c.spv;
+  with_tb(c, [&](auto tb) {
+    constexpr int TB = decltype(tb)::value;
+    if (stamp) {
+#define L(W)                                                                                                      \
+  hipExtLaunchKernelGGL(k_cg_pq<NVC, W, TB>, dim3(G), dim3(TB), 0, c.stream, ea, eb, 0, c.M, it, dg, sv, zc, pc, pnew, \
+                        q, pU, G, pR, pbuf(c, 1), c.ksr, c.ks)
+      FVK_WS(c.M.Ws, L);
 #undef L
-    return;
-  }
-#define L(W)                                                                                                    \
-  k_cg_pq<NVC, W><<<G, RB64, 0, c.stream>>>(c.M, it, c.diag, c.spv, z, pold, pnew, q, pU, G, pR, G, pbuf(c, 1), \
-                                          c.ksr, c.ks)
-  FVK_WS(c.M.Ws, L);
+    } else {
+#define L(W)                                                                                                      \
+  k_cg_pq<NVC, W, TB><<<G, TB, 0, c.stream>>>(c.M, it, dg, sv, zc, pc, pnew, q, pU, G, pR, pbuf(c, 1), \
+                                              c.ksr, c.ks)
+      FVK_WS(c.M.Ws, L);
 #undef L
+    }
+  });
 }
 template <int NVC>
 static void launch_cg_upd(Ctx &c, int G, int it, double *x, double *r, double *p, double *q, int jac, double *z) {
-  k_cg_upd<NVC><<<G, RB64, 0, c.stream>>>(c.n, it, x, r, p, q, c.pc_c, jac, z, pbuf(c, 1), G, pbuf(c, 0), c.ksr);
+  with_tb(c, [&](auto tb) {
+    constexpr int TB = decltype(tb)::value;
+    k_cg_upd<NVC, TB><<<G, TB, 0, c.stream>>>(c.n, it, x, r, p, q, c.pc_c, jac, z, pbuf(c, 1), G, pbuf(c, 0), c.ksr);
+  });
+}
+
+// z = M^-1 r and the partials of r.z
+static int precond_dot(Ctx &c, int imat, int nvc, const double *r, double *z, const KS *gate) {
+  const int rc = precond_apply(c, imat, nvc, r, z, gate);
+  if (rc) return rc;
+  const int G = red_grid64(c.n);
+  with_tb(c, [&](auto tb) {
+    constexpr int TB = decltype(tb)::value;
+    k_dot<TB><<<G, TB, 0, c.stream>>>(c.n, nvc, r, z, pbuf(c, 2), gate);
+  });
+  return 0;
 }
 
 // PCG: r0 holds b on entry, b - A x0 (the initial residual) on exit; x is
@@ -1046,18 +1143,19 @@ static int cg_run(Ctx &c, int imat, double reduc, int n_iter, int nvc, double *x
   }
   // both direction buffers (slots 2 and 3)
   if (fill(c, P, wk_ld(n) + (size_t)3 * n, 0.0)) return FVK_ERR_HIP;
+  with_tb(c, [&](auto tb) {
+  constexpr int TB = decltype(tb)::value;
 #define L(W)                                                                                                \
-  k_residual<W><<<G, RB64, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r0, not_r0 ? 1 : 0, jac ? 1 : 0, c.pc_c, z, \
+  k_residual<W, TB><<<G, TB, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r0, not_r0 ? 1 : 0, jac ? 1 : 0, c.pc_c, z, \
                                         pbuf(c, 0))
   FVK_WS(c.M.Ws, L);
 #undef L
+  });
   if (copy_d(c, r0, r, (size_t)nvc * n)) return FVK_ERR_HIP;
-  const double *pR = nullptr;
+  const double *pR = jac ? nullptr : pbuf(c, 2);
   if (!jac) {
-    int rc = precond_apply(c, imat, nvc, r, z, nullptr);
+    int rc = precond_dot(c, imat, nvc, r, z, nullptr);
     if (rc) return rc;
-    k_dot<<<G, RB64, 0, c.stream>>>(n, nvc, r, z, pbuf(c, 2), nullptr);
-    pR = pbuf(c, 2);
   }
   Poller Pl(c);
   int it = 0, next_poll = chunk;
@@ -1070,9 +1168,8 @@ static int cg_run(Ctx &c, int imat, double reduc, int n_iter, int nvc, double *x
     else if (nvc == 2) launch_cg_upd<2>(c, G, it, x, r, pnew, q, jac, z);
     else launch_cg_upd<3>(c, G, it, x, r, pnew, q, jac, z);
     if (!jac) {
-      int rc = precond_apply(c, imat, nvc, r, z, c.ksr + (it & 1) * 3);
+      int rc = precond_dot(c, imat, nvc, r, z, c.ksr + (it & 1) * 3);
       if (rc) return rc;
-      k_dot<<<G, RB64, 0, c.stream>>>(n, nvc, r, z, pbuf(c, 2), c.ksr + (it & 1) * 3);
     }
     if (chunk > 0 && it + 1 == next_poll && it + 1 < n_iter) {
       bool done;
@@ -1088,7 +1185,7 @@ static int cg_run(Ctx &c, int imat, double reduc, int n_iter, int nvc, double *x
       next_poll = it + 1 + next;
     }
   }
-  k_cg_final<<<1, RB64, 0, c.stream>>>(it, nvc, pbuf(c, 0), G, pR, G, c.ksr, c.ks);
+  k_cg_final<<<1, RB64, 0, c.stream>>>(it, nvc, pbuf(c, 0), G, pR, c.ksr, c.ks);
   FVK_HIP(hipGetLastError());
   if (T && T->flush()) return FVK_ERR_HIP;
   return 0;
@@ -1104,26 +1201,35 @@ static int bicg_run(Ctx &c, int imat, int n_iter, int nvc, double *x, double *r0
   }
   // slots 1-4
   if (fill(c, p, (size_t)3 * wk_ld(n) + (size_t)3 * n, 0.0)) return FVK_ERR_HIP;
+  with_tb(c, [&](auto tb) {
+  constexpr int TB = decltype(tb)::value;
 #define L(W)                                                                                              \
-  k_residual<W><<<G, RB64, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r0, not_r0 ? 1 : 0, 2, nullptr, nullptr, \
+  k_residual<W, TB><<<G, TB, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r0, not_r0 ? 1 : 0, 2, nullptr, nullptr, \
                                         pbuf(c, 0))
   FVK_WS(c.M.Ws, L);
 #undef L
+  });
   if (copy_d(c, r0, r, (size_t)nvc * n)) return FVK_ERR_HIP;
   int it = 0;
   for (; it < n_iter; ++it) {
     const KS *gate = c.ksr + (it & 1) * 3;
-    k_bi_p<<<G, RB64, 0, c.stream>>>(n, it, nvc, r, p, u, c.pc_c, jac, z, pbuf(c, 0), G, c.ksr, c.ks);
+    with_tb(c, [&](auto tb) { k_bi_p<decltype(tb)::value><<<G, decltype(tb)::value, 0, c.stream>>>(n, it, nvc, r, p, u, c.pc_c, jac, z, pbuf(c, 0), G, c.ksr, c.ks); });
     if (!jac && precond_apply(c, imat, nvc, p, z, gate)) return FVK_ERR_HIP;
-#define L(W) k_bi_spmv<W><<<G, RB64, 0, c.stream>>>(c.M, it, nvc, 0, c.diag, c.spv, z, u, r0, pbuf(c, 1), c.ksr)
+  with_tb(c, [&](auto tb) {
+  constexpr int TB = decltype(tb)::value;
+#define L(W) k_bi_spmv<W, TB><<<G, TB, 0, c.stream>>>(c.M, it, nvc, 0, c.diag, c.spv, z, u, r0, pbuf(c, 1), c.ksr)
     FVK_WS(c.M.Ws, L);
 #undef L
-    k_bi_upd1<<<G, RB64, 0, c.stream>>>(n, it, nvc, x, r, z, u, c.pc_c, jac, pbuf(c, 1), G, c.ksr);
+  });
+    with_tb(c, [&](auto tb) { k_bi_upd1<decltype(tb)::value><<<G, decltype(tb)::value, 0, c.stream>>>(n, it, nvc, x, r, z, u, c.pc_c, jac, pbuf(c, 1), G, c.ksr); });
     if (!jac && precond_apply(c, imat, nvc, r, z, gate)) return FVK_ERR_HIP;
-#define L(W) k_bi_spmv<W><<<G, RB64, 0, c.stream>>>(c.M, it, nvc, 1, c.diag, c.spv, z, v, r, pbuf(c, 2), c.ksr)
+  with_tb(c, [&](auto tb) {
+  constexpr int TB = decltype(tb)::value;
+#define L(W) k_bi_spmv<W, TB><<<G, TB, 0, c.stream>>>(c.M, it, nvc, 1, c.diag, c.spv, z, v, r, pbuf(c, 2), c.ksr)
     FVK_WS(c.M.Ws, L);
 #undef L
-    k_bi_upd2<<<G, RB64, 0, c.stream>>>(n, it, nvc, x, r, z, v, r0, pbuf(c, 2), G, pbuf(c, 0), c.ksr);
+  });
+    with_tb(c, [&](auto tb) { k_bi_upd2<decltype(tb)::value><<<G, decltype(tb)::value, 0, c.stream>>>(n, it, nvc, x, r, z, v, r0, pbuf(c, 2), G, pbuf(c, 0), c.ksr); });
   }
   k_bi_final<<<1, RB64, 0, c.stream>>>(it, nvc, pbuf(c, 0), G, c.ksr, c.ks);
   FVK_HIP(hipGetLastError());
@@ -1171,9 +1277,12 @@ int pcg_tol(Ctx &c, int imat, const double *b, double *x, double tol, int max_it
 
 int true_residual(Ctx &c, const double *x, const double *b, double *dev_out4, double *host_out4) {
   const int G = red_grid64(c.n);
-#define L(W) k_true_res<W><<<G, RB64, 0, c.stream>>>(c.M, c.diag, c.spv, x, b, pbuf(c, 3))
+  with_tb(c, [&](auto tb) {
+  constexpr int TB = decltype(tb)::value;
+#define L(W) k_true_res<W, TB><<<G, TB, 0, c.stream>>>(c.M, c.diag, c.spv, x, b, pbuf(c, 3))
   FVK_WS(c.M.Ws, L);
 #undef L
+  });
   k_totals4<<<1, RB64, 0, c.stream>>>(pbuf(c, 3), G, dev_out4);
   FVK_HIP(hipGetLastError());
   FVK_HIP(hipMemcpyAsync(host_out4, dev_out4, 4 * sizeof(double), hipMemcpyDeviceToHost, c.stream));

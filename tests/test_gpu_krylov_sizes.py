@@ -1,0 +1,75 @@
+"""The FP64 Krylov kernels around the sizes where their launch changes: a
+block that is not full, one row more than a block of 256, the last size whose
+rows all fall on a thread's first pass (1024 blocks of 256), the next one, and
+both sides of the change to blocks of 1024 (512 * 1024 rows)."""
+import numpy as np
+import pytest
+
+from tests.helpers import require_lib
+from tests.test_gpu_sweeps import random_matrix
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(float).eps
+
+
+def mult(m, pl, gp, gn):
+    t = m.topology()
+    inner = t["fce_in"] > 0
+    a, b, gp, gn = t["fce_ip"][inner] - 1, t["fce_in"][inner] - 1, gp[inner], gn[inner]
+    n = m.n_vol
+    return lambda x: pl * x + np.bincount(a, gp * x[b], n) + np.bincount(b, gn * x[a], n)
+
+
+def pcg(A, c, b, steps):
+    x, r = np.zeros_like(b), b.copy()
+    z = c * r
+    p, s = z.copy(), r @ z
+    for _ in range(steps):
+        q = A(p)
+        al = s / (p @ q)
+        x += al * p
+        r -= al * q
+        z = c * r
+        s, so = r @ z, s
+        p = z + s / so * p
+    return x
+
+
+@pytest.mark.parametrize("dims", [(3, 1, 1), (257, 1, 1), (64, 64, 64), (4097, 8, 8), (64, 64, 128), (4097, 8, 16)])
+def test_two_steps(dims):
+    fvk = require_lib()
+    print("krylov sizes:", dims, flush=True)
+    m = fvk.Mesh.box(*dims, jitter=0.0, seed=1)
+    n = m.n_vol
+    ctx = fvk.grd_solv(m)
+    pl, gp, gn = random_matrix(m, 5)
+    b = np.random.default_rng(n).standard_normal((n, 3))
+    # a rounding error per addition of a reduction, four reductions; the
+    # rows' own errors are below 1e-14
+    tol = 4 * n * EPS + 1e-14
+
+    pls = pl + 6.0  # dominant for the symmetric matrix too
+    fvk.set_matrix(ctx, pls, gp, gp)
+    A = mult(m, pls, gp, gp)
+    for k in (1, 2, 3):
+        x, r = np.zeros((n, k)), b[:, :k].copy()
+        fvk.solv_cg(ctx, 0, 1e-30, 2, x, r)
+        assert np.array_equal(r, b[:, :k])  # from x = 0 the initial residual is b
+        for q in range(k):
+            want = pcg(A, 1.0 / pls, b[:, q], 2)
+            assert np.abs(x[:, q] - want).max() <= tol * np.abs(want).max(), (k, q)
+
+    fvk.set_matrix(ctx, pl, gp, gn)
+    A = mult(m, pl, gp, gn)
+    x, r = np.zeros((n, 3)), b.copy()
+    fvk.solv_bicg(ctx, 0, 1e-30, 1, x, r)
+    for q in range(3):
+        # one step: p = r = b, gamma = r.r0 / u.r0, omega = v.s / v.v
+        b0, c = b[:, q], 1.0 / pl
+        u = A(c * b0)
+        g = b0 @ b0 / (u @ b0)
+        s = b0 - g * u
+        v = A(c * s)
+        want = g * c * b0 + (v @ s) / (v @ v) * c * s
+        assert np.abs(x[:, q] - want).max() <= tol * np.abs(want).max(), q
+    ctx.destroy()
