@@ -207,13 +207,13 @@ template <int WS>
 __device__ __forceinline__ int nslots(const DMesh &M) { return WS > 0 ? WS : M.Ws; }
 
 // Grid of the reduction kernels: at most RG blocks of RB threads, a multiple
-// of 8 once there are enough rows (XCD-contiguous row chunks).
+// of 8 once there are enough rows (XCD-contiguous row chunks), rounded up:
+// with one block fewer than the rows need every block takes a second pass.
 inline int red_grid(int n) {
   int g = (n + RB - 1) / RB;
   if (g < 1) g = 1;
-  if (g > RG) g = RG;
-  if (g >= 16) g = g / 8 * 8;
-  return g;
+  if (g >= 16) g = (g + 7) / 8 * 8;
+  return g > RG ? RG : g;
 }
 inline int grid_for(int n) { return n > 0 ? (n + BS - 1) / BS : 1; }
 
@@ -229,24 +229,23 @@ __device__ __forceinline__ int xcd_block() {
   return b < per * kXcd ? (b % kXcd) * per + b / kXcd : b;
 }
 
-// The FP64 Krylov kernels (krylov.hip): blocks of TB64 threads up to
-// kSmall64 rows, where blocks of RB64 would leave compute units without one
-// and a launch lasts as long as one block (48^3, per CG iteration with the
-// gaps: 22.8 us with RB64, 10.7 us with TB64); above, RB64 threads and at
-// most RG64 blocks (2.6 % faster than 512 x 512 on the plain FP64 solve at
-// 128^3).
+// The FP64 Krylov kernels (krylov.hip): blocks of 256 threads where 1024
+// blocks give every row a thread, then blocks of 512 likewise.  Larger
+// blocks would leave compute units without one, and a launch lasts as long
+// as one block's chain of loads (48^3, per CG iteration with the gaps: 22.8
+// us with blocks of 1024, 10.7 us with 256; 281k rows, k_cg_pq: 13.9 us with
+// 256, two rows a thread, 10.5 us with 512).  Above, blocks of 1024 and at most
+// 512 of them (2.6 % faster than 512 x 512 on the plain FP64 solve at 128^3).
 constexpr int RB64 = 1024;
 constexpr int RG64 = 512;
-constexpr int TB64 = 256;
-constexpr int kSmall64 = 512 * 1024;
-inline bool small64(int n) { return n <= kSmall64; }
+inline int red_block64(int n) { return n <= RG * 256 ? 256 : n <= RG * 512 ? 512 : RB64; }
+// rounded as red_grid is
 inline int red_grid64(int n) {
-  const int tb = small64(n) ? TB64 : RB64, most = small64(n) ? RG : RG64;
+  const int tb = red_block64(n), most = tb < RB64 ? RG : RG64;
   int g = (n + tb - 1) / tb;
   if (g < 1) g = 1;
-  if (g > most) g = most;
-  if (g >= 16) g = g / 8 * 8;
-  return g;
+  if (g >= 16) g = (g + 7) / 8 * 8;
+  return g > most ? most : g;
 }
 
 // Stride of the slot-major FP64 tables: n plus 128 KiB + 512 B of doubles

@@ -335,8 +335,8 @@ __global__ __launch_bounds__(BS) void k_spmv(DMesh M, int nvc, const double *__r
 // r = b - A x (or r = b) with partials {|r|_1[q], s2[q]} where s2 = r.(c r)
 // and z = c r (mode 1, Jacobi PCG), s2 = r.r (mode 2, BiCGStab) or 0.
 // (solv_res.f90; solv_cg.f90:19-33; solv_bicg.f90:19-38)
-template <int WS, int TB>
-__global__ __launch_bounds__(TB) void k_residual(DMesh M, int nvc, const double *__restrict__ diag,
+template <int NVC, int WS, int TB>
+__global__ __launch_bounds__(TB) void k_residual(DMesh M, const double *__restrict__ diag,
                                                  const double *__restrict__ spv, const double *__restrict__ x,
                                                  double *__restrict__ r, int not_r0, int mode,
                                                  const double *__restrict__ c, double *__restrict__ z,
@@ -345,29 +345,37 @@ __global__ __launch_bounds__(TB) void k_residual(DMesh M, int nvc, const double 
   double a[6] = {0, 0, 0, 0, 0, 0};
   int r0, r1;
   block_rows<TB>(n, r0, r1);
-  for (int i = r0 + threadIdx.x; i < r1; i += TB)
-    for (int q = 0; q < nvc; ++q) {
-      double v = r[q * n + i];
-      if (!not_r0) {
-        const double *xq = x + q * n;
-        v = v - diag[i] * xq[i];
+  for (int i = r0 + threadIdx.x; i < r1; i += TB) {
+    double v[NVC];
 #pragma unroll
-        for (int k = 0; k < nslots<WS>(M); ++k) {
-          const int j = M.spc[(size_t)k * M.ld + i];
-          const double a = spv[(size_t)k * M.ld + i];
-          if (j >= 0) v = v - a * xq[j];
-        }
-        r[q * n + i] = v;
+    for (int q = 0; q < NVC; ++q) v[q] = r[q * n + i];
+    if (!not_r0) {
+      const double d = diag[i];
+#pragma unroll
+      for (int q = 0; q < NVC; ++q) v[q] = v[q] - d * x[q * n + i];
+#pragma unroll
+      for (int k = 0; k < nslots<WS>(M); ++k) {
+        const int j = M.spc[(size_t)k * M.ld + i];
+        const double s = spv[(size_t)k * M.ld + i];
+        if (j >= 0)
+#pragma unroll
+          for (int q = 0; q < NVC; ++q) v[q] = v[q] - s * x[q * n + j];
       }
-      a[q] += fabs(v);
+#pragma unroll
+      for (int q = 0; q < NVC; ++q) r[q * n + i] = v[q];
+    }
+#pragma unroll
+    for (int q = 0; q < NVC; ++q) {
+      a[q] += fabs(v[q]);
       if (mode == 1) {
-        const double zi = v * c[i];
+        const double zi = v[q] * c[i];
         z[q * n + i] = zi;
-        a[3 + q] += v * zi;
+        a[3 + q] += v[q] * zi;
       } else if (mode == 2) {
-        a[3 + q] += v * v;
+        a[3 + q] += v[q] * v[q];
       }
     }
+  }
   store_partials<6, TB>(a, part);
 }
 
@@ -445,7 +453,7 @@ __global__ __launch_bounds__(TB) void k_cg_pq(DMesh M, int it, const double *__r
   int r0, r1;
   block_rows<TB>(n, r0, r1);
   int i = r0 + threadIdx.x;
-  constexpr bool ahead = NVC == 1 && WS > 0 && TB == TB64;
+  constexpr bool ahead = NVC == 1 && WS > 0 && TB < RB64;
   CgRow<WS> first;
   if (ahead && i < r1) first.load(M, i, diag, spv, z, pold);
   // |r|_1 (components 0..NVC) and, for Jacobi, r.z (components 3..3+NVC)
@@ -512,7 +520,7 @@ __global__ __launch_bounds__(TB) void k_cg_upd(int n, int it, double *__restrict
   block_rows<TB>(n, r0, r1);
   int i = r0 + threadIdx.x;
   // the first row's loads before the partials are reduced
-  constexpr bool ahead = NVC == 1 && TB == TB64;
+  constexpr bool ahead = NVC == 1 && TB < RB64;
   double x0 = 0.0, p0 = 0.0, ri0 = 0.0, q0 = 0.0, c0 = 0.0;
   if (ahead && i < r1) {
     x0 = x[i];
@@ -619,32 +627,43 @@ __device__ __forceinline__ void bi_decide(int it, int nvc, const double *L1, con
   }
 }
 
+// The BiCGStab kernels have the number of right-hand sides as a template
+// argument: with a loop bound known at run time only, the scalars of the
+// components lay in scratch memory and a row of A was loaded once per
+// component (281k rows, 3 components: k_bi_p 23.3 -> 10.7 us, k_bi_spmv
+// 12.8 -> 7.4 us on average over active and finished iterations).
+
 // Decide iteration it ; p = r + w6 (p - w2 u) ; Jacobi: z = c p
-template <int TB>
-__global__ __launch_bounds__(TB) void k_bi_p(int n, int it, int nvc, const double *__restrict__ r,
-                                             double *__restrict__ p, const double *__restrict__ u,
-                                             const double *__restrict__ c, int jacobi, double *__restrict__ z,
-                                             const double *__restrict__ partU, int PU, KS *ring, KS *out) {
+template <int NVC, int TB>
+__global__ __launch_bounds__(TB) void k_bi_p(int n, int it, const double *__restrict__ r, double *__restrict__ p,
+                                             const double *__restrict__ u, const double *__restrict__ c, int jacobi,
+                                             double *__restrict__ z, const double *__restrict__ partU, int PU, KS *ring,
+                                             KS *out) {
   double t[6];
   load_totals<6, TB>(partU, PU, t);
   __shared__ KS sk[3];
   if (threadIdx.x == 0) {
-    bi_decide(it, nvc, t, t + 3, ring + ((it + 1) & 1) * 3, sk);
+    bi_decide(it, NVC, t, t + 3, ring + ((it + 1) & 1) * 3, sk);
     if (blockIdx.x == 0)
-      for (int q = 0; q < nvc; ++q) ring[(it & 1) * 3 + q] = out[q] = sk[q];
+      for (int q = 0; q < NVC; ++q) ring[(it & 1) * 3 + q] = out[q] = sk[q];
   }
   __syncthreads();
-  double w6[3] = {0, 0, 0}, w2[3] = {0, 0, 0};
-  int dn[3] = {1, 1, 1};
-  for (int q = 0; q < nvc; ++q) {
+  double w6[NVC], w2[NVC];
+  int dn[NVC];
+  bool any = false;
+#pragma unroll
+  for (int q = 0; q < NVC; ++q) {
     w6[q] = sk[q].w6;
     w2[q] = sk[q].w2;
     dn[q] = sk[q].done;
+    any = any || !dn[q];
   }
+  if (!any) return;
   int r0, r1;
   block_rows<TB>(n, r0, r1);
   for (int i = r0 + threadIdx.x; i < r1; i += TB)
-    for (int q = 0; q < nvc; ++q) {
+#pragma unroll
+    for (int q = 0; q < NVC; ++q) {
       if (dn[q]) continue;
       const int o = q * n + i;
       const double pi = r[o] + w6[q] * (p[o] - w2[q] * u[o]);
@@ -654,55 +673,76 @@ __global__ __launch_bounds__(TB) void k_bi_p(int n, int it, int nvc, const doubl
 }
 
 // y = A z with partials y.other (and y.y when mode = 1)
-template <int WS, int TB>
-__global__ __launch_bounds__(TB) void k_bi_spmv(DMesh M, int it, int nvc, int mode, const double *__restrict__ diag,
+template <int NVC, int WS, int TB>
+__global__ __launch_bounds__(TB) void k_bi_spmv(DMesh M, int it, int mode, const double *__restrict__ diag,
                                                 const double *__restrict__ spv, const double *__restrict__ z,
                                                 double *__restrict__ y, const double *__restrict__ other,
                                                 double *__restrict__ part, const KS *ring) {
   const KS *cur = ring + (it & 1) * 3;
+  int dn[NVC];
+  bool any = false;
+#pragma unroll
+  for (int q = 0; q < NVC; ++q) {
+    dn[q] = cur[q].done;
+    any = any || !dn[q];
+  }
+  if (!any) return;  // nobody reads the partials of a finished solve
   double a[6] = {0, 0, 0, 0, 0, 0};
-  if (!all_done(cur, nvc)) {
-    const int n = M.n;
-    int r0, r1;
-    block_rows<TB>(n, r0, r1);
-    for (int i = r0 + threadIdx.x; i < r1; i += TB)
-      for (int q = 0; q < nvc; ++q) {
-        if (cur[q].done) continue;
-        const double yi = row_spmv<WS>(M, diag, spv, z + q * n, i);
-        y[q * n + i] = yi;
-        a[q] += yi * other[q * n + i];
-        if (mode) a[3 + q] += yi * yi;
-      }
+  const int n = M.n;
+  int r0, r1;
+  block_rows<TB>(n, r0, r1);
+  for (int i = r0 + threadIdx.x; i < r1; i += TB) {
+    const double d = diag[i];
+    double v[NVC];
+#pragma unroll
+    for (int q = 0; q < NVC; ++q) v[q] = d * z[q * n + i];
+#pragma unroll
+    for (int k = 0; k < nslots<WS>(M); ++k) {
+      const int j = M.spc[(size_t)k * M.ld + i];
+      const double s = spv[(size_t)k * M.ld + i];
+      if (j >= 0)
+#pragma unroll
+        for (int q = 0; q < NVC; ++q) v[q] = v[q] + s * z[q * n + j];
+    }
+#pragma unroll
+    for (int q = 0; q < NVC; ++q) {
+      if (dn[q]) continue;
+      y[q * n + i] = v[q];
+      a[q] += v[q] * other[q * n + i];
+      if (mode) a[3 + q] += v[q] * v[q];
+    }
   }
   store_partials<6, TB>(a, part);
 }
 
 // gam = beta/(u.r0 + small) ; x += gam z ; r -= gam u ; Jacobi: z = c r
-template <int TB>
-__global__ __launch_bounds__(TB) void k_bi_upd1(int n, int it, int nvc, double *__restrict__ x,
-                                                double *__restrict__ r, double *__restrict__ z,
-                                                const double *__restrict__ u, const double *__restrict__ c, int jacobi,
+template <int NVC, int TB>
+__global__ __launch_bounds__(TB) void k_bi_upd1(int n, int it, double *__restrict__ x, double *__restrict__ r,
+                                                double *__restrict__ z, const double *__restrict__ u,
+                                                const double *__restrict__ c, int jacobi,
                                                 const double *__restrict__ partB, int PB, KS *ring) {
   KS *cur = ring + (it & 1) * 3;
-  if (all_done(cur, nvc)) return;
-  double t[6];
-  load_totals<6, TB>(partB, PB, t);
-  double w5[3];
-  int dn[3];
-  for (int q = 0; q < nvc; ++q) {
+  if (all_done(cur, NVC)) return;
+  double t[NVC];
+  load_totals<NVC, TB>(partB, PB, t);
+  double w5[NVC];
+  int dn[NVC];
+#pragma unroll
+  for (int q = 0; q < NVC; ++q) {
     dn[q] = cur[q].done;
-    w5[q] = t[q];
-    w5[q] = cur[q].w4 / (w5[q] + SMALL);
+    w5[q] = cur[q].w4 / (t[q] + SMALL);
   }
   // every block has read cur[] above; only w5 is written, which no block of
   // this kernel reads
   if (blockIdx.x == 0 && threadIdx.x == 0)
-    for (int q = 0; q < nvc; ++q)
+#pragma unroll
+    for (int q = 0; q < NVC; ++q)
       if (!dn[q]) cur[q].w5 = w5[q];
   int r0, r1;
   block_rows<TB>(n, r0, r1);
   for (int i = r0 + threadIdx.x; i < r1; i += TB)
-    for (int q = 0; q < nvc; ++q) {
+#pragma unroll
+    for (int q = 0; q < NVC; ++q) {
       if (dn[q]) continue;
       const int o = q * n + i;
       x[o] = x[o] + w5[q] * z[o];
@@ -713,41 +753,41 @@ __global__ __launch_bounds__(TB) void k_bi_upd1(int n, int it, int nvc, double *
 }
 
 // omega = (v.r)/(v.v + small) ; x += omega z ; r -= omega v ; partials |r|_1, r.r0
-template <int TB>
-__global__ __launch_bounds__(TB) void k_bi_upd2(int n, int it, int nvc, double *__restrict__ x,
-                                                double *__restrict__ r, const double *__restrict__ z,
-                                                const double *__restrict__ v, const double *__restrict__ r0v,
-                                                const double *__restrict__ partD, int PD, double *__restrict__ partU,
-                                                KS *ring) {
+template <int NVC, int TB>
+__global__ __launch_bounds__(TB) void k_bi_upd2(int n, int it, double *__restrict__ x, double *__restrict__ r,
+                                                const double *__restrict__ z, const double *__restrict__ v,
+                                                const double *__restrict__ r0v, const double *__restrict__ partD, int PD,
+                                                double *__restrict__ partU, KS *ring) {
   KS *cur = ring + (it & 1) * 3;
+  if (all_done(cur, NVC)) return;  // the next decision takes nothing from the partials
   double a[6] = {0, 0, 0, 0, 0, 0};
-  if (!all_done(cur, nvc)) {
-    double t[6];
-    load_totals<6, TB>(partD, PD, t);
-    double w1[3], w2[3];
-    int dn[3];
-    for (int q = 0; q < nvc; ++q) {
-      dn[q] = cur[q].done;
-      w1[q] = t[q];
-      w2[q] = t[3 + q];
-      w2[q] = w1[q] / (w2[q] + SMALL);
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-      for (int q = 0; q < nvc; ++q)
-        if (!dn[q]) { cur[q].w1 = w1[q]; cur[q].w2 = w2[q]; }
-    int r0, r1;
-    block_rows<TB>(n, r0, r1);
-    for (int i = r0 + threadIdx.x; i < r1; i += TB)
-      for (int q = 0; q < nvc; ++q) {
-        if (dn[q]) continue;
-        const int o = q * n + i;
-        x[o] = x[o] + w2[q] * z[o];
-        const double ri = r[o] - w2[q] * v[o];
-        r[o] = ri;
-        a[q] += fabs(ri);
-        a[3 + q] += ri * r0v[o];
-      }
+  double t[6];
+  load_totals<6, TB>(partD, PD, t);
+  double w1[NVC], w2[NVC];
+  int dn[NVC];
+#pragma unroll
+  for (int q = 0; q < NVC; ++q) {
+    dn[q] = cur[q].done;
+    w1[q] = t[q];
+    w2[q] = w1[q] / (t[3 + q] + SMALL);
   }
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+#pragma unroll
+    for (int q = 0; q < NVC; ++q)
+      if (!dn[q]) { cur[q].w1 = w1[q]; cur[q].w2 = w2[q]; }
+  int r0, r1;
+  block_rows<TB>(n, r0, r1);
+  for (int i = r0 + threadIdx.x; i < r1; i += TB)
+#pragma unroll
+    for (int q = 0; q < NVC; ++q) {
+      if (dn[q]) continue;
+      const int o = q * n + i;
+      x[o] = x[o] + w2[q] * z[o];
+      const double ri = r[o] - w2[q] * v[o];
+      r[o] = ri;
+      a[q] += fabs(ri);
+      a[3 + q] += ri * r0v[o];
+    }
   store_partials<6, TB>(a, partU);
 }
 
@@ -997,10 +1037,20 @@ int precond_apply(Ctx &c, int imat, int nvc, const double *b, double *x, const K
     default: F(0); break; \
   }
 
+// f(number of right-hand sides)
+template <class F>
+static void with_nvc(int nvc, F f) {
+  if (nvc == 1) f(std::integral_constant<int, 1>{});
+  else if (nvc == 2) f(std::integral_constant<int, 2>{});
+  else f(std::integral_constant<int, 3>{});
+}
+
 // f(block size) of the reduction kernels at the context's size
 template <class F>
 static void with_tb(const Ctx &c, F f) {
-  if (small64(c.n)) f(std::integral_constant<int, TB64>{});
+  const int tb = red_block64(c.n);
+  if (tb == 256) f(std::integral_constant<int, 256>{});
+  else if (tb == 512) f(std::integral_constant<int, 512>{});
   else f(std::integral_constant<int, RB64>{});
 }
 
@@ -1024,11 +1074,13 @@ static int ks_init(Ctx &c, int nvc, double reduc, int n_iter, bool bicg) {
 int residual(Ctx &c, int nvc, const double *x, double *r, bool not_r0) {
   const int G = red_grid64(c.n);
   with_tb(c, [&](auto tb) {
-  constexpr int TB = decltype(tb)::value;
+    with_nvc(nvc, [&](auto nv) {
+      constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
 #define L(W) \
-  k_residual<W, TB><<<G, TB, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r, not_r0 ? 1 : 0, 0, nullptr, nullptr, pbuf(c, 0))
+  k_residual<NVC, W, TB><<<G, TB, 0, c.stream>>>(c.M, c.diag, c.spv, x, r, not_r0 ? 1 : 0, 0, nullptr, nullptr, pbuf(c, 0))
   FVK_WS(c.M.Ws, L);
 #undef L
+    });
   });
   k_res_final<<<1, RB64, 0, c.stream>>>(nvc, pbuf(c, 0), G, c.ks);
   FVK_HIP(hipGetLastError());
@@ -1053,11 +1105,13 @@ int residual_to(Ctx &c, int nvc, const double *x, double *r, bool not_r0, double
     return FVK_ERR_ARG;
   }
   with_tb(c, [&](auto tb) {
-  constexpr int TB = decltype(tb)::value;
+    with_nvc(nvc, [&](auto nv) {
+      constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
 #define L(W) \
-  k_residual<W, TB><<<G, TB, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r, not_r0 ? 1 : 0, 0, nullptr, nullptr, part)
+  k_residual<NVC, W, TB><<<G, TB, 0, c.stream>>>(c.M, c.diag, c.spv, x, r, not_r0 ? 1 : 0, 0, nullptr, nullptr, part)
   FVK_WS(c.M.Ws, L);
 #undef L
+    });
   });
   k_res_final_to<<<1, RB64, 0, c.stream>>>(nvc, part, G, out_dev);
   FVK_HIP(hipGetLastError());
@@ -1144,12 +1198,14 @@ static int cg_run(Ctx &c, int imat, double reduc, int n_iter, int nvc, double *x
   // both direction buffers (slots 2 and 3)
   if (fill(c, P, wk_ld(n) + (size_t)3 * n, 0.0)) return FVK_ERR_HIP;
   with_tb(c, [&](auto tb) {
-  constexpr int TB = decltype(tb)::value;
+    with_nvc(nvc, [&](auto nv) {
+      constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
 #define L(W)                                                                                                \
-  k_residual<W, TB><<<G, TB, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r0, not_r0 ? 1 : 0, jac ? 1 : 0, c.pc_c, z, \
+  k_residual<NVC, W, TB><<<G, TB, 0, c.stream>>>(c.M, c.diag, c.spv, x, r0, not_r0 ? 1 : 0, jac ? 1 : 0, c.pc_c, z, \
                                         pbuf(c, 0))
   FVK_WS(c.M.Ws, L);
 #undef L
+    });
   });
   if (copy_d(c, r0, r, (size_t)nvc * n)) return FVK_ERR_HIP;
   const double *pR = jac ? nullptr : pbuf(c, 2);
@@ -1202,34 +1258,55 @@ static int bicg_run(Ctx &c, int imat, int n_iter, int nvc, double *x, double *r0
   // slots 1-4
   if (fill(c, p, (size_t)3 * wk_ld(n) + (size_t)3 * n, 0.0)) return FVK_ERR_HIP;
   with_tb(c, [&](auto tb) {
-  constexpr int TB = decltype(tb)::value;
+    with_nvc(nvc, [&](auto nv) {
+      constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
 #define L(W)                                                                                              \
-  k_residual<W, TB><<<G, TB, 0, c.stream>>>(c.M, nvc, c.diag, c.spv, x, r0, not_r0 ? 1 : 0, 2, nullptr, nullptr, \
+  k_residual<NVC, W, TB><<<G, TB, 0, c.stream>>>(c.M, c.diag, c.spv, x, r0, not_r0 ? 1 : 0, 2, nullptr, nullptr, \
                                         pbuf(c, 0))
   FVK_WS(c.M.Ws, L);
 #undef L
+    });
   });
   if (copy_d(c, r0, r, (size_t)nvc * n)) return FVK_ERR_HIP;
   int it = 0;
   for (; it < n_iter; ++it) {
     const KS *gate = c.ksr + (it & 1) * 3;
-    with_tb(c, [&](auto tb) { k_bi_p<decltype(tb)::value><<<G, decltype(tb)::value, 0, c.stream>>>(n, it, nvc, r, p, u, c.pc_c, jac, z, pbuf(c, 0), G, c.ksr, c.ks); });
+    with_tb(c, [&](auto tb) {
+      with_nvc(nvc, [&](auto nv) {
+        constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
+        k_bi_p<NVC, TB><<<G, TB, 0, c.stream>>>(n, it, r, p, u, c.pc_c, jac, z, pbuf(c, 0), G, c.ksr, c.ks);
+      });
+    });
     if (!jac && precond_apply(c, imat, nvc, p, z, gate)) return FVK_ERR_HIP;
   with_tb(c, [&](auto tb) {
-  constexpr int TB = decltype(tb)::value;
-#define L(W) k_bi_spmv<W, TB><<<G, TB, 0, c.stream>>>(c.M, it, nvc, 0, c.diag, c.spv, z, u, r0, pbuf(c, 1), c.ksr)
+    with_nvc(nvc, [&](auto nv) {
+      constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
+#define L(W) k_bi_spmv<NVC, W, TB><<<G, TB, 0, c.stream>>>(c.M, it, 0, c.diag, c.spv, z, u, r0, pbuf(c, 1), c.ksr)
     FVK_WS(c.M.Ws, L);
 #undef L
+    });
   });
-    with_tb(c, [&](auto tb) { k_bi_upd1<decltype(tb)::value><<<G, decltype(tb)::value, 0, c.stream>>>(n, it, nvc, x, r, z, u, c.pc_c, jac, pbuf(c, 1), G, c.ksr); });
+    with_tb(c, [&](auto tb) {
+      with_nvc(nvc, [&](auto nv) {
+        constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
+        k_bi_upd1<NVC, TB><<<G, TB, 0, c.stream>>>(n, it, x, r, z, u, c.pc_c, jac, pbuf(c, 1), G, c.ksr);
+      });
+    });
     if (!jac && precond_apply(c, imat, nvc, r, z, gate)) return FVK_ERR_HIP;
   with_tb(c, [&](auto tb) {
-  constexpr int TB = decltype(tb)::value;
-#define L(W) k_bi_spmv<W, TB><<<G, TB, 0, c.stream>>>(c.M, it, nvc, 1, c.diag, c.spv, z, v, r, pbuf(c, 2), c.ksr)
+    with_nvc(nvc, [&](auto nv) {
+      constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
+#define L(W) k_bi_spmv<NVC, W, TB><<<G, TB, 0, c.stream>>>(c.M, it, 1, c.diag, c.spv, z, v, r, pbuf(c, 2), c.ksr)
     FVK_WS(c.M.Ws, L);
 #undef L
+    });
   });
-    with_tb(c, [&](auto tb) { k_bi_upd2<decltype(tb)::value><<<G, decltype(tb)::value, 0, c.stream>>>(n, it, nvc, x, r, z, v, r0, pbuf(c, 2), G, pbuf(c, 0), c.ksr); });
+    with_tb(c, [&](auto tb) {
+      with_nvc(nvc, [&](auto nv) {
+        constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
+        k_bi_upd2<NVC, TB><<<G, TB, 0, c.stream>>>(n, it, x, r, z, v, r0, pbuf(c, 2), G, pbuf(c, 0), c.ksr);
+      });
+    });
   }
   k_bi_final<<<1, RB64, 0, c.stream>>>(it, nvc, pbuf(c, 0), G, c.ksr, c.ks);
   FVK_HIP(hipGetLastError());
