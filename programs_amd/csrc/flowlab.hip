@@ -68,6 +68,13 @@ struct FlCtx {
   // Krylov work: 6 vectors x 3 components, partials, scalars
   double *wk = nullptr, *pc = nullptr, *part = nullptr;
   FlKS *ks = nullptr;
+  // the matrix of a solve by slots (slot k of row i at k*n + i, column -1:
+  // none) when no row has more than 8 entries; ew: slots, 0: CSR only
+  int ew = 0;
+  int *ecol = nullptr;
+  double *eval = nullptr;
+  // a solve's end as the host sees it (FlWatch)
+  unsigned long long *watch = nullptr, watch_tag = 0;
   double *scal = nullptr;  // c_rat and scratch scalars
   // workspaces of the calls on host arrays, kept once made: matrix values,
   // solution and right-hand side; boundary values and boundary faces
@@ -336,11 +343,49 @@ __global__ __launch_bounds__(BS) void k_fl_grad_bnd(int nbf, const int *__restri
 }
 
 // ---------------------------------------------------------------- Krylov
-// csr_matvec_prod (matrix_utils_m.f90:70-82): y(i) = 0 + sum a x in CSR order
-__device__ __forceinline__ double fl_row_mv(const int *ia, const int *ja, const double *a, const double *x, int i) {
-  double y = 0.0;
-  for (int k = ia[i]; k < ia[i + 1]; ++k) y = y + a[k] * x[ja[k]];
-  return y;
+// The matrix of a solve.  A thread per row of the CSR arrays reads addresses
+// a row apart; by slots neighbouring threads read neighbouring addresses.
+struct FlMat {
+  int n;
+  const int *ia, *ja, *ecol;
+  const double *a, *eval;
+};
+
+__global__ __launch_bounds__(BS) void k_fl_slots(FlMat M, int ew, int *__restrict__ ecol, double *__restrict__ eval) {
+  const int i = blockIdx.x * BS + threadIdx.x;
+  if (i >= M.n) return;
+  const int k0 = M.ia[i], nk = M.ia[i + 1] - k0;
+  for (int k = 0; k < ew; ++k) {
+    const size_t o = (size_t)k * M.n + i;
+    if (ecol) ecol[o] = k < nk ? M.ja[k0 + k] : -1;
+    if (eval) eval[o] = k < nk ? M.a[k0 + k] : 0.0;
+  }
+}
+
+// csr_matvec_prod (matrix_utils_m.f90:70-82): y(i) = 0 + sum a x in CSR
+// order, x(q, j) the value of component q at row j; WS: slots, 0: CSR
+template <int NC, int WS, class X>
+__device__ __forceinline__ void fl_row_mv(const FlMat &M, int i, X x, double (&y)[NC]) {
+#pragma unroll
+  for (int q = 0; q < NC; ++q) y[q] = 0.0;
+  if (WS > 0) {
+#pragma unroll
+    for (int k = 0; k < WS; ++k) {
+      const size_t o = (size_t)k * M.n + i;
+      const int j = M.ecol[o];
+      const double a = M.eval[o];
+      if (j >= 0)
+#pragma unroll
+        for (int q = 0; q < NC; ++q) y[q] = y[q] + a * x(q, j);
+    }
+  } else {
+    for (int k = M.ia[i]; k < M.ia[i + 1]; ++k) {
+      const int j = M.ja[k];
+      const double a = M.a[k];
+#pragma unroll
+      for (int q = 0; q < NC; ++q) y[q] = y[q] + a * x(q, j);
+    }
+  }
 }
 
 // preconditioner (solv_m.f90:224-250) over one level of rows
@@ -404,177 +449,15 @@ __global__ __launch_bounds__(BS) void k_fl_bwd_level(const int *__restrict__ row
   }
 }
 
-// Block partial sums of NV per-row terms per component, stored at
-// part[(c*NV + j)*RG + block]
-template <int NV, class F>
-__device__ __forceinline__ void fl_partials(int n, int ncmp, const FlKS *ks, double *part, F term) {
-  int r0, r1;
-  block_rows<RB>(n, r0, r1);
-  for (int c = 0; c < 3; ++c) {
-    if (c >= ncmp) break;
-    double v[NV];
-#pragma unroll
-    for (int j = 0; j < NV; ++j) v[j] = 0.0;
-    if (!ks[c].done)
-      for (int i = r0 + (int)threadIdx.x; i < r1; i += RB) term(c, i, v);
-    rblock_sum<NV, RB>(v);
-    if (threadIdx.x == 0)
-#pragma unroll
-      for (int j = 0; j < NV; ++j) part[(size_t)(c * NV + j) * RG + blockIdx.x] = v[j];
-  }
-}
-
-// initial residual: wk1 = A phi; res = res - wk1; wk1 = res; partial |res|
-__global__ __launch_bounds__(RB) void k_fl_init(int n, int ncmp, const int *__restrict__ ia, const int *__restrict__ ja,
-                                                const double *__restrict__ a, const double *__restrict__ phi,
-                                                double *res, double *w1, const FlKS *ks, double *part) {
-  fl_partials<1>(n, ncmp, ks, part, [&](int c, int i, double *v) {
-    const double y = fl_row_mv(ia, ja, a, phi + (size_t)c * n, i);
-    const double r = res[(size_t)c * n + i] - y;
-    res[(size_t)c * n + i] = r;
-    w1[(size_t)c * n + i] = r;
-    v[0] += fabs(r);
-  });
-}
-
-// s = sum x*y (two vectors)
-__global__ __launch_bounds__(RB) void k_fl_dot(int n, int ncmp, const double *__restrict__ x,
-                                               const double *__restrict__ y, const FlKS *ks, double *part) {
-  fl_partials<1>(n, ncmp, ks, part, [&](int c, int i, double *v) {
-    v[0] += x[(size_t)c * n + i] * y[(size_t)c * n + i];
-  });
-}
-
-// q = A p and sum p*q (CG)
-__global__ __launch_bounds__(RB) void k_fl_mv_dot(int n, int ncmp, const int *__restrict__ ia,
-                                                  const int *__restrict__ ja, const double *__restrict__ a,
-                                                  const double *__restrict__ p, double *q, const double *__restrict__ d,
-                                                  const FlKS *ks, double *part) {
-  fl_partials<1>(n, ncmp, ks, part, [&](int c, int i, double *v) {
-    const double y = fl_row_mv(ia, ja, a, p + (size_t)c * n, i);
-    q[(size_t)c * n + i] = y;
-    v[0] += d[(size_t)c * n + i] * y;
-  });
-}
-
-// v = A z, sum v*r and sum (v+small)^2 (BiCGStab, solv_m.f90:190-196)
-__global__ __launch_bounds__(RB) void k_fl_mv_dot2(int n, int ncmp, const int *__restrict__ ia,
-                                                   const int *__restrict__ ja, const double *__restrict__ a,
-                                                   const double *__restrict__ z, double *vv,
-                                                   const double *__restrict__ r, const FlKS *ks, double *part) {
-  fl_partials<2>(n, ncmp, ks, part, [&](int c, int i, double *v) {
-    const double y = fl_row_mv(ia, ja, a, z + (size_t)c * n, i);
-    vv[(size_t)c * n + i] = y;
-    v[0] += y * r[(size_t)c * n + i];
-    v[1] += (y + SMALL) * (y + SMALL);
-  });
-}
-
-// phi += alpha p; r -= alpha q; partial |r| (alpha = cof[ai])
-__global__ __launch_bounds__(RB) void k_fl_upd(int n, int ncmp, int ai, double *phi, const double *__restrict__ p,
-                                               double *r, const double *__restrict__ q, const FlKS *ks, double *part,
-                                               int with_norm) {
-  fl_partials<1>(n, ncmp, ks, part, [&](int c, int i, double *v) {
-    const double al = ks[c].cof[ai];
-    phi[(size_t)c * n + i] = phi[(size_t)c * n + i] + al * p[(size_t)c * n + i];
-    const double rr = r[(size_t)c * n + i] - al * q[(size_t)c * n + i];
-    r[(size_t)c * n + i] = rr;
-    if (with_norm) v[0] += fabs(rr);
-  });
-}
-
-// p = z + beta p (CG) or p = r + omega (p - alpha u) (BiCGStab)
-__global__ __launch_bounds__(BS) void k_fl_dir(int n, int ncmp, int bicg, double *p, const double *__restrict__ z,
-                                               const double *__restrict__ u, const FlKS *ks) {
-  const int i = blockIdx.x * BS + threadIdx.x;
-  if (i >= n) return;
-  for (int c = 0; c < ncmp; ++c) {
-    if (ks[c].done) continue;
-    const size_t o = (size_t)c * n + i;
-    if (bicg) p[o] = z[o] + ks[c].cof[6] * (p[o] - ks[c].cof[2] * u[o]);
-    else p[o] = z[o] + ks[c].cof[3] * p[o];
-  }
-}
-
-__device__ __forceinline__ double fl_total(const double *part, int P, int comp) {
-  double v[1];
-  v[0] = 0.0;
-  for (int b = threadIdx.x; b < P; b += RB) v[0] += part[(size_t)comp * RG + b];
-  rblock_sum<1, RB>(v);
-  return v[0];
-}
-
-// scalar steps of cg_solver / bicg_solver; one block, thread 0 writes.
-// stage: 0 initial norm, 10 CG s/beta, 11 CG alpha, 12 CG norm/exit,
-// 20 BiCG beta/omega, 21 BiCG gamma, 22 BiCG alpha, 23 BiCG norm/exit
-__global__ __launch_bounds__(RB) void k_fl_scal(int stage, int ncmp, int P, int NV, const double *part, FlKS *ks,
-                                                double reduc, int bicg) {
-  for (int c = 0; c < ncmp; ++c) {
-    const double t0 = fl_total(part, P, c * NV);
-    const double t1 = NV > 1 ? fl_total(part, P, c * NV + 1) : 0.0;
-    if (threadIdx.x != 0) continue;
-    FlKS &k = ks[c];
-    if (stage == 0) {
-      for (int j = 0; j < 7; ++j) k.cof[j] = 0.0;
-      k.norm = t0;
-      k.norm0 = t0;
-      k.iter = 0;
-      k.done = 0;
-      if (bicg) {
-        k.cof[2] = 1.0;
-        k.cof[3] = 1.0;
-        k.cof[5] = 1.0;
-      } else {
-        k.cof[4] = 1.0 / SMALL;
-      }
-      continue;
-    }
-    if (k.done) continue;
-    switch (stage) {
-      case 10: {
-        k.cof[1] = 0.0;
-        k.cof[3] = 1.0 / (k.cof[4] + SMALL);
-        k.cof[4] = t0;
-        k.cof[3] = k.cof[3] * k.cof[4];
-        break;
-      }
-      case 11: k.cof[2] = k.cof[4] / (t0 + SMALL); break;
-      case 12:
-      case 23: {
-        k.norm = t0;
-        k.cof[1] = t0 / (k.norm0 + SMALL);
-        k.iter += 1;
-        if (k.cof[1] < reduc) k.done = 1;
-        break;
-      }
-      case 20: {
-        k.cof[1] = 0.0;
-        k.cof[4] = t0;
-        k.cof[6] = k.cof[4] * k.cof[5] / (k.cof[2] * k.cof[3] + SMALL);
-        k.cof[3] = k.cof[4];
-        break;
-      }
-      case 21: k.cof[5] = k.cof[4] / (t0 + SMALL); break;
-      case 22: {
-        k.cof[1] = t0;
-        k.cof[2] = t1;
-        k.cof[2] = k.cof[1] / (k.cof[2] + SMALL);
-        break;
-      }
-    }
-  }
-}
-
-// a new solve: every component open (the initial residual kernel is gated
-// like the others)
-__global__ void k_fl_ks_open(FlKS *ks, int ncmp) {
-  if (threadIdx.x == 0)
-    for (int c = 0; c < ncmp; ++c) ks[c].done = 0;
-}
-
-static int fl_pgrid(int n) { return red_grid(n); }
-
-// ---------------------------------------------------------------- one-launch sweeps
+// The Krylov kernels leave a partial per block of NC (or NC pairs of) sums;
+// the kernel that uses a sum adds the partials itself, every block in the same
+// tree, so that a scalar step costs no launch of its own.  Only the end of an
+// iteration is a launch (k_fl_end): the sweeps after it are skipped once every
+// component is done.  A CG iteration takes 6 launches, a BiCGStab iteration
+// 10; with a launch per scalar step they were 9 and 15, and on the momentum
+// systems, which end after one iteration, most of them found nothing to do
+// (96^3, three outer iterations: 38.3 -> 30.4 ms; there the products by slots
+// take 24.9 us with the direction update, by CSR they took 35.6 us without).
 __device__ __forceinline__ bool fl_all_done(const FlKS *ks, int ncmp) {
   if (!ks) return false;
   for (int c = 0; c < ncmp; ++c)
@@ -582,6 +465,285 @@ __device__ __forceinline__ bool fl_all_done(const FlKS *ks, int ncmp) {
   return true;
 }
 
+// f(component, index into a vector's components, row) for this block's rows
+// of the components that are not done
+template <int NC, class F>
+__device__ __forceinline__ void fl_rows(int n, const int (&dn)[NC], F f) {
+  int r0, r1;
+  block_rows<RB>(n, r0, r1);
+  for (int i = r0 + (int)threadIdx.x; i < r1; i += RB)
+#pragma unroll
+    for (int q = 0; q < NC; ++q)
+      if (!dn[q]) f(q, (size_t)q * n + i);
+}
+template <int NC>
+__device__ __forceinline__ bool fl_open(const FlKS *ks, int (&dn)[NC]) {
+  bool any = false;
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    dn[q] = ks[q].done;
+    any = any || !dn[q];
+  }
+  return any;
+}
+
+// initial residual: res = res - A phi; w1 = res; sums |res| and (BiCGStab)
+// res.res; the search direction p (and u) start at zero
+template <int NC, int WS>
+__global__ __launch_bounds__(RB) void k_fl_init(FlMat M, const double *__restrict__ phi, double *res, double *w1,
+                                                double *p, double *u, double *part) {
+  const int n = M.n;
+  double v[2 * NC];
+#pragma unroll
+  for (int q = 0; q < 2 * NC; ++q) v[q] = 0.0;
+  int r0, r1;
+  block_rows<RB>(n, r0, r1);
+  for (int i = r0 + (int)threadIdx.x; i < r1; i += RB) {
+    double y[NC];
+    fl_row_mv<NC, WS>(M, i, [&](int q, int j) { return phi[(size_t)q * n + j]; }, y);
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      const size_t o = (size_t)q * n + i;
+      const double r = res[o] - y[q];
+      res[o] = r;
+      w1[o] = r;
+      p[o] = 0.0;
+      if (u) u[o] = 0.0;
+      v[q] += fabs(r);
+      v[NC + q] += r * r;
+    }
+  }
+  store_partials<2 * NC, RB>(v, part);
+}
+
+// sum x.y
+template <int NC>
+__global__ __launch_bounds__(RB) void k_fl_dot(int n, const double *__restrict__ x, const double *__restrict__ y,
+                                               const FlKS *ks, double *part) {
+  int dn[NC];
+  if (!fl_open<NC>(ks, dn)) return;
+  double v[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) v[q] = 0.0;
+  fl_rows<NC>(n, dn, [&](int q, size_t o) { v[q] += x[o] * y[o]; });
+  store_partials<NC, RB>(v, part);
+}
+
+// CG: beta from z.r (partS) ; p = z + beta p ; q = A p ; sum p.q.  The
+// neighbours' p is formed from z and the old p.  cof[0]: z.r for k_fl_end
+// (the other blocks still read the old one, cof[4]).
+template <int NC, int WS>
+__global__ __launch_bounds__(RB) void k_fl_cg_pq(FlMat M, const double *__restrict__ z, const double *__restrict__ pold,
+                                                 double *__restrict__ pnew, double *__restrict__ qv,
+                                                 const double *__restrict__ partS, int P, FlKS *ks, double *part) {
+  int dn[NC];
+  if (!fl_open<NC>(ks, dn)) return;
+  const int n = M.n;
+  double s[NC], beta[NC], v[NC];
+  load_totals<NC, RB>(partS, P, s);
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    beta[q] = 1.0 / (ks[q].cof[4] + SMALL);
+    beta[q] = beta[q] * s[q];
+    v[q] = 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && !dn[q]) ks[q].cof[0] = s[q];
+  }
+  int r0, r1;
+  block_rows<RB>(n, r0, r1);
+  for (int i = r0 + (int)threadIdx.x; i < r1; i += RB) {
+    double y[NC];
+    fl_row_mv<NC, WS>(M, i, [&](int q, int j) {
+      const size_t o = (size_t)q * n + j;
+      return z[o] + beta[q] * pold[o];
+    }, y);
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      if (dn[q]) continue;
+      const size_t o = (size_t)q * n + i;
+      const double pi = z[o] + beta[q] * pold[o];
+      pnew[o] = pi;
+      qv[o] = y[q];
+      v[q] += pi * y[q];
+    }
+  }
+  store_partials<NC, RB>(v, part);
+}
+
+// CG: alpha = z.r / p.q (partQ) ; phi += alpha p ; r -= alpha q ; sum |r|
+template <int NC>
+__global__ __launch_bounds__(RB) void k_fl_cg_upd(int n, double *__restrict__ phi, const double *__restrict__ p,
+                                                  double *__restrict__ r, const double *__restrict__ qv,
+                                                  const double *__restrict__ partQ, int P, const FlKS *ks,
+                                                  double *part) {
+  int dn[NC];
+  if (!fl_open<NC>(ks, dn)) return;
+  double t[NC], al[NC], v[NC];
+  load_totals<NC, RB>(partQ, P, t);
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    al[q] = ks[q].cof[0] / (t[q] + SMALL);
+    v[q] = 0.0;
+  }
+  fl_rows<NC>(n, dn, [&](int q, size_t o) {
+    phi[o] = phi[o] + al[q] * p[o];
+    const double rr = r[o] - al[q] * qv[o];
+    r[o] = rr;
+    v[q] += fabs(rr);
+  });
+  store_partials<NC, RB>(v, part);
+}
+
+// BiCGStab: p = r + omega (p - alpha u)
+template <int NC>
+__global__ __launch_bounds__(BS) void k_fl_bi_dir(int n, double *p, const double *__restrict__ r,
+                                                  const double *__restrict__ u, const FlKS *ks) {
+  const int i = blockIdx.x * BS + threadIdx.x;
+  if (i >= n) return;
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    if (ks[q].done) continue;
+    const size_t o = (size_t)q * n + i;
+    p[o] = r[o] + ks[q].cof[6] * (p[o] - ks[q].cof[2] * u[o]);
+  }
+}
+
+// BiCGStab: y = A z ; sum y.d, and with SQ sum (y + small)^2 (solv_m.f90:190-196)
+template <int NC, int WS, bool SQ>
+__global__ __launch_bounds__(RB) void k_fl_bi_mv(FlMat M, const double *__restrict__ z, double *__restrict__ y,
+                                                 const double *__restrict__ d, const FlKS *ks, double *part) {
+  int dn[NC];
+  if (!fl_open<NC>(ks, dn)) return;
+  const int n = M.n;
+  constexpr int NV = SQ ? 2 * NC : NC;
+  double v[NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) v[q] = 0.0;
+  int r0, r1;
+  block_rows<RB>(n, r0, r1);
+  for (int i = r0 + (int)threadIdx.x; i < r1; i += RB) {
+    double w[NC];
+    fl_row_mv<NC, WS>(M, i, [&](int q, int j) { return z[(size_t)q * n + j]; }, w);
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      if (dn[q]) continue;
+      const size_t o = (size_t)q * n + i;
+      y[o] = w[q];
+      v[q] += w[q] * d[o];
+      if (SQ) v[NV - NC + q] += (w[q] + SMALL) * (w[q] + SMALL);
+    }
+  }
+  store_partials<NV, RB>(v, part);
+}
+
+// BiCGStab, first half: gamma = beta / u.r0 (partT) ; phi += gamma z ;
+// r -= gamma u
+template <int NC>
+__global__ __launch_bounds__(RB) void k_fl_bi_upd1(int n, double *__restrict__ phi, const double *__restrict__ z,
+                                                   double *__restrict__ r, const double *__restrict__ u,
+                                                   const double *__restrict__ partT, int P, FlKS *ks) {
+  int dn[NC];
+  if (!fl_open<NC>(ks, dn)) return;
+  double t[NC], g[NC];
+  load_totals<NC, RB>(partT, P, t);
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    g[q] = ks[q].cof[4] / (t[q] + SMALL);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && !dn[q]) ks[q].cof[5] = g[q];
+  }
+  fl_rows<NC>(n, dn, [&](int q, size_t o) {
+    phi[o] = phi[o] + g[q] * z[o];
+    r[o] = r[o] - g[q] * u[o];
+  });
+}
+
+// BiCGStab, second half: alpha from partD ; phi += alpha z ; r -= alpha v ;
+// sums |r| and r.r0 (the next iteration's beta)
+template <int NC>
+__global__ __launch_bounds__(RB) void k_fl_bi_upd2(int n, double *__restrict__ phi, const double *__restrict__ z,
+                                                   double *__restrict__ r, const double *__restrict__ vv,
+                                                   const double *__restrict__ r0v, const double *__restrict__ partD,
+                                                   int P, FlKS *ks, double *part) {
+  int dn[NC];
+  if (!fl_open<NC>(ks, dn)) return;
+  double t[2 * NC], al[NC], v[2 * NC];
+  load_totals<2 * NC, RB>(partD, P, t);
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    al[q] = t[q] / (t[NC + q] + SMALL);
+    v[q] = v[NC + q] = 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && !dn[q]) ks[q].cof[2] = al[q];
+  }
+  fl_rows<NC>(n, dn, [&](int q, size_t o) {
+    phi[o] = phi[o] + al[q] * z[o];
+    const double rr = r[o] - al[q] * vv[o];
+    r[o] = rr;
+    v[q] += fabs(rr);
+    v[NC + q] += rr * r0v[o];
+  });
+  store_partials<2 * NC, RB>(v, part);
+}
+
+// The scalar steps between two iterations of cg_solver / bicg_solver (one
+// block): the start (first) or the norm and the exit test, then for BiCGStab
+// the next beta and omega.  part: NV totals per component, |r| and (BiCGStab,
+// start) a second one.  watch: where the host finds tag and whether every
+// component is done.
+template <int NC, bool BICG>
+__global__ __launch_bounds__(RB) void k_fl_end(int first, int P, const double *__restrict__ part, FlKS *ks, double reduc,
+                                               unsigned long long *watch, unsigned long long tag) {
+  double t[2 * NC];
+#pragma unroll
+  for (int q = 0; q < 2 * NC; ++q) t[q] = 0.0;
+  bool open = true;
+  if (!first) open = !fl_all_done(ks, NC);
+  if (open) {
+    if (BICG) {
+      load_totals<2 * NC, RB>(part, P, t);
+    } else {
+      double t1[NC];
+      load_totals<NC, RB>(part, P, t1);
+#pragma unroll
+      for (int q = 0; q < NC; ++q) t[q] = t1[q];
+    }
+  }
+  if (threadIdx.x != 0) return;
+  bool all = true;
+  if (open)
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      FlKS &k = ks[q];
+      if (first) {
+        for (int j = 0; j < 7; ++j) k.cof[j] = 0.0;
+        k.norm = k.norm0 = t[q];
+        k.iter = 0;
+        k.done = 0;
+        if (BICG) k.cof[2] = k.cof[3] = k.cof[5] = 1.0;
+        else k.cof[4] = 1.0 / SMALL;
+      } else {
+        if (k.done) continue;
+        k.norm = t[q];
+        k.cof[1] = t[q] / (k.norm0 + SMALL);
+        k.iter += 1;
+        if (k.cof[1] < reduc) {
+          k.done = 1;
+          continue;
+        }
+        if (!BICG) k.cof[4] = k.cof[0];
+      }
+      all = false;
+      if (BICG) {
+        k.cof[1] = 0.0;
+        k.cof[4] = t[NC + q];
+        k.cof[6] = k.cof[4] * k.cof[5] / (k.cof[2] * k.cof[3] + SMALL);
+        k.cof[3] = k.cof[4];
+      }
+    }
+  __hip_atomic_store(watch, tag << 1 | (all ? 1ull : 0ull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+static int fl_pgrid(int n) { return red_grid(n); }
+
+// ---------------------------------------------------------------- one-launch sweeps
 __global__ __launch_bounds__(BS) void k_fl_mark(size_t cnt, double *out, int *ticket, const FlKS *ks, int ncmp) {
   if (fl_all_done(ks, ncmp)) return;
   unsigned long long *o = (unsigned long long *)out;
@@ -862,48 +1024,86 @@ static int fl_direct(FlCtx &c, int ncmp, const double *a, const double *b, doubl
   return 0;
 }
 
+// Whether an iteration's k_fl_end found every component done.  It stores the
+// answer in pinned memory, where the host looks for it while the next
+// iteration is queued already: the device stays busy and at most one iteration
+// is queued after the end, whose launches find nothing to do.  The wait ends
+// when the stream has nothing left to run.
+static int fl_watch(FlCtx &c, unsigned long long tag, bool &done) {
+  const unsigned long long *w = c.watch + (tag & 1);
+  for (unsigned spin = 1;; ++spin) {
+    const unsigned long long v = __atomic_load_n(w, __ATOMIC_ACQUIRE);
+    if (v >> 1 == tag) {
+      done = (v & 1) != 0;
+      return 0;
+    }
+    if (spin % 4096 == 0) {
+      const hipError_t e = hipStreamQuery(c.stream);
+      if (e == hipErrorNotReady) continue;
+      FVK_HIP(e);
+      const unsigned long long last = __atomic_load_n(w, __ATOMIC_ACQUIRE);
+      done = last >> 1 == tag && (last & 1);
+      return 0;
+    }
+  }
+}
+
+template <int NC, int WS>
+static int fl_solve_run(FlCtx &c, const FlMat &M, bool bicg, const double *a, double *phi, double *res, int n_iter,
+                        double reduc) {
+  const int n = c.n, P = fl_pgrid(n), G = grid_for(n);
+  double *w1 = wkv(c, 0), *w2 = wkv(c, 1), *w3 = wkv(c, 2), *w4 = wkv(c, 3), *w5 = wkv(c, 4), *wt = wkv(c, 5);
+  double *pa = c.part, *pb = c.part + (size_t)6 * RG;
+  auto end = [&](int first, const double *part) {
+    const unsigned long long tag = ++c.watch_tag;
+    if (bicg) k_fl_end<NC, true><<<1, RB, 0, c.stream>>>(first, P, part, c.ks, reduc, c.watch + (tag & 1), tag);
+    else k_fl_end<NC, false><<<1, RB, 0, c.stream>>>(first, P, part, c.ks, reduc, c.watch + (tag & 1), tag);
+  };
+  k_fl_init<NC, WS><<<P, RB, 0, c.stream>>>(M, phi, res, w1, w2, bicg ? w3 : nullptr, pa);
+  end(1, pa);
+  int rc = fl_precond(c, a);
+  if (rc) return rc;
+  for (int it = 0; it < n_iter; ++it) {
+    if (!bicg) {
+      double *po = it & 1 ? w5 : w2, *pn = it & 1 ? w2 : w5;
+      if ((rc = fl_direct(c, NC, a, w1, wt, w3, c.ks))) return rc;
+      k_fl_dot<NC><<<P, RB, 0, c.stream>>>(n, w1, w3, c.ks, pa);
+      k_fl_cg_pq<NC, WS><<<P, RB, 0, c.stream>>>(M, w3, po, pn, w4, pa, P, c.ks, pb);
+      k_fl_cg_upd<NC><<<P, RB, 0, c.stream>>>(n, phi, pn, w1, w4, pb, P, c.ks, pa);
+      end(0, pa);
+    } else {
+      k_fl_bi_dir<NC><<<G, BS, 0, c.stream>>>(n, w2, w1, w3, c.ks);
+      if ((rc = fl_direct(c, NC, a, w2, wt, w5, c.ks))) return rc;
+      k_fl_bi_mv<NC, WS, false><<<P, RB, 0, c.stream>>>(M, w5, w3, res, c.ks, pb);
+      k_fl_bi_upd1<NC><<<P, RB, 0, c.stream>>>(n, phi, w5, w1, w3, pb, P, c.ks);
+      if ((rc = fl_direct(c, NC, a, w1, wt, w5, c.ks))) return rc;
+      k_fl_bi_mv<NC, WS, true><<<P, RB, 0, c.stream>>>(M, w5, w4, w1, c.ks, pa);
+      k_fl_bi_upd2<NC><<<P, RB, 0, c.stream>>>(n, phi, w5, w1, w4, res, pa, P, c.ks, pb);
+      end(0, pb);
+    }
+    bool done = false;
+    if (it > 0 && it + 1 < n_iter && (rc = fl_watch(c, c.watch_tag - 1, done))) return rc;
+    if (done) break;
+  }
+  FVK_HIP(hipGetLastError());
+  return 0;
+}
+
 // lin_eqns_solver (solv_m.f90:10-30) for ncmp right-hand sides sharing the
 // matrix a (device, CSR of the context): phi and res (the right-hand side
 // in, the initial residual out) component-major on the device; norms to
 // ks[c].norm.  isol 1: cg_solver, 2: bicg_solver.
 static int fl_solve(FlCtx &c, int isol, int ncmp, const double *a, double *phi, double *res, int n_iter,
                     double reduc) {
-  const int n = c.n, P = fl_pgrid(n), G = grid_for(n);
-  double *w1 = wkv(c, 0), *w2 = wkv(c, 1), *w3 = wkv(c, 2), *w4 = wkv(c, 3), *w5 = wkv(c, 4), *wt = wkv(c, 5);
-  const bool bicg = isol == 2;
-  FVK_HIP(hipMemsetAsync(c.wk, 0, sizeof(double) * 5 * 3 * (size_t)n, c.stream));
-  k_fl_ks_open<<<1, 64, 0, c.stream>>>(c.ks, ncmp);
-  k_fl_init<<<P, RB, 0, c.stream>>>(n, ncmp, c.ia, c.ja, a, phi, res, w1, c.ks, c.part);
-  k_fl_scal<<<1, RB, 0, c.stream>>>(0, ncmp, P, 1, c.part, c.ks, reduc, bicg ? 1 : 0);
-  int rc = fl_precond(c, a);
-  if (rc) return rc;
-  for (int it = 0; it < n_iter; ++it) {
-    if (!bicg) {
-      if ((rc = fl_direct(c, ncmp, a, w1, wt, w3, c.ks))) return rc;
-      k_fl_dot<<<P, RB, 0, c.stream>>>(n, ncmp, w1, w3, c.ks, c.part);
-      k_fl_scal<<<1, RB, 0, c.stream>>>(10, ncmp, P, 1, c.part, c.ks, reduc, 0);
-      k_fl_dir<<<G, BS, 0, c.stream>>>(n, ncmp, 0, w2, w3, nullptr, c.ks);
-      k_fl_mv_dot<<<P, RB, 0, c.stream>>>(n, ncmp, c.ia, c.ja, a, w2, w3, w2, c.ks, c.part);
-      k_fl_scal<<<1, RB, 0, c.stream>>>(11, ncmp, P, 1, c.part, c.ks, reduc, 0);
-      k_fl_upd<<<P, RB, 0, c.stream>>>(n, ncmp, 2, phi, w2, w1, w3, c.ks, c.part, 1);
-      k_fl_scal<<<1, RB, 0, c.stream>>>(12, ncmp, P, 1, c.part, c.ks, reduc, 0);
-    } else {
-      k_fl_dot<<<P, RB, 0, c.stream>>>(n, ncmp, w1, res, c.ks, c.part);
-      k_fl_scal<<<1, RB, 0, c.stream>>>(20, ncmp, P, 1, c.part, c.ks, reduc, 1);
-      k_fl_dir<<<G, BS, 0, c.stream>>>(n, ncmp, 1, w2, w1, w3, c.ks);
-      if ((rc = fl_direct(c, ncmp, a, w2, wt, w5, c.ks))) return rc;
-      k_fl_mv_dot<<<P, RB, 0, c.stream>>>(n, ncmp, c.ia, c.ja, a, w5, w3, res, c.ks, c.part);
-      k_fl_scal<<<1, RB, 0, c.stream>>>(21, ncmp, P, 1, c.part, c.ks, reduc, 1);
-      k_fl_upd<<<P, RB, 0, c.stream>>>(n, ncmp, 5, phi, w5, w1, w3, c.ks, c.part, 0);
-      if ((rc = fl_direct(c, ncmp, a, w1, wt, w5, c.ks))) return rc;
-      k_fl_mv_dot2<<<P, RB, 0, c.stream>>>(n, ncmp, c.ia, c.ja, a, w5, w4, w1, c.ks, c.part);
-      k_fl_scal<<<1, RB, 0, c.stream>>>(22, ncmp, P, 2, c.part, c.ks, reduc, 1);
-      k_fl_upd<<<P, RB, 0, c.stream>>>(n, ncmp, 2, phi, w5, w1, w4, c.ks, c.part, 1);
-      k_fl_scal<<<1, RB, 0, c.stream>>>(23, ncmp, P, 1, c.part, c.ks, reduc, 1);
-    }
-  }
-  FVK_HIP(hipGetLastError());
-  return 0;
+  const FlMat M{c.n, c.ia, c.ja, c.ecol, a, c.eval};
+  if (c.ew) k_fl_slots<<<grid_for(c.n), BS, 0, c.stream>>>(M, c.ew, nullptr, c.eval);
+  const bool bi = isol == 2;
+#define RUN(W)                                                                                    \
+  (ncmp == 1   ? fl_solve_run<1, W>(c, M, bi, a, phi, res, n_iter, reduc)                         \
+   : ncmp == 2 ? fl_solve_run<2, W>(c, M, bi, a, phi, res, n_iter, reduc)                         \
+               : fl_solve_run<3, W>(c, M, bi, a, phi, res, n_iter, reduc))
+  return c.ew == 4 ? RUN(4) : c.ew == 5 ? RUN(5) : c.ew == 7 ? RUN(7) : c.ew == 8 ? RUN(8) : RUN(0);
+#undef RUN
 }
 
 // ---------------------------------------------------------------- SIMPLE
@@ -1176,8 +1376,9 @@ __global__ __launch_bounds__(RB) void k_fl_inout(int nbf, const int *__restrict_
 }
 
 __global__ __launch_bounds__(RB) void k_fl_crat(int P, const double *part, double *scal) {
-  const double ci = fl_total(part, P, 0);
-  const double co = fl_total(part, P, 1);
+  double t[2];
+  load_totals<2, RB>(part, P, t);
+  const double ci = t[0], co = t[1];
   if (threadIdx.x == 0) {
     double r = ci / (co + SMALL);
     r = fabs(r);
@@ -1330,7 +1531,7 @@ static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
 #define A(ptr, cnt_) if (!rc) rc = fl_alloc(c, &ptr, cnt_)
 #define U(ptr, vec) if (!rc) rc = fl_up(c, &ptr, vec)
   U(c.ia, ia); U(c.ja, ja); U(c.kii, kii); U(c.klo, klo); U(c.kup, kup); U(c.tpos, tpos);
-  A(c.wk, (size_t)6 * 3 * n); A(c.pc, n); A(c.part, (size_t)6 * RG); A(c.ks, 3); A(c.scal, 8);
+  A(c.wk, (size_t)6 * 3 * n); A(c.pc, n); A(c.part, (size_t)12 * RG); A(c.ks, 3); A(c.scal, 8);
   A(c.sweep_int, 4);
 #undef A
 #undef U
@@ -1344,6 +1545,30 @@ static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
   if (c.one_launch) {
     if ((rc = fl_parts_setup(c))) return rc;
     c.parts = true;
+  }
+  FVK_HIP(hipHostMalloc((void **)&c.watch, 2 * sizeof *c.watch, hipHostMallocDefault));
+  c.watch[0] = c.watch[1] = 0;
+  // rows of 4, 5 or 7 entries: triangles, quadrangles, hexahedra; by slots
+  // unless half of them would be empty or there is no memory for them
+  int w = 0;
+  for (int i = 0; i < n; ++i) w = std::max(w, ia[i + 1] - ia[i]);
+  w = w <= 4 ? 4 : w == 6 ? 7 : w;
+  if (w <= 8 && (size_t)w * n <= 2 * (size_t)c.nnz) {
+    void *q = nullptr, *v = nullptr;
+    if (hipMalloc(&q, (size_t)w * n * sizeof(int)) == hipSuccess &&
+        hipMalloc(&v, (size_t)w * n * sizeof(double)) == hipSuccess) {
+      c.owned.push_back(q);
+      c.owned.push_back(v);
+      c.ecol = (int *)q;
+      c.eval = (double *)v;
+      c.ew = w;
+      k_fl_slots<<<grid_for(n), BS, 0, c.stream>>>(FlMat{n, c.ia, c.ja, nullptr, nullptr, nullptr}, w, c.ecol, nullptr);
+      FVK_HIP(hipGetLastError());
+      FVK_HIP(hipStreamSynchronize(c.stream));
+    } else {
+      (void)hipGetLastError();
+      if (q) (void)hipFree(q);
+    }
   }
   return 0;
 }
@@ -1446,6 +1671,8 @@ static void fl_ctx_free(FlCtx &c) {
   c.owned.clear();
   sweep_exec_free(c.sw);
   c.io.free();
+  if (c.watch) (void)hipHostFree(c.watch);
+  c.watch = nullptr;
   if (c.stream) hipStreamDestroy(c.stream);
   c.stream = nullptr;
 }
