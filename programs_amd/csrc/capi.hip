@@ -245,6 +245,7 @@ static int ctx_build(Ctx &c, const Topo &t, int device, int flags) {
   c.io.stream = c.stream;
   FVK_HIP(hipEventCreate(&c.ev0));
   FVK_HIP(hipEventCreate(&c.ev1));
+  FVK_HIP(c.watch.init());
   FVK_HIP(hipHostMalloc((void **)&c.poll_h, 2 * sizeof(KS), hipHostMallocDefault));
   for (int k = 0; k < 2; ++k) FVK_HIP(hipEventCreateWithFlags(&c.poll_ev[k], hipEventDisableTiming));
   const int n = t.n, nf = t.nf;
@@ -372,6 +373,7 @@ static void ctx_free(Ctx &c) {
   if (c.ev1) hipEventDestroy(c.ev1);
   for (int k = 0; k < 2; ++k)
     if (c.poll_ev[k]) hipEventDestroy(c.poll_ev[k]);
+  c.watch.free();
   if (c.poll_h) hipHostFree(c.poll_h);
   c.poll_h = nullptr;
   if (c.stream) hipStreamDestroy(c.stream);
@@ -746,7 +748,7 @@ static int solve_common(fvk_ctx *cc, int kind, int imat, double reduc, int n_ite
   GUARD(cells_in(c, phi, n_vc, dx));
   GUARD(cols_in(c, res0, n_vc, dr));
   FVK_HIP(hipEventRecord(c.ev0, c.stream));
-  GUARD(krylov(c, kind, imat, reduc, n_iter, n_vc, dx, dr, not_r0 != 0));
+  GUARD(krylov(c, kind, imat, reduc, n_iter, n_vc, dx, dr, not_r0 != 0, kWatch));
   FVK_HIP(hipEventRecord(c.ev1, c.stream));
   GUARD(cells_out(c, dx, n_vc, phi));
   GUARD(cols_out(c, dr, n_vc, res0));

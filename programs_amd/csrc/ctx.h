@@ -11,6 +11,7 @@
 #include "dev.h"
 #include "hostio.h"
 #include "sweepexec.h"
+#include "watch.h"
 
 namespace fvk {
 
@@ -120,6 +121,8 @@ struct Ctx {
   double *bnd_buf = nullptr;      // 3 x n_bf boundary values (fvk_solv_grad)
   Mix mx;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // the end of a short solve (kWatch)
+  DoneWatch watch;
   // host polls of a solve's decisions: two pinned slots and their events
   KS *poll_h = nullptr;
   hipEvent_t poll_ev[2] = {nullptr, nullptr};
@@ -282,7 +285,10 @@ struct KTimer {
 
 // kind 0: PCG, 1: BiCGStab.  x, r0: nvc component vectors in device rows;
 // r0 holds the RHS on entry and the initial residual on exit.  chunk > 0:
-// stop queueing iterations once converged (checked every chunk iterations).
+// stop queueing iterations once converged (checked every chunk iterations);
+// kWatch: checked every iteration, for solves of few iterations (not while the
+// stream is captured).
+constexpr int kWatch = -1;
 int krylov(Ctx &c, int kind, int imat, double reduc, int n_iter, int nvc, double *x, double *r0, bool not_r0,
            int chunk = 0, KTimer *T = nullptr);
 int true_residual(Ctx &c, const double *x, const double *b, double *dev_out4, double *host_out4);

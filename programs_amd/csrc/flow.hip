@@ -715,7 +715,8 @@ int mom_setup(Flow &F, int it, bool &skipped) {
                                                c.spv, F.rhs, F.cs, F.frc_vol);
   FVK_HIP(hipGetLastError());
   matrix_changed(c);
-  rc = krylov(c, 1, F.cfg.imat_u, F.cfg.reduc_u, F.cfg.n_bicg, nvc, F.u, F.rhs, false);
+  rc = krylov(c, 1, F.cfg.imat_u, F.cfg.reduc_u, F.cfg.n_bicg, nvc, F.u, F.rhs, false,
+              F.capture ? 0 : kWatch);
   if (rc) return rc;
   k_mom_norm<<<1, 1, 0, c.stream>>>(it, nvc, c.ks, F.sc);
   FVK_HIP(hipGetLastError());
@@ -843,7 +844,7 @@ static int pp_solve(Flow &F, double *x, double *b) {
   switch (F.cfg.p_solver) {
     case 0:
       return krylov(c, 0, F.cfg.imat_p, F.cfg.reduc_p, F.cfg.n_cg, 1, x, b, true,
-                    F.cfg.n_cg > 64 ? chunk : 0);
+                    F.cfg.n_cg > 64 || F.capture ? chunk : kWatch);
     case 3: {
       KS h;
       NullSpace N;

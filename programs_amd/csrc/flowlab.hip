@@ -73,8 +73,7 @@ struct FlCtx {
   int ew = 0;
   int *ecol = nullptr;
   double *eval = nullptr;
-  // a solve's end as the host sees it (FlWatch)
-  unsigned long long *watch = nullptr, watch_tag = 0;
+  DoneWatch watch;
   double *scal = nullptr;  // c_rat and scratch scalars
   // workspaces of the calls on host arrays, kept once made: matrix values,
   // solution and right-hand side; boundary values and boundary faces
@@ -686,11 +685,10 @@ __global__ __launch_bounds__(RB) void k_fl_bi_upd2(int n, double *__restrict__ p
 // The scalar steps between two iterations of cg_solver / bicg_solver (one
 // block): the start (first) or the norm and the exit test, then for BiCGStab
 // the next beta and omega.  part: NV totals per component, |r| and (BiCGStab,
-// start) a second one.  watch: where the host finds tag and whether every
-// component is done.
+// start) a second one.
 template <int NC, bool BICG>
 __global__ __launch_bounds__(RB) void k_fl_end(int first, int P, const double *__restrict__ part, FlKS *ks, double reduc,
-                                               unsigned long long *watch, unsigned long long tag) {
+                                               DoneSlot slot) {
   double t[2 * NC];
 #pragma unroll
   for (int q = 0; q < 2 * NC; ++q) t[q] = 0.0;
@@ -738,7 +736,7 @@ __global__ __launch_bounds__(RB) void k_fl_end(int first, int P, const double *_
         k.cof[3] = k.cof[4];
       }
     }
-  __hip_atomic_store(watch, tag << 1 | (all ? 1ull : 0ull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  done_store(slot, all);
 }
 
 static int fl_pgrid(int n) { return red_grid(n); }
@@ -1024,30 +1022,6 @@ static int fl_direct(FlCtx &c, int ncmp, const double *a, const double *b, doubl
   return 0;
 }
 
-// Whether an iteration's k_fl_end found every component done.  It stores the
-// answer in pinned memory, where the host looks for it while the next
-// iteration is queued already: the device stays busy and at most one iteration
-// is queued after the end, whose launches find nothing to do.  The wait ends
-// when the stream has nothing left to run.
-static int fl_watch(FlCtx &c, unsigned long long tag, bool &done) {
-  const unsigned long long *w = c.watch + (tag & 1);
-  for (unsigned spin = 1;; ++spin) {
-    const unsigned long long v = __atomic_load_n(w, __ATOMIC_ACQUIRE);
-    if (v >> 1 == tag) {
-      done = (v & 1) != 0;
-      return 0;
-    }
-    if (spin % 4096 == 0) {
-      const hipError_t e = hipStreamQuery(c.stream);
-      if (e == hipErrorNotReady) continue;
-      FVK_HIP(e);
-      const unsigned long long last = __atomic_load_n(w, __ATOMIC_ACQUIRE);
-      done = last >> 1 == tag && (last & 1);
-      return 0;
-    }
-  }
-}
-
 template <int NC, int WS>
 static int fl_solve_run(FlCtx &c, const FlMat &M, bool bicg, const double *a, double *phi, double *res, int n_iter,
                         double reduc) {
@@ -1055,9 +1029,9 @@ static int fl_solve_run(FlCtx &c, const FlMat &M, bool bicg, const double *a, do
   double *w1 = wkv(c, 0), *w2 = wkv(c, 1), *w3 = wkv(c, 2), *w4 = wkv(c, 3), *w5 = wkv(c, 4), *wt = wkv(c, 5);
   double *pa = c.part, *pb = c.part + (size_t)6 * RG;
   auto end = [&](int first, const double *part) {
-    const unsigned long long tag = ++c.watch_tag;
-    if (bicg) k_fl_end<NC, true><<<1, RB, 0, c.stream>>>(first, P, part, c.ks, reduc, c.watch + (tag & 1), tag);
-    else k_fl_end<NC, false><<<1, RB, 0, c.stream>>>(first, P, part, c.ks, reduc, c.watch + (tag & 1), tag);
+    const DoneSlot w = c.watch.next();
+    if (bicg) k_fl_end<NC, true><<<1, RB, 0, c.stream>>>(first, P, part, c.ks, reduc, w);
+    else k_fl_end<NC, false><<<1, RB, 0, c.stream>>>(first, P, part, c.ks, reduc, w);
   };
   k_fl_init<NC, WS><<<P, RB, 0, c.stream>>>(M, phi, res, w1, w2, bicg ? w3 : nullptr, pa);
   end(1, pa);
@@ -1081,8 +1055,9 @@ static int fl_solve_run(FlCtx &c, const FlMat &M, bool bicg, const double *a, do
       k_fl_bi_upd2<NC><<<P, RB, 0, c.stream>>>(n, phi, w5, w1, w4, res, pa, P, c.ks, pb);
       end(0, pb);
     }
+    // the iteration before this one, while this one runs
     bool done = false;
-    if (it > 0 && it + 1 < n_iter && (rc = fl_watch(c, c.watch_tag - 1, done))) return rc;
+    if (it > 0 && it + 1 < n_iter) FVK_HIP(c.watch.wait(c.stream, c.watch.tag - 1, done));
     if (done) break;
   }
   FVK_HIP(hipGetLastError());
@@ -1546,8 +1521,7 @@ static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
     if ((rc = fl_parts_setup(c))) return rc;
     c.parts = true;
   }
-  FVK_HIP(hipHostMalloc((void **)&c.watch, 2 * sizeof *c.watch, hipHostMallocDefault));
-  c.watch[0] = c.watch[1] = 0;
+  FVK_HIP(c.watch.init());
   // rows of 4, 5 or 7 entries: triangles, quadrangles, hexahedra; by slots
   // unless half of them would be empty or there is no memory for them
   int w = 0;
@@ -1671,8 +1645,7 @@ static void fl_ctx_free(FlCtx &c) {
   c.owned.clear();
   sweep_exec_free(c.sw);
   c.io.free();
-  if (c.watch) (void)hipHostFree(c.watch);
-  c.watch = nullptr;
+  c.watch.free();
   if (c.stream) hipStreamDestroy(c.stream);
   c.stream = nullptr;
 }

@@ -448,7 +448,7 @@ __global__ __launch_bounds__(TB) void k_cg_pq(DMesh M, int it, const double *__r
                                               const double *__restrict__ pold, double *__restrict__ pnew,
                                               double *__restrict__ qv, const double *__restrict__ partU, int P,
                                               const double *__restrict__ partR, double *__restrict__ partQ, KS *ring,
-                                              KS *out) {
+                                              KS *out, DoneSlot slot) {
   const int n = M.n;
   int r0, r1;
   block_rows<TB>(n, r0, r1);
@@ -471,8 +471,10 @@ __global__ __launch_bounds__(TB) void k_cg_pq(DMesh M, int it, const double *__r
   __shared__ KS sk[3];
   if (threadIdx.x == 0) {
     cg_decide(it, NVC, L1, rz, ring + ((it + 1) & 1) * 3, sk);
-    if (blockIdx.x == 0)
+    if (blockIdx.x == 0) {
       for (int q = 0; q < NVC; ++q) ring[(it & 1) * 3 + q] = out[q] = sk[q];
+      done_store(slot, all_done(sk, NVC));
+    }
   }
   __syncthreads();
   double beta[NVC];
@@ -638,14 +640,16 @@ template <int NVC, int TB>
 __global__ __launch_bounds__(TB) void k_bi_p(int n, int it, const double *__restrict__ r, double *__restrict__ p,
                                              const double *__restrict__ u, const double *__restrict__ c, int jacobi,
                                              double *__restrict__ z, const double *__restrict__ partU, int PU, KS *ring,
-                                             KS *out) {
+                                             KS *out, DoneSlot slot) {
   double t[6];
   load_totals<6, TB>(partU, PU, t);
   __shared__ KS sk[3];
   if (threadIdx.x == 0) {
     bi_decide(it, NVC, t, t + 3, ring + ((it + 1) & 1) * 3, sk);
-    if (blockIdx.x == 0)
+    if (blockIdx.x == 0) {
       for (int q = 0; q < NVC; ++q) ring[(it & 1) * 3 + q] = out[q] = sk[q];
+      done_store(slot, all_done(sk, NVC));
+    }
   }
   __syncthreads();
   double w6[NVC], w2[NVC];
@@ -1143,7 +1147,7 @@ static int all_done_host(Ctx &c, int nvc, bool &done) {
 
 template <int NVC>
 static void launch_cg_pq(Ctx &c, int G, int it, double *z, double *pold, double *pnew, double *q, const double *pU,
-                         const double *pR, KTimer *T) {
+                         const double *pR, KTimer *T, DoneSlot slot) {
   hipEvent_t ea, eb;
   const bool stamp = T && T->take(ea, eb);
   const double *zc = z, *pc = pold, *dg = c.diag, *sv = c.spv;
@@ -1152,13 +1156,13 @@ static void launch_cg_pq(Ctx &c, int G, int it, double *z, double *pold, double 
     if (stamp) {
 #define L(W)                                                                                                      \
   hipExtLaunchKernelGGL(k_cg_pq<NVC, W, TB>, dim3(G), dim3(TB), 0, c.stream, ea, eb, 0, c.M, it, dg, sv, zc, pc, pnew, \
-                        q, pU, G, pR, pbuf(c, 1), c.ksr, c.ks)
+                        q, pU, G, pR, pbuf(c, 1), c.ksr, c.ks, slot)
       FVK_WS(c.M.Ws, L);
 #undef L
     } else {
 #define L(W)                                                                                                      \
   k_cg_pq<NVC, W, TB><<<G, TB, 0, c.stream>>>(c.M, it, dg, sv, zc, pc, pnew, q, pU, G, pR, pbuf(c, 1), \
-                                              c.ksr, c.ks)
+                                              c.ksr, c.ks, slot)
       FVK_WS(c.M.Ws, L);
 #undef L
     }
@@ -1216,16 +1220,25 @@ static int cg_run(Ctx &c, int imat, double reduc, int n_iter, int nvc, double *x
   Poller Pl(c);
   int it = 0, next_poll = chunk;
   for (; it < n_iter; ++it) {
+    const DoneSlot slot = chunk == kWatch ? c.watch.next() : DoneSlot{};
     double *pold = P + (size_t)(it & 1) * wk_ld(n), *pnew = P + (size_t)((it + 1) & 1) * wk_ld(n);
-    if (nvc == 1) launch_cg_pq<1>(c, G, it, z, pold, pnew, q, pbuf(c, 0), pR, T);
-    else if (nvc == 2) launch_cg_pq<2>(c, G, it, z, pold, pnew, q, pbuf(c, 0), pR, T);
-    else launch_cg_pq<3>(c, G, it, z, pold, pnew, q, pbuf(c, 0), pR, T);
+    if (nvc == 1) launch_cg_pq<1>(c, G, it, z, pold, pnew, q, pbuf(c, 0), pR, T, slot);
+    else if (nvc == 2) launch_cg_pq<2>(c, G, it, z, pold, pnew, q, pbuf(c, 0), pR, T, slot);
+    else launch_cg_pq<3>(c, G, it, z, pold, pnew, q, pbuf(c, 0), pR, T, slot);
     if (nvc == 1) launch_cg_upd<1>(c, G, it, x, r, pnew, q, jac, z);
     else if (nvc == 2) launch_cg_upd<2>(c, G, it, x, r, pnew, q, jac, z);
     else launch_cg_upd<3>(c, G, it, x, r, pnew, q, jac, z);
     if (!jac) {
       int rc = precond_dot(c, imat, nvc, r, z, c.ksr + (it & 1) * 3);
       if (rc) return rc;
+    }
+    // iteration it's decision comes with its first launch: what is queued
+    // behind it (sweeps; or the next two iterations) runs while the host looks
+    const int lag = jac ? 2 : 0;
+    if (chunk == kWatch && it >= lag && it + 1 < n_iter) {
+      bool done;
+      FVK_HIP(c.watch.wait(c.stream, slot.tag - lag, done));
+      if (done) { ++it; break; }
     }
     if (chunk > 0 && it + 1 == next_poll && it + 1 < n_iter) {
       bool done;
@@ -1247,7 +1260,7 @@ static int cg_run(Ctx &c, int imat, double reduc, int n_iter, int nvc, double *x
   return 0;
 }
 
-static int bicg_run(Ctx &c, int imat, int n_iter, int nvc, double *x, double *r0, bool not_r0) {
+static int bicg_run(Ctx &c, int imat, int n_iter, int nvc, double *x, double *r0, bool not_r0, bool watch) {
   const int n = c.n, G = red_grid64(n);
   double *r = wv(c, 0), *p = wv(c, 1), *u = wv(c, 2), *v = wv(c, 3), *z = wv(c, 4);
   const int jac = imat == 0;
@@ -1271,10 +1284,11 @@ static int bicg_run(Ctx &c, int imat, int n_iter, int nvc, double *x, double *r0
   int it = 0;
   for (; it < n_iter; ++it) {
     const KS *gate = c.ksr + (it & 1) * 3;
+    const DoneSlot slot = watch ? c.watch.next() : DoneSlot{};
     with_tb(c, [&](auto tb) {
       with_nvc(nvc, [&](auto nv) {
         constexpr int TB = decltype(tb)::value, NVC = decltype(nv)::value;
-        k_bi_p<NVC, TB><<<G, TB, 0, c.stream>>>(n, it, r, p, u, c.pc_c, jac, z, pbuf(c, 0), G, c.ksr, c.ks);
+        k_bi_p<NVC, TB><<<G, TB, 0, c.stream>>>(n, it, r, p, u, c.pc_c, jac, z, pbuf(c, 0), G, c.ksr, c.ks, slot);
       });
     });
     if (!jac && precond_apply(c, imat, nvc, p, z, gate)) return FVK_ERR_HIP;
@@ -1307,6 +1321,11 @@ static int bicg_run(Ctx &c, int imat, int n_iter, int nvc, double *x, double *r0
         k_bi_upd2<NVC, TB><<<G, TB, 0, c.stream>>>(n, it, x, r, z, v, r0, pbuf(c, 2), G, pbuf(c, 0), c.ksr);
       });
     });
+    if (watch && it + 1 < n_iter) {
+      bool done;
+      FVK_HIP(c.watch.wait(c.stream, slot.tag, done));
+      if (done) { ++it; break; }
+    }
   }
   k_bi_final<<<1, RB64, 0, c.stream>>>(it, nvc, pbuf(c, 0), G, c.ksr, c.ks);
   FVK_HIP(hipGetLastError());
@@ -1318,7 +1337,7 @@ int krylov(Ctx &c, int kind, int imat, double reduc, int n_iter, int nvc, double
   int rc = ks_init(c, nvc, reduc, n_iter, kind == 1);
   if (rc) return rc;
   if (kind == 0) return cg_run(c, imat, reduc, n_iter, nvc, x, r0, not_r0, chunk, T);
-  return bicg_run(c, imat, n_iter, nvc, x, r0, not_r0);
+  return bicg_run(c, imat, n_iter, nvc, x, r0, not_r0, chunk == kWatch);
 }
 
 __global__ __launch_bounds__(BS) void k_scale64(size_t n, double *__restrict__ a, const double *__restrict__ b,

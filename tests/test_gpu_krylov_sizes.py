@@ -73,3 +73,35 @@ def test_two_steps(dims):
         want = g * c * b0 + (v @ s) / (v @ v) * c * s
         assert np.abs(x[:, q] - want).max() <= tol * np.abs(want).max(), q
     ctx.destroy()
+
+
+@pytest.mark.parametrize("imat", [0, 1])
+@pytest.mark.parametrize("fn,n_iter", [("solv_cg", 30), ("solv_bicg", 12)])
+def test_stops_as_if_told_the_iterations(fn, n_iter, imat):
+    """A solve that meets its tolerance after k iterations leaves the bits of
+    a solve of exactly k iterations, for an end at the start, in the middle
+    and at the last iteration allowed (the host sees the end while later
+    iterations are queued)."""
+    fvk = require_lib()
+    m = fvk.Mesh.box(20, 17, 13, jitter=0.05, seed=2)
+    ctx = fvk.grd_solv(m)
+    pl, gp, gn = random_matrix(m, 9)
+    sym = fn == "solv_cg"
+    fvk.set_matrix(ctx, pl + 6.0 * sym, gp, gp if sym else gn)
+    b = np.random.default_rng(1).standard_normal((m.n_vol, 2))
+    pc = imat if sym else 2 * imat
+
+    def run(reduc, its):
+        x, r = np.zeros((m.n_vol, 2)), b.copy()
+        rn, st = getattr(fvk, fn)(ctx, pc, reduc, its, x, r)
+        return x, r, list(st.iters[:2])
+
+    seen = set()
+    for reduc in (2.0, 0.3, 1e-2, 1e-4, 1e-30):
+        x, r, k = run(reduc, n_iter)
+        seen.update(k)
+        for q in range(2):
+            xk, rk, kk = run(0.0, k[q])
+            assert kk[q] == k[q] and np.array_equal(xk[:, q], x[:, q]) and np.array_equal(rk[:, q], r[:, q])
+    assert 1 in seen and n_iter in seen and len(seen) > 3
+    ctx.destroy()
