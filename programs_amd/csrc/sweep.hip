@@ -28,16 +28,22 @@
 // the bound they record the error, the compute wave runs through what is
 // left on what is there and the block stops taking parts.
 //
-// What bounds it: the chain of chunks a path runs through (0.11 us a chunk:
-// LDS read, five dependent FP64 operations, LDS write) and the crossings
-// between parts (1 us: store, poll, reload), not bandwidth.  One application
-// of DIC to one right-hand side (both sweeps), against the form it replaced
-// (ranges of 4096 consecutive rows, a level at a time): 24^3 42 us (177),
-// 96^3 189 us (620), 128^3 294 us (1232); DILU to three at 128^3 445 us
-// (1823); 40,000 triangles of a Delaunay channel 64 us (155).
+// What bounds it: the chain of chunks a path runs through (LDS read, five
+// dependent FP64 operations, LDS write) and the crossings between parts
+// (store, poll, reload), not bandwidth.  A chunk is 42 instructions of one
+// wave, each at least four cycles: records whose words are LDS addresses as
+// they are and are taken apart in the shadow of the LDS reads, a wait loop out
+// of line, and loads first issued in the loop's order (else a ring of chunks
+// begins by waiting for loads two chunks old) took 15 instructions and those
+// waits out: 42 -> 38 us at 24^3, 189 -> 163 at 96^3, 294 -> 250 at 128^3.
+// One application of DIC to one right-hand side (both sweeps), against the
+// form it replaced (ranges of 4096 consecutive rows, a level at a time): 24^3
+// 38 us (177), 96^3 163 us (620), 128^3 250 us (1232); DILU to three at 128^3
+// 417 us (1823).
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <cstdint>
 
 #include "ctx.h"
 #include "sweep.h"
@@ -56,6 +62,7 @@ constexpr int sweep_ahead(int MW, int KIND) {
 
 struct SweepArgs {
   int P, np, slots, NE, NEo, n;
+  unsigned shared;            // LDS address of the block's shared scalars
   const int *part, *prow, *ppos, *hsrc;
   const unsigned short *pslot, *rec;
   const double *a, *a2, *c;   // by position
@@ -68,13 +75,19 @@ struct SweepArgs {
   SweepGate gate;
 };
 
-// LDS scalars shared by a block's waves
-struct SweepShared {
-  int q, have, abort;
-};
-
-__device__ __forceinline__ int lds_get(const int *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+// A block's LDS, by byte address from 0 (the kernels have no static LDS, which
+// the host checks): values of component q at slot offset + q ld, the halo's
+// sources, and the scalars shared by the block's waves at Shared.  Plain
+// addresses, so that a record's 16-bit offset is an address as it is.
+enum { SH_PART = 0, SH_HAVE = 4, SH_ABORT = 8, kShared = 16 };
+template <class T>
+using lds_t = __attribute__((address_space(3))) T;
+__device__ __forceinline__ double lds_value(unsigned at) { return *(lds_t<double> *)(uintptr_t)at; }
+__device__ __forceinline__ void lds_put(unsigned at, double v) { *(lds_t<double> *)(uintptr_t)at = v; }
+__device__ __forceinline__ int lds_int(unsigned at) { return *(lds_t<int> *)(uintptr_t)at; }
+__device__ __forceinline__ void lds_put(unsigned at, int v) { *(lds_t<int> *)(uintptr_t)at = v; }
+__device__ __forceinline__ int lds_get(unsigned at) {
+  return __hip_atomic_load((lds_t<int> *)(uintptr_t)at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // this wave's LDS operations so far are done
 __device__ __forceinline__ void lds_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
@@ -85,6 +98,13 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 template <class T>
 __device__ __forceinline__ T ld_at(global_p base, unsigned byte) {
   return *(const __attribute__((address_space(1))) T *)(base + byte);
+}
+
+typedef __attribute__((address_space(1))) char *global_w;
+// agent scope, as st_agent
+__device__ __forceinline__ void st_at(global_w base, unsigned byte, double v) {
+  __hip_atomic_store((__attribute__((address_space(1))) unsigned long long *)(base + byte),
+                     (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // what a lane needs to run its row of a chunk
@@ -134,8 +154,7 @@ __device__ __forceinline__ void sweep_load(const SweepBase<MW> &B, unsigned bo, 
 // stage that the chunk before has freed, while this chunk's LDS reads are
 // on their way.
 template <bool FWD, int NC, int MW, int KIND>
-__device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nch, char *lv, unsigned ld,
-                                              SweepShared &sh) {
+__device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nch, unsigned ld) {
   constexpr int kAhead = sweep_ahead(MW, KIND), kRing = kAhead + 1;
   SweepBase<MW> B;
   B.rec = opaque(A.rec);
@@ -153,34 +172,48 @@ __device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nc
   };
   SweepStage<MW> S[kRing];
 #pragma unroll
-  for (int u = 0; u < kAhead; ++u) sweep_load<MW, KIND>(B, at(u), S[u]);
+  for (int u = 0; u < kAhead; ++u) {
+    sweep_load<MW, KIND>(B, at(u), S[u]);
+    // in the loop's order: else its waits count on the other order as well
+    __builtin_amdgcn_sched_barrier(0);
+  }
   int have = 0;
   // the chunk about to run: its LDS addresses and halo need, taken while
   // the reads of the chunk before are on their way
-  unsigned off[MW + 1];
+  unsigned off[MW + 1], eoff = 0;
   int nd = 0;
+  global_w E[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) E[q] = (global_w)opaque(A.E + (size_t)q * A.NE);
+  // (opaque: taken apart here and not between this chunk's write and the next
+  // chunk's reads, which is on the chain)
   auto prep = [&](const SweepStage<MW> &Y) {
 #pragma unroll
-    for (int t = 0; t <= MW; ++t) off[t] = Y.word(t);
+    for (int t = 0; t <= MW; ++t) {
+      off[t] = Y.word(t);
+      asm volatile("" : "+v"(off[t]));
+    }
+    eoff = (unsigned)Y.exp() << 3;
+    asm volatile("" : "+v"(eoff));
     nd = __builtin_amdgcn_readfirstlane(Y.need());
   };
   auto run = [&](const SweepStage<MW> &X, const SweepStage<MW> &Y, auto ahead) {
-    while (nd > have) {
-      have = __builtin_amdgcn_readfirstlane(lds_get(&sh.have));
+    while (__builtin_expect(nd > have, 0)) {
+      have = __builtin_amdgcn_readfirstlane(lds_get(A.shared + SH_HAVE));
       // the halo waves gave up: the rest of the part runs on what is there
-      if (nd > have && __builtin_amdgcn_readfirstlane(lds_get(&sh.abort))) have = INT_MAX;
+      if (nd > have && __builtin_amdgcn_readfirstlane(lds_get(A.shared + SH_ABORT))) have = INT_MAX;
     }
     asm volatile("" ::: "memory");
     double acc[NC], v[MW][NC], r[NC];
 #pragma unroll
-    for (int q = 0; q < NC; ++q) acc[q] = *(const double *)(lv + (off[0] + q * ld));
+    for (int q = 0; q < NC; ++q) acc[q] = lds_value(off[0] + q * ld);
 #pragma unroll
     for (int t = 0; t < MW; ++t)
 #pragma unroll
-      for (int q = 0; q < NC; ++q) v[t][q] = *(const double *)(lv + (off[1 + t] + q * ld));
+      for (int q = 0; q < NC; ++q) v[t][q] = lds_value(off[1 + t] + q * ld);
     __builtin_amdgcn_sched_barrier(0);
     ahead();
-    const unsigned own = off[0];
+    const unsigned own = off[0], eo = eoff;
     prep(Y);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -193,15 +226,14 @@ __device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nc
       }
     if (KIND == 0) {
 #pragma unroll
-      for (int q = 0; q < NC; ++q) *(double *)(lv + (own + q * ld)) = r[q] = acc[q] * X.c;
+      for (int q = 0; q < NC; ++q) lds_put(own + q * ld, r[q] = acc[q] * X.c);
     } else {
-      *(double *)(lv + own) = r[0] = 1.0 / (acc[0] + SMALL);
-      *(double *)(lv + (own + ld)) = acc[0];
+      lds_put(own, r[0] = 1.0 / (acc[0] + SMALL));
+      lds_put(own + ld, acc[0]);
     }
-    const int e = X.exp();
-    if (e >= 0)
+    if (X.exp() >= 0)
 #pragma unroll
-      for (int q = 0; q < NC; ++q) st_agent(A.E + (size_t)q * A.NE + e, r[q]);
+      for (int q = 0; q < NC; ++q) st_at(E[q], eo, r[q]);
     __builtin_amdgcn_sched_barrier(0);
   };
   prep(S[0]);
@@ -219,15 +251,14 @@ __device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nc
 }
 
 template <int NC>
-__device__ __forceinline__ void sweep_halo(const SweepArgs &A, int nh, int nr, char *lv, unsigned ld, const int *s_hsrc,
-                                           SweepShared &sh) {
+__device__ __forceinline__ void sweep_halo(const SweepArgs &A, int nh, int nr, unsigned ld, unsigned hsrc) {
   const int lane = threadIdx.x & 63, ng = (nh + 63) / 64;
   int src[kHaloWin];
   bool pend[kHaloWin];
   auto start = [&](int g, int &s, bool &p) {
     const int e = g * 64 + lane;
     p = e < nh;
-    s = p ? s_hsrc[e] : 0;
+    s = p ? lds_int(hsrc + 4u * e) : 0;
   };
 #pragma unroll
   for (int w = 0; w < kHaloWin; ++w) start(w, src[w], pend[w]);
@@ -249,7 +280,7 @@ __device__ __forceinline__ void sweep_halo(const SweepArgs &A, int nh, int nr, c
         if (ready) {
           const unsigned o = (unsigned)(nr + (g + w) * 64 + lane) * 8u;
 #pragma unroll
-          for (int q = 0; q < NC; ++q) *(double *)(lv + (o + q * ld)) = __longlong_as_double((long long)v[w][q]);
+          for (int q = 0; q < NC; ++q) lds_put(o + q * ld, __longlong_as_double((long long)v[w][q]));
           pend[w] = false;
         }
       }
@@ -269,11 +300,11 @@ __device__ __forceinline__ void sweep_halo(const SweepArgs &A, int nh, int nr, c
       pub = have;
       spin = 0;
       lds_done();
-      __hip_atomic_fetch_max(&sh.have, have, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_fetch_max((lds_t<int> *)(uintptr_t)(A.shared + SH_HAVE), have, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     } else if (++spin > kSweepSpin ||
                ((spin & 255u) == 0 && __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
       __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(&sh.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_store((lds_t<int> *)(uintptr_t)(A.shared + SH_ABORT), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       return;
     }
   }
@@ -286,12 +317,9 @@ __global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
     for (int q = 0; q < A.gate.n; ++q) all = all && A.gate.done[q * A.gate.stride];
     if (all) return;
   }
-  extern __shared__ double lds[];
-  __shared__ SweepShared sh;
   constexpr int NV = KIND == 0 ? NC : 2;  // values per slot (factor: c and d)
   const unsigned ld = (unsigned)A.slots * 8u;
-  char *lv = (char *)lds;
-  int *s_hsrc = (int *)(lv + (size_t)NV * ld);
+  const unsigned hsrc = NV * ld;
   const int tid = threadIdx.x, wave = tid >> 6;
   if (KIND == 0) {
     // the other direction's export buffer, for the launch after this one
@@ -300,14 +328,14 @@ __global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
       ((unsigned long long *)A.Eo)[i] = kSweepMark;
     if (blockIdx.x == 0 && tid == 0) *A.ticket_o = 0;
   }
-  if (tid == 0) sh.abort = 0;
+  if (tid == 0) lds_put(A.shared + SH_ABORT, 0);
   for (;;) {
     if (tid == 0) {
-      sh.q = atomicAdd(A.ticket, 1);
-      sh.have = 0;
+      lds_put(A.shared + SH_PART, atomicAdd(A.ticket, 1));
+      lds_put(A.shared + SH_HAVE, 0);
     }
     __syncthreads();
-    const int o = __builtin_amdgcn_readfirstlane(sh.q);
+    const int o = __builtin_amdgcn_readfirstlane(lds_int(A.shared + SH_PART));
     if (o >= A.P) return;
     const int q = FWD ? o : A.P - 1 - o;
     const int *Q = A.part + 8 * q;
@@ -334,26 +362,26 @@ __global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
       for (int i = 0; i < 4; ++i)
         if (k0 + i * SW_TB < nr)
 #pragma unroll
-          for (int c = 0; c < NC; ++c) *(double *)(lv + (off[i] + c * ld)) = FWD ? v[i][c] : v[i][c] * s[i];
+          for (int c = 0; c < NC; ++c) lds_put(off[i] + c * ld, FWD ? v[i][c] : v[i][c] * s[i]);
     }
-    for (int h = tid; h < nh; h += SW_TB) s_hsrc[h] = A.hsrc[h0 + h];
-    if (tid < 2 * NV) *(double *)(lv + ((unsigned)(nr + nh + (tid & 1)) * 8u + (tid >> 1) * ld)) = 0.0;
+    for (int h = tid; h < nh; h += SW_TB) lds_put(hsrc + 4u * h, A.hsrc[h0 + h]);
+    if (tid < 2 * NV) lds_put((unsigned)(nr + nh + (tid & 1)) * 8u + (tid >> 1) * ld, 0.0);
     __syncthreads();
     // the halo waves of other blocks poll on the same SIMD
     if (wave == 0) __builtin_amdgcn_s_setprio(3);
-    if (wave == 0) sweep_compute<FWD, NC, MW, KIND>(A, c0, nch, lv, ld, sh);
-    else sweep_halo<NC>(A, nh, nr, lv, ld, s_hsrc, sh);
+    if (wave == 0) sweep_compute<FWD, NC, MW, KIND>(A, c0, nch, ld);
+    else sweep_halo<NC>(A, nh, nr, ld, hsrc);
     __syncthreads();
-    if (sh.abort) return;
+    if (lds_int(A.shared + SH_ABORT)) return;
     for (int k = tid; k < nr; k += SW_TB) {
       const unsigned off = A.pslot[r0 + k];
       if (KIND == 0) {
         const int z = FWD ? r0 + k : A.prow[r0 + k];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) A.dst[(size_t)c * A.n + z] = *(const double *)(lv + (off + c * ld));
+        for (int c = 0; c < NC; ++c) A.dst[(size_t)c * A.n + z] = lds_value(off + c * ld);
       } else {
         const int row = A.prow[r0 + k];
-        const double c = *(const double *)(lv + off), d = *(const double *)(lv + (off + ld));
+        const double c = lds_value(off), d = lds_value(off + ld);
         A.crow[row] = c;
         if (A.drow) A.drow[row] = d;
         A.cpos[A.ppos[r0 + k]] = c;
@@ -433,7 +461,12 @@ static int allow_lds() {
                      (const void *)k_sweep<true, 3, MW, 0>,  (const void *)k_sweep<false, 1, MW, 0>,
                      (const void *)k_sweep<false, 2, MW, 0>, (const void *)k_sweep<false, 3, MW, 0>,
                      (const void *)k_sweep<true, 1, MW, 1>,  (const void *)k_sweep<true, 1, MW, 2>};
-  for (const void *f : k) FVK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kSweepLds));
+  for (const void *f : k) {
+    hipFuncAttributes at;
+    FVK_HIP(hipFuncGetAttributes(&at, f));
+    if (at.sharedSizeBytes) { set_error("a sweep kernel has static LDS"); return FVK_ERR_STATE; }
+    FVK_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kSweepLds + kShared));
+  }
   return 0;
 }
 
@@ -500,9 +533,11 @@ static int grid(const SweepExec &X, size_t lds) {
 }
 
 template <bool FWD, int NC, int KIND>
-static void launch(const SweepExec &X, const SweepArgs &A, hipStream_t s) {
-  const size_t lds = X.lds_[KIND == 0 ? NC : 2];
+static void launch(const SweepExec &X, const SweepArgs &args, hipStream_t s) {
+  const size_t room = (X.lds_[KIND == 0 ? NC : 2] + 15) / 16 * 16, lds = room + kShared;
   const int G = grid(X, lds);
+  SweepArgs A = args;
+  A.shared = (unsigned)room;
   if (X.MW == 3) k_sweep<FWD, NC, 3, KIND><<<G, SW_TB, lds, s>>>(A);
   else if (X.MW == 4) k_sweep<FWD, NC, 4, KIND><<<G, SW_TB, lds, s>>>(A);
   else k_sweep<FWD, NC, 8, KIND><<<G, SW_TB, lds, s>>>(A);
