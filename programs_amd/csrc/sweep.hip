@@ -14,11 +14,9 @@
 //     stored by position, so that a chunk's loads are consecutive, and are
 //     issued up to eight chunks ahead.  Values that other parts need go to
 //     the export buffer at once (agent scope).
-//   waves 1 and 2 fetch the halo: each polls the export buffer for the
-//     values of other parts, in the order in which the chunks need them,
-//     puts them into LDS and publishes how many are there.  Two waves poll
-//     twice as often as one (the wait for the next poll is part of every
-//     crossing).
+//   wave 1 fetches the halo: it polls the export buffer for the values of
+//     other parts, in the order in which the chunks need them, puts them
+//     into LDS and publishes how many are there.
 // Results go from LDS to memory by all waves when the part is done.
 //
 // Export slots hold kSweepMark (a signalling NaN: no arithmetic result has
@@ -36,10 +34,11 @@
 // of line, and loads first issued in the loop's order (else a ring of chunks
 // begins by waiting for loads two chunks old) took 15 instructions and those
 // waits out: 42 -> 38 us at 24^3, 189 -> 163 at 96^3, 294 -> 250 at 128^3.
-// One application of DIC to one right-hand side (both sweeps), against the
-// form it replaced (ranges of 4096 consecutive rows, a level at a time): 24^3
-// 38 us (177), 96^3 163 us (620), 128^3 250 us (1232); DILU to three at 128^3
-// 417 us (1823).
+// Bricks of 8 x 8 columns, one poll in flight a block and more threads beside
+// the chunks took them to 32, 137 and 207 us.  One application of DIC to one
+// right-hand side (both sweeps), against the form it replaced (ranges of 4096
+// consecutive rows, a level at a time): 24^3 32 us (177), 96^3 137 us (620),
+// 128^3 207 us (1232); DILU to three at 128^3 314 us (1823).
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -51,8 +50,9 @@
 
 namespace fvk {
 
-constexpr int SW_TB = 192;   // one compute wave, two halo waves
-constexpr int kHaloWin = 2;  // groups of 64 halo values polled together
+// a compute wave, a halo wave, and six that help to load a part and to store
+// it (both sweeps, 24^3 / 96^3 / 128^3: 33.8 / 144 / 233 us with 192 threads)
+constexpr int SW_TB = 512;
 // chunks whose loads are in flight: at most 8, and at most 56 loads and
 // exports (a wave counts 63)
 constexpr int sweep_ahead(int MW, int KIND) {
@@ -89,6 +89,9 @@ __device__ __forceinline__ void lds_put(unsigned at, int v) { *(lds_t<int> *)(ui
 __device__ __forceinline__ int lds_get(unsigned at) {
   return __hip_atomic_load((lds_t<int> *)(uintptr_t)at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+__device__ __forceinline__ void lds_post(unsigned at, int v) {
+  __hip_atomic_store((lds_t<int> *)(uintptr_t)at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 // this wave's LDS operations so far are done
 __device__ __forceinline__ void lds_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
@@ -101,7 +104,11 @@ __device__ __forceinline__ T ld_at(global_p base, unsigned byte) {
 }
 
 typedef __attribute__((address_space(1))) char *global_w;
-// agent scope, as st_agent
+// agent scope, as ld_agent and st_agent
+__device__ __forceinline__ unsigned long long ld_agent_at(global_p base, unsigned byte) {
+  return __hip_atomic_load((const __attribute__((address_space(1))) unsigned long long *)(base + byte), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void st_at(global_w base, unsigned byte, double v) {
   __hip_atomic_store((__attribute__((address_space(1))) unsigned long long *)(base + byte),
                      (unsigned long long)__double_as_longlong(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -250,61 +257,55 @@ __device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nc
     if (j0 + u < nch) run(S[u], S[(u + 1) % kRing], [] {});
 }
 
+// The halo of a part: lane l fetches the values l, l + 64, ... of the part's
+// list, in the order in which the chunks need them.  One wave with one poll in
+// flight: polls are misses to the fabric, and more of them (two waves, several
+// polls in flight, two values a lane) delay the answers by more than they save,
+// while fewer lanes cannot keep up with the chunks (DIC at 96^3, both sweeps,
+// with 192 threads: 141 us; two polls in flight 145; two values a lane 150; two
+// waves 151, with two, four, eight polls in flight 156, 187, 279; 32 lanes 199).
 template <int NC>
 __device__ __forceinline__ void sweep_halo(const SweepArgs &A, int nh, int nr, unsigned ld, unsigned hsrc) {
-  const int lane = threadIdx.x & 63, ng = (nh + 63) / 64;
-  int src[kHaloWin];
-  bool pend[kHaloWin];
-  auto start = [&](int g, int &s, bool &p) {
-    const int e = g * 64 + lane;
-    p = e < nh;
-    s = p ? lds_int(hsrc + 4u * e) : 0;
-  };
-#pragma unroll
-  for (int w = 0; w < kHaloWin; ++w) start(w, src[w], pend[w]);
+  if (nh == 0) return;
+  const int lane = threadIdx.x & 63;
+  auto source = [&](int e) { return (unsigned)lds_int(hsrc + 4u * min(e, nh - 1)) << 3; };
+  int cur = lane;  // the value this lane is at; past the last, nothing is asked of the answers
+  unsigned src = source(lane), nxt = source(lane + 64);
+  int at = 0, pub = 0;  // every lane is at its value number at / 64 or beyond; published
   unsigned spin = 0;
-  int g = 0, pub = 0;
-  while (g < ng) {
-    unsigned long long v[kHaloWin][NC];
+  global_p E[NC];
 #pragma unroll
-    for (int w = 0; w < kHaloWin; ++w)
-      if (pend[w])
+  for (int q = 0; q < NC; ++q) E[q] = opaque(A.E + (size_t)q * A.NE);
+  for (;;) {
+    unsigned long long v[NC];
+    bool ready = cur < nh;
 #pragma unroll
-        for (int q = 0; q < NC; ++q) v[w][q] = ld_agent(A.E + (size_t)q * A.NE + src[w]);
+    for (int q = 0; q < NC; ++q) v[q] = ld_agent_at(E[q], src);
 #pragma unroll
-    for (int w = 0; w < kHaloWin; ++w)
-      if (pend[w]) {
-        bool ready = true;
+    for (int q = 0; q < NC; ++q) ready = ready && v[q] != kSweepMark;
+    if (ready) {
+      const unsigned o = (unsigned)(nr + cur) * 8u;
 #pragma unroll
-        for (int q = 0; q < NC; ++q) ready = ready && v[w][q] != kSweepMark;
-        if (ready) {
-          const unsigned o = (unsigned)(nr + (g + w) * 64 + lane) * 8u;
-#pragma unroll
-          for (int q = 0; q < NC; ++q) lds_put(o + q * ld, __longlong_as_double((long long)v[w][q]));
-          pend[w] = false;
-        }
-      }
-    unsigned long long m = __ballot(pend[0]);
-    while (m == 0 && g < ng) {
-      ++g;
-#pragma unroll
-      for (int w = 0; w + 1 < kHaloWin; ++w) {
-        pend[w] = pend[w + 1];
-        src[w] = src[w + 1];
-      }
-      start(g + kHaloWin - 1, src[kHaloWin - 1], pend[kHaloWin - 1]);
-      m = __ballot(pend[0]);
+      for (int q = 0; q < NC; ++q) lds_put(o + q * ld, __longlong_as_double((long long)v[q]));
+      cur += 64;
+      src = nxt;
+      nxt = source(cur + 64);
     }
-    const int have = min(nh, g * 64 + (m ? __builtin_ctzll(m) : 0));
+    // a lane takes one step at most, so `at` takes one at most
+    unsigned long long m = __ballot(cur < at + 64);
+    at = m ? at : at + 64;
+    m = m ? m : __ballot(cur < at + 64);
+    const int have = min(nh, at + (m ? __builtin_ctzll(m) : 64));
     if (have > pub) {
       pub = have;
       spin = 0;
       lds_done();
-      __hip_atomic_fetch_max((lds_t<int> *)(uintptr_t)(A.shared + SH_HAVE), have, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      lds_post(A.shared + SH_HAVE, have);
+      if (pub == nh) return;
     } else if (++spin > kSweepSpin ||
                ((spin & 255u) == 0 && __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
       __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store((lds_t<int> *)(uintptr_t)(A.shared + SH_ABORT), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      lds_post(A.shared + SH_ABORT, 1);
       return;
     }
   }
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
     // the halo waves of other blocks poll on the same SIMD
     if (wave == 0) __builtin_amdgcn_s_setprio(3);
     if (wave == 0) sweep_compute<FWD, NC, MW, KIND>(A, c0, nch, ld);
-    else sweep_halo<NC>(A, nh, nr, ld, hsrc);
+    else if (wave == 1) sweep_halo<NC>(A, nh, nr, ld, hsrc);
     __syncthreads();
     if (lds_int(A.shared + SH_ABORT)) return;
     for (int k = tid; k < nr; k += SW_TB) {

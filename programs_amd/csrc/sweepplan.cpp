@@ -63,22 +63,56 @@ int main_distances(const SweepGraph &g, int (&d)[3]) {
 
 }  // namespace
 
+// The chunks on the longest path through a grid of bricks of these sides
+// (cells each), as one compute wave a brick runs them: the chunks of the last
+// brick, and for every crossing in a direction the chunks by which a brick
+// lags behind the one before it plus the crossing itself.
+// kCross: a crossing in chunks (1.4 us against 0.1 us, from boxes of 12^3 to
+// 96^3 cut into bricks of 8^3 and 12^3).
+static double brick_path(int m, const int *side, const int *cells) {
+  constexpr double kCross = 14.0;
+  // rows of a brick by level, and the chunks up to a level
+  std::vector<int> cnt(1, 1);
+  for (int c = 0; c < m; ++c) {
+    const int had = (int)cnt.size();
+    std::vector<int> t(had + side[c] - 1);
+    for (int l = 0, sum = 0; l < (int)t.size(); ++l) {
+      if (l < had) sum += cnt[l];
+      if (l >= side[c]) sum -= cnt[l - side[c]];
+      t[l] = sum;
+    }
+    cnt.swap(t);
+  }
+  int all = 0;
+  for (int &v : cnt) v = all += (v + kChunk - 1) / kChunk;
+  double path = all;
+  for (int c = 0; c < m; ++c) {
+    int lag = 0;
+    for (size_t l = 0; l + side[c] - 1 < cnt.size(); ++l)
+      lag = std::max(lag, cnt[l + side[c] - 1] - (l ? cnt[l - 1] : 0));
+    path += (cells[c] - 1) * (lag + kCross);
+  }
+  return path;
+}
+
 // Parts.  An acyclic split with few crossings on a path: for each of the
 // main rank distances d, phi_d(row) is the largest number of entries of
 // distance d on any path that ends at the row.  Each phi_d never decreases
 // along an entry, so cells of a grid over the phi_d ("bricks") depend on
 // each other only in the direction of growing cell indices, and taking them
 // by the sum of the indices is a valid order.  On a box in natural order
-// the phi_d are the cell's coordinates and the bricks are cubes: a path
-// through an N^3 box crosses 3 N / B of them instead of one range of
-// consecutive rows per plane.  kBrickRows: smaller bricks cross more often,
-// larger ones have levels wider than a chunk, which their one compute wave
-// runs one after the other (DIC, both sweeps, 96^3 / 128^3: 512 rows 243 /
-// 395 us, 1000 204 / 354, 1728 205 / 350, 2744 226 / 354, 4096 261 / 423).
+// the phi_d are the cell's coordinates, and a path through it crosses a few
+// bricks in each direction instead of one range of consecutive rows per
+// plane.  The sides are those with the shortest path: few crossings, but no
+// levels much wider than a chunk, which the one compute wave runs one after
+// the other and which the next brick waits for.  On boxes that gives 8 x 8
+// columns (whose levels have at most 64 rows) of up to kBrickRows rows (DIC,
+// both sweeps, 24^3 / 96^3 / 128^3, with two halo waves: 35.3 / 153 / 235 us;
+// cubes of at most 1728 rows 38 / 163 / 250, of 512 rows 37 / 173).
 // Without main distances (unstructured numberings) the parts are ranges of
 // consecutive rows, few and large: a path crosses them about once a level
 // anyway.
-constexpr int kBrickRows = 1728;
+constexpr int kBrickRows = 4096;
 
 static bool brick_parts(const SweepGraph &g, int max_rows, std::vector<int> &part, int &P) {
   max_rows = std::min(max_rows, kBrickRows);
@@ -107,23 +141,34 @@ static bool brick_parts(const SweepGraph &g, int max_rows, std::vector<int> &par
     }
     ext[c] = top + 1;
   }
-  // sides: equal, within the extents, their product at most max_rows
+  // sides: the shortest path of all that are even within a direction and have
+  // at most max_rows rows a brick
   int side[3] = {1, 1, 1}, cells[3] = {1, 1, 1};
-  for (int s = 1;; ++s) {
-    long r = 1;
-    for (int c = 0; c < m; ++c) r *= std::min(s, ext[c]);
-    if (r > max_rows) break;
-    bool grew = false;
-    for (int c = 0; c < m; ++c) {
-      grew = grew || side[c] < std::min(s, ext[c]);
-      side[c] = std::min(s, ext[c]);
+  double best = -1.0;
+  std::vector<int> cand[3];
+  for (int c = 0; c < 3; ++c)
+    for (int w = 1; w <= ext[c]; ++w) {
+      const int k = (ext[c] + w - 1) / w, e = (ext[c] + k - 1) / k;
+      if (e == w && (w >= 4 || w == ext[c])) cand[c].push_back(w);
     }
-    if (s > 1 && !grew) break;
-  }
+  for (int s0 : cand[0])
+    for (int s1 : cand[1]) {
+      if ((long)s0 * s1 > max_rows) break;
+      for (int s2 : cand[2]) {
+        if ((long)s0 * s1 * s2 > max_rows) break;
+        const int s[3] = {s0, s1, s2};
+        int k[3];
+        for (int c = 0; c < 3; ++c) k[c] = (ext[c] + s[c] - 1) / s[c];
+        const double t = brick_path(m, s, k);
+        if (best < 0 || t < best) {
+          best = t;
+          std::copy(s, s + 3, side);
+        }
+      }
+    }
+  if (best < 0) return false;
   long grid = 1;
   for (int c = 0; c < m; ++c) {
-    cells[c] = (ext[c] + side[c] - 1) / side[c];
-    side[c] = (ext[c] + cells[c] - 1) / cells[c];  // even sides
     cells[c] = (ext[c] + side[c] - 1) / side[c];
     grid *= cells[c];
   }
