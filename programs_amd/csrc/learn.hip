@@ -85,10 +85,13 @@ __device__ void load_weights(const float *__restrict__ th, WLds &s, bool bwd) {
       s.w3[k] = o4 < 2 ? bf16(th[OFF_W3 + i4 * 2 + o4]) : (short)0;
     }
   }
+  // 8 x 8 tiles a wave: 32 bytes of a row of memory, and 8 lanes at most on an
+  // LDS bank (a row or a column a wave: 64 lines of memory, or 64 lanes)
   for (int k = threadIdx.x; k < 64 * 64; k += blockDim.x) {
-    const int o = k / 64, i = k % 64;
-    s.w2t[k] = bf16(th[OFF_W2 + i * 64 + o]);
-    if (bwd) s.w2[k] = bf16(th[OFF_W2 + k]);
+    const int l = k % 64, o = (k / 64) % 8 * 8 + l % 8, i = k / 512 * 8 + l / 8;
+    const short v = bf16(th[OFF_W2 + i * 64 + o]);
+    s.w2t[o * 64 + i] = v;
+    if (bwd) s.w2[i * 64 + o] = v;
   }
   for (int k = threadIdx.x; k < 64; k += blockDim.x) {
     s.b1[k] = th[OFF_B1 + k];
@@ -529,15 +532,26 @@ __global__ __launch_bounds__(RB) void k_loss_grad(FaceIn F, const double *__rest
   }
 }
 
-// Sum of the block partials (fixed order), then Adam (Kingma and Ba 2015).
-__global__ __launch_bounds__(BS) void k_adam(float *__restrict__ theta, float *__restrict__ m1,
+// Sum of the block partials (fixed order), then Adam (Kingma and Ba 2015).  A
+// wave per 64 parameters and 64 partials in flight: with the partials loaded a
+// few at a time the 256 of them were one chain of waits (48 us; 15 us).
+constexpr int ADAM_B = 64;
+__global__ __launch_bounds__(ADAM_B) void k_adam(float *__restrict__ theta, float *__restrict__ m1,
                                              float *__restrict__ m2, const float *__restrict__ gpart, int nblk,
                                              float *__restrict__ gout, int update, float lr, float b1, float b2,
                                              float eps, float c1, float c2) {
-  const int k = blockIdx.x * BS + threadIdx.x;
+  const int k = blockIdx.x * ADAM_B + threadIdx.x;
   if (k >= NPARAM) return;
   float gk = 0.f;
-  for (int b = 0; b < nblk; ++b) gk += gpart[(size_t)b * NPARAM + k];
+  int b = 0;
+  for (; b + 64 <= nblk; b += 64) {
+    float v[64];
+#pragma unroll
+    for (int t = 0; t < 64; ++t) v[t] = gpart[(size_t)(b + t) * NPARAM + k];
+#pragma unroll
+    for (int t = 0; t < 64; ++t) gk += v[t];
+  }
+  for (; b < nblk; ++b) gk += gpart[(size_t)b * NPARAM + k];
   if (gout) gout[k] = gk;
   if (!update) return;
   const float m = b1 * m1[k] + (1.f - b1) * gk, v = b2 * m2[k] + (1.f - b2) * gk * gk;
@@ -682,7 +696,7 @@ int learned_train(Ctx &c, fvk_model *m, int steps, double lr, double *last_loss)
     if ((rc = run_loss_grad(m, c, B, nblk))) return rc;
     m->step += 1;
     const float c1 = 1.f - std::pow(b1, (float)m->step), c2 = 1.f - std::pow(b2, (float)m->step);
-    k_adam<<<(NPARAM + BS - 1) / BS, BS, 0, c.stream>>>(m->theta, m->m1, m->m2, m->gpart, nblk, nullptr, 1,
+    k_adam<<<(NPARAM + ADAM_B - 1) / ADAM_B, ADAM_B, 0, c.stream>>>(m->theta, m->m1, m->m2, m->gpart, nblk, nullptr, 1,
                                                         (float)lr, b1, b2, eps, c1, c2);
     FVK_HIP(hipGetLastError());
   }
@@ -841,7 +855,7 @@ int fvk_model_loss(fvk_model *m, fvk_ctx *cc, double *J, float *grad, float *dl,
   LossBufs B;
   int nblk = 0;
   GUARD_L(run_loss_grad(m, c, B, nblk));
-  k_adam<<<(NPARAM + BS - 1) / BS, BS, 0, c.stream>>>(m->theta, m->m1, m->m2, m->gpart, nblk, m->grad, 0, 0.f, 0.f,
+  k_adam<<<(NPARAM + ADAM_B - 1) / ADAM_B, ADAM_B, 0, c.stream>>>(m->theta, m->m1, m->m2, m->gpart, nblk, m->grad, 0, 0.f, 0.f,
                                                       0.f, 0.f, 1.f, 1.f);
   FVK_HIP(hipGetLastError());
   double jt[2];
@@ -878,7 +892,7 @@ int fvk_model_train(fvk_model *m, fvk_ctx *cc, int steps, double lr, double *los
     GUARD_L(run_loss_grad(m, c, B, nblk));
     m->step += 1;
     const float c1 = 1.f - std::pow(b1, (float)m->step), c2 = 1.f - std::pow(b2, (float)m->step);
-    k_adam<<<(NPARAM + BS - 1) / BS, BS, 0, c.stream>>>(m->theta, m->m1, m->m2, m->gpart, nblk, nullptr, 1,
+    k_adam<<<(NPARAM + ADAM_B - 1) / ADAM_B, ADAM_B, 0, c.stream>>>(m->theta, m->m1, m->m2, m->gpart, nblk, nullptr, 1,
                                                         (float)lr, b1, b2, eps, c1, c2);
     FVK_HIP(hipGetLastError());
     if (loss) {
