@@ -286,7 +286,7 @@ def simple_leg(fvk, args, model):
     # the reference's shipped configuration (cfd_setup.f90:528,581,662,742):
     # SIMPLER pressure, DILU momentum and DIC pressure preconditioners, urf_p
     # 0.1; factor and triangular sweeps in one launch each (the default:
-    # blocks owning ranges of rows, values inside a range through LDS), and
+    # blocks walking parts of the rows, values inside a part through LDS), and
     # for comparison one launch with rows taken in level order in chunks and
     # one launch per level.  First one application of the DIC / DILU factor
     # (both sweeps) in the three forms.
@@ -508,7 +508,7 @@ def flowlab_leg(fvk, args):
     """flowlab's serial CSR SIMPLE (flowlab/src/navierstokes.f90:515-641) on
     an n^3 lid-driven cavity (+-10% jitter, Re 100, urf 0.7 / 0.3, blending
     0.5): outer iterations per second with the factor and sweeps in one
-    launch each (blocks owning row ranges; rows in level order in chunks)
+    launch each (blocks walking parts of the rows; rows in level order in chunks)
     and with one launch per level, beside one outer iteration of flowlab's
     own Fortran (flang -O2, one core) on the same mesh."""
     from programs_amd import flowlab as fl
@@ -525,7 +525,7 @@ def flowlab_leg(fvk, args):
     out = dict(workload="flowlab CSR SIMPLE, %d^3 lid-driven cavity (+-10%% jitter), Re 100, momentum BiCGStab and "
                         "pressure CG (25 iterations, reduction 0.01) with flowlab's factor" % n,
                cells=m.n_dmn, faces=m.n_fce, nnz=m.nnz, mesh_build_s=t_mesh, context_s=t_ctx)
-    # one launch per sweep with row ranges owned by blocks (the default), with
+    # one launch per sweep with blocks walking parts ("ranges", the default), with
     # rows taken in level order in chunks, and one launch per level
     forms = args.flowlab_forms.split(",")
     for key, one, parts in (("one_launch", 1, 1), ("one_launch_chunks", 1, 0), ("per_level_launches", 0, 0)):
