@@ -286,6 +286,7 @@ static int ctx_build(Ctx &c, const Topo &t, int device, int flags) {
   for (int f = 0; f < nf; ++f) {
     fip[f] = c.iperm[t.fip[f]];
     fin[f] = t.fin[f] >= 0 ? c.iperm[t.fin[f]] : -1;
+    c.reversed = c.reversed || (t.fin[f] >= 0 && t.fip[f] > t.fin[f]);
   }
   c.h_fip = fip; c.h_fin = fin; c.h_fib = t.fib; c.h_fbty = t.fbty;
   std::vector<double> cx(n), cy(n), cz(n), v(n), vr(n);

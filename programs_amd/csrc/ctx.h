@@ -85,6 +85,7 @@ struct Ctx {
   int n = 0, nf = 0, nbf = 0, W = 0, Ws = 0, ndx = 0;
   std::vector<int> perm, iperm;  // perm[row] = reference cell (0-based)
   std::vector<int> h_fip, h_fin, h_fib, h_fbty;  // rows
+  bool reversed = false;  // an interior face has fce_ip > fce_in (create_arrays takes any; the mesh builders make none)
   HostIo io;
   int *where = nullptr;           // device: row of each reference cell (null: the same)
   DMesh M{};

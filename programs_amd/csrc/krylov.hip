@@ -964,11 +964,18 @@ int precond_build(Ctx &c, int imat) {
   if (imat == 0) {
     k_precond_jacobi<<<grid_for(n), BS, 0, c.stream>>>(n, c.diag, c.pc_c, c.pc_cr);
   } else if (c.sweep_one_launch && c.sweep_parts) {
+    // The factor takes ngn of the entry's face whichever side the row is on
+    // (solv_precond.f90:17-23), the sweeps the row's own coefficient: the same
+    // where every face runs from the lower cell to the higher one.
     int rc = sweep_pack_matrix(c);
+    c.sw_mat = false;
+    if (!rc && c.reversed) rc = sweep_lower(c.sw, c.stream, c.ngn, true);
     if (!rc)
       rc = sweep_factor(c.sw, c.stream, imat == 1 ? SWEEP_DIC : SWEEP_DILU, c.diag, nullptr, c.pc_c, c.pc_cr,
                         c.sweep_int + 3);
+    if (!rc && c.reversed) rc = sweep_lower(c.sw, c.stream, c.spv, false);
     if (rc) return rc;
+    c.sw_mat = true;
   } else if (c.sweep_one_launch) {
     k_sweep_mark<<<mark_grid(n), BS, 0, c.stream>>>(n, c.pc_c, c.sweep_int + 2, nullptr, 1);
     k_precond_sf<<<sweep_grid(c), BS, 0, c.stream>>>(c.M, c.lf.rows, c.sweep_lmask, imat, c.diag, c.ngp, c.ngn,

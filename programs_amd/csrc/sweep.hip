@@ -420,6 +420,12 @@ __global__ __launch_bounds__(BS) void k_sweep_pack(int np, int MW, const int *__
   }
 }
 
+__global__ __launch_bounds__(BS) void k_sweep_lower(size_t cnt, const int *__restrict__ idx,
+                                                    const double *__restrict__ vals, double *__restrict__ a) {
+  const size_t i = blockIdx.x * (size_t)BS + threadIdx.x;
+  if (i < cnt) a[i] = idx[i] >= 0 ? vals[idx[i]] : 0.0;
+}
+
 __global__ __launch_bounds__(BS) void k_sweep_factor_from(int n, const int *__restrict__ prow,
                                                           const int *__restrict__ ppos,
                                                           const double *__restrict__ crow,
@@ -548,6 +554,13 @@ int sweep_pack(SweepExec &X, hipStream_t s, const double *vals, const double *tv
   const int cnt = std::max(X.np, X.d[0].NE);
   k_sweep_pack<<<(cnt + BS - 1) / BS, BS, 0, s>>>(X.np, X.MW, X.d[0].val, X.d[1].val, X.tval, vals, tvals, X.d[0].a,
                                                   X.d[1].a, X.aT, X.d[0].NE, X.Ec, X.ticket + 2);
+  FVK_HIP(hipGetLastError());
+  return 0;
+}
+
+int sweep_lower(SweepExec &X, hipStream_t s, const double *vals, bool transposed) {
+  const size_t cnt = (size_t)X.MW * X.np;
+  k_sweep_lower<<<(unsigned)((cnt + BS - 1) / BS), BS, 0, s>>>(cnt, transposed ? X.tval : X.d[0].val, vals, X.d[0].a);
   FVK_HIP(hipGetLastError());
   return 0;
 }

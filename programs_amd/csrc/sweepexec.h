@@ -46,6 +46,9 @@ void sweep_exec_free(SweepExec &X);
 // entries tvals[...] (may be null: not needed by factor kind 0).  Opens the
 // export buffer of a factorisation.
 int sweep_pack(SweepExec &X, hipStream_t s, const double *vals, const double *tvals);
+// The lower entries alone: vals[val index], or by the transposed entries'
+// indices vals[tval]
+int sweep_lower(SweepExec &X, hipStream_t s, const double *vals, bool transposed);
 enum { SWEEP_DIC = 0, SWEEP_DILU = 1, SWEEP_FL = 2 };
 // The factor of the packed matrix (sweep_pack before each): c = 1/(d+small)
 // by row to crow, d to drow (null: not wanted); diag[dix ? dix[row] : row].

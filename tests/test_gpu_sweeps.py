@@ -126,6 +126,43 @@ def test_sweeps_on_tetrahedra_bitwise(rcm, tmp_path):
     m.free()
 
 
+@pytest.mark.parametrize("rcm", [False, True])
+@pytest.mark.parametrize("dims", [(9, 8, 7), (40, 13, 1)])
+def test_reversed_faces_bitwise(dims, rcm):
+    """A context from arrays with half of the interior faces running from the
+    higher cell to the lower one: the factor takes ng_p and ng_n by face
+    (solv_precond.f90:17-23, restated here), in every form."""
+    fvk = require_lib()
+    say("sweeps: reversed faces, box %s rcm %s" % (dims, rcm))
+    m = fvk.Mesh.box(*dims, jitter=0.0, seed=3)
+    t, g = m.topology(), m.geometry()
+    rng = np.random.default_rng(23)
+    rev = (t["fce_in"] > 0) & (rng.random(m.n_fce) < 0.5)
+    t["fce_ip"][rev], t["fce_in"][rev] = t["fce_in"][rev], t["fce_ip"][rev].copy()
+    ctx = fvk.grd_solv_arrays(t, g, m.n_dx, m.n_bf, rcm=rcm)
+    gp, gn = -rng.uniform(0.5, 1.5, (2, m.n_fce))
+    pl = rng.uniform(8.0, 9.0, m.n_vol)
+    fvk.set_matrix(ctx, pl, gp, gn)
+    b = rng.standard_normal(m.n_vol)
+    small = float.fromhex("0x1.79ca10c924224p-67")
+    for imat in (1, 2):
+        c, d = np.zeros(m.n_vol), pl.copy()
+        for i in range(m.n_vol):
+            for s in range(t["cell_ptr"][i], t["cell_ptr"][i + 1]):
+                f = t["fce_lst"][s] - 1
+                j = t["fce_ip"][f] + t["fce_in"][f] - i - 2
+                if t["fce_in"][f] > 0 and j < i:
+                    d[i] -= gn[f] * gn[f] * c[j] if imat == 1 else gp[f] * c[j] * gn[f]
+            c[i] = 1.0 / (d[i] + small)
+        for label, (c1, cr1) in all_modes(fvk, ctx, lambda: fvk.solv_precond(ctx, imat)):
+            assert np.array_equal(c, c1) and np.array_equal(d, cr1), ("factor", imat, label)
+        x = all_modes(fvk, ctx, lambda: fvk.solv_direct(ctx, imat, b))
+        for label, x1 in x[1:]:
+            assert np.array_equal(x[0][1], x1), ("sweeps", imat, label)
+    ctx.destroy()
+    m.free()
+
+
 def test_krylov_on_one_launch_sweeps_bitwise():
     fvk = require_lib()
     n = 48
