@@ -261,7 +261,9 @@ int fvk_sys_get_x(fvk_ctx *ctx, double *x);
    that a sweep's wait ran past its bound, as a wait that never ends would;
    parts that wait give up within 256 polls, blocks stop taking parts, and
    this and every later factorisation or sweep of the
-   context returns FVK_ERR_HIP. */
+   context returns FVK_ERR_HIP.  "sweep_positions" (a test of what follows;
+   0, default: the kernels' own limit): patterns whose tables need more
+   positions (fvk_sweep_positions) take the chunks of "sweep_parts" 0. */
 int fvk_ctx_set_param(fvk_ctx *ctx, const char *name, double value);
 /* How the one-launch sweeps split a pattern (1-based CSR with its diagonal,
    as solv_m receives it): parts of at most max_rows rows that depend on
@@ -274,6 +276,11 @@ int fvk_ctx_set_param(fvk_ctx *ctx, const char *name, double value);
    three right-hand sides, values passed between parts forward and backward.
    Host only; no counterpart in the reference. */
 int fvk_sweep_plan(int n, const int *ia, const int *ja, int max_rows, int *info);
+/* The positions of that plan's tables, rows and padding (a chunk has 64
+   whatever its rows).  FVK_ERR_ARG when there are more than limit (0: than the
+   kernels' 32-bit offsets reach, 2^28, or 2^27 where a row has more than four
+   lower or upper entries).  Host only. */
+int fvk_sweep_positions(int n, const int *ia, const int *ja, int max_rows, int64_t limit, int64_t *positions);
 
 /* The factorised preconditioner z = G G^T r, G = D^-1/2 (I + L) Delta, with
    D the diagonal of the current matrix, L strictly lower triangular on the
@@ -520,7 +527,7 @@ void fvk_fl_ctx_destroy(fvk_fl_ctx *ctx);
    chunks.  "sweep_blocks" (0: one per CU): blocks of the
    one-launch kernels.  All give the same bits.  "sweep_fail" 1 (a test of
    the failure path): as fvk_ctx_set_param's; the context's solves then
-   return FVK_ERR_HIP.  No counterpart in the reference. */
+   return FVK_ERR_HIP.  "sweep_positions": as there.  No counterpart in the reference. */
 int fvk_fl_ctx_set_param(fvk_fl_ctx *ctx, const char *name, double value);
 /* xdmn%x_vc (n_dim x n_dmn), vol, x_fc, norm, area, x_pc, x_nc, l_pn, w_fp
    (per face), ls (n_dim x n_dim x n_dmn); NULL skips */

@@ -992,6 +992,11 @@ int fvk_ctx_set_param(fvk_ctx *cc, const char *name, double value) {
     const int rc = sweep_parts_build(cc->c);
     if (rc) return rc;
   }
+  else if (!std::strcmp(name, "sweep_positions") && value >= 0 && value <= 1 << 28 && value == (long)value) {
+    cc->c.sweep_positions = (long)value;
+    const int rc = sweep_parts_build(cc->c);
+    if (rc) return rc;
+  }
   else if (!std::strcmp(name, "sweep_blocks_per_cu") && value >= 1 && value <= 8 && value == (int)value)
     cc->c.sweep_blocks_per_cu = (int)value;
   else if (!std::strcmp(name, "sweep_fail") && value == 1 && cc->c.sweep_int) {

@@ -109,6 +109,7 @@ struct Ctx {
   SweepExec sw;
   bool sweep_parts = true;
   int sweep_part_rows = 4096;     // rows of a part at most
+  long sweep_positions = 0;       // positions of its tables at most (0: the kernels' limit)
   // the packed copies in sw are of the current matrix / of pc_c, pc_cr
   bool sw_mat = false, sw_fac = false;
   // Krylov workspace (3 components)

@@ -63,6 +63,8 @@ struct FlCtx {
   SweepExec sw;
   bool parts = false;
   int part_rows = 4096;  // rows of a part at most
+  long positions = 0;    // positions of its tables at most (0: the kernels' limit)
+  bool narrow = false;   // no row has more than kSweepSlots lower or upper entries
   std::vector<int> h_kii, h_klo, h_kup, h_tpos;
   int *sweep_int = nullptr;  // tickets: forward, backward, factor; [3] wait-bound error
   // Krylov work: 6 vectors x 3 components, partials, scalars
@@ -930,8 +932,8 @@ static int fl_parts_setup(FlCtx &c) {
   sweep_exec_free(c.sw);
   const SweepGraph g = fl_sweep_graph(c.n, c.h_ia, c.h_ja, c.h_klo, c.h_kup, c.h_tpos);
   SweepPlan p;
-  const std::string e = sweep_plan(g, c.part_rows, p);
-  if (!e.empty()) { set_error(e); return FVK_ERR_ARG; }
+  // no plan: the rows are taken in level order in chunks (fl_parts_on)
+  if (!sweep_plan(g, c.part_rows, p, c.positions).empty()) return 0;
   c.sw.n_cu = c.n_cu;
   return sweep_exec_build(c.sw, p, c.stream);
 }
@@ -964,8 +966,10 @@ static int fl_sweep_grid(const FlCtx &c) {
 }
 static int fl_mark_grid(size_t cnt) { return (int)std::max<size_t>(1, std::min<size_t>((cnt + BS - 1) / BS, 4096)); }
 
+static bool fl_parts_on(const FlCtx &c) { return c.one_launch && c.parts && c.sw.built(); }
+
 static int fl_precond(FlCtx &c, const double *a) {
-  if (c.one_launch && c.parts) {
+  if (fl_parts_on(c)) {
     const int rc = sweep_pack(c.sw, c.stream, a, a);
     return rc ? rc : sweep_factor(c.sw, c.stream, SWEEP_FL, a, c.kii, c.pc, nullptr, c.sweep_int + 3);
   }
@@ -987,7 +991,7 @@ static int fl_precond(FlCtx &c, const double *a) {
 
 // x = M^-1 b (direct_solve), t: scratch
 static int fl_direct(FlCtx &c, int ncmp, const double *a, const double *b, double *t, double *x, const FlKS *ks) {
-  if (c.one_launch && c.parts) {
+  if (fl_parts_on(c)) {
     SweepGate G;
     if (ks) G = SweepGate{&ks->done, (int)(sizeof(FlKS) / sizeof(int)), ncmp};
     return sweep_apply(c.sw, c.stream, ncmp, b, x, G, c.sweep_int + 3);
@@ -1495,7 +1499,7 @@ static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
   c.nnz = (int)p.ja.size();
   const std::vector<int> &ia = p.ia, &ja = p.ja, &kii = p.kii, &klo = p.klo, &kup = p.kup, &tpos = p.tpos;
   const int mx = p.widest;
-  c.one_launch = mx <= kSweepSlots;
+  c.one_launch = c.narrow = mx <= kSweepSlots;
   c.h_ia = ia;
   c.h_ja = ja;
   c.h_kii = kii;
@@ -1932,6 +1936,18 @@ int fvk_sweep_plan(int n, const int *ia, const int *ja, int max_rows, int *info)
   return FVK_OK;
 }
 
+int fvk_sweep_positions(int n, const int *ia, const int *ja, int max_rows, int64_t limit, int64_t *positions) {
+  if (!ia || !ja || !positions || n < 1 || max_rows < 64 || limit < 0) { set_error("bad argument"); return FVK_ERR_ARG; }
+  FlPattern q;
+  const int rc = fl_pattern(n, ia, ja, q);
+  if (rc) return rc;
+  SweepPlan p;
+  const std::string e = sweep_plan(fl_sweep_graph(n, q.ia, q.ja, q.klo, q.kup, q.tpos), max_rows, p, (long)limit);
+  if (!e.empty()) { set_error(e); return FVK_ERR_ARG; }
+  *positions = p.np;
+  return FVK_OK;
+}
+
 int fvk_fl_csr_matches(const fvk_fl_ctx *cc, int n, const int *ia, const int *ja) {
   if (!cc || !ia || !ja) return 0;
   const FlCtx &c = cc->c;
@@ -2035,14 +2051,20 @@ int fvk_fl_ctx_set_param(fvk_fl_ctx *cc, const char *name, double value) {
     return FVK_OK;
   }
   if (!std::strcmp(name, "sweep_parts") && (value == 0 || value == 1)) {
-    if (value == 1 && !c.sw.built()) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
+    if (value == 1 && !c.narrow) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
     c.parts = value != 0;
     return FVK_OK;
   }
   if (!std::strcmp(name, "sweep_part_rows") && value >= 256 && value <= 6400 && value == (int)value) {
-    if (!c.sw.built()) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
+    if (!c.narrow) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
     FVK_HIP(hipStreamSynchronize(c.stream));
     c.part_rows = (int)value;
+    return fl_parts_setup(c);
+  }
+  if (!std::strcmp(name, "sweep_positions") && value >= 0 && value <= 1 << 28 && value == (long)value) {
+    if (!c.narrow) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
+    FVK_HIP(hipStreamSynchronize(c.stream));
+    c.positions = (long)value;
     return fl_parts_setup(c);
   }
   if (!std::strcmp(name, "sweep_blocks") && value >= 0 && value <= 65536 && value == (int)value) {

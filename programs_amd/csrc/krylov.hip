@@ -944,14 +944,13 @@ int sweep_parts_build(Ctx &c) {
     }
   }
   SweepPlan p;
-  const std::string e = sweep_plan(g, c.sweep_part_rows, p);
-  if (!e.empty()) {
-    set_error(e);
-    return FVK_ERR_ARG;
-  }
+  // no plan: the rows are taken in level order in chunks (parts_on)
+  if (!sweep_plan(g, c.sweep_part_rows, p, c.sweep_positions).empty()) return 0;
   c.sw.n_cu = c.n_cu;
   return sweep_exec_build(c.sw, p, c.stream);
 }
+
+static bool parts_on(const Ctx &c) { return c.sweep_one_launch && c.sweep_parts && c.sw.built(); }
 
 static int sweep_pack_matrix(Ctx &c) {
   const int rc = sweep_pack(c.sw, c.stream, c.spv, c.ngp);
@@ -963,7 +962,7 @@ int precond_build(Ctx &c, int imat) {
   const int n = c.n;
   if (imat == 0) {
     k_precond_jacobi<<<grid_for(n), BS, 0, c.stream>>>(n, c.diag, c.pc_c, c.pc_cr);
-  } else if (c.sweep_one_launch && c.sweep_parts) {
+  } else if (parts_on(c)) {
     // The factor takes ngn of the entry's face whichever side the row is on
     // (solv_precond.f90:17-23), the sweeps the row's own coefficient: the same
     // where every face runs from the lower cell to the higher one.
@@ -990,7 +989,7 @@ int precond_build(Ctx &c, int imat) {
   FVK_HIP(hipGetLastError());
   c.pc_imat = imat;
   c.pc_valid = true;
-  c.sw_fac = imat != 0 && c.sweep_one_launch && c.sweep_parts;
+  c.sw_fac = imat != 0 && parts_on(c);
   return 0;
 }
 
@@ -998,7 +997,7 @@ int precond_apply(Ctx &c, int imat, int nvc, const double *b, double *x, const K
   const int n = c.n;
   if (imat == 0) {
     k_jacobi_apply<<<grid_for(n), BS, 0, c.stream>>>(n, nvc, c.pc_c, b, x, gate);
-  } else if (c.sweep_one_launch && c.sweep_parts) {
+  } else if (parts_on(c)) {
     // a factor that another form built, or that the caller gave
     int rc = c.sw_mat ? 0 : sweep_pack_matrix(c);
     if (!rc && !c.sw_fac) {

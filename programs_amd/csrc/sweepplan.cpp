@@ -203,7 +203,8 @@ static bool brick_parts(const SweepGraph &g, int max_rows, std::vector<int> &par
   return true;
 }
 
-static bool plan_with(const SweepGraph &g, int max_rows, SweepPlan &p) {
+enum PlanEnd { PLAN_OK, PLAN_LDS, PLAN_POSITIONS };
+static PlanEnd plan_with(const SweepGraph &g, int max_rows, long limit, SweepPlan &p) {
   const int n = g.n;
   std::vector<int> part;
   int P = 0;
@@ -293,8 +294,8 @@ static bool plan_with(const SweepGraph &g, int max_rows, SweepPlan &p) {
   });
   std::vector<int> cb(P + 1, 0);
   for (int q = 0; q < P; ++q) cb[q + 1] = cb[q] + nch[q];
-  const int C = cb[P];
-  p.np = C * kChunk;
+  if ((long)cb[P] * kChunk > limit) return PLAN_POSITIONS;
+  p.np = cb[P] * kChunk;
   // exports, numbered part by part in the order the direction runs
   std::vector<int> eslot[2];
   for (int dir = 0; dir < 2; ++dir) {
@@ -383,7 +384,7 @@ static bool plan_with(const SweepGraph &g, int max_rows, SweepPlan &p) {
           for (; t < MW; ++t) ix[1 + t] = (unsigned short)(zero * 8);
         }
     });
-    if (slots.load() * 8 > 65535) return false;
+    if (slots.load() * 8 > 65535) return PLAN_LDS;
     // lanes without a row write the last slot and export nothing
     parallel_for(P, 8, [&](int q) {
       const int other = (pbeg[q + 1] - pbeg[q] + (int)halo[q].size() + 1) * 8;
@@ -410,7 +411,7 @@ static bool plan_with(const SweepGraph &g, int max_rows, SweepPlan &p) {
     });
   }
   p.slots = slots.load();
-  if (p.lds(3) > (size_t)kSweepLds) return false;
+  if (p.lds(3) > (size_t)kSweepLds) return PLAN_LDS;
   // rows of each part by device row
   p.prow.resize(n);
   p.ppos.resize(n);
@@ -431,10 +432,10 @@ static bool plan_with(const SweepGraph &g, int max_rows, SweepPlan &p) {
       p.pslot[pbeg[q] + t] = (unsigned short)(slot[k] * 8);
     }
   });
-  return true;
+  return PLAN_OK;
 }
 
-std::string sweep_plan(const SweepGraph &g, int max_rows, SweepPlan &p) {
+std::string sweep_plan(const SweepGraph &g, int max_rows, SweepPlan &p, long limit) {
   int W = 1;
   for (int k = 0; k < g.n; ++k) W = std::max({W, g.lptr[k + 1] - g.lptr[k], g.uptr[k + 1] - g.uptr[k]});
   if (W > 8) return "a row has more lower or upper entries than one launch holds";
@@ -444,13 +445,17 @@ std::string sweep_plan(const SweepGraph &g, int max_rows, SweepPlan &p) {
     p = SweepPlan();
     p.W = W;
     p.MW = W <= 3 ? 3 : W <= 4 ? 4 : 8;
-    if (plan_with(g, r, p)) return "";
+    const long most = (1L << 32) / (2 * p.nrec());
+    const PlanEnd e = plan_with(g, r, limit > 0 ? std::min(limit, most) : most, p);
+    if (e == PLAN_OK) return "";
+    if (e == PLAN_POSITIONS) return "the pattern needs more positions than the sweep tables hold";
   }
   return "no plan";
 }
 
 std::string sweep_plan_check(const SweepGraph &g, const SweepPlan &p) {
   const int NI = p.nrec(), ND = p.at_need();
+  if ((long)p.np * 2 * NI > 1L << 32) return "a record's byte offset";
   // rank at each position
   std::vector<int> rank_of_row(g.n, -1), rank_at(p.np, -1);
   for (int k = 0; k < g.n; ++k) rank_of_row[g.row[k]] = k;

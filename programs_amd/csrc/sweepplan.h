@@ -56,9 +56,12 @@ struct SweepPlan {
   size_t lds(int nc) const { return (size_t)8 * nc * slots + (size_t)4 * maxh; }
 };
 
-// max_rows: rows of a part at most.  Empty string, or why there is no plan
-// (a row with more than 8 entries on one side).
-std::string sweep_plan(const SweepGraph &g, int max_rows, SweepPlan &p);
+// max_rows: rows of a part at most.  limit: positions at most (0, or more
+// than the kernels take: what a 32-bit byte offset into the records reaches,
+// 2^28 positions, 2^27 of rows with more than four entries a side).  Empty
+// string, or why there is no plan: a row with more than 8 entries on one
+// side, or too many positions.
+std::string sweep_plan(const SweepGraph &g, int max_rows, SweepPlan &p, long limit = 0);
 
 // Walks the plan as the kernels do and checks that every value is there
 // when it is read, that a part only needs parts taken before it, and that

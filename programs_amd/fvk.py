@@ -150,6 +150,7 @@ def lib():
         "fvk_sys_get_x": [_vp, _dp],
         "fvk_ctx_set_param": [_vp, C.c_char_p, C.c_double],
         "fvk_sweep_plan": [C.c_int, _ip, _ip, C.c_int, _ip],
+        "fvk_sweep_positions": [C.c_int, _ip, _ip, C.c_int, C.c_int64, C.POINTER(C.c_int64)],
         "fvk_factor_set": [_vp, _fp, _fp],
         "fvk_factor_apply": [_vp, _dp, _dp],
         "fvk_factor_get": [_vp, _fp, _fp],
@@ -527,6 +528,15 @@ def sweep_plan(ia, ja, max_rows=4096):
     o = np.zeros(8, np.int32)
     _check(lib().fvk_sweep_plan(len(a) - 1, _i(a), _i(b), max_rows, _i(o)))
     return dict(zip(("parts", "chunks", "levels", "bricks", "lds1", "lds3", "passed_fwd", "passed_bwd"), map(int, o)))
+
+
+def sweep_positions(ia, ja, max_rows=4096, limit=0):
+    """Positions of the plan's tables; FvkError when there are more than limit
+    (0: than the kernels reach).  Host only."""
+    a, b = np.ascontiguousarray(ia, np.int32), np.ascontiguousarray(ja, np.int32)
+    o = C.c_int64()
+    _check(lib().fvk_sweep_positions(len(a) - 1, _i(a), _i(b), max_rows, limit, C.byref(o)))
+    return o.value
 
 
 def factor_set(ctx: Ctx, l, sig):

@@ -124,3 +124,30 @@ def test_solves_by_row_width(n, width, full):
             assert np.abs(x - wx).max() <= tol * np.abs(wx).max(), (isol, n_iter)
             assert abs(norm[0] - wn) <= tol * np.abs(wr).sum(), (isol, n_iter)
     L.fvk_fl_ctx_destroy(h)
+
+
+def test_sweep_forms_bitwise():
+    """One launch per level, chunks, parts, and a pattern with more positions
+    than the parts' tables may hold ("sweep_positions"), which takes chunks."""
+    fvk = require_lib()
+    ia, ja = pattern(900, 7, True, 3)
+    rows = np.repeat(np.arange(900), np.diff(ia))
+    rng = np.random.default_rng(5)
+    a, b = rng.uniform(-1.0, -0.2, len(ja)), rng.standard_normal(900)
+    a[rows == ja - 1] = 9.0
+    L = fvk.lib()
+    h = C.c_void_p()
+    ip = lambda v: v.ctypes.data_as(C.POINTER(C.c_int))
+    dp = lambda v: v.ctypes.data_as(C.POINTER(C.c_double))
+    assert L.fvk_fl_csr_create(900, ip(ia), ip(ja), 0, C.byref(h)) == 0
+    first = None
+    for params in ((), ((b"sweep_positions", 64),), ((b"sweep_positions", 0),), ((b"sweep_parts", 0),),
+                   ((b"sweep_positions", 64), (b"sweep_parts", 1)), ((b"sweep_one_launch", 0),)):
+        print("flowlab sweeps:", params, flush=True)
+        for k, v in params:
+            assert L.fvk_fl_ctx_set_param(h, k, C.c_double(v)) == 0
+        x, r, norm = np.zeros(900), b.copy(), np.zeros(1)
+        assert L.fvk_fl_lin_eqns_solver(h, dp(a), dp(x), dp(r), dp(norm), 4, C.c_double(0.0), 2) == 0
+        first = x if first is None else first
+        assert np.array_equal(x, first), params
+    L.fvk_fl_ctx_destroy(h)

@@ -163,6 +163,26 @@ def test_reversed_faces_bitwise(dims, rcm):
     m.free()
 
 
+def test_pattern_beyond_the_tables_bitwise():
+    """A pattern whose plan has more positions than its tables may hold
+    ("sweep_positions") takes the chunks, and the parts again without it."""
+    fvk = require_lib()
+    say("sweeps: more positions than the tables hold")
+    m = fvk.Mesh.box(19, 6, 5, jitter=0.0, seed=3)
+    ctx = fvk.grd_solv(m)
+    pl, ngp, ngn = random_matrix(m, 29)
+    fvk.set_matrix(ctx, pl, ngp, ngn)
+    b = np.random.default_rng(1).standard_normal(m.n_vol)
+    want = [(fvk.solv_precond(ctx, k), fvk.solv_direct(ctx, k, b)) for k in (1, 2)]
+    for limit in (64, 0):
+        fvk.set_param(ctx, "sweep_positions", limit)
+        for k, (f, x) in zip((2, 1), want[::-1]):
+            assert np.array_equal(fvk.solv_direct(ctx, k, b), x), (limit, k)
+            assert all(np.array_equal(p, q) for p, q in zip(fvk.solv_precond(ctx, k), f)), (limit, k)
+    ctx.destroy()
+    m.free()
+
+
 def test_krylov_on_one_launch_sweeps_bitwise():
     fvk = require_lib()
     n = 48

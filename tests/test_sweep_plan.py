@@ -69,3 +69,13 @@ def test_unstructured(n, span, width, rows):
 def test_too_many_entries_is_refused():
     with pytest.raises(fvk.FvkError):
         fvk.sweep_plan(*csr(10, [(9, j) for j in range(9)]), 64)
+
+
+@pytest.mark.parametrize("n,pairs", [(3000, [(i, i - 1) for i in range(1, 3000)]), box(25, 24, 23),
+                                     (3000, [(i, i - j) for i in range(3000) for j in range(1, 9) if i >= j])])
+def test_positions_are_limited(n, pairs):
+    ia, ja = csr(n, [(int(i), int(j)) for i, j in pairs])
+    p = fvk.sweep_positions(ia, ja)
+    assert p >= n and fvk.sweep_positions(ia, ja, limit=p) == p
+    with pytest.raises(fvk.FvkError):
+        fvk.sweep_positions(ia, ja, limit=p - 1)
