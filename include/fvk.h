@@ -276,8 +276,9 @@ int fvk_ctx_set_param(fvk_ctx *ctx, const char *name, double value);
    three right-hand sides, values passed between parts forward and backward.
    Host only; no counterpart in the reference. */
 int fvk_sweep_plan(int n, const int *ia, const int *ja, int max_rows, int *info);
-/* The positions of that plan's tables, rows and padding (a chunk has 64
-   whatever its rows).  FVK_ERR_ARG when there are more than limit (0: than the
+/* The positions of that plan's tables, rows and padding: chunks times the rows
+   a chunk may have, which is 64, or less where that would make more than 8
+   positions a row.  FVK_ERR_ARG when there are more than limit (0: than the
    kernels' 32-bit offsets reach, 2^28, or 2^27 where a row has more than four
    lower or upper entries).  Host only. */
 int fvk_sweep_positions(int n, const int *ia, const int *ja, int max_rows, int64_t limit, int64_t *positions);

@@ -1931,7 +1931,7 @@ int fvk_sweep_plan(int n, const int *ia, const int *ja, int max_rows, int *info)
   if (!e.empty()) { set_error(e); return FVK_ERR_ARG; }
   e = sweep_plan_check(g, p);
   if (!e.empty()) { set_error("sweep plan: " + e); return FVK_ERR_STATE; }
-  const int v[8] = {p.P, p.np / kChunk, p.levels, p.bricks ? 1 : 0, (int)p.lds(1), (int)p.lds(3), p.d[0].NE, p.d[1].NE};
+  const int v[8] = {p.P, p.np / p.width, p.levels, p.bricks ? 1 : 0, (int)p.lds(1), (int)p.lds(3), p.d[0].NE, p.d[1].NE};
   std::copy(v, v + 8, info);
   return FVK_OK;
 }

@@ -7,7 +7,7 @@
 // A block takes parts of the plan from a ticket counter, in an order in
 // which a part only needs values of parts taken before it (no deadlock
 // whatever the residency), and runs a part with three waves:
-//   wave 0 computes: it walks the part's chunks (64 rows that do not depend
+//   wave 0 computes: it walks the part's chunks (up to 64 rows that do not depend
 //     on each other) in order.  All values it reads sit in LDS, its own
 //     rows' and the halo's; a wave's LDS operations are in order, so chunk
 //     after chunk needs no barrier.  Matrix entries, factor and records are
@@ -61,7 +61,7 @@ constexpr int sweep_ahead(int MW, int KIND) {
 }
 
 struct SweepArgs {
-  int P, np, slots, NE, NEo, n;
+  int P, np, slots, NE, NEo, n, width;
   unsigned shared;            // LDS address of the block's shared scalars
   const int *part, *prow, *ppos, *hsrc;
   const unsigned short *pslot, *rec;
@@ -171,11 +171,15 @@ __device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nc
     if (KIND == 2) B.a2[t] = opaque(A.a2 + (size_t)t * A.np);
   }
   if (KIND == 0) B.c = opaque(A.c);
-  const unsigned lane8 = threadIdx.x * 8u;
+  // lanes beyond the width repeat its last lane: the same row, the same values
+  const unsigned lane8 = min((int)threadIdx.x, A.width - 1) * 8u;
+  // a power of two, in a vector register: one instruction shifts and adds
+  unsigned shift = 31u - __builtin_clz((unsigned)A.width * 8u);
+  asm volatile("" : "+v"(shift));
   // byte offset of the j-th chunk in the sweep's direction (clamped to the part's last)
   auto at = [&](int j) {
     const int jj = min(j, nch - 1);
-    return (unsigned)(FWD ? c0 + jj : c0 + nch - 1 - jj) * (kChunk * 8u) + lane8;
+    return ((unsigned)(FWD ? c0 + jj : c0 + nch - 1 - jj) << shift) + lane8;
   };
   SweepStage<MW> S[kRing];
 #pragma unroll
@@ -478,7 +482,7 @@ static int allow_lds() {
 }
 
 int sweep_exec_build(SweepExec &X, const SweepPlan &p, hipStream_t s) {
-  X.n = p.n; X.P = p.P; X.MW = p.MW; X.np = p.np; X.slots = p.slots; X.bricks = p.bricks;
+  X.n = p.n; X.P = p.P; X.MW = p.MW; X.np = p.np; X.slots = p.slots; X.width = p.width; X.bricks = p.bricks;
   for (int k = 1; k <= 3; ++k) X.lds_[k] = p.lds(k);
   int rc = 0;
 #define U(dst, src) if (!rc) rc = up(X, &dst, src)
@@ -517,6 +521,7 @@ static SweepArgs args(const SweepExec &X, int dir) {
   SweepArgs A;
   const SweepExec::Dir &D = X.d[dir], &O = X.d[1 - dir];
   A.P = X.P; A.np = X.np; A.slots = X.slots; A.NE = D.NE; A.NEo = O.NE; A.n = X.n;
+  A.width = X.width;
   A.part = X.part; A.prow = X.prow; A.ppos = X.ppos; A.pslot = X.pslot;
   A.rec = D.rec; A.hsrc = D.hsrc;
   A.a = D.a; A.a2 = nullptr; A.c = X.c; A.src = nullptr; A.cr = X.cr; A.dix = nullptr; A.dst = nullptr;

@@ -16,7 +16,7 @@ struct SweepGate {
 };
 
 struct SweepExec {
-  int n = 0, P = 0, MW = 0, np = 0, slots = 0, n_cu = 256, blocks = 0;  // blocks: launch size, 0: what fits
+  int n = 0, P = 0, MW = 0, np = 0, slots = 0, width = kChunk, n_cu = 256, blocks = 0;  // blocks: launch size, 0: what fits
   size_t lds_[4] = {0, 0, 0, 0};
   bool bricks = false;
   std::vector<void *> mem;

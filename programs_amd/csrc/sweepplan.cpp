@@ -263,39 +263,47 @@ static PlanEnd plan_with(const SweepGraph &g, int max_rows, long limit, SweepPla
   // chunks: rows in level order; a new chunk when one is full or the next
   // row depends on a row of the chunk being filled
   std::vector<int> chunk(n), lane(n), slot(n), nch(P);
-  std::vector<int> dep(g.symmetric ? 0 : n, -1);  // asymmetric: newest chunk that reaches a row from an upper entry
+  std::vector<int> dep(g.symmetric ? 0 : n);  // asymmetric: newest chunk that reaches a row from an upper entry
   std::vector<int> ne[2] = {std::vector<int>(P), std::vector<int>(P)};
-  parallel_for(P, 8, [&](int q) {
-    int c = 0, fill = 0, e0 = 0, e1 = 0;
-    for (int t = pbeg[q]; t < pbeg[q + 1]; ++t) {
-      const int k = order[t];
-      bool next = fill == kChunk;
-      for (int z = g.lptr[k]; !next && z < g.lptr[k + 1]; ++z) {
-        const int j = g.lcol[z];
-        next = part[j] == q && chunk[j] == c;
+  for (p.width = kChunk;; p.width /= 2) {
+    const int width = p.width;
+    std::fill(dep.begin(), dep.end(), -1);
+    parallel_for(P, 8, [&](int q) {
+      int c = 0, fill = 0, e0 = 0, e1 = 0;
+      for (int t = pbeg[q]; t < pbeg[q + 1]; ++t) {
+        const int k = order[t];
+        bool next = fill == width;
+        for (int z = g.lptr[k]; !next && z < g.lptr[k + 1]; ++z) {
+          const int j = g.lcol[z];
+          next = part[j] == q && chunk[j] == c;
+        }
+        if (!next && !g.symmetric) next = dep[k] == c;
+        if (next) {
+          ++c;
+          fill = 0;
+        }
+        chunk[k] = c;
+        lane[k] = fill++;
+        slot[k] = t - pbeg[q];
+        if (!g.symmetric)
+          for (int z = g.uptr[k]; z < g.uptr[k + 1]; ++z)
+            if (part[g.ucol[z]] == q) dep[g.ucol[z]] = c;
+        e0 += exported(k, 0);
+        e1 += exported(k, 1);
       }
-      if (!next && !g.symmetric) next = dep[k] == c;
-      if (next) {
-        ++c;
-        fill = 0;
-      }
-      chunk[k] = c;
-      lane[k] = fill++;
-      slot[k] = t - pbeg[q];
-      if (!g.symmetric)
-        for (int z = g.uptr[k]; z < g.uptr[k + 1]; ++z)
-          if (part[g.ucol[z]] == q) dep[g.ucol[z]] = c;
-      e0 += exported(k, 0);
-      e1 += exported(k, 1);
-    }
-    nch[q] = c + 1;
-    ne[0][q] = e0;
-    ne[1][q] = e1;
-  });
+      nch[q] = c + 1;
+      ne[0][q] = e0;
+      ne[1][q] = e1;
+    });
+    long positions = 0;
+    for (int q = 0; q < P; ++q) positions += (long)nch[q] * width;
+    if (positions <= (long)kPadding * n || width <= kPadding) break;
+  }
   std::vector<int> cb(P + 1, 0);
   for (int q = 0; q < P; ++q) cb[q + 1] = cb[q] + nch[q];
-  if ((long)cb[P] * kChunk > limit) return PLAN_POSITIONS;
-  p.np = cb[P] * kChunk;
+  const int width = p.width;
+  if ((long)cb[P] * width > limit) return PLAN_POSITIONS;
+  p.np = cb[P] * width;
   // exports, numbered part by part in the order the direction runs
   std::vector<int> eslot[2];
   for (int dir = 0; dir < 2; ++dir) {
@@ -355,7 +363,7 @@ static PlanEnd plan_with(const SweepGraph &g, int max_rows, long limit, SweepPla
       };
       for (int s = a; s < b; ++s) {
         const int k = order[dir == 0 ? s : a + b - 1 - s];
-        const size_t pos = (size_t)(cb[q] + chunk[k]) * kChunk + lane[k];
+        const size_t pos = (size_t)(cb[q] + chunk[k]) * width + lane[k];
         unsigned short *ix = &D.rec[pos * NI];
         ix[0] = (unsigned short)(slot[k] * 8);
         ix[ND + 1] = (unsigned short)((unsigned)eslot[dir][k] & 0xffffu);
@@ -375,8 +383,8 @@ static PlanEnd plan_with(const SweepGraph &g, int max_rows, long limit, SweepPla
       if (used * 8 > 65535) return;  // no plan: see below
       // padding entries read the zero slot; the need is the chunk's in every lane
       for (int c = 0; c < nch[q]; ++c)
-        for (int l = 0; l < kChunk; ++l) {
-          const size_t pos = (size_t)(cb[q] + c) * kChunk + l;
+        for (int l = 0; l < width; ++l) {
+          const size_t pos = (size_t)(cb[q] + c) * width + l;
           unsigned short *ix = &D.rec[pos * NI];
           ix[ND] = (unsigned short)need[c];
           int t = 0;
@@ -391,8 +399,8 @@ static PlanEnd plan_with(const SweepGraph &g, int max_rows, long limit, SweepPla
       std::vector<int> fill(nch[q], 0);
       for (int t = pbeg[q]; t < pbeg[q + 1]; ++t) fill[chunk[order[t]]] = lane[order[t]] + 1;
       for (int c = 0; c < nch[q]; ++c)
-        for (int l = fill[c]; l < kChunk; ++l) {
-          unsigned short *ix = &D.rec[((size_t)(cb[q] + c) * kChunk + l) * NI];
+        for (int l = fill[c]; l < width; ++l) {
+          unsigned short *ix = &D.rec[((size_t)(cb[q] + c) * width + l) * NI];
           ix[0] = (unsigned short)other;
           ix[ND + 1] = ix[ND + 2] = 0xffffu;
         }
@@ -428,7 +436,7 @@ static PlanEnd plan_with(const SweepGraph &g, int max_rows, long limit, SweepPla
     for (size_t t = 0; t < r.size(); ++t) {
       const int k = r[t].second;
       p.prow[pbeg[q] + t] = r[t].first;
-      p.ppos[pbeg[q] + t] = (cb[q] + chunk[k]) * kChunk + lane[k];
+      p.ppos[pbeg[q] + t] = (cb[q] + chunk[k]) * width + lane[k];
       p.pslot[pbeg[q] + t] = (unsigned short)(slot[k] * 8);
     }
   });
@@ -478,15 +486,15 @@ std::string sweep_plan_check(const SweepGraph &g, const SweepPlan &p) {
       int have = 0;
       for (int c = 0; c < Q[1]; ++c) {
         const int ch = Q[0] + (dir == 0 ? c : Q[1] - 1 - c);
-        const int need = D.rec[(size_t)ch * kChunk * NI + ND];
+        const int need = D.rec[(size_t)ch * p.width * NI + ND];
         if (need > nh) return "halo count";
         for (; have < need; ++have) {
           const int e = D.hsrc[h0 + have];
           if (e < 0 || e >= D.NE || exported[e] < 0) return "a halo value of a part not taken before";
           lds[Q[3] + have] = exported[e];
         }
-        for (int l = 0; l < kChunk; ++l) {
-          const size_t pos = (size_t)ch * kChunk + l;
+        for (int l = 0; l < p.width; ++l) {
+          const size_t pos = (size_t)ch * p.width + l;
           const int k = rank_at[pos];
           const unsigned short *ix = &D.rec[pos * NI];
           if (ix[ND] != need) return "the need differs between lanes";
@@ -502,8 +510,8 @@ std::string sweep_plan_check(const SweepGraph &g, const SweepPlan &p) {
           for (; t < p.MW; ++t)
             if (ix[1 + t] / 8 != zero || D.val[(size_t)t * p.np + pos] >= 0) return "padding entry";
         }
-        for (int l = 0; l < kChunk; ++l) {
-          const size_t pos = (size_t)ch * kChunk + l;
+        for (int l = 0; l < p.width; ++l) {
+          const size_t pos = (size_t)ch * p.width + l;
           const int k = rank_at[pos];
           if (k < 0) continue;
           const unsigned short *ix = &D.rec[pos * NI];

@@ -20,22 +20,31 @@ struct SweepGraph {
   bool symmetric = false;        // the upper entries are the lower ones transposed
 };
 
-// kChunk rows are run together by the lanes of one wave
+// at most kChunk rows are run together by the lanes of one wave
 constexpr int kChunk = 64;
+// positions a row at most (SweepPlan::width)
+constexpr int kPadding = 8;
 // LDS of one block: 160 KiB less the kernel's few shared scalars
 constexpr int kSweepLds = 163840 - 256;
 
 // The parts, in the order in which the forward sweep may take them (the
 // backward sweep takes them from the last to the first).  A part's rows are
-// packed into chunks of at most kChunk rows that do not depend on each
+// packed into chunks of at most `width` rows that do not depend on each
 // other, in an order in which every row follows the rows it depends on; the
 // backward sweep walks the chunks from the last to the first.  Position p =
-// 64 chunk + lane.  Inside a part a row's value sits in an LDS slot: own
+// width chunk + lane.  Inside a part a row's value sits in an LDS slot: own
 // rows first, then (per direction) the halo, values of rows of other parts
 // in the order in which the chunks need them, a slot that stays zero (for
 // padding entries) and one that padding lanes write.
+// The width is kChunk unless padding would then take more than kPadding
+// positions a row: a chunk of a narrow pattern has few rows (one on a chain),
+// and a position costs 148 bytes of tables and more.  Then it is the largest
+// power of two that keeps to kPadding; 8 always does.  (A chain of 20,000 rows:
+// 64 positions a row -> 8, its context made in 27 ms -> 9, DIC, both sweeps,
+// 3.74 ms -> 3.77, for a vector register that holds the shift; 128^3, which
+// stays at 64: 205 us both.)
 struct SweepPlan {
-  int n = 0, P = 0, W = 0, MW = 0, np = 0, levels = 0;
+  int n = 0, P = 0, W = 0, MW = 0, np = 0, levels = 0, width = kChunk;
   int slots = 0, maxh = 0;                 // the most LDS slots and halo values of a part
   bool bricks = false;
   std::vector<int> part;                   // 8 ints a part: first chunk, chunks, first row, rows,

@@ -76,6 +76,6 @@ def test_too_many_entries_is_refused():
 def test_positions_are_limited(n, pairs):
     ia, ja = csr(n, [(int(i), int(j)) for i, j in pairs])
     p = fvk.sweep_positions(ia, ja)
-    assert p >= n and fvk.sweep_positions(ia, ja, limit=p) == p
+    assert n <= p <= 8 * n and fvk.sweep_positions(ia, ja, limit=p) == p
     with pytest.raises(fvk.FvkError):
         fvk.sweep_positions(ia, ja, limit=p - 1)
