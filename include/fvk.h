@@ -263,7 +263,9 @@ int fvk_sys_get_x(fvk_ctx *ctx, double *x);
    this and every later factorisation or sweep of the
    context returns FVK_ERR_HIP.  "sweep_positions" (a test of what follows;
    0, default: the kernels' own limit): patterns whose tables need more
-   positions (fvk_sweep_positions) take the chunks of "sweep_parts" 0. */
+   positions (fvk_sweep_positions), or more device memory than there is, take
+   the chunks of "sweep_parts" 0; "sweep_fail" 2: the next tables find no
+   memory. */
 int fvk_ctx_set_param(fvk_ctx *ctx, const char *name, double value);
 /* How the one-launch sweeps split a pattern (1-based CSR with its diagonal,
    as solv_m receives it): parts of at most max_rows rows that depend on
@@ -528,7 +530,7 @@ void fvk_fl_ctx_destroy(fvk_fl_ctx *ctx);
    chunks.  "sweep_blocks" (0: one per CU): blocks of the
    one-launch kernels.  All give the same bits.  "sweep_fail" 1 (a test of
    the failure path): as fvk_ctx_set_param's; the context's solves then
-   return FVK_ERR_HIP.  "sweep_positions": as there.  No counterpart in the reference. */
+   return FVK_ERR_HIP.  "sweep_positions", "sweep_fail" 2: as there.  No counterpart in the reference. */
 int fvk_fl_ctx_set_param(fvk_fl_ctx *ctx, const char *name, double value);
 /* xdmn%x_vc (n_dim x n_dmn), vol, x_fc, norm, area, x_pc, x_nc, l_pn, w_fp
    (per face), ls (n_dim x n_dim x n_dmn); NULL skips */

@@ -354,12 +354,13 @@ static int ctx_build(Ctx &c, const Topo &t, int device, int flags) {
   FVK_HIP(hipDeviceGetAttribute(&c.n_cu, hipDeviceAttributeMultiprocessorCount, c.device));
   if (Ws > 8) c.sweep_one_launch = false;  // slot masks hold 8 slots
   if ((rc = sweep_masks_build(c))) return rc;
-  if ((rc = sweep_parts_build(c))) return rc;
   if ((rc = dalloc(c, &c.wk, (size_t)8 * wk_ld(n)))) return rc;
   if ((rc = dalloc(c, &c.ks, 3))) return rc;
   if ((rc = dalloc(c, &c.ksr, 6))) return rc;
   if ((rc = dalloc(c, &c.part, (size_t)4 * RG * 8))) return rc;
   if ((rc = dalloc(c, &c.stage, (size_t)3 * std::max(n, nf)))) return rc;
+  // last: without memory for its tables the sweeps take another form
+  if ((rc = sweep_parts_build(c))) return rc;
   FVK_HIP(hipStreamSynchronize(c.stream));
   return 0;
 }
@@ -999,6 +1000,7 @@ int fvk_ctx_set_param(fvk_ctx *cc, const char *name, double value) {
   }
   else if (!std::strcmp(name, "sweep_blocks_per_cu") && value >= 1 && value <= 8 && value == (int)value)
     cc->c.sweep_blocks_per_cu = (int)value;
+  else if (!std::strcmp(name, "sweep_fail") && value == 2) cc->c.sw.deny = true;
   else if (!std::strcmp(name, "sweep_fail") && value == 1 && cc->c.sweep_int) {
     const int one = 1;
     FVK_HIP(hipMemcpyAsync(cc->c.sweep_int + 3, &one, sizeof one, hipMemcpyHostToDevice, cc->c.stream));

@@ -932,7 +932,8 @@ static int fl_parts_setup(FlCtx &c) {
   sweep_exec_free(c.sw);
   const SweepGraph g = fl_sweep_graph(c.n, c.h_ia, c.h_ja, c.h_klo, c.h_kup, c.h_tpos);
   SweepPlan p;
-  // no plan: the rows are taken in level order in chunks (fl_parts_on)
+  // no plan, or no room for its tables: the rows are taken in level order in
+  // chunks (fl_parts_on)
   if (!sweep_plan(g, c.part_rows, p, c.positions).empty()) return 0;
   c.sw.n_cu = c.n_cu;
   return sweep_exec_build(c.sw, p, c.stream);
@@ -966,7 +967,7 @@ static int fl_sweep_grid(const FlCtx &c) {
 }
 static int fl_mark_grid(size_t cnt) { return (int)std::max<size_t>(1, std::min<size_t>((cnt + BS - 1) / BS, 4096)); }
 
-static bool fl_parts_on(const FlCtx &c) { return c.one_launch && c.parts && c.sw.built(); }
+static bool fl_parts_on(const FlCtx &c) { return c.one_launch && c.parts && c.sw.built; }
 
 static int fl_precond(FlCtx &c, const double *a) {
   if (fl_parts_on(c)) {
@@ -2069,6 +2070,10 @@ int fvk_fl_ctx_set_param(fvk_fl_ctx *cc, const char *name, double value) {
   }
   if (!std::strcmp(name, "sweep_blocks") && value >= 0 && value <= 65536 && value == (int)value) {
     c.sweep_blocks = c.sw.blocks = (int)value;
+    return FVK_OK;
+  }
+  if (!std::strcmp(name, "sweep_fail") && value == 2) {
+    c.sw.deny = true;
     return FVK_OK;
   }
   if (!std::strcmp(name, "sweep_fail") && value == 1 && c.sweep_int) {

@@ -899,6 +899,7 @@ int sweep_masks_build(Ctx &c) {
 // The sweeps' pattern in the reference numbering: entry values are places in
 // the slot table spv, transposed ones faces (ngp of the entry's face).
 int sweep_parts_build(Ctx &c) {
+  FVK_HIP(hipStreamSynchronize(c.stream));
   sweep_exec_free(c.sw);
   c.sw_mat = c.sw_fac = false;
   if (!c.sweep_one_launch) return 0;
@@ -906,7 +907,6 @@ int sweep_parts_build(Ctx &c) {
   const size_t ld = (size_t)c.M.ld;
   std::vector<int> rank(n), spc((size_t)Ws * ld), spf((size_t)Ws * ld);
   std::vector<unsigned char> lm(n), um(n);
-  FVK_HIP(hipStreamSynchronize(c.stream));
   FVK_HIP(hipMemcpy(rank.data(), c.M.rank, (size_t)n * sizeof(int), hipMemcpyDeviceToHost));
   FVK_HIP(hipMemcpy(spc.data(), c.M.spc, spc.size() * sizeof(int), hipMemcpyDeviceToHost));
   FVK_HIP(hipMemcpy(spf.data(), c.M.spf, spf.size() * sizeof(int), hipMemcpyDeviceToHost));
@@ -944,13 +944,14 @@ int sweep_parts_build(Ctx &c) {
     }
   }
   SweepPlan p;
-  // no plan: the rows are taken in level order in chunks (parts_on)
+  // no plan, or no room for its tables: the rows are taken in level order in
+  // chunks (parts_on)
   if (!sweep_plan(g, c.sweep_part_rows, p, c.sweep_positions).empty()) return 0;
   c.sw.n_cu = c.n_cu;
   return sweep_exec_build(c.sw, p, c.stream);
 }
 
-static bool parts_on(const Ctx &c) { return c.sweep_one_launch && c.sweep_parts && c.sw.built(); }
+static bool parts_on(const Ctx &c) { return c.sweep_one_launch && c.sweep_parts && c.sw.built; }
 
 static int sweep_pack_matrix(Ctx &c) {
   const int rc = sweep_pack(c.sw, c.stream, c.spv, c.ngp);

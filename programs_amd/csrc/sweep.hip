@@ -442,11 +442,22 @@ __global__ __launch_bounds__(BS) void k_sweep_factor_from(int n, const int *__re
 }
 
 // ---------------------------------------------------------------- host
+constexpr int kNoRoom = 1;
+static int take(SweepExec &X, void **q, size_t bytes) {
+  const hipError_t e = X.deny && X.mem.size() == 8 ? hipErrorOutOfMemory : hipMalloc(q, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return kNoRoom;
+  }
+  FVK_HIP(e);
+  X.mem.push_back(*q);
+  return 0;
+}
 template <class T>
-static int up(SweepExec &X, T **d, const std::vector<T> &v, size_t extra = 0) {
+static int up(SweepExec &X, T **d, const std::vector<T> &v) {
   void *q = nullptr;
-  FVK_HIP(hipMalloc(&q, std::max<size_t>(1, v.size() + extra) * sizeof(T)));
-  X.mem.push_back(q);
+  const int rc = take(X, &q, std::max<size_t>(1, v.size()) * sizeof(T));
+  if (rc) return rc;
   if (!v.empty()) FVK_HIP(hipMemcpy(q, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
   *d = (T *)q;
   return 0;
@@ -454,8 +465,8 @@ static int up(SweepExec &X, T **d, const std::vector<T> &v, size_t extra = 0) {
 // zeroed; the clear has finished when the build returns (it ends with a wait)
 static int room(SweepExec &X, double **d, size_t n, hipStream_t s) {
   void *q = nullptr;
-  FVK_HIP(hipMalloc(&q, std::max<size_t>(1, n) * sizeof(double)));
-  X.mem.push_back(q);
+  const int rc = take(X, &q, std::max<size_t>(1, n) * sizeof(double));
+  if (rc) return rc;
   FVK_HIP(hipMemsetAsync(q, 0, std::max<size_t>(1, n) * sizeof(double), s));
   *d = (double *)q;
   return 0;
@@ -481,7 +492,7 @@ static int allow_lds() {
   return 0;
 }
 
-int sweep_exec_build(SweepExec &X, const SweepPlan &p, hipStream_t s) {
+static int exec_build(SweepExec &X, const SweepPlan &p, hipStream_t s) {
   X.n = p.n; X.P = p.P; X.MW = p.MW; X.np = p.np; X.slots = p.slots; X.width = p.width; X.bricks = p.bricks;
   for (int k = 1; k <= 3; ++k) X.lds_[k] = p.lds(k);
   int rc = 0;
@@ -509,12 +520,25 @@ int sweep_exec_build(SweepExec &X, const SweepPlan &p, hipStream_t s) {
   return 0;
 }
 
+int sweep_exec_build(SweepExec &X, const SweepPlan &p, hipStream_t s) {
+  const int rc = exec_build(X, p, s);
+  if (rc) {
+    (void)hipStreamSynchronize(s);  // clears and marks still queued
+    sweep_exec_free(X);
+  }
+  X.built = rc == 0;
+  X.deny = false;
+  return rc == kNoRoom ? 0 : rc;
+}
+
 void sweep_exec_free(SweepExec &X) {
   for (void *q : X.mem) hipFree(q);
   const int n_cu = X.n_cu, blocks = X.blocks;
+  const bool deny = X.deny;
   X = SweepExec();
   X.n_cu = n_cu;
   X.blocks = blocks;
+  X.deny = deny;
 }
 
 static SweepArgs args(const SweepExec &X, int dir) {

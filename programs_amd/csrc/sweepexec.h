@@ -36,9 +36,12 @@ struct SweepExec {
   double *Ec = nullptr;        // exported values of the factorisation (NE of d[0])
   double *t = nullptr;         // forward sweep's result, rows in part order (3 x n)
   int *ticket = nullptr;       // forward, backward, factor
-  bool built() const { return part != nullptr; }
+  bool built = false;          // all of the above is there
+  bool deny = false;           // the next build finds no memory (a test of that)
 };
 
+// Not built when there is no device memory for the tables (the caller then
+// takes another form) or on an error; nothing is left allocated then.
 int sweep_exec_build(SweepExec &X, const SweepPlan &p, hipStream_t s);
 void sweep_exec_free(SweepExec &X);
 

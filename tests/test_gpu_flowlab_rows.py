@@ -128,7 +128,8 @@ def test_solves_by_row_width(n, width, full):
 
 def test_sweep_forms_bitwise():
     """One launch per level, chunks, parts, and a pattern with more positions
-    than the parts' tables may hold ("sweep_positions"), which takes chunks."""
+    than the parts' tables may hold ("sweep_positions") or tables that find no
+    memory ("sweep_fail" 2), which take chunks."""
     fvk = require_lib()
     ia, ja = pattern(900, 7, True, 3)
     rows = np.repeat(np.arange(900), np.diff(ia))
@@ -142,7 +143,8 @@ def test_sweep_forms_bitwise():
     assert L.fvk_fl_csr_create(900, ip(ia), ip(ja), 0, C.byref(h)) == 0
     first = None
     for params in ((), ((b"sweep_positions", 64),), ((b"sweep_positions", 0),), ((b"sweep_parts", 0),),
-                   ((b"sweep_positions", 64), (b"sweep_parts", 1)), ((b"sweep_one_launch", 0),)):
+                   ((b"sweep_positions", 64), (b"sweep_parts", 1)), ((b"sweep_fail", 2), (b"sweep_positions", 0)),
+                   ((b"sweep_part_rows", 300),), ((b"sweep_one_launch", 0),)):
         print("flowlab sweeps:", params, flush=True)
         for k, v in params:
             assert L.fvk_fl_ctx_set_param(h, k, C.c_double(v)) == 0

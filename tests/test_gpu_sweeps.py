@@ -165,7 +165,8 @@ def test_reversed_faces_bitwise(dims, rcm):
 
 def test_pattern_beyond_the_tables_bitwise():
     """A pattern whose plan has more positions than its tables may hold
-    ("sweep_positions") takes the chunks, and the parts again without it."""
+    ("sweep_positions"), or whose tables find no memory ("sweep_fail" 2, when
+    half of them are made), takes the chunks, and the parts again without it."""
     fvk = require_lib()
     say("sweeps: more positions than the tables hold")
     m = fvk.Mesh.box(19, 6, 5, jitter=0.0, seed=3)
@@ -174,11 +175,12 @@ def test_pattern_beyond_the_tables_bitwise():
     fvk.set_matrix(ctx, pl, ngp, ngn)
     b = np.random.default_rng(1).standard_normal(m.n_vol)
     want = [(fvk.solv_precond(ctx, k), fvk.solv_direct(ctx, k, b)) for k in (1, 2)]
-    for limit in (64, 0):
-        fvk.set_param(ctx, "sweep_positions", limit)
+    for name, value in (("sweep_positions", 64), ("sweep_positions", 0), ("sweep_fail", 2), ("sweep_part_rows", 512),
+                        ("sweep_part_rows", 300)):
+        fvk.set_param(ctx, name, value)
         for k, (f, x) in zip((2, 1), want[::-1]):
-            assert np.array_equal(fvk.solv_direct(ctx, k, b), x), (limit, k)
-            assert all(np.array_equal(p, q) for p, q in zip(fvk.solv_precond(ctx, k), f)), (limit, k)
+            assert np.array_equal(fvk.solv_direct(ctx, k, b), x), (name, value, k)
+            assert all(np.array_equal(p, q) for p, q in zip(fvk.solv_precond(ctx, k), f)), (name, value, k)
     ctx.destroy()
     m.free()
 
