@@ -3,9 +3,9 @@
 
 #include <algorithm>
 #include <cstring>
-#include <thread>
 
 #include "ctx.h"
+#include "threads.h"
 
 namespace fvk {
 
@@ -47,14 +47,10 @@ static void copy_bytes(void *dst, const void *src, size_t n) {
     return;
   }
   constexpr int T = 4;
-  std::thread th[T - 1];
-  auto part = [=](int t) {
+  on_threads(T, [=](int t) {
     const size_t a = n / T * t, b = t == T - 1 ? n : n / T * (t + 1);
     std::memcpy((char *)dst + a, (const char *)src + a, b - a);
-  };
-  for (int t = 1; t < T; ++t) th[t - 1] = std::thread(part, t);
-  part(0);
-  for (auto &t : th) t.join();
+  });
 }
 
 void HostIo::drain(int b) {

@@ -5,6 +5,8 @@
 #include <atomic>
 #include <thread>
 
+#include "threads.h"
+
 namespace fvk {
 
 namespace {
@@ -14,17 +16,10 @@ template <class F>
 void parallel_for(int n, int grain, F f) {
   const int hw = std::max(1u, std::thread::hardware_concurrency());
   const int nt = std::max(1, std::min({hw, 8, n / std::max(1, grain)}));
-  if (nt == 1) {
-    for (int i = 0; i < n; ++i) f(i);
-    return;
-  }
-  std::vector<std::thread> th;
-  for (int t = 0; t < nt; ++t)
-    th.emplace_back([=] {
-      const int a = (int)((long)n * t / nt), b = (int)((long)n * (t + 1) / nt);
-      for (int i = a; i < b; ++i) f(i);
-    });
-  for (auto &t : th) t.join();
+  on_threads(nt, [&](int t) {
+    const int a = (int)((long)n * t / nt), b = (int)((long)n * (t + 1) / nt);
+    for (int i = a; i < b; ++i) f(i);
+  });
 }
 
 // The (at most three) rank distances that carry most lower entries, when

@@ -5,10 +5,15 @@ before it is there, when a part needs a part taken after it, or when a row
 is not run once; the cases are where that can go wrong: one row, one part,
 ragged boxes, chains, unstructured and unsorted patterns, rows with one to
 eight entries on a side."""
+import resource
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 from programs_amd import fvk
+from tests.helpers import ROOT
 
 LDS = 163840  # bytes of LDS of a compute unit
 
@@ -79,3 +84,25 @@ def test_positions_are_limited(n, pairs):
     assert n <= p <= 8 * n and fvk.sweep_positions(ia, ja, limit=p) == p
     with pytest.raises(fvk.FvkError):
         fvk.sweep_positions(ia, ja, limit=p - 1)
+
+
+def test_without_threads():
+    """Where no thread can be started (here for want of address space for its
+    stack) the calling thread does their work."""
+    code = """
+import resource
+from programs_amd import fvk
+from tests.test_sweep_plan import box, csr
+n, pairs = box(40, 33, 5)
+pattern = csr(n, pairs.tolist())
+want = fvk.sweep_plan(*pattern, 64)
+size = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (size + (256 << 20),) * 2)
+assert fvk.sweep_plan(*pattern, 64) == want and want["parts"] >= 16
+"""
+    stack = 1 << 30
+    hard = resource.getrlimit(resource.RLIMIT_STACK)[1]
+    if hard != resource.RLIM_INFINITY and hard < stack:
+        pytest.skip("the stack limit cannot be raised")
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=ROOT, timeout=120,
+                   preexec_fn=lambda: resource.setrlimit(resource.RLIMIT_STACK, (stack, hard)))
