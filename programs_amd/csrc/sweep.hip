@@ -393,6 +393,11 @@ __global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
         A.crr[r0 + k] = A.drow ? d : 1.0 / (c + SMALL);
       }
     }
+    // Keeps the loop above, whose trip count is a thread's own, apart from
+    // thread 0's ticket: a compiler may join a branch at the end of a loop's
+    // body with one at its head, and the threads that skip both would then go
+    // round to the barrier without a ticket.  A barrier is never duplicated.
+    __syncthreads();
   }
 }
 
