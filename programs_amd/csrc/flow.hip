@@ -678,9 +678,13 @@ int mom_setup(Flow &F, int it, bool &skipped) {
   MomPar P{F.cfg.rho, F.cfg.mu, F.cfg.c_bl, F.cfg.urf_u, F.cfg.c_sch};
   skipped = false;
   if (fill(c, &F.sc->phi_mx_cell, 2, 0.0)) return FVK_ERR_HIP;
-  // few blocks: their atomics on one address take turns (102k cells, three
-  // components: 12 us with 128 blocks, 28 us with one per 256 cells)
-  k_absmax<<<std::min(grid_for(std::max(n, c.nbf)), 128), BS, 0, c.stream>>>(n, nvc, F.u, c.nbf, F.ub,
+  // Blocks: their atomics on one address take turns, about 25 ns a block, and
+  // the loads take as long as one thread's share of them, so the best number
+  // grows with the square root of the values (three components, with 128 /
+  // 512 / 2048 blocks: 110k cells 6 / 12 / 12 us, 885k 24 / 19 / 51, 2.1M 54 /
+  // 26 / 55, 8M 315 / 92 / 76; by the rule 126, 358, 552 and 1078 blocks).
+  const int most = 1 + (int)(0.22 * std::sqrt((double)nvc * std::max(n, c.nbf)));
+  k_absmax<<<std::min(grid_for(std::max(n, c.nbf)), most), BS, 0, c.stream>>>(n, nvc, F.u, c.nbf, F.ub,
                                                                            &F.sc->phi_mx_cell, &F.sc->phi_mx_all);
   // the early return when every velocity is zero (cfd_setup.f90:170-171);
   // a captured iteration follows one that did not take it, and with fixed
