@@ -54,6 +54,18 @@ def test_boxes(dims, rows):
         assert p["passed_fwd"] < n or rows < 100
 
 
+def test_sampled_distances():
+    """A box as wide as the rows are sampled apart (every eighth of 423,200) is
+    still recognised by all three distances: with parts of 64 rows a brick
+    cannot hold whole lines of 8 cells in two directions."""
+    n, e = box(8, 230, 230)
+    k = np.arange(n)
+    r, c = np.concatenate([e[:, 0], e[:, 1], k]), np.concatenate([e[:, 1], e[:, 0], k])
+    o = np.lexsort((c, r))
+    ia = 1 + np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))])
+    assert fvk.sweep_plan(ia, c[o] + 1, 64)["bricks"] == 1
+
+
 @pytest.mark.parametrize("rows", [64, 300, 4096])
 @pytest.mark.parametrize("n,span,width", [(50, 1, 1), (700, 3, 2), (3000, 40, 3), (3000, 3000, 4), (2000, 900, 8)])
 def test_unstructured(n, span, width, rows):
