@@ -253,10 +253,12 @@ int fvk_sys_get_x(fvk_ctx *ctx, double *x);
    restart, default).  DIC / DILU factor and sweeps (solv_precond,
    solv_direct): "sweep_one_launch" (1, default when no row has more than 8
    slots: one launch each, rows waiting for their values; 0: one launch per
-   level), "sweep_parts" (1, default: each block walks parts of at most
-   "sweep_part_rows" rows, default 4096, 256..6400, values inside a part
-   passing through LDS (fvk_sweep_plan); 0: rows taken in level order in
-   chunks by "sweep_blocks_per_cu" resident blocks per CU, default 1).  All
+   level), "sweep_parts" (2: each block walks parts of at most
+   "sweep_part_rows" rows, default 4096, 256..6400 (bricks have at most 4096
+   rows and ranges 2048, whatever it says), values inside a part passing
+   through LDS (fvk_sweep_plan); 0: rows taken in level order in chunks by
+   "sweep_blocks_per_cu" resident blocks per CU, default 1; 1, default: the
+   faster of the two by the pattern (fvk_sweep_times)).  All
    give the same bits.  "sweep_fail" 1 (a test of the failure path): records
    that a sweep's wait ran past its bound, as a wait that never ends would;
    parts that wait give up within 256 polls, blocks stop taking parts, and
@@ -270,9 +272,9 @@ int fvk_ctx_set_param(fvk_ctx *ctx, const char *name, double value);
 /* How the one-launch sweeps split a pattern (1-based CSR with its diagonal,
    as solv_m receives it): parts of at most max_rows rows that depend on
    each other in one direction only, grid cells over the paths' entry
-   distances ("bricks") where a few distances carry nearly all entries, else
-   ranges of consecutive rows; inside a part chunks of up to 64 independent
-   rows.  Builds the plan and walks it as the kernels do: FVK_ERR_STATE when
+   distances ("bricks") where a few distances carry nearly all entries, or
+   ranges of consecutive rows where those are faster; inside a part chunks of
+   up to 64 independent rows.  Builds the plan and walks it as the kernels do: FVK_ERR_STATE when
    a value would be read before it is there.  info: parts, chunks,
    dependency levels, 1 for bricks, LDS bytes of a block with one and with
    three right-hand sides, values passed between parts forward and backward.
@@ -284,6 +286,9 @@ int fvk_sweep_plan(int n, const int *ia, const int *ja, int max_rows, int *info)
    kernels' 32-bit offsets reach, 2^28, or 2^27 where a row has more than four
    lower or upper entries).  Host only. */
 int fvk_sweep_positions(int n, const int *ia, const int *ja, int max_rows, int64_t limit, int64_t *positions);
+/* What the choice between the forms rests on: us of both sweeps by that plan
+   and by chunks of the level order, one right-hand side.  Host only. */
+int fvk_sweep_times(int n, const int *ia, const int *ja, int max_rows, double *us);
 
 /* The factorised preconditioner z = G G^T r, G = D^-1/2 (I + L) Delta, with
    D the diagonal of the current matrix, L strictly lower triangular on the
@@ -523,11 +528,9 @@ int fvk_fl_csr_matches(const fvk_fl_ctx *ctx, int n, const int *ia, const int *j
 void fvk_fl_ctx_destroy(fvk_fl_ctx *ctx);
 /* "sweep_one_launch" 1 (default when every row has at most 8 lower and 8
    upper entries): the factor and direct_solve's sweeps in one launch each,
-   rows waiting for their values; 0: one launch per level.  "sweep_parts" 1
-   (default with one launch): each block of the launch walks parts of at most
-   "sweep_part_rows" rows (default 4096, 256..6400), values inside a part
-   passing through LDS (fvk_sweep_plan); 0: rows taken in level order in
-   chunks.  "sweep_blocks" (0: one per CU): blocks of the
+   rows waiting for their values; 0: one launch per level.  "sweep_parts" 0,
+   1 (default with one launch), 2 and "sweep_part_rows": as
+   fvk_ctx_set_param's.  "sweep_blocks" (0: one per CU): blocks of the
    one-launch kernels.  All give the same bits.  "sweep_fail" 1 (a test of
    the failure path): as fvk_ctx_set_param's; the context's solves then
    return FVK_ERR_HIP.  "sweep_positions", "sweep_fail" 2: as there.  No counterpart in the reference. */

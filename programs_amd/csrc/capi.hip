@@ -986,8 +986,14 @@ int fvk_ctx_set_param(fvk_ctx *cc, const char *name, double value) {
       const int rc = sweep_parts_build(cc->c);
       if (rc) return rc;
     }
-  } else if (!std::strcmp(name, "sweep_parts") && (value == 0 || value == 1))
-    cc->c.sweep_parts = value != 0;
+  } else if (!std::strcmp(name, "sweep_parts") && (value == 0 || value == 1 || value == 2)) {
+    const bool plan = (value == 2) != (cc->c.sweep_parts == 2);
+    cc->c.sweep_parts = (int)value;
+    if (plan) {
+      const int rc = sweep_parts_build(cc->c);
+      if (rc) return rc;
+    }
+  }
   else if (!std::strcmp(name, "sweep_part_rows") && value >= 256 && value <= 6400 && value == (int)value) {
     cc->c.sweep_part_rows = (int)value;
     const int rc = sweep_parts_build(cc->c);

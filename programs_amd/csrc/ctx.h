@@ -107,7 +107,7 @@ struct Ctx {
   unsigned char *sweep_lmask = nullptr, *sweep_umask = nullptr;  // lower / upper slots of each row
   // the default form: parts of rows, each walked by one block (sweep.hip)
   SweepExec sw;
-  bool sweep_parts = true;
+  int sweep_parts = 1;            // 1: where they are the faster form, 2: always, 0: never
   int sweep_part_rows = 4096;     // rows of a part at most
   long sweep_positions = 0;       // positions of its tables at most (0: the kernels' limit)
   // the packed copies in sw are of the current matrix / of pc_c, pc_cr

@@ -61,7 +61,7 @@ struct FlCtx {
   int sweep_blocks = 0;  // blocks of the one-launch kernels (0: one per CU)
   // the default form: parts of rows, each walked by one block (sweep.hip)
   SweepExec sw;
-  bool parts = false;
+  int parts = 0;         // 1: where they are the faster form, 2: always, 0: never
   int part_rows = 4096;  // rows of a part at most
   long positions = 0;    // positions of its tables at most (0: the kernels' limit)
   bool narrow = false;   // no row has more than kSweepSlots lower or upper entries
@@ -932,9 +932,10 @@ static int fl_parts_setup(FlCtx &c) {
   sweep_exec_free(c.sw);
   const SweepGraph g = fl_sweep_graph(c.n, c.h_ia, c.h_ja, c.h_klo, c.h_kup, c.h_tpos);
   SweepPlan p;
-  // no plan, or no room for its tables: the rows are taken in level order in
-  // chunks (fl_parts_on)
+  // no plan, a slower one, or no room for its tables: the rows are taken in
+  // level order in chunks (fl_parts_on)
   if (!sweep_plan(g, c.part_rows, p, c.positions).empty()) return 0;
+  if (p.chunks_faster() && c.parts < 2) return 0;
   c.sw.n_cu = c.n_cu;
   return sweep_exec_build(c.sw, p, c.stream);
 }
@@ -1523,8 +1524,8 @@ static int fl_csr_setup(FlCtx &c, int n, const int *ngp, const int *ngc) {
   fl_levels(ia, ja, n, false, c.lb_ptr, lrows);
   if ((rc = fl_up(c, &c.lb_rows, lrows))) return rc;
   if (c.one_launch) {
+    c.parts = 1;
     if ((rc = fl_parts_setup(c))) return rc;
-    c.parts = true;
   }
   FVK_HIP(c.watch.init());
   // rows of 4, 5 or 7 entries: triangles, quadrangles, hexahedra; by slots
@@ -1949,6 +1950,19 @@ int fvk_sweep_positions(int n, const int *ia, const int *ja, int max_rows, int64
   return FVK_OK;
 }
 
+int fvk_sweep_times(int n, const int *ia, const int *ja, int max_rows, double *us) {
+  if (!ia || !ja || !us || n < 1 || max_rows < 64) { set_error("bad argument"); return FVK_ERR_ARG; }
+  FlPattern q;
+  const int rc = fl_pattern(n, ia, ja, q);
+  if (rc) return rc;
+  SweepPlan p;
+  const std::string e = sweep_plan(fl_sweep_graph(n, q.ia, q.ja, q.klo, q.kup, q.tpos), max_rows, p);
+  if (!e.empty()) { set_error(e); return FVK_ERR_ARG; }
+  us[0] = p.us;
+  us[1] = p.chunk_us;
+  return FVK_OK;
+}
+
 int fvk_fl_csr_matches(const fvk_fl_ctx *cc, int n, const int *ia, const int *ja) {
   if (!cc || !ia || !ja) return 0;
   const FlCtx &c = cc->c;
@@ -2051,10 +2065,13 @@ int fvk_fl_ctx_set_param(fvk_fl_ctx *cc, const char *name, double value) {
     c.one_launch = value != 0;
     return FVK_OK;
   }
-  if (!std::strcmp(name, "sweep_parts") && (value == 0 || value == 1)) {
-    if (value == 1 && !c.narrow) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
-    c.parts = value != 0;
-    return FVK_OK;
+  if (!std::strcmp(name, "sweep_parts") && (value == 0 || value == 1 || value == 2)) {
+    if (value != 0 && !c.narrow) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }
+    const bool plan = (value == 2) != (c.parts == 2);
+    c.parts = (int)value;
+    if (!plan) return FVK_OK;
+    FVK_HIP(hipStreamSynchronize(c.stream));
+    return fl_parts_setup(c);
   }
   if (!std::strcmp(name, "sweep_part_rows") && value >= 256 && value <= 6400 && value == (int)value) {
     if (!c.narrow) { set_error("a row has more lower or upper entries than one launch holds"); return FVK_ERR_ARG; }

@@ -944,9 +944,10 @@ int sweep_parts_build(Ctx &c) {
     }
   }
   SweepPlan p;
-  // no plan, or no room for its tables: the rows are taken in level order in
-  // chunks (parts_on)
+  // no plan, a slower one, or no room for its tables: the rows are taken in
+  // level order in chunks (parts_on)
   if (!sweep_plan(g, c.sweep_part_rows, p, c.sweep_positions).empty()) return 0;
+  if (p.chunks_faster() && c.sweep_parts < 2) return 0;
   c.sw.n_cu = c.n_cu;
   return sweep_exec_build(c.sw, p, c.stream);
 }

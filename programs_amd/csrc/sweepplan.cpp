@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <functional>
 #include <thread>
 
 #include "threads.h"
@@ -22,13 +23,18 @@ void parallel_for(int n, int grain, F f) {
   });
 }
 
+// An entry of rank distance x is of a direction's: within a quarter of its
+// distance, so that rows left out, added or out of order, which shift the
+// distances between lines and planes, do not hide a structured numbering.
+inline bool near_distance(int x, int d) { return std::abs(x - d) <= d / 4; }
+
 // The (at most three) rank distances that carry most lower entries, when
-// they carry nearly all of them: a structured numbering.  Sampled rows, one of
-// every `step` at no fixed distance: every 224th row of a box 224 cells wide
-// has no neighbour at distance 1.
-int main_distances(const SweepGraph &g, int (&d)[3]) {
+// they carry nearly all of them: a structured numbering.  exact: without the
+// quarter.  Sampled rows, one of every `step` at no fixed distance: every 224th
+// row of a box 224 cells wide has no neighbour at distance 1.
+int main_distances(const SweepGraph &g, int (&d)[3], bool &exact) {
   constexpr int T = 64;
-  int key[T], cnt[T], used = 0;
+  int key[T], cnt[T], same[T], used = 0;
   long total = 0;
   const int step = std::max(1, g.n / 50021);
   unsigned h = 1;
@@ -39,17 +45,19 @@ int main_distances(const SweepGraph &g, int (&d)[3]) {
       const int x = k - g.lcol[q];
       ++total;
       int s = 0;
-      while (s < used && key[s] != x) ++s;
+      while (s < used && !near_distance(x, key[s])) ++s;
       if (s == used) {
         if (used == T) continue;
         key[used] = x;
-        cnt[used++] = 0;
+        cnt[used] = same[used] = 0;
+        ++used;
       }
       ++cnt[s];
+      same[s] += x == key[s];
     }
   }
   int m = 0;
-  long sum = 0;
+  long sum = 0, alike = 0;
   while (m < 3) {
     int best = -1;
     for (int s = 0; s < used; ++s)
@@ -57,8 +65,10 @@ int main_distances(const SweepGraph &g, int (&d)[3]) {
     if (best < 0 || cnt[best] * 20L < total) break;
     d[m++] = key[best];
     sum += cnt[best];
+    alike += same[best];
     cnt[best] = 0;
   }
+  exact = alike * 10 >= total * 9;
   return m > 1 && sum * 10 >= total * 9 ? m : 0;
 }
 
@@ -98,7 +108,7 @@ static double brick_path(int m, const int *side, const int *cells) {
 
 // Parts.  An acyclic split with few crossings on a path: for each of the
 // main rank distances d, phi_d(row) is the largest number of entries of
-// distance d on any path that ends at the row.  Each phi_d never decreases
+// distance d (near_distance) on any path that ends at the row.  Each phi_d never decreases
 // along an entry, so cells of a grid over the phi_d ("bricks") depend on
 // each other only in the direction of growing cell indices, and taking them
 // by the sum of the indices is a valid order.  On a box in natural order
@@ -111,17 +121,19 @@ static double brick_path(int m, const int *side, const int *cells) {
 // both sweeps, 24^3 / 96^3 / 128^3, with two halo waves: 35.3 / 153 / 235 us;
 // cubes of at most 1728 rows 38 / 163 / 250, of 512 rows 37 / 173).
 // Without main distances (unstructured numberings) the parts are ranges of
-// consecutive rows: a path crosses them about once a level anyway, and short
-// ones are loaded sooner (DIC, both sweeps, 20k / 40k / 200k triangles in RCM
-// order: ranges of 512 rows 53 / 65 / 93 us, 1024 45 / 57 / 87, 2048 51 / 61 /
-// 92, 4096 51 / 61 / 92).
+// consecutive rows, of whichever size plan_us finds faster: a path through
+// triangles crosses them about once a level anyway, and short ones are loaded
+// sooner (DIC, both sweeps, 20k / 40k / 200k triangles in RCM order: ranges of
+// 512 rows 53 / 65 / 93 us, 1024 45 / 57 / 87, 2048 51 / 61 / 92), where long
+// ones save crossings elsewhere (an iteration of CG on 24k tetrahedra 172 -> 123
+// us, on a 64^3 box of which a fiftieth is numbered at random 1090 -> 574).
 constexpr int kBrickRows = 4096;
-constexpr int kRangeRows = 1024;
+constexpr int kRangeRows[] = {1024, 2048};
 
-static bool brick_parts(const SweepGraph &g, int max_rows, std::vector<int> &part, int &P) {
+static bool brick_parts(const SweepGraph &g, int max_rows, std::vector<int> &part, int &P, bool &exact) {
   max_rows = std::min(max_rows, kBrickRows);
   int dist[3] = {0, 0, 0};
-  const int m = main_distances(g, dist), n = g.n;
+  const int m = main_distances(g, dist, exact), n = g.n;
   if (m == 0) return false;
   std::vector<int> phi[3];
   int ext[3] = {1, 1, 1};
@@ -133,59 +145,64 @@ static bool brick_parts(const SweepGraph &g, int max_rows, std::vector<int> &par
       int v = f[k];
       for (int q = g.lptr[k]; q < g.lptr[k + 1]; ++q) {
         const int j = g.lcol[q];
-        v = std::max(v, f[j] + (k - j == dist[c] ? 1 : 0));
+        v = std::max(v, f[j] + (near_distance(k - j, dist[c]) ? 1 : 0));
       }
       f[k] = v;
       top = std::max(top, v);
       if (!g.symmetric)
         for (int q = g.uptr[k]; q < g.uptr[k + 1]; ++q) {
           const int i = g.ucol[q];
-          f[i] = std::max(f[i], v + (i - k == dist[c] ? 1 : 0));
+          f[i] = std::max(f[i], v + (near_distance(i - k, dist[c]) ? 1 : 0));
         }
     }
     ext[c] = top + 1;
   }
   // sides: the shortest path of all that are even within a direction and have
-  // at most max_rows rows a brick
+  // at most `rows` rows a brick of a box; fewer when a brick then has more than
+  // max_rows after all, as on irregular numberings
   int side[3] = {1, 1, 1}, cells[3] = {1, 1, 1};
-  double best = -1.0;
-  std::vector<int> cand[3];
+  std::vector<int> cand[3], cnt;
   for (int c = 0; c < 3; ++c)
     for (int w = 1; w <= ext[c]; ++w) {
       const int k = (ext[c] + w - 1) / w, e = (ext[c] + k - 1) / k;
       if (e == w && (w >= 4 || w == ext[c])) cand[c].push_back(w);
     }
-  for (int s0 : cand[0])
-    for (int s1 : cand[1]) {
-      if ((long)s0 * s1 > max_rows) break;
-      for (int s2 : cand[2]) {
-        if ((long)s0 * s1 * s2 > max_rows) break;
-        const int s[3] = {s0, s1, s2};
-        int k[3];
-        for (int c = 0; c < 3; ++c) k[c] = (ext[c] + s[c] - 1) / s[c];
-        const double t = brick_path(m, s, k);
-        if (best < 0 || t < best) {
-          best = t;
-          std::copy(s, s + 3, side);
+  long grid = 1;
+  part.resize(n);
+  for (int rows = max_rows;; rows = rows * 3 / 4) {
+    double best = -1.0;
+    for (int s0 : cand[0])
+      for (int s1 : cand[1]) {
+        if ((long)s0 * s1 > rows) break;
+        for (int s2 : cand[2]) {
+          if ((long)s0 * s1 * s2 > rows) break;
+          const int s[3] = {s0, s1, s2};
+          int k[3];
+          for (int c = 0; c < 3; ++c) k[c] = (ext[c] + s[c] - 1) / s[c];
+          const double t = brick_path(m, s, k);
+          if (best < 0 || t < best) {
+            best = t;
+            std::copy(s, s + 3, side);
+          }
         }
       }
+    if (best < 0) return false;
+    grid = 1;
+    for (int c = 0; c < m; ++c) {
+      cells[c] = (ext[c] + side[c] - 1) / side[c];
+      grid *= cells[c];
     }
-  if (best < 0) return false;
-  long grid = 1;
-  for (int c = 0; c < m; ++c) {
-    cells[c] = (ext[c] + side[c] - 1) / side[c];
-    grid *= cells[c];
+    if (grid > n) return false;
+    cnt.assign(grid, 0);
+    for (int k = 0; k < n; ++k) {
+      int id = 0;
+      for (int c = m - 1; c >= 0; --c) id = id * cells[c] + phi[c][k] / side[c];
+      part[k] = id;
+      ++cnt[id];
+    }
+    if (*std::max_element(cnt.begin(), cnt.end()) <= max_rows) break;
+    if (rows < max_rows / 8) return false;
   }
-  if (grid > n) return false;
-  part.resize(n);
-  std::vector<int> cnt(grid, 0);
-  for (int k = 0; k < n; ++k) {
-    int id = 0;
-    for (int c = m - 1; c >= 0; --c) id = id * cells[c] + phi[c][k] / side[c];
-    part[k] = id;
-    ++cnt[id];
-  }
-  if (*std::max_element(cnt.begin(), cnt.end()) > max_rows) return false;
   std::vector<std::pair<int, int>> order;
   for (int id = 0; id < (int)grid; ++id) {
     if (!cnt[id]) continue;
@@ -204,14 +221,17 @@ static bool brick_parts(const SweepGraph &g, int max_rows, std::vector<int> &par
   return true;
 }
 
-enum PlanEnd { PLAN_OK, PLAN_LDS, PLAN_POSITIONS };
-static PlanEnd plan_with(const SweepGraph &g, int max_rows, long limit, SweepPlan &p) {
+enum PlanEnd { PLAN_OK, PLAN_LDS, PLAN_POSITIONS, PLAN_NONE };
+// range_rows 0: bricks
+static PlanEnd plan_with(const SweepGraph &g, int max_rows, int range_rows, long limit, SweepPlan &p, bool &exact) {
   const int n = g.n;
   std::vector<int> part;
   int P = 0;
-  p.bricks = brick_parts(g, max_rows, part, P);
-  if (!p.bricks) {
-    const int rows = std::min(max_rows, kRangeRows);
+  p.bricks = range_rows == 0;
+  if (p.bricks) {
+    if (!brick_parts(g, max_rows, part, P, exact)) return PLAN_NONE;
+  } else {
+    const int rows = std::min(max_rows, range_rows);
     part.resize(n);
     for (int k = 0; k < n; ++k) part[k] = k / rows;
     P = (n + rows - 1) / rows;
@@ -444,22 +464,94 @@ static PlanEnd plan_with(const SweepGraph &g, int max_rows, long limit, SweepPla
   return PLAN_OK;
 }
 
+// Time of both sweeps with one right-hand side in us, by walking the plan as
+// the kernels do: blocks take parts as they come free, a chunk takes 0.1 us
+// from the one before or from its last halo value, a lane of the halo wave
+// fetches one value in 0.5 us, 0.7 us after it was passed on at the earliest,
+// and a part is loaded and stored in 1.4 us.  Within 10 % of the sweeps in 50
+// patterns (boxes, triangles, tetrahedra; natural, RCM, Morton, red-black and
+// random orders) with ranges of 256 to 4096 rows, from 10 us to 9.5 ms, and low
+// by up to 1.7 where many blocks wait long, as polls then hinder each other.
+// Chunks of the level order (sweep.h) take 4.2 us a level for both sweeps, 3 to
+// 5.4 in those patterns, or 0.32 ns a row.  They are the faster form where a
+// part needs many values from many others: an iteration of CG, parts / chunks:
+// 48^3 box numbered at random 408 / 116 us, 80^3 949 / 214, 200k triangles at
+// random 248 / 91, 64^3 in RCM order 821 / 608; but 60k triangles as they are
+// 85 / 121, 64^3 in natural order 112 / 1028.
+static double plan_us(const SweepPlan &p) {
+  constexpr int kCus = 256;
+  const int NI = p.nrec(), ND = p.at_need();
+  const int blocks = std::min(p.P, kCus * std::max(1, std::min(4, (int)(163840 / (p.lds(1) + 512)))));
+  double sum = 0;
+  for (int dir = 0; dir < 2; ++dir) {
+    const SweepPlan::Dir &D = p.d[dir];
+    std::vector<float> passed(D.NE, 0.f);    // when a value was passed on
+    std::vector<double> idle(blocks, 0.0);   // when a block comes free, the first at the heap's head
+    double end = 0;
+    for (int o = 0; o < p.P; ++o) {
+      const int q = dir == 0 ? o : p.P - 1 - o, *Q = &p.part[8 * q];
+      const int *src = D.hsrc.data() + Q[4 + 2 * dir];
+      std::pop_heap(idle.begin(), idle.end(), std::greater<double>());
+      double t = idle.back() + 1.4, there = t, lane[64];
+      std::fill(lane, lane + 64, t);
+      int have = 0;
+      for (int c = 0; c < Q[1]; ++c) {
+        const int ch = Q[0] + (dir == 0 ? c : Q[1] - 1 - c);
+        const unsigned short *rec = &D.rec[(size_t)ch * p.width * NI];
+        for (; have < rec[ND]; ++have) {
+          double &l = lane[have % 64];
+          l = std::max(l + 0.5, passed[src[have]] + 0.7);
+          there = std::max(there, l);
+        }
+        t = std::max(t, there) + 0.1;
+        for (int k = 0; k < p.width; ++k) {
+          const int e = (int)((unsigned)rec[k * NI + ND + 1] | (unsigned)rec[k * NI + ND + 2] << 16);
+          if (e >= 0) passed[e] = (float)t;
+        }
+      }
+      idle.back() = t + 1.4;
+      std::push_heap(idle.begin(), idle.end(), std::greater<double>());
+      end = std::max(end, t);
+    }
+    sum += end;
+  }
+  return sum;
+}
+
 std::string sweep_plan(const SweepGraph &g, int max_rows, SweepPlan &p, long limit) {
   int W = 1;
   for (int k = 0; k < g.n; ++k) W = std::max({W, g.lptr[k + 1] - g.lptr[k], g.uptr[k + 1] - g.uptr[k]});
   if (W > 8) return "a row has more lower or upper entries than one launch holds";
+  const int MW = W <= 3 ? 3 : W <= 4 ? 4 : 8;
   // smaller parts until every part and its halo fit the LDS (a part of R
   // rows has at most 8 R halo values, so this ends)
-  for (int r = max_rows; r >= 64; r /= 2) {
-    p = SweepPlan();
-    p.W = W;
-    p.MW = W <= 3 ? 3 : W <= 4 ? 4 : 8;
-    const long most = (1L << 32) / (2 * p.nrec());
-    const PlanEnd e = plan_with(g, r, limit > 0 ? std::min(limit, most) : most, p);
-    if (e == PLAN_OK) return "";
-    if (e == PLAN_POSITIONS) return "the pattern needs more positions than the sweep tables hold";
-  }
-  return "no plan";
+  bool exact = false;
+  auto fit = [&](int range, SweepPlan &q) {
+    for (int r = range ? std::min(max_rows, range) : max_rows; r >= 64; r /= 2) {
+      q = SweepPlan();
+      q.W = W;
+      q.MW = W <= 3 ? 3 : W <= 4 ? 4 : 8;
+      const long most = (1L << 32) / (2 * q.nrec());
+      const PlanEnd e = plan_with(g, r, range, limit > 0 ? std::min(limit, most) : most, q, exact);
+      if (e == PLAN_OK) q.us = plan_us(q);
+      if (e != PLAN_LDS) return e;
+    }
+    return PLAN_NONE;
+  };
+  // bricks of an exactly structured numbering, else the fastest of the forms
+  PlanEnd e = fit(0, p);
+  if (e != PLAN_OK || !exact)
+    for (int range : kRangeRows) {
+      if (range > kRangeRows[0] && (e == PLAN_POSITIONS || max_rows <= kRangeRows[0] || p.P == 1)) break;
+      SweepPlan q;
+      const PlanEnd f = fit(range, q);
+      if (f == PLAN_OK && (e != PLAN_OK || q.us < p.us)) p = std::move(q);
+      if (e != PLAN_OK) e = f;
+    }
+  if (e == PLAN_POSITIONS) return "the pattern needs more positions than the sweep tables hold";
+  if (e != PLAN_OK) return "no plan";
+  p.chunk_us = std::max(4.2 * p.levels, 3.2e-4 * p.n);
+  return "";
 }
 
 std::string sweep_plan_check(const SweepGraph &g, const SweepPlan &p) {

@@ -47,6 +47,8 @@ struct SweepPlan {
   int n = 0, P = 0, W = 0, MW = 0, np = 0, levels = 0, width = kChunk;
   int slots = 0, maxh = 0;                 // the most LDS slots and halo values of a part
   bool bricks = false;
+  double us = 0, chunk_us = 0;             // both sweeps by this plan and by chunks of the level order (plan_us)
+  bool chunks_faster() const { return 1.25 * us > chunk_us; }
   std::vector<int> part;                   // 8 ints a part: first chunk, chunks, first row, rows,
                                            // first forward halo, count, first backward halo, count
   std::vector<int> prow, ppos;             // rows of each part ascending: device row, position

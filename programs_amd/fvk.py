@@ -150,6 +150,7 @@ def lib():
         "fvk_sys_get_x": [_vp, _dp],
         "fvk_ctx_set_param": [_vp, C.c_char_p, C.c_double],
         "fvk_sweep_plan": [C.c_int, _ip, _ip, C.c_int, _ip],
+        "fvk_sweep_times": [C.c_int, _ip, _ip, C.c_int, _dp],
         "fvk_sweep_positions": [C.c_int, _ip, _ip, C.c_int, C.c_int64, C.POINTER(C.c_int64)],
         "fvk_factor_set": [_vp, _fp, _fp],
         "fvk_factor_apply": [_vp, _dp, _dp],
@@ -537,6 +538,15 @@ def sweep_positions(ia, ja, max_rows=4096, limit=0):
     o = C.c_int64()
     _check(lib().fvk_sweep_positions(len(a) - 1, _i(a), _i(b), max_rows, limit, C.byref(o)))
     return o.value
+
+
+def sweep_times(ia, ja, max_rows=4096):
+    """us of both sweeps that the choice of their form rests on: by the plan's
+    parts and by chunks of the level order.  Host only."""
+    a, b = np.ascontiguousarray(ia, np.int32), np.ascontiguousarray(ja, np.int32)
+    o = np.zeros(2)
+    _check(lib().fvk_sweep_times(len(a) - 1, _i(a), _i(b), max_rows, _d(o)))
+    return tuple(map(float, o))
 
 
 def factor_set(ctx: Ctx, l, sig):

@@ -126,29 +126,40 @@ def test_solves_by_row_width(n, width, full):
     L.fvk_fl_ctx_destroy(h)
 
 
-def test_sweep_forms_bitwise():
+def scattered(nx):
+    """The pattern of a box of nx^3 cells numbered at random."""
+    k = np.random.default_rng(2).permutation(nx ** 3).reshape(nx, nx, nx)
+    e = np.concatenate([np.stack([a.ravel(), b.ravel()], 1) for a, b in ((k[1:], k[:-1]), (k[:, 1:], k[:, :-1]),
+                                                                        (k[:, :, 1:], k[:, :, :-1]))])
+    r, c = np.concatenate([e[:, 0], e[:, 1], k.ravel()]), np.concatenate([e[:, 1], e[:, 0], k.ravel()])
+    o = np.lexsort((c, r))
+    return (1 + np.concatenate([[0], np.cumsum(np.bincount(r))])).astype(np.int32), (c[o] + 1).astype(np.int32)
+
+
+@pytest.mark.parametrize("ia,ja", [pattern(900, 7, True, 3), scattered(16)])
+def test_sweep_forms_bitwise(ia, ja):
     """One launch per level, chunks, parts, and a pattern with more positions
     than the parts' tables may hold ("sweep_positions") or tables that find no
     memory ("sweep_fail" 2), which take chunks."""
     fvk = require_lib()
-    ia, ja = pattern(900, 7, True, 3)
-    rows = np.repeat(np.arange(900), np.diff(ia))
+    n = len(ia) - 1
+    rows = np.repeat(np.arange(n), np.diff(ia))
     rng = np.random.default_rng(5)
-    a, b = rng.uniform(-1.0, -0.2, len(ja)), rng.standard_normal(900)
+    a, b = rng.uniform(-1.0, -0.2, len(ja)), rng.standard_normal(n)
     a[rows == ja - 1] = 9.0
     L = fvk.lib()
     h = C.c_void_p()
     ip = lambda v: v.ctypes.data_as(C.POINTER(C.c_int))
     dp = lambda v: v.ctypes.data_as(C.POINTER(C.c_double))
-    assert L.fvk_fl_csr_create(900, ip(ia), ip(ja), 0, C.byref(h)) == 0
+    assert L.fvk_fl_csr_create(n, ip(ia), ip(ja), 0, C.byref(h)) == 0
     first = None
-    for params in ((), ((b"sweep_positions", 64),), ((b"sweep_positions", 0),), ((b"sweep_parts", 0),),
-                   ((b"sweep_positions", 64), (b"sweep_parts", 1)), ((b"sweep_fail", 2), (b"sweep_positions", 0)),
+    for params in ((), ((b"sweep_positions", 64),), ((b"sweep_positions", 0),), ((b"sweep_parts", 0),), ((b"sweep_parts", 2),),
+                   ((b"sweep_positions", 64), (b"sweep_parts", 2)), ((b"sweep_fail", 2), (b"sweep_positions", 0)),
                    ((b"sweep_part_rows", 300),), ((b"sweep_one_launch", 0),)):
         print("flowlab sweeps:", params, flush=True)
         for k, v in params:
             assert L.fvk_fl_ctx_set_param(h, k, C.c_double(v)) == 0
-        x, r, norm = np.zeros(900), b.copy(), np.zeros(1)
+        x, r, norm = np.zeros(n), b.copy(), np.zeros(1)
         assert L.fvk_fl_lin_eqns_solver(h, dp(a), dp(x), dp(r), dp(norm), 4, C.c_double(0.0), 2) == 0
         first = x if first is None else first
         assert np.array_equal(x, first), params

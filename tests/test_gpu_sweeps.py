@@ -1,11 +1,11 @@
 """DIC / DILU factor and triangular sweeps in one launch each against the
-level-by-level launches and the oracle.  One launch: blocks owning ranges of
-rows consecutive in the reference numbering, walked level by level with the
-values inside a range passing through LDS (the default; ranges of 4096 rows,
-and of 256 rows so that each block takes many ranges), or rows taken in level
-order in chunks; rows wait for the values they need from elsewhere.
+level-by-level launches and the oracle.  One launch: blocks walking parts of
+the rows with the values inside a part passing through LDS (bricks of the
+dependency grid or ranges of the numbering; at most 4096 rows, and at most 256
+so that each block takes many), or rows taken in level order in chunks; rows
+wait for the values they need from elsewhere.
 
-Bar: bitwise.  Both forms perform the same operations in the same order for
+Bar: bitwise.  All forms perform the same operations in the same order for
 every row (solv_precond.f90:10-29, solv_direct.f90:11-42); only the
 scheduling differs.  Cases: jittered hex boxes up to 96^3 (884,736 rows,
 286 levels per sweep) in natural and reverse Cuthill-McKee order, one and
@@ -49,8 +49,8 @@ def random_matrix(m, seed):
 MODES = [
     ("one launch per level", {"sweep_one_launch": 0}),
     ("chunks in level order", {"sweep_one_launch": 1, "sweep_parts": 0}),
-    ("ranges of 4096 rows", {"sweep_one_launch": 1, "sweep_parts": 1, "sweep_part_rows": 4096}),
-    ("ranges of 256 rows", {"sweep_one_launch": 1, "sweep_parts": 1, "sweep_part_rows": 256}),
+    ("parts of at most 4096 rows", {"sweep_one_launch": 1, "sweep_parts": 2, "sweep_part_rows": 4096}),
+    ("parts of at most 256 rows", {"sweep_one_launch": 1, "sweep_parts": 2, "sweep_part_rows": 256}),
 ]
 
 
@@ -249,9 +249,8 @@ def test_shipped_simple_one_launch_bitwise(graph):
 
 def test_sweep_wait_failure_is_reported():
     """The failure path of the one-launch factor and sweeps, forced from the
-    host: with the wait-bound flag raised ("sweep_fail"), rows of the ranges
-    form that wait give up within 256 passes, blocks stop taking ranges, the
-    launches end, and the factorisation and sweeps report FVK_ERR_HIP; a new
+    host: with the wait-bound flag raised ("sweep_fail"), parts that wait give
+    up within 256 polls, blocks stop taking parts, the launches end, and the factorisation and sweeps report FVK_ERR_HIP; a new
     context on the same mesh gives the bits of the first."""
     fvk = require_lib()
     n = 32

@@ -54,16 +54,43 @@ def test_boxes(dims, rows):
         assert p["passed_fwd"] < n or rows < 100
 
 
+def arrays(n, e):
+    """1-based CSR of the pattern as csr() gives it, for large ones."""
+    k = np.arange(n)
+    r, c = np.concatenate([e[:, 0], e[:, 1], k]), np.concatenate([e[:, 1], e[:, 0], k])
+    o = np.lexsort((c, r))
+    return 1 + np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))]), c[o] + 1
+
+
 def test_sampled_distances():
     """A box as wide as the rows are sampled apart (every eighth of 423,200) is
     still recognised by all three distances: with parts of 64 rows a brick
     cannot hold whole lines of 8 cells in two directions."""
-    n, e = box(8, 230, 230)
+    assert fvk.sweep_plan(*arrays(*box(8, 230, 230)), 64)["bricks"] == 1
+
+
+@pytest.mark.parametrize("holes", ["block", "cells"])
+def test_irregular_boxes_are_bricks(holes):
+    """Cells left out of a box shift the distances between lines and planes; a
+    brick of a full box has as many rows as a part may have."""
+    n, e = box(40, 40, 64)
     k = np.arange(n)
-    r, c = np.concatenate([e[:, 0], e[:, 1], k]), np.concatenate([e[:, 1], e[:, 0], k])
-    o = np.lexsort((c, r))
-    ia = 1 + np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))])
-    assert fvk.sweep_plan(ia, c[o] + 1, 64)["bricks"] == 1
+    x, y, z = k % 40, k // 40 % 40, k // 1600
+    keep = ~((abs(x - 20) < 6) & (abs(y - 12) < 5) & (abs(z - 30) < 9)) if holes == "block" else k % 101 != 0
+    new = np.cumsum(keep) - 1
+    e = new[e[keep[e].all(1)]]
+    for rows in (512, 4096):
+        assert fvk.sweep_plan(*arrays(int(keep.sum()), e), rows)["bricks"] == 1
+
+
+def test_choice_of_form():
+    """Parts on ordered numberings; chunks where the rows are numbered at random
+    and a part needs values from nearly all others."""
+    n, e = box(30, 30, 30)
+    parts, chunks = fvk.sweep_times(*arrays(n, e))
+    assert 4 * parts < chunks
+    parts, chunks = fvk.sweep_times(*arrays(n, np.random.default_rng(0).permutation(n)[e]))
+    assert parts > 1.5 * chunks
 
 
 @pytest.mark.parametrize("rows", [64, 300, 4096])
