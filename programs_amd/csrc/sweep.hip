@@ -6,7 +6,7 @@
 //
 // A block takes parts of the plan from a ticket counter, in an order in
 // which a part only needs values of parts taken before it (no deadlock
-// whatever the residency), and runs a part with three waves:
+// whatever the residency), and runs a part with eight waves:
 //   wave 0 computes: it walks the part's chunks (up to 64 rows that do not depend
 //     on each other) in order.  All values it reads sit in LDS, its own
 //     rows' and the halo's; a wave's LDS operations are in order, so chunk
@@ -17,14 +17,15 @@
 //   wave 1 fetches the halo: it polls the export buffer for the values of
 //     other parts, in the order in which the chunks need them, puts them
 //     into LDS and publishes how many are there.
-// Results go from LDS to memory by all waves when the part is done.
+// All waves load a part's tables and first values into LDS, and store its
+// results from there when it is done.
 //
 // Export slots hold kSweepMark (a signalling NaN: no arithmetic result has
 // this pattern) until their value arrives.  A launch marks the buffer of the
-// other direction, so no launch is spent on marking.  The halo waves'
-// waits are bounded (kSweepSpin polls; 256 once an error is recorded); past
-// the bound they record the error, the compute wave runs through what is
-// left on what is there and the block stops taking parts.
+// other direction, so no launch is spent on marking.  A halo wave's waits
+// are bounded (kSweepSpin polls; 256 once an error is recorded); past the
+// bound it records the error, the compute wave runs through what is left on
+// what is there and the block stops taking parts.
 //
 // What bounds it: the chain of chunks a path runs through (LDS read, five
 // dependent FP64 operations, LDS write) and the crossings between parts
@@ -211,7 +212,7 @@ __device__ __forceinline__ void sweep_compute(const SweepArgs &A, int c0, int nc
   auto run = [&](const SweepStage<MW> &X, const SweepStage<MW> &Y, auto ahead) {
     while (__builtin_expect(nd > have, 0)) {
       have = __builtin_amdgcn_readfirstlane(lds_get(A.shared + SH_HAVE));
-      // the halo waves gave up: the rest of the part runs on what is there
+      // the halo wave gave up: the rest of the part runs on what is there
       if (nd > have && __builtin_amdgcn_readfirstlane(lds_get(A.shared + SH_ABORT))) have = INT_MAX;
     }
     asm volatile("" ::: "memory");
@@ -560,15 +561,17 @@ static SweepArgs args(const SweepExec &X, int dir) {
   return A;
 }
 
-// Blocks of a launch.  A block that waits for its part's first values polls,
-// which slows the ones at work, so of a brick plan no more are resident than
-// run at a time: the front through the brick grid is about 2.25 P^(2/3)
-// parts wide.  At least one per CU, at most what their LDS lets reside.
-// Measured (DIC, both sweeps, 128^3, 1331 bricks: 272 blocks by the rule):
-// 256 blocks 294 us, 512 309 us, 1024 334 us; 96^3 (512 bricks): 189 us
-// with 256, 199 us with 512.
+// Blocks of a launch, at most one a part and as many as can be resident by
+// their LDS and 512 threads each.  Of a brick plan no more than one per CU or
+// than run at a time (the front through the brick grid is about 2.25 P^(2/3)
+// parts wide): those that wait poll.  Fewer than one per CU leave CUs without
+// work, and more make little difference (DIC, both sweeps, us, with 128 / 192 /
+// 256 / 512 / 1024 blocks: 96^3, 288 bricks, 256 blocks by the rule, 136.5 /
+// 136.9 / 138.0 / 138.1 / 137.7; 128^3, 512 bricks, 256: 239 / 213 / 208 / 208 /
+// 208; 192^3, 1728 bricks, 324: 630 / 504 / 448 / 447 / 445; 1M triangles, 980
+// ranges, 768: 237 / 188 / 164 / 164 / 164).
 static int grid(const SweepExec &X, size_t lds) {
-  const int fit = X.n_cu * std::max(1, std::min(8, (int)(163840 / (lds + 512))));
+  const int fit = X.n_cu * std::max(1, std::min(4, (int)(163840 / (lds + 512))));
   const int front = X.bricks ? std::max(X.n_cu, (int)(2.25 * std::cbrt((double)X.P * X.P))) : fit;
   return std::max(1, std::min({X.P, fit, X.blocks > 0 ? X.blocks : front}));
 }
