@@ -334,12 +334,19 @@ __global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
       ((unsigned long long *)A.Eo)[i] = kSweepMark;
     if (blockIdx.x == 0 && tid == 0) *A.ticket_o = 0;
   }
-  if (tid == 0) lds_put(A.shared + SH_ABORT, 0);
-  for (;;) {
+  // Between a barrier and the loop that stores a part, and not after that loop,
+  // whose trip count is a thread's own: the compiler may join a branch at the
+  // end of a loop's body with one that follows, and threads that skip both then
+  // reach the next barrier without a ticket.  The stores hide its latency.
+  auto ticket = [&] {
     if (tid == 0) {
       lds_put(A.shared + SH_PART, atomicAdd(A.ticket, 1));
       lds_put(A.shared + SH_HAVE, 0);
     }
+  };
+  if (tid == 0) lds_put(A.shared + SH_ABORT, 0);
+  ticket();
+  for (;;) {
     __syncthreads();
     const int o = __builtin_amdgcn_readfirstlane(lds_int(A.shared + SH_PART));
     if (o >= A.P) return;
@@ -378,7 +385,8 @@ __global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
     if (wave == 0) sweep_compute<FWD, NC, MW, KIND>(A, c0, nch, ld);
     else if (wave == 1) sweep_halo<NC>(A, nh, nr, ld, hsrc);
     __syncthreads();
-    if (lds_int(A.shared + SH_ABORT)) return;
+    if (__builtin_amdgcn_readfirstlane(lds_int(A.shared + SH_ABORT))) return;
+    ticket();
     for (int k = tid; k < nr; k += SW_TB) {
       const unsigned off = A.pslot[r0 + k];
       if (KIND == 0) {
@@ -394,11 +402,6 @@ __global__ __launch_bounds__(SW_TB) void k_sweep(SweepArgs A) {
         A.crr[r0 + k] = A.drow ? d : 1.0 / (c + SMALL);
       }
     }
-    // Keeps the loop above, whose trip count is a thread's own, apart from
-    // thread 0's ticket: a compiler may join a branch at the end of a loop's
-    // body with one at its head, and the threads that skip both would then go
-    // round to the barrier without a ticket.  A barrier is never duplicated.
-    __syncthreads();
   }
 }
 
