@@ -1958,7 +1958,7 @@ int fvk_sweep_times(int n, const int *ia, const int *ja, int max_rows, double *u
   SweepPlan p;
   const std::string e = sweep_plan(fl_sweep_graph(n, q.ia, q.ja, q.klo, q.kup, q.tpos), max_rows, p);
   if (!e.empty()) { set_error(e); return FVK_ERR_ARG; }
-  us[0] = p.us;
+  us[0] = sweep_plan_us(p);
   us[1] = p.chunk_us;
   return FVK_OK;
 }

@@ -121,7 +121,7 @@ static double brick_path(int m, const int *side, const int *cells) {
 // both sweeps, 24^3 / 96^3 / 128^3, with two halo waves: 35.3 / 153 / 235 us;
 // cubes of at most 1728 rows 38 / 163 / 250, of 512 rows 37 / 173).
 // Without main distances (unstructured numberings) the parts are ranges of
-// consecutive rows, of whichever size plan_us finds faster: a path through
+// consecutive rows, of whichever size sweep_plan_us finds faster: a path through
 // triangles crosses them about once a level anyway, and short ones are loaded
 // sooner (DIC, both sweeps, 20k / 40k / 200k triangles in RCM order: ranges of
 // 512 rows 53 / 65 / 93 us, 1024 45 / 57 / 87, 2048 51 / 61 / 92), where long
@@ -478,7 +478,7 @@ static PlanEnd plan_with(const SweepGraph &g, int max_rows, int range_rows, long
 // 48^3 box numbered at random 408 / 116 us, 80^3 949 / 214, 200k triangles at
 // random 248 / 91, 64^3 in RCM order 821 / 608; but 60k triangles as they are
 // 85 / 121, 64^3 in natural order 112 / 1028.
-static double plan_us(const SweepPlan &p) {
+double sweep_plan_us(const SweepPlan &p) {
   constexpr int kCus = 256;
   const int NI = p.nrec(), ND = p.at_need();
   const int blocks = std::min(p.P, kCus * std::max(1, std::min(4, (int)(163840 / (p.lds(1) + 512)))));
@@ -533,7 +533,7 @@ std::string sweep_plan(const SweepGraph &g, int max_rows, SweepPlan &p, long lim
       q.MW = W <= 3 ? 3 : W <= 4 ? 4 : 8;
       const long most = (1L << 32) / (2 * q.nrec());
       const PlanEnd e = plan_with(g, r, range, limit > 0 ? std::min(limit, most) : most, q, exact);
-      if (e == PLAN_OK) q.us = plan_us(q);
+      if (e == PLAN_OK && !(range == 0 && exact)) q.us = sweep_plan_us(q);
       if (e != PLAN_LDS) return e;
     }
     return PLAN_NONE;

@@ -47,7 +47,8 @@ struct SweepPlan {
   int n = 0, P = 0, W = 0, MW = 0, np = 0, levels = 0, width = kChunk;
   int slots = 0, maxh = 0;                 // the most LDS slots and halo values of a part
   bool bricks = false;
-  double us = 0, chunk_us = 0;             // both sweeps by this plan and by chunks of the level order (plan_us)
+  double us = 0, chunk_us = 0;             // both sweeps by this plan (0: bricks of an exactly structured
+                                           // numbering) and by chunks of the level order (sweep_plan_us)
   bool chunks_faster() const { return 1.25 * us > chunk_us; }
   std::vector<int> part;                   // 8 ints a part: first chunk, chunks, first row, rows,
                                            // first forward halo, count, first backward halo, count
@@ -73,6 +74,9 @@ struct SweepPlan {
 // string, or why there is no plan: a row with more than 8 entries on one
 // side, or too many positions.
 std::string sweep_plan(const SweepGraph &g, int max_rows, SweepPlan &p, long limit = 0);
+
+// us of both sweeps by this plan with one right-hand side, by a model
+double sweep_plan_us(const SweepPlan &p);
 
 // Walks the plan as the kernels do and checks that every value is there
 // when it is read, that a part only needs parts taken before it, and that
